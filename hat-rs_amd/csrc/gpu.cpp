@@ -3,6 +3,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <deque>
 #include <memory>
 #include <atomic>
 #include <thread>
@@ -2128,42 +2129,92 @@ void GpuBackend::forward(int h, int w, const float* in, float* out)
 
 namespace {
 
-struct DevBuf {
-    float* p = nullptr;
-    DevBuf(size_t n) { p = (float*)Runtime::get().alloc(n * sizeof(float)); }
-    DevBuf(const float* src, size_t n) : DevBuf(n) { Runtime::get().h2d(p, src, n * sizeof(float)); }
-    ~DevBuf() { Runtime::get().free(p); }
-    DevBuf(const DevBuf&) = delete;
-    DevBuf& operator=(const DevBuf&) = delete;
+// An op's device buffers: one allocation, and one upload for everything small.
+// The ops run once per call on buffers of their own, so a hipMalloc and hipFree
+// a buffer and a blocking copy a weight were much of a call's host time (SW-MSA
+// at 128 x 128, 180 channels: 2.32 -> 2.11 ms a call, most of what is left the
+// two copies of the plane; OCAB at 96 x 160, 144 channels: 3.24 -> 1.88, the
+// weights that only the unfused kernels read no longer packed as well). add()
+// before commit(), ptr() after it.
+class OpArena {
+public:
+    // n floats, from src if set (kept by the caller until commit)
+    size_t add(size_t n, const float* src = nullptr) { return add_bytes(n * sizeof(float), src); }
+    // n floats or 16-bit values the arena keeps until commit
+    size_t keep(std::vector<float> v)
+    {
+        kept_f_.push_back(std::move(v));
+        return add(kept_f_.back().size(), kept_f_.back().data());
+    }
+    size_t keep(std::vector<unsigned short> v)
+    {
+        kept_u_.push_back(std::move(v));
+        return add_bytes(kept_u_.back().size() * sizeof(unsigned short), kept_u_.back().data());
+    }
+    void commit()
+    {
+        Runtime& rt = Runtime::get();
+        // the small uploads first, side by side, so that one copy takes them
+        size_t off = 0;
+        for (int pass = 0; pass < 2; ++pass)
+            for (Req& r : reqs_)
+                if ((pass == 0) == (r.src && r.bytes <= kSmall)) {
+                    r.off = off;
+                    off += (r.bytes + 255) / 256 * 256;
+                    if (pass == 0) small_ = off;
+                }
+        base_ = (char*)rt.alloc(off);
+        std::vector<char> stage(small_);
+        for (const Req& r : reqs_)
+            if (r.src && r.bytes <= kSmall) memcpy(&stage[r.off], r.src, r.bytes);
+        if (small_) rt.h2d(base_, stage.data(), small_);
+        for (const Req& r : reqs_)
+            if (r.src && r.bytes > kSmall) rt.h2d(base_ + r.off, r.src, r.bytes);
+        kept_f_.clear();
+        kept_u_.clear();
+    }
+    float* ptr(size_t i) const { return (float*)(base_ + reqs_[i].off); }
+    OpArena() = default;
+    ~OpArena()
+    {
+        if (base_) Runtime::get().free(base_);
+    }
+    OpArena(const OpArena&) = delete;
+    OpArena& operator=(const OpArena&) = delete;
+
+private:
+    static constexpr size_t kSmall = 4u << 20;
+    struct Req {
+        size_t bytes, off;
+        const void* src;
+    };
+    size_t add_bytes(size_t bytes, const void* src)
+    {
+        reqs_.push_back(Req{bytes, 0, src});
+        return reqs_.size() - 1;
+    }
+    std::vector<Req> reqs_;
+    std::deque<std::vector<float>> kept_f_;
+    std::deque<std::vector<unsigned short>> kept_u_;
+    char* base_ = nullptr;
+    size_t small_ = 0;
 };
 
-// Device copy of a host bf16 array (DevBuf's units are floats).
-static std::unique_ptr<DevBuf> dev_u16(const std::vector<unsigned short>& v)
-{
-    std::unique_ptr<DevBuf> d(new DevBuf((v.size() + 1) / 2));
-    Runtime::get().h2d(d->p, v.data(), v.size() * sizeof(unsigned short));
-    return d;
-}
-
 // A linear of the op entry points, packed as the backend packs it
-// (upload_linear): the FP32 rows, and for the shapes a split-bf16 kernel
-// takes (the qkv of 144 / 180 channels, the 144 / 180 projection) the split
-// weights too, so that an op runs the forward's kernels.
+// (upload_linear): for the shapes a split-bf16 kernel takes (the qkv of 144 /
+// 180 channels, the 144 / 180 projection) the split weights, so that an op runs
+// the forward's kernels; for the others (and with kBias, where only the bias is
+// read, neither) the FP32 rows.
 struct OpLinear {
-    enum Split { kNone, kQkv, kProj };
-    DevBuf w, b;
-    std::unique_ptr<DevBuf> x;
+    enum Split { kNone, kQkv, kProj, kBias };
     DevLinear L;
-    OpLinear(const float* wt, const float* bias, int N, int K, Split sp = kNone) : w(1), b(bias, N)
+    size_t iw = 0, ib = 0, ix = 0;
+    bool fp32 = false, split = false;
+    OpLinear(OpArena& ar, const float* wt, const float* bias, int N, int K, Split sp = kNone)
     {
         L.N = N;
         L.K = K;
-        std::vector<float> pk = pack_linear(wt, N, K, &L.Kp);
-        Runtime::get().free(w.p);
-        w.p = (float*)Runtime::get().alloc(pk.size() * sizeof(float));
-        Runtime::get().h2d(w.p, pk.data(), pk.size() * sizeof(float));
-        L.w = w.p;
-        L.b = b.p;
+        ib = ar.add(N, bias);
         std::vector<unsigned short> xs;
         if (sp == kQkv && ((N == 432 && K == 144) || (N == 540 && K == 180)))
             xs = pack_linear_ws(wt, bias, N, K);
@@ -2171,38 +2222,41 @@ struct OpLinear {
             xs = pack_linear_x(wt, N, K);
         else if (sp == kProj && N == 180 && K == 180)
             xs = pack_linear_x180(wt);
-        if (!xs.empty()) {
-            x = dev_u16(xs);
-            L.wx = (unsigned short*)x->p;
-        }
+        L.Kp = (K + 15) / 16 * 16;
+        if ((split = !xs.empty())) ix = ar.keep(std::move(xs));
+        else if ((fp32 = sp != kBias)) iw = ar.keep(pack_linear(wt, N, K, &L.Kp));
+    }
+    void bind(const OpArena& ar)
+    {
+        if (fp32) L.w = ar.ptr(iw);
+        L.b = ar.ptr(ib);
+        if (split) L.wx = (unsigned short*)ar.ptr(ix);
     }
 };
 
-// An op's MLP pre-split for hat_mlpx (C = 144) or hat_mlpx180 (C = 180), as
-// upload_mlpx packs it; other shapes leave m.w null (the FP32 kernels).
+// An op's MLP pre-split for the fused tails (hat_habx, hat_habx180), as
+// upload_mlpx packs it; other shapes (fused false) run the FP32 kernels.
 struct OpMlpX {
-    std::unique_ptr<DevBuf> buf, fbuf, bbuf;
     DevMlpX m;
-    OpMlpX(const float* w1, const float* b1, const float* w2, int c, size_t hid)
+    size_t iwf = 0, ib1 = 0;
+    bool fused = false;
+    OpMlpX(OpArena& ar, const float* w1, const float* b1, const float* w2, int c, size_t hid)
     {
-        std::vector<unsigned short> w, wf;
+        std::vector<unsigned short> wf;
         std::vector<float> b1x;
-        if (c == 144 && hid == 288) {
-            pack_mlp_x(w1, b1, w2, &w);
-            pack_mlp_xf(w1, b1, w2, &wf, &b1x);
-        } else if (c == 180 && hid == 360) {
-            pack_mlp_x180(w1, b1, w2, &w);
-            pack_mlp_xf180(w1, b1, w2, &wf, &b1x);
-        } else {
-            return;
-        }
-        fbuf = dev_u16(wf);
-        m.wf = (unsigned short*)fbuf->p;
-        bbuf.reset(new DevBuf(b1x.data(), b1x.size()));
-        m.b1x = bbuf->p;
+        if (c == 144 && hid == 288) pack_mlp_xf(w1, b1, w2, &wf, &b1x);
+        else if (c == 180 && hid == 360) pack_mlp_xf180(w1, b1, w2, &wf, &b1x);
+        else return;
+        fused = true;
         m.C = c;
-        buf = dev_u16(w);
-        m.w = (unsigned short*)buf->p;
+        iwf = ar.keep(std::move(wf));
+        ib1 = ar.keep(std::move(b1x));
+    }
+    void bind(const OpArena& ar)
+    {
+        if (!fused) return;
+        m.wf = (unsigned short*)ar.ptr(iwf);
+        m.b1x = ar.ptr(ib1);
     }
 };
 
@@ -2243,18 +2297,25 @@ void op_swmsa(const float* x, float* out, int hp, int wp, int c, int heads, int 
     Runtime& rt = Runtime::get();
     const HipApi& api = rt.api();
     const size_t T = (size_t)hp * wp;
+    // the null stream: the op is synchronous, as are its copies, and a stream
+    // of its own would be created and destroyed on each call
     hipStream_t s = nullptr;
-    rt.check(api.StreamCreate(&s), "hipStreamCreate");
     {
-        DevBuf dx(x, T * c), dq(3 * T * c), dao(T * c), dout(T * c), dtab(table, 961 * (size_t)heads);
+        OpArena ar;
+        const size_t ix = ar.add(T * c, x), iq = ar.add(3 * T * c), iao = ar.add(T * c), iout = ar.add(T * c),
+                     itab = ar.add(961 * (size_t)heads, table);
         // qkv as in the forward; the projection here has no residual, a form the
         // forward never runs, so it stays on the FP32 store epilogue
-        OpLinear qkv(qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv), proj(proj_w, proj_b, c, c);
+        OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv), proj(ar, proj_w, proj_b, c, c);
+        ar.commit();
+        qkv.bind(ar);
+        proj.bind(ar);
+        float *dx = ar.ptr(ix), *dq = ar.ptr(iq), *dao = ar.ptr(iao), *dout = ar.ptr(iout), *dtab = ar.ptr(itab);
         const GemmEpilogue none;
         auto run = [&]() {
-            run_gemm(s, qkv.L, dx.p, c, (long)T, dq.p, 0, EPI_QKV, none, heads, D, 0.f);
-            run_attn(s, dq.p, dtab.p, dao.p, pl, heads, D, false, shift);
-            run_gemm(s, proj.L, dao.p, c, (long)T, dout.p, c, EPI_STORE, none, heads, D, 0.f);
+            run_gemm(s, qkv.L, dx, c, (long)T, dq, 0, EPI_QKV, none, heads, D, 0.f);
+            run_attn(s, dq, dtab, dao, pl, heads, D, false, shift);
+            run_gemm(s, proj.L, dao, c, (long)T, dout, c, EPI_STORE, none, heads, D, 0.f);
         };
         run();
         rt.check(api.StreamSynchronize(s), "swmsa");
@@ -2264,7 +2325,7 @@ void op_swmsa(const float* x, float* out, int hp, int wp, int c, int heads, int 
             for (int i = 0; i < iters; ++i) run();
             api.EventRecord(t.b, s);
             api.EventRecord(ta.a, s);
-            for (int i = 0; i < iters; ++i) run_attn(s, dq.p, dtab.p, dao.p, pl, heads, D, false, shift);
+            for (int i = 0; i < iters; ++i) run_attn(s, dq, dtab, dao, pl, heads, D, false, shift);
             api.EventRecord(ta.b, s);
             rt.check(api.EventSynchronize(ta.b), "swmsa timing");
             float e = 0.f;
@@ -2273,9 +2334,8 @@ void op_swmsa(const float* x, float* out, int hp, int wp, int c, int heads, int 
             api.EventElapsedTime(&e, ta.a, ta.b);
             if (attn_ms) *attn_ms = e / iters;
         }
-        rt.d2h(out, dout.p, T * c * sizeof(float));
+        rt.d2h(out, dout, T * c * sizeof(float));
     }
-    api.StreamDestroy(s);
 }
 
 void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int mlp_ratio,
@@ -2297,47 +2357,57 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
     Runtime& rt = Runtime::get();
     const HipApi& api = rt.api();
     const size_t T = (size_t)hp * wp, hid = (size_t)c * mlp_ratio;
-    hipStream_t s = nullptr;
-    rt.check(api.StreamCreate(&s), "hipStreamCreate");
+    hipStream_t s = nullptr;  // the null stream, as in op_swmsa
     {
-        DevBuf dx(x, T * c), dwork(T * c), dxn(T * c), dq(3 * T * c), dao(T * c), dh(T * hid),
-            dtab(table, 1521 * (size_t)heads), d1w(n1w, c), d1b(n1b, c), d2w(n2w, c), d2b(n2b, c);
-        OpLinear qkv(qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv), proj(proj_w, proj_b, c, c, OpLinear::kProj),
-            fc1(fc1_w, fc1_b, (int)hid, c), fc2(fc2_w, fc2_b, c, (int)hid);
-        const OpMlpX mx(fc1_w, fc1_b, fc2_w, c, hid);
+        OpArena ar;
+        const size_t ix = ar.add(T * c, x), iwork = ar.add(T * c), ixn = ar.add(T * c), iq = ar.add(3 * T * c),
+                     iao = ar.add(T * c), itab = ar.add(1521 * (size_t)heads, table), i1w = ar.add(c, n1w),
+                     i1b = ar.add(c, n1b), i2w = ar.add(c, n2w), i2b = ar.add(c, n2b);
+        OpMlpX mx(ar, fc1_w, fc1_b, fc2_w, c, hid);
+        // the split tails read only fc2's bias of these two
+        const OpLinear::Split mlp = mx.fused ? OpLinear::kBias : OpLinear::kNone;
+        OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv),
+            proj(ar, proj_w, proj_b, c, c, mx.fused ? OpLinear::kProj : OpLinear::kNone),
+            fc1(ar, fc1_w, fc1_b, (int)hid, c, mlp), fc2(ar, fc2_w, fc2_b, c, (int)hid, mlp);
+        const size_t ih = ar.add(mx.fused || mlp_fused(fc1.L, fc2.L) ? 1 : T * hid);
+        ar.commit();
+        mx.bind(ar);
+        for (OpLinear* l : {&qkv, &proj, &fc1, &fc2}) l->bind(ar);
+        float *dx = ar.ptr(ix), *dwork = ar.ptr(iwork), *dxn = ar.ptr(ixn), *dq = ar.ptr(iq), *dao = ar.ptr(iao),
+              *dtab = ar.ptr(itab), *d1w = ar.ptr(i1w), *d1b = ar.ptr(i1b), *d2w = ar.ptr(i2w), *d2b = ar.ptr(i2b);
         const GemmEpilogue none;
         GemmEpilogue resid_ln;
-        resid_ln.res = dx.p;
-        resid_ln.xn = dxn.p;
-        resid_ln.nw = d2w.p;
-        resid_ln.nb = d2b.p;
+        resid_ln.res = dx;
+        resid_ln.xn = dxn;
+        resid_ln.nw = d2w;
+        resid_ln.nb = d2b;
         // The backend's OCAB sequence (GpuBackend::ocab): norm1, qkv, attention,
         // proj + shortcut (which also writes norm2), then the MLP + residual.
         auto run = [&]() {
-            run_ln(s, dx.p, dxn.p, d1w.p, d1b.p, (long)T, c);
-            run_gemm(s, qkv.L, dxn.p, c, (long)T, dq.p, 0, EPI_QKV, none, heads, D, 0.f);
-            run_attn(s, dq.p, dtab.p, dao.p, pl, heads, D, true, 0);
-            if (proj.L.wx && mx.m.w && c == 144) {
-                run_tailx(s, false, proj.L, mx.m, fc2.L.b, dao.p, dx.p, dwork.p, dxn.p, nullptr, nullptr, proj.L.b,
-                          d2w.p, d2b.p, nullptr, nullptr, hp, wp);
-            } else if (proj.L.wx && mx.m.w && c == 180) {
-                run_tailx180(s, proj.L, mx.m, fc2.L.b, dao.p, dx.p, dwork.p, nullptr, d2w.p, d2b.p, nullptr, nullptr, 0.f,
+            run_ln(s, dx, dxn, d1w, d1b, (long)T, c);
+            run_gemm(s, qkv.L, dxn, c, (long)T, dq, 0, EPI_QKV, none, heads, D, 0.f);
+            run_attn(s, dq, dtab, dao, pl, heads, D, true, 0);
+            if (mx.fused && c == 144) {
+                run_tailx(s, false, proj.L, mx.m, fc2.L.b, dao, dx, dwork, dxn, nullptr, nullptr, proj.L.b, d2w, d2b,
+                          nullptr, nullptr, hp, wp);
+            } else if (mx.fused) {
+                run_tailx180(s, proj.L, mx.m, fc2.L.b, dao, dx, dwork, nullptr, d2w, d2b, nullptr, nullptr, 0.f,
                              nullptr, nullptr, (long)T);
             } else {
-                run_gemm(s, proj.L, dao.p, c, (long)T, dwork.p, c, EPI_RESID_LN, resid_ln, heads, D, 0.f);
-                run_mlp(s, fc1.L, fc2.L, dxn.p, (long)T, dwork.p, dwork.p, EPI_RESID, none, dh.p);
+                run_gemm(s, proj.L, dao, c, (long)T, dwork, c, EPI_RESID_LN, resid_ln, heads, D, 0.f);
+                run_mlp(s, fc1.L, fc2.L, dxn, (long)T, dwork, dwork, EPI_RESID, none, ar.ptr(ih));
             }
         };
         run();
         rt.check(api.StreamSynchronize(s), "ocab");
-        rt.d2h(out, dwork.p, T * c * sizeof(float));
+        rt.d2h(out, dwork, T * c * sizeof(float));
         if (iters > 0 && (ms || attn_ms)) {
             Timer t, ta;
             api.EventRecord(t.a, s);
             for (int i = 0; i < iters; ++i) run();
             api.EventRecord(t.b, s);
             api.EventRecord(ta.a, s);
-            for (int i = 0; i < iters; ++i) run_attn(s, dq.p, dtab.p, dao.p, pl, heads, D, true, 0);
+            for (int i = 0; i < iters; ++i) run_attn(s, dq, dtab, dao, pl, heads, D, true, 0);
             api.EventRecord(ta.b, s);
             rt.check(api.EventSynchronize(ta.b), "ocab timing");
             float e = 0.f;
@@ -2347,7 +2417,6 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
             if (attn_ms) *attn_ms = e / iters;
         }
     }
-    api.StreamDestroy(s);
 }
 
 }  // namespace hat
