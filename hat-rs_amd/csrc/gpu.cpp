@@ -437,6 +437,58 @@ std::vector<unsigned short> pack_cab_conv1(const float* w)
     return out;
 }
 
+float f16_scale(double bound)
+{
+    if (!(bound > 0.0) || !std::isfinite(bound)) return 1.0f;
+    int e = 0;
+    std::frexp(bound, &e);  // bound in [2^(e-1), 2^e)
+    return std::ldexp(1.0f, std::max(-60, std::min(60, 15 - e)));
+}
+
+double ln_linear_bound(const float* w, const float* b, const float* lnw, const float* lnb, int n0, int n1, int C)
+{
+    double worst = 0.0;
+    for (int n = n0; n < n1; ++n) {
+        const float* r = w + (size_t)n * C;
+        double sq = 0.0, off = b ? b[n] : 0.0;
+        for (int c = 0; c < C; ++c) {
+            const double x = (double)r[c] * lnw[c];
+            sq += x * x;
+            off += (double)r[c] * lnb[c];
+        }
+        const double v = std::sqrt(sq * C) + std::fabs(off);
+        if (std::isnan(v)) return v;
+        worst = std::max(worst, v);
+    }
+    return worst;
+}
+
+double ln_bound(const float* lnw, const float* lnb, int C)
+{
+    double worst = 0.0;
+    for (int c = 0; c < C; ++c) {
+        const double v = std::sqrt((double)C) * std::fabs((double)lnw[c]) + std::fabs((double)lnb[c]);
+        if (std::isnan(v)) return v;
+        worst = std::max(worst, v);
+    }
+    return worst;
+}
+
+QkvScale qkv_scale(double bq, double bk, double bv, int head_dim)
+{
+    QkvScale s;
+    bq *= 1.4426950408889634 / std::sqrt((double)head_dim);  // the kernels split q times this
+    if (!std::isfinite(bq) || !std::isfinite(bk) || !std::isfinite(bv)) return s;
+    int a = 0;
+    if (bq > 0.0 && bk > 0.0) a = (int)std::lround(0.5 * std::log2(bk / bq));
+    if (std::abs(a) > 60 || std::ldexp(bq, a) > 32768.0 || std::ldexp(bk, -a) > 32768.0) return s;
+    s.q = std::ldexp(1.0f, a);
+    s.k = std::ldexp(1.0f, -a);
+    s.v = f16_scale(bv);
+    s.ok = true;
+    return s;
+}
+
 // ---------------------------------------------------------------------------
 // Launch helpers shared by the backend and the op entry points.
 
@@ -1033,7 +1085,7 @@ void run_convw(hipStream_t s, const DevConv& C, const float* in, int cin_stride,
 }
 
 void run_attn(hipStream_t s, const float* qkv, const float* table, float* out, const Plan& pl,
-              int heads, int D, bool oca, int shift, const CabGateArgs* gate = nullptr,
+              int heads, int D, bool oca, int shift, bool f16, const CabGateArgs* gate = nullptr,
               const SeArgs* se = nullptr)
 {
     if (se && oca) throw Error("attention: the SE gate rides on SW launches only");
@@ -1047,16 +1099,14 @@ void run_attn(hipStream_t s, const float* qkv, const float* table, float* out, c
         throw Error("attention: shift " + std::to_string(shift) + " is not supported (0" +
                     (oca ? "" : " or " + std::to_string(pl.shift)) + ")");
     const char* name = nullptr;
-    // The split-bf16 kernels (attnx.hip), one (window, head) item per block.
-    if (D == 24) {
-        name = oca ? "hat_attnx_oca_d24" : "hat_attnx_sw_d24";
-    } else if (D == 30) {
-        // SW in four parts of 64 keys (two blocks per CU; the whole-item form
-        // hat_attnx_sw_d30 needs 114 KB of LDS, one block per CU)
-        name = oca ? "hat_attnx_oca_d30" : "hat_attnx_swp_d30";
-    } else {
+    // The split-f16 kernels (attnx.hip), one (window, head) item per block,
+    // where q, k and v are known to lie inside f16's range; else the FP32 ones.
+    if (D != 24 && D != 30)
         throw Error("attention: head_dim " + std::to_string(D) + " has no kernel (24 and 30 do)");
-    }
+    if (f16) name = oca ? (D == 24 ? "hat_attnx_oca_d24" : "hat_attnx_oca_d30")
+                        : (D == 24 ? "hat_attnx_sw_d24" : "hat_attnx_sw_d30");
+    else name = oca ? (D == 24 ? "hat_attn_oca_d24" : "hat_attn_oca_d30")
+                    : (D == 24 ? "hat_attn_sw_d24" : "hat_attn_sw_d30");
     AttnArgs p{};
     p.qkv = qkv;
     p.table = table;
@@ -1080,6 +1130,11 @@ void run_attn(hipStream_t s, const float* qkv, const float* table, float* out, c
     if (se && se->gate) {
         p.with_se = 1;
         p.se = *se;
+    }
+    if (!f16 && attn_persistent(D, oca)) {
+        static const int cus = std::max(1, Runtime::get().cu_count());
+        launch(s, name, (unsigned)std::min<long>((long)pl.nw() * heads, cus), 1, 1, 512, p);
+        return;
     }
     launch(s, name, (unsigned)pl.nw(), (unsigned)heads, 1, 512, p);
 }
@@ -1151,31 +1206,58 @@ void GpuBackend::upload_raw(const std::string& name)
     raw_[name] = upload(wt_.t(name), ti.numel());
 }
 
-void GpuBackend::upload_linear(const std::string& name)
+void GpuBackend::upload_linear(const std::string& name, const std::vector<float>* row_scale, float all, bool split)
 {
     const TensorInfo& ti = wt_.info(name + ".weight");
     DevLinear L;
     L.N = (int)ti.shape[0];
     L.K = (int)ti.shape[1];
-    std::vector<float> pk = pack_linear(wt_.t(name + ".weight"), L.N, L.K, &L.Kp);
+    const float *w = wt_.t(name + ".weight"), *bias = wt_.t(name + ".bias");
+    std::vector<float> ws, bs;
+    if (row_scale || all != 1.0f) {
+        ws.assign(w, w + (size_t)L.N * L.K);
+        bs.assign(bias, bias + L.N);
+        for (int n = 0; n < L.N; ++n) {
+            const float f = row_scale ? (*row_scale)[n] : 1.0f;
+            for (int k = 0; k < L.K; ++k) ws[(size_t)n * L.K + k] *= f * all;
+            bs[n] *= f;
+        }
+        w = ws.data();
+        bias = bs.data();
+    }
+    std::vector<float> pk = pack_linear(w, L.N, L.K, &L.Kp);
     L.w = upload(pk.data(), pk.size());
-    L.b = upload(wt_.t(name + ".bias"), L.N);
+    L.b = upload(bias, L.N);
     auto ends = [&](const char* t) {
         const size_t n = strlen(t);
         return name.size() >= n && name.compare(name.size() - n, n, t) == 0;
     };
-    if (L.K == 180 && L.N == 180 && ends("proj")) {
+    if (split && L.K == 180 && L.N == 180 && ends("proj")) {
         // the C = 180 projection tails (hat_projx180*)
-        std::vector<unsigned short> x = pack_linear_x180(wt_.t(name + ".weight"));
+        std::vector<unsigned short> x = pack_linear_x180(w);
         L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
     }
-    if ((L.K == 180 && L.N == 540 && ends(".qkv")) || (L.K == 144 && ((L.N == 432 && ends(".qkv")) || (L.N == 144 && ends("proj"))))) {
+    if (split && ((L.K == 180 && L.N == 540 && ends(".qkv")) || (L.K == 144 && ((L.N == 432 && ends(".qkv")) || (L.N == 144 && ends("proj")))))) {
         // qkv: the weight-stationary layout of hat_gemmx_qkv; proj: streamed chunks (tailx)
-        std::vector<unsigned short> x = ends(".qkv") ? pack_linear_ws(wt_.t(name + ".weight"), wt_.t(name + ".bias"), L.N, L.K)
-                                                     : pack_linear_x(wt_.t(name + ".weight"), L.N, L.K);
+        std::vector<unsigned short> x = ends(".qkv") ? pack_linear_ws(w, bias, L.N, L.K) : pack_linear_x(w, L.N, L.K);
         L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
     }
     lin_[name] = L;
+}
+
+void GpuBackend::upload_attn(const std::string& qkv, const std::string& proj, const std::string& ln,
+                             const std::string& table)
+{
+    const int C = wt_.embed;
+    const float *w = wt_.t(qkv + ".weight"), *b = wt_.t(qkv + ".bias"), *lw = wt_.t(ln + ".weight"),
+                *lb = wt_.t(ln + ".bias");
+    const QkvScale s = qkv_scale(ln_linear_bound(w, b, lw, lb, 0, C, C), ln_linear_bound(w, b, lw, lb, C, 2 * C, C),
+                                 ln_linear_bound(w, b, lw, lb, 2 * C, 3 * C, C), wt_.head_dim);
+    std::vector<float> rows((size_t)3 * C);
+    for (int n = 0; n < 3 * C; ++n) rows[n] = n < C ? s.q : n < 2 * C ? s.k : s.v;
+    upload_linear(qkv, &rows);
+    upload_linear(proj, nullptr, 1.0f / s.v);
+    attn_f16_[table] = s.ok;
 }
 
 // The C = 144 MLP, pre-split for hat_mlpx (other widths keep the FP32 kernels).
@@ -1279,8 +1361,7 @@ void GpuBackend::upload_all()
                                   ".conv_block.cab.3.attention.3.weight",
                                   ".conv_block.cab.3.attention.3.bias"})
                 upload_raw(p + n);
-            upload_linear(p + ".attn.qkv");
-            upload_linear(p + ".attn.proj");
+            upload_attn(p + ".attn.qkv", p + ".attn.proj", p + ".norm1", p + ".attn.relative_position_bias_table");
             upload_linear(p + ".mlp.fc1");
             upload_linear(p + ".mlp.fc2");
             upload_mlpx(p + ".mlp");
@@ -1307,8 +1388,7 @@ void GpuBackend::upload_all()
         for (const char* n : {".norm1.weight", ".norm1.bias", ".norm2.weight", ".norm2.bias",
                               ".relative_position_bias_table"})
             upload_raw(p + n);
-        upload_linear(p + ".qkv");
-        upload_linear(p + ".proj");
+        upload_attn(p + ".qkv", p + ".proj", p + ".norm1", p + ".relative_position_bias_table");
         upload_linear(p + ".mlp.fc1");
         upload_linear(p + ".mlp.fc2");
         upload_mlpx(p + ".mlp");
@@ -1563,7 +1643,8 @@ void GpuBackend::conv(const DevConv& C, const float* in, int cin_stride, int H, 
 void GpuBackend::attention(const std::string& table, bool oca, int shift, const CabGateArgs* gate,
                            const SeArgs* se)
 {
-    run_attn(stream_, a_.qkv, raw_.at(table), a_.ao, plan_, wt_.heads, wt_.head_dim, oca, shift, gate, se);
+    run_attn(stream_, a_.qkv, raw_.at(table), a_.ao, plan_, wt_.heads, wt_.head_dim, oca, shift,
+             attn_f16_.at(table), gate, se);
 }
 
 // HAB.forward (hat_arch.py:266-309; cpu.rs:1090-1166):
@@ -1580,13 +1661,14 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
         // CAB, folded: conv1 + GELU here, the gate inside the attention
         // launch (its first block), conv2 inside the tail's projection.
         const DevLinear& proj = lin_.at(p + ".attn.proj");
+        auto mx = mlpx_.find(p + ".mlp");
+        const bool split = proj.wx && C == 144 && mx != mlpx_.end();  // the split tail runs
         CabGateArgs gate{};
         run_cab(stream_, cab_.at(p), a_.xn, H, W, proj.b, wt_.conv_scale, wt_.squeezed, a_.t1, a_.cab_part,
                 a_.w2g, a_.bias2, a_.gate, (unsigned short*)a_.w2gx, &gate);
         gemm(lin_.at(p + ".attn.qkv"), a_.xn, C, T, a_.qkv, 0, EPI_QKV);
         attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, &gate);
-        auto mx = mlpx_.find(p + ".mlp");
-        if (proj.wx && C == 144 && mx != mlpx_.end()) {
+        if (split) {
             // split-bf16: proj + gated conv2 + shortcut + norm2, then the MLP + next norm1
             run_tailx(stream_, true, proj, mx->second, lin_.at(p + ".mlp.fc2").b, a_.ao, x_in, x_out, a_.xn, a_.t1,
                       (const unsigned short*)a_.w2gx, a_.bias2, raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"),
@@ -2210,11 +2292,27 @@ struct OpLinear {
     DevLinear L;
     size_t iw = 0, ib = 0, ix = 0;
     bool fp32 = false, split = false;
-    OpLinear(OpArena& ar, const float* wt, const float* bias, int N, int K, Split sp = kNone)
+    // out, in: as GpuBackend::upload_linear's
+    OpLinear(OpArena& ar, const float* wt, const float* bias, int N, int K, Split sp = kNone, const float* out = nullptr,
+             float in = 1.0f)
     {
         L.N = N;
         L.K = K;
-        ib = ar.add(N, bias);
+        std::vector<float> ws, bs;
+        if (out || in != 1.0f) {
+            ws.assign(wt, wt + (size_t)N * K);
+            bs.assign(bias, bias + N);
+            for (int n = 0; n < N; ++n) {
+                const float f = out ? out[n / (N / 3)] : 1.0f;
+                for (int k = 0; k < K; ++k) ws[(size_t)n * K + k] *= f * in;
+                bs[n] *= f;
+            }
+            wt = ws.data();
+            bias = bs.data();
+            ib = ar.keep(bs);
+        } else {
+            ib = ar.add(N, bias);
+        }
         std::vector<unsigned short> xs;
         if (sp == kQkv && ((N == 432 && K == 144) || (N == 540 && K == 180)))
             xs = pack_linear_ws(wt, bias, N, K);
@@ -2260,6 +2358,20 @@ struct OpMlpX {
     }
 };
 
+// The largest |row . x + bias| for rows [n0, n1) over every x with |x_k| <= mx.
+double op_linear_bound(const float* w, const float* b, int n0, int n1, int K, double mx)
+{
+    double worst = 0.0;
+    for (int n = n0; n < n1; ++n) {
+        double v = 0.0;
+        for (int k = 0; k < K; ++k) v += std::fabs((double)w[(size_t)n * K + k]);
+        v = v * mx + std::fabs((double)b[n]);
+        if (std::isnan(v)) return v;
+        worst = std::max(worst, v);
+    }
+    return worst;
+}
+
 struct Timer {
     hipEvent_t a = nullptr, b = nullptr;
     Timer()
@@ -2301,20 +2413,36 @@ void op_swmsa(const float* x, float* out, int hp, int wp, int c, int heads, int 
     // of its own would be created and destroyed on each call
     hipStream_t s = nullptr;
     {
+        // the planes first, and the input's largest finite |x|, which is what
+        // bounds q, k and v here (no norm comes before them)
         OpArena ar;
+        const float zero = 0.0f;
         const size_t ix = ar.add(T * c, x), iq = ar.add(3 * T * c), iao = ar.add(T * c), iout = ar.add(T * c),
-                     itab = ar.add(961 * (size_t)heads, table);
+                     imax = ar.add(1, &zero);
+        ar.commit();
+        float *dx = ar.ptr(ix), *dq = ar.ptr(iq), *dao = ar.ptr(iao), *dout = ar.ptr(iout);
+        AbsMaxArgs am{dx, (unsigned*)ar.ptr(imax), (long)(T * c)};
+        launch(s, "hat_absmax", (unsigned)std::min<size_t>((T * c + 4095) / 4096, 512), 1, 1, 256, am);
+        float mx = 0.0f;
+        rt.d2h(&mx, ar.ptr(imax), sizeof mx);
+        const QkvScale sc = qkv_scale(op_linear_bound(qkv_w, qkv_b, 0, c, c, mx),
+                                      op_linear_bound(qkv_w, qkv_b, c, 2 * c, c, mx),
+                                      op_linear_bound(qkv_w, qkv_b, 2 * c, 3 * c, c, mx), D);
+        const float osc[3] = {sc.q, sc.k, sc.v};
         // qkv as in the forward; the projection here has no residual, a form the
         // forward never runs, so it stays on the FP32 store epilogue
-        OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv), proj(ar, proj_w, proj_b, c, c);
-        ar.commit();
-        qkv.bind(ar);
-        proj.bind(ar);
-        float *dx = ar.ptr(ix), *dq = ar.ptr(iq), *dao = ar.ptr(iao), *dout = ar.ptr(iout), *dtab = ar.ptr(itab);
+        OpArena wr;
+        const size_t itab = wr.add(961 * (size_t)heads, table);
+        OpLinear qkv(wr, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc),
+            proj(wr, proj_w, proj_b, c, c, OpLinear::kNone, nullptr, 1.0f / sc.v);
+        wr.commit();
+        qkv.bind(wr);
+        proj.bind(wr);
+        const float* dtab = wr.ptr(itab);
         const GemmEpilogue none;
         auto run = [&]() {
             run_gemm(s, qkv.L, dx, c, (long)T, dq, 0, EPI_QKV, none, heads, D, 0.f);
-            run_attn(s, dq, dtab, dao, pl, heads, D, false, shift);
+            run_attn(s, dq, dtab, dao, pl, heads, D, false, shift, sc.ok);
             run_gemm(s, proj.L, dao, c, (long)T, dout, c, EPI_STORE, none, heads, D, 0.f);
         };
         run();
@@ -2325,7 +2453,7 @@ void op_swmsa(const float* x, float* out, int hp, int wp, int c, int heads, int 
             for (int i = 0; i < iters; ++i) run();
             api.EventRecord(t.b, s);
             api.EventRecord(ta.a, s);
-            for (int i = 0; i < iters; ++i) run_attn(s, dq, dtab, dao, pl, heads, D, false, shift);
+            for (int i = 0; i < iters; ++i) run_attn(s, dq, dtab, dao, pl, heads, D, false, shift, sc.ok);
             api.EventRecord(ta.b, s);
             rt.check(api.EventSynchronize(ta.b), "swmsa timing");
             float e = 0.f;
@@ -2364,10 +2492,14 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
                      iao = ar.add(T * c), itab = ar.add(1521 * (size_t)heads, table), i1w = ar.add(c, n1w),
                      i1b = ar.add(c, n1b), i2w = ar.add(c, n2w), i2b = ar.add(c, n2b);
         OpMlpX mx(ar, fc1_w, fc1_b, fc2_w, c, hid);
+        const QkvScale sc = qkv_scale(ln_linear_bound(qkv_w, qkv_b, n1w, n1b, 0, c, c),
+                                      ln_linear_bound(qkv_w, qkv_b, n1w, n1b, c, 2 * c, c),
+                                      ln_linear_bound(qkv_w, qkv_b, n1w, n1b, 2 * c, 3 * c, c), D);
+        const float osc[3] = {sc.q, sc.k, sc.v};
         // the split tails read only fc2's bias of these two
         const OpLinear::Split mlp = mx.fused ? OpLinear::kBias : OpLinear::kNone;
-        OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv),
-            proj(ar, proj_w, proj_b, c, c, mx.fused ? OpLinear::kProj : OpLinear::kNone),
+        OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc),
+            proj(ar, proj_w, proj_b, c, c, mx.fused ? OpLinear::kProj : OpLinear::kNone, nullptr, 1.0f / sc.v),
             fc1(ar, fc1_w, fc1_b, (int)hid, c, mlp), fc2(ar, fc2_w, fc2_b, c, (int)hid, mlp);
         const size_t ih = ar.add(mx.fused || mlp_fused(fc1.L, fc2.L) ? 1 : T * hid);
         ar.commit();
@@ -2386,7 +2518,7 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
         auto run = [&]() {
             run_ln(s, dx, dxn, d1w, d1b, (long)T, c);
             run_gemm(s, qkv.L, dxn, c, (long)T, dq, 0, EPI_QKV, none, heads, D, 0.f);
-            run_attn(s, dq, dtab, dao, pl, heads, D, true, 0);
+            run_attn(s, dq, dtab, dao, pl, heads, D, true, 0, sc.ok);
             if (mx.fused && c == 144) {
                 run_tailx(s, false, proj.L, mx.m, fc2.L.b, dao, dx, dwork, dxn, nullptr, nullptr, proj.L.b, d2w, d2b,
                           nullptr, nullptr, hp, wp);
@@ -2407,7 +2539,7 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
             for (int i = 0; i < iters; ++i) run();
             api.EventRecord(t.b, s);
             api.EventRecord(ta.a, s);
-            for (int i = 0; i < iters; ++i) run_attn(s, dq, dtab, dao, pl, heads, D, true, 0);
+            for (int i = 0; i < iters; ++i) run_attn(s, dq, dtab, dao, pl, heads, D, true, 0, sc.ok);
             api.EventRecord(ta.b, s);
             rt.check(api.EventSynchronize(ta.b), "ocab timing");
             float e = 0.f;

@@ -66,6 +66,29 @@ struct DevConv {
     int CI = 0, CIp = 0, CO = 0, COp = 0, r = 0;
 };
 
+// ---- Power-of-two scales for the split-f16 kernels (common.h), which need
+// their operands inside f16's range. Every scale is exact in fp32, so the
+// results do not depend on it while nothing leaves that range.
+
+// The largest power of two s with bound * s <= 2^15 (half of f16's range: room
+// for the roundings the bound leaves out); 1 for a bound that is 0 or not finite.
+float f16_scale(double bound);
+// A vector that a LayerNorm (w, b over C channels) can produce is n o w + b with
+// |n|_2 <= sqrt(C), and |n_c| <= sqrt(C). Bounds over every such vector: of
+// |row . y + bias| for rows [n0, n1) of a linear [N][C] (the largest), and of
+// |y_c| over the channels.
+double ln_linear_bound(const float* w, const float* b, const float* lnw, const float* lnb, int n0, int n1, int C);
+double ln_bound(const float* lnw, const float* lnb, int C);
+// The scales of an attention's q, k and v rows (folded into the qkv weights):
+// q and k by inverse powers of two that balance their bounds, so that the scores
+// do not change, v by its own (the projection's weights take it out). ok: the
+// balanced bounds fit; otherwise the FP32 kernels run and every scale is 1.
+struct QkvScale {
+    float q = 1.0f, k = 1.0f, v = 1.0f;
+    bool ok = false;
+};
+QkvScale qkv_scale(double bq, double bk, double bv, int head_dim);
+
 // Host-side repacking (also used by the selftest and the op entry points).
 std::vector<float> pack_linear(const float* w, int N, int K, int* Kp);
 // [N][144] -> per 144-row slice, five weight chunks (one per 32-k step) of
@@ -179,6 +202,7 @@ private:
     std::map<std::string, DevConv> conv_;
     std::map<std::string, DevCab> cab_;
     std::map<std::string, DevMlpX> mlpx_;  // C = 144 MLPs (blocks and OCABs) for hat_mlpx
+    std::map<std::string, bool> attn_f16_;  // by bias table name: the split-f16 attention runs
     bool cab_fold_ = false;  // the C = 144, 6-channel CAB runs folded
     std::vector<void*> owned_;
     size_t weight_bytes_ = 0;
@@ -229,7 +253,13 @@ private:
     float* upload(const float* src, size_t n);
     void* upload_bytes(const void* src, size_t bytes);
     void upload_raw(const std::string& name);
-    void upload_linear(const std::string& name);
+    // row_scale (if set): each weight row's and bias entry's factor; all: every
+    // weight's (the bias is not touched). split: whether the split copy is made.
+    void upload_linear(const std::string& name, const std::vector<float>* row_scale = nullptr, float all = 1.0f,
+                       bool split = true);
+    // An attention's qkv and projection behind norm `ln`, scaled for the
+    // split-f16 attention where the bounds allow it (attn_f16_ of its table).
+    void upload_attn(const std::string& qkv, const std::string& proj, const std::string& ln, const std::string& table);
     void upload_conv(const std::string& name, int r = 0);
     void upload_mlpx(const std::string& name);
     void ensure_plan(int h, int w);

@@ -105,7 +105,7 @@ struct CabGateArgs {
     const float* wb;     // excite [144][sq]
     const float* bb;     // [144]
     const float* bproj;  // attention projection bias [144]
-    float* w2g;          // out: cscale * gate[c] * conv2 weight, [144][CAB_K2] (k = tap*6 + ci)
+    float* w2g;          // out (if set): cscale * gate[c] * conv2 weight, [144][CAB_K2] (k = tap*6 + ci)
     float* bias2;        // out: bproj + cscale * gate * b2, [144]
     float* gate;         // out: the gate itself [144]
     float cscale;
@@ -340,6 +340,14 @@ struct CopyArgs {
     const float* src;
     float* dst;
     long n4;
+};
+
+// out[0] = max(out[0], bits of the largest finite |x[i]|), i < n (a multiple of
+// 4): the bits of non-negative floats order as unsigned integers do.
+struct AbsMaxArgs {
+    const float* x;
+    unsigned* out;
+    long n;
 };
 
 // Column sums of a [nrows][stride] matrix in row blocks: out[blk][c] = sum of

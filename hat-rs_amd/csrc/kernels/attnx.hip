@@ -1,21 +1,28 @@
-// Shifted-window attention on BF16 MFMA with fp32 accuracy: QK^T + relative-
-// position bias + shift mask + softmax + PV for one (window, head) per block.
+// Window attention on F16 MFMA with fp32 accuracy: QK^T + relative-position
+// bias + shift mask + softmax + PV for one (window, head) per block.
 //
 // The same operator as attn.hip (cpu.rs:772-844; hat.cu:246-316) on gfx950's
-// BF16 matrix path, whose peak is 16x the FP32 MFMA rate. VALU and MFMA work
-// share a SIMD's issue time (measured: they do not overlap, from one wave or
-// from two), so the splits and exponentials below cost their full time. Every fp32
-// operand x enters as three bf16 parts, x = x0 + x1 + x2 + e with |e| <=
-// 2^-27 |x| (each part the round-to-nearest of what the earlier ones leave),
-// and a product as the six terms a_i b_j with i + j <= 2, accumulated in fp32
-// by v_mfma_f32_32x32x16_bf16; the terms dropped (i + j >= 3) are below
-// 2^-26 |ab|. Measured at K = 144 against a double reference: worst error
-// 1.25e-7 of sum|ab| against 1.42e-7 for FP32 MFMA.
+// 16-bit matrix path, whose peak is 16x the FP32 MFMA rate. VALU and MFMA work
+// share a SIMD's issue time (measured: they hardly overlap, from one wave or
+// from two), so the splits and exponentials below cost their full time. Every
+// fp32 operand enters as two f16 parts and a product as three MFMA terms
+// (common.h states the split's accuracy); q, k and v must lie inside f16's
+// range, which the host sees to by folding powers of two into the qkv weights
+// (qkv_scale), and networks whose bounds do not allow it run attn.hip.
 //
-// Layout (all per item, in LDS): K as three bf16 planes [256 keys][KS] and V^T
-// as three planes [D + 1][VS] whose key order is permuted within each 16 so
+// What bounds it: issue time, MFMA and VALU together. Per 32-key tile and wave
+// at head_dim 24, 11 MFMAs of 32 cycles (5 for QK^T, 6 for PV), 16 exponentials
+// and ~90 other VALU instructions; the three-part bf16 split that this replaced
+// took 21 MFMAs and ~120. HAT-S 512 x 512 (1024 windows, 6 heads): SW 252.6 ->
+// 178.2 us a launch, OCA 574 -> 383; HAT 512 x 512 OCA 664 -> 458; head_dim 30
+// SW as whole items (two planes fit two blocks a CU; the bf16 planes did not).
+// Parts of 288 keys for OCA at head_dim 24 spilled 34 registers (446 us), parts
+// of 192 at 30 27 of them (154 us at 256 x 256 against 122).
+//
+// Layout (all per item, in LDS): K as two f16 planes [256 keys][KS] and V^T
+// as two planes [D + 1][VS] whose key order is permuted within each 16 so
 // that a lane's eight keys of one MFMA step are contiguous; row D of V^T is
-// ones in the high plane and zeros in the others, so row D of O^T is the
+// ones in the high plane and zeros in the other, so row D of O^T is the
 // softmax denominator. The bias table of the head is kept in log2 units. Wave
 // w owns queries [32w, 32w+32). Scores are computed transposed, S^T = K Q^T
 // (A = a 32-key tile of K, B = the wave's q, split in registers): lane l holds
@@ -26,16 +33,20 @@
 
 using namespace hatk;
 
+// What the max-subtracted softmax adds to its base: P up to 2^(8 + 6), so that
+// the smallest probabilities stay clear of f16's subnormals.
+#define ATTNX_SAFE_UP 6.0f
+
 template <int D>
 struct AttnXShape {
     static constexpr int NK = 256;
-    // K row stride in bf16: 24 (48 B) and 40 (80 B) put the 16 rows a ds_read_b128
+    // K row stride in f16: 24 (48 B) and 40 (80 B) put the 16 rows a ds_read_b128
     // phase touches on distinct banks.
     static constexpr int KS = D == 24 ? 24 : 40;
     static constexpr int VS = NK + 8;  // V^T row stride (528 B: rows 4 banks apart)
     static constexpr int KPL = NK * KS, VPL = (D + 1) * VS;  // elements per plane
     static constexpr int TROWS = 961;
-    static constexpr int LDS_BYTES = 2 * 3 * (KPL + VPL) + 4 * TROWS;
+    static constexpr int LDS_BYTES = 2 * 2 * (KPL + VPL) + 4 * TROWS;
 };
 
 // Position of key k in the V^T planes: within each 16 keys, bits 2 and 3
@@ -70,28 +81,25 @@ __device__ __forceinline__ void attnx_stash(unsigned short* Kp, unsigned short* 
             }
 #pragma unroll
             for (int j = 0; j < S::U; j += 2) {
-                unsigned k0, k1, k2, v0, v1, v2;
-                split3_pk(kv[j], kv[j + 1], k0, k1, k2);
+                unsigned k0, k1, v0, v1;
+                split2_pk(kv[j], kv[j + 1], k0, k1);
                 *(unsigned*)(Kp + 0 * X::KPL + k * X::KS + d + j) = k0;
                 *(unsigned*)(Kp + 1 * X::KPL + k * X::KS + d + j) = k1;
-                *(unsigned*)(Kp + 2 * X::KPL + k * X::KS + d + j) = k2;
-                split3_pk(vv[j], vv[j + 1], v0, v1, v2);
+                split2_pk(vv[j], vv[j + 1], v0, v1);
                 const int pos = vpos(k);
                 Vp[0 * X::VPL + (d + j) * X::VS + pos] = (unsigned short)v0;
                 Vp[0 * X::VPL + (d + j + 1) * X::VS + pos] = (unsigned short)(v0 >> 16);
                 Vp[1 * X::VPL + (d + j) * X::VS + pos] = (unsigned short)v1;
                 Vp[1 * X::VPL + (d + j + 1) * X::VS + pos] = (unsigned short)(v1 >> 16);
-                Vp[2 * X::VPL + (d + j) * X::VS + pos] = (unsigned short)v2;
-                Vp[2 * X::VPL + (d + j + 1) * X::VS + pos] = (unsigned short)(v2 >> 16);
             }
         }
     }
-    for (int e = threadIdx.x; e < 3 * (S::NK / 2); e += 512) {
+    for (int e = threadIdx.x; e < 2 * (S::NK / 2); e += 512) {
         const int pl = e / (S::NK / 2), k2 = e - pl * (S::NK / 2);
-        *(unsigned*)(Vp + pl * X::VPL + D * X::VS + 2 * k2) = pl == 0 ? 0x3f803f80u : 0u;  // bf16 1.0 pairs
+        *(unsigned*)(Vp + pl * X::VPL + D * X::VS + 2 * k2) = pl == 0 ? 0x3c003c00u : 0u;  // f16 1.0 pairs
     }
     if (D == 30) {
-        for (int e = threadIdx.x; e < 3 * S::NK; e += 512) {
+        for (int e = threadIdx.x; e < 2 * S::NK; e += 512) {
             const int pl = e / S::NK, k = e - pl * S::NK;
             *(unsigned*)(Kp + pl * X::KPL + k * X::KS + 30) = 0u;
         }
@@ -100,10 +108,9 @@ __device__ __forceinline__ void attnx_stash(unsigned short* Kp, unsigned short* 
 
 // The lane's q, pre-scaled and split: qb[s][part] = dims 16s + 8h .. 16s + 8h
 // + 7 of its query (zeros past D). For D = 24 the second step is packed (see
-// AttnxKRows): qb[1][0] = dims 16..23 of part h ? 0 : 2, qb[1][1] = of part
-// h ? 0 : 1.
+// AttnxKRows): qb[1][0] = dims 16..23 of part h.
 template <int D>
-__device__ __forceinline__ int attnx_query(const AttnArgs& p, int wi, int head, u32x4 (&qb)[2][3])
+__device__ __forceinline__ int attnx_query(const AttnArgs& p, int wi, int head, u32x4 (&qb)[2][2])
 {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, in a scalar register
@@ -139,49 +146,38 @@ __device__ __forceinline__ int attnx_query(const AttnArgs& p, int wi, int head, 
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) qv[s][j] *= p.qscale;
-        split3_x8(qv[s], qb[s]);
+        split2_x8(qv[s], qb[s]);
     }
-    if constexpr (D == 24) {
-        const u32x4 q0 = qb[1][0], q1 = qb[1][1], q2 = qb[1][2];
-        qb[1][0] = h ? q0 : q2;
-        qb[1][1] = h ? q0 : q1;
-    }
+    if constexpr (D == 24) qb[1][0] = h ? qb[1][1] : qb[1][0];
     return qpix;
 }
 
-// The lane's K rows for S^T = K Q^T over 32-key tiles of three planes [keys][KS]
+// The lane's K rows for S^T = K Q^T over 32-key tiles of two planes [keys][KS]
 // (A = 32 keys x 16 dims: lane l gives key l % 32, dims 8h .. 8h + 7 of the step).
-// Step 0 (dims 0..15) is the six products of mfma6. For D = 24, step 1 has only
-// dims 16..23, so each MFMA carries two of the six products, one per lane half:
-// [k1 | k2] . [q1 | q0], [k0 | k1] . [q2 | q0], [k0 | k0] . [q1 | q0] (half 0 |
-// half 1): the same terms in three MFMAs instead of six. For D = 30 step 1 is
-// dims 16..31 (30, 31 zero) as step 0.
+// Step 0 (dims 0..15) is the three products of mfma3. For D = 24, step 1 has only
+// dims 16..23, so each MFMA carries two products, one per lane half: [k1 | k1] .
+// [q0 | q1], then [k0 | k0] . [q0 | q1] (half 0 | half 1), two MFMAs for the
+// three products (k1 q1 comes along). For D = 30 step 1 is dims 16..31 (30, 31
+// zero) as step 0.
 template <int D, int KS, int KPL>
 struct AttnxKRows {
-    const unsigned short *r0, *r12, *r3;
+    const unsigned short *r0, *r1;
     __device__ __forceinline__ void init(const unsigned short* Kp, int ql, int h)
     {
         r0 = Kp + ql * KS + 8 * h;
-        r12 = Kp + ql * KS + 16 + h * KPL;  // plane h (+1)
-        r3 = Kp + ql * KS + 16;             // plane 0
+        r1 = Kp + ql * KS + 16 + (D == 24 ? 0 : 8 * h);
     }
     // s += K Q^T for the tile whose first key row is koff elements in
-    __device__ __forceinline__ f32x16 qk(int koff, const u32x4 (&qb)[2][3], f32x16 s) const
+    __device__ __forceinline__ f32x16 qk(int koff, const u32x4 (&qb)[2][2], f32x16 s) const
     {
-        u32x4 ka[3];
-#pragma unroll
-        for (int pl = 0; pl < 3; ++pl) ka[pl] = *(const u32x4*)(r0 + pl * KPL + koff);
-        s = mfma6(ka, qb[0], s);
+        const u32x4 k0[2] = {*(const u32x4*)(r0 + koff), *(const u32x4*)(r0 + KPL + koff)};
+        const u32x4 k1[2] = {*(const u32x4*)(r1 + koff), *(const u32x4*)(r1 + KPL + koff)};
+        s = mfma3(k0, qb[0], s);
         if constexpr (D == 24) {
-            const u32x4 a12 = *(const u32x4*)(r12 + KPL + koff), a01 = *(const u32x4*)(r12 + koff),
-                        a00 = *(const u32x4*)(r3 + koff);
-            s = mfma_bf16(a12, qb[1][1], s);
-            s = mfma_bf16(a01, qb[1][0], s);
-            return mfma_bf16(a00, qb[1][1], s);
+            s = mfma_f16(k1[1], qb[1][0], s);
+            return mfma_f16(k1[0], qb[1][0], s);
         } else {
-#pragma unroll
-            for (int pl = 0; pl < 3; ++pl) ka[pl] = *(const u32x4*)(r0 + pl * KPL + koff + 16);
-            return mfma6(ka, qb[1], s);
+            return mfma3(k1, qb[1], s);
         }
     }
 };
@@ -196,13 +192,13 @@ struct AttnxKRows {
 // Either way o / o[row D] is the softmax-weighted sum, the same quantity.
 template <int D, bool MASKED, bool SAFE>
 __device__ __forceinline__ f32x16 attnx_tiles(const AttnArgs& p, const unsigned char* lds, int wi,
-                                              const u32x4 (&qb)[2][3])
+                                              const u32x4 (&qb)[2][2])
 {
     using X = AttnXShape<D>;
     constexpr int NKT = X::NK / 32;
     const unsigned short* Kp = (const unsigned short*)lds;
-    const unsigned short* Vp = Kp + 3 * X::KPL;
-    const float* Tb = (const float*)(Vp + 3 * X::VPL);
+    const unsigned short* Vp = Kp + 2 * X::KPL;
+    const float* Tb = (const float*)(Vp + 2 * X::VPL);
 
     const int wy = wi / p.nx, wx = wi - (wi / p.nx) * p.nx;
     const int lane = threadIdx.x & 63;
@@ -264,29 +260,32 @@ __device__ __forceinline__ f32x16 attnx_tiles(const AttnArgs& p, const unsigned 
         for (int st = 0; st < 2; ++st) {
             float pv[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pv[j] = fast_exp2(SAFE ? s[8 * st + j] - mrun : s[8 * st + j]);
-            u32x4 pb[3], va[3];
-            split3_x8(pv, pb);
+            for (int j = 0; j < 8; ++j) pv[j] = fast_exp2(SAFE ? s[8 * st + j] - (mrun - ATTNX_SAFE_UP) : s[8 * st + j]);
+            u32x4 pb[2], va[2];
+            split2_x8(pv, pb);
 #pragma unroll
-            for (int pl = 0; pl < 3; ++pl) va[pl] = *(const u32x4*)(vrow + pl * X::VPL + kt * 32 + 16 * st);
-            o = mfma6(va, pb, o);
+            for (int pl = 0; pl < 2; ++pl) va[pl] = *(const u32x4*)(vrow + pl * X::VPL + kt * 32 + 16 * st);
+            o = mfma3(va, pb, o);
         }
     }
     return o;
 }
 
 // Whether an item's base-0 pass (attnx_tiles with SAFE false) may stand, for
-// every query of the wave: the denominator within [2^-60, 2^100] (no
-// overflow, and far from the range where P's split parts would underflow;
-// with the row maximum subtracted it lies in [1, 256 * 2^8]) and every
-// accumulator finite. Wave-uniform.
+// every query of the wave: the denominator within [32, 65504] and every
+// accumulator finite. The upper end means that no probability left f16's range
+// (they are positive, and one that did is infinite, as is then the sum). The
+// lower end bounds what the subnormal parts of the probabilities lose: up to
+// 2^-25 of each of at most 576, under 1e-8 of the denominator. A window of 256
+// scores around 0 has denominator 256; with the row maximum subtracted
+// (ATTNX_SAFE_UP above it) it lies in [2^6, 576 * 2^14]. Wave-uniform.
 template <int D>
 __device__ __forceinline__ bool attnx_item_done(const f32x16& o)
 {
     constexpr int RH = (D % 8) / 4, RR = (D / 8) * 4 + D % 4;
     const int ql = threadIdx.x & 31;
     const float ltot = __shfl(o[RR], ql + 32 * RH, 64);
-    bool ok = ltot >= 0x1p-60f && ltot <= 0x1p100f;
+    bool ok = ltot >= 32.0f && ltot <= 65504.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) ok = ok && __builtin_isfinite(o[i]);
     return __all(ok);
@@ -319,7 +318,7 @@ __device__ __forceinline__ void attnx_store(const AttnArgs& p, int head, int qpi
 
 template <int D, bool MASKED>
 __device__ __forceinline__ void attnx_compute(const AttnArgs& p, const unsigned char* lds, int wi, int head,
-                                              const u32x4 (&qb)[2][3], int qpix)
+                                              const u32x4 (&qb)[2][2], int qpix)
 {
     f32x16 o = attnx_tiles<D, MASKED, false>(p, lds, wi, qb);
     if (!attnx_item_done<D>(o)) {  // wave-uniform
@@ -349,9 +348,9 @@ __device__ __forceinline__ void attnx_item_kernel(const AttnArgs& p, unsigned ch
         __syncthreads();
     }
     unsigned short* Kp = (unsigned short*)lds;
-    unsigned short* Vp = Kp + 3 * X::KPL;
-    float* Tb = (float*)(Vp + 3 * X::VPL);
-    u32x4 qb[2][3];
+    unsigned short* Vp = Kp + 2 * X::KPL;
+    float* Tb = (float*)(Vp + 2 * X::VPL);
+    u32x4 qb[2][2];
     int qpix;
     {
         typename S::vec ks[S::NE], vs[S::NE];
@@ -381,32 +380,28 @@ __device__ __forceinline__ void attnx_item_kernel(const AttnArgs& p, unsigned ch
 // most 80 KB of LDS and 128 VGPRs, so that two blocks share a CU and one's
 // staging overlaps the other's MFMAs.
 
-// SW: the same part-wise staging for shifted-window attention (256 keys of the
-// rolled window, the shift mask on the last window row and column, the 961-row
-// table), which head_dim 30 needs for two blocks per CU: its whole item, K and
-// V^T in three planes, takes 114 KB of LDS, two parts of 128 keys 60 KB.
-template <int D, int NK, bool SW = false>
+template <int D, int NK>
 struct AttnXOcaShape {
-    static constexpr int NKEYS = SW ? 256 : 576;
+    static constexpr int NKEYS = 576;
     static_assert(NKEYS % NK == 0 && NK % 32 == 0, "whole 32-key tiles, whole parts");
     static constexpr int NPART = NKEYS / NK;
     static constexpr int KS = D == 24 ? 24 : 40;
     static constexpr int VS = NK + 8;                 // V^T row stride: 16 rows of a phase on distinct banks
     static constexpr int KPL = NK * KS, VPL = (D + 1) * VS;
-    static constexpr int TROWS = SW ? 961 : 1521;
-    static constexpr int LDS_BYTES = 2 * 3 * (KPL + VPL) + 4 * TROWS;
+    static constexpr int TROWS = 1521;
+    static constexpr int LDS_BYTES = 2 * 2 * (KPL + VPL) + 4 * TROWS;
     static constexpr int U = D % 4 == 0 ? 4 : 2;       // floats per staging unit
     static constexpr int NE = (NK * D / U + 511) / 512;
     using vec = typename pick_t<U == 4, float4, float2>::type;
 };
 
 // This thread's share of part `part` of item (wi, head): K and V units.
-template <int D, int NK, bool SW = false>
+template <int D, int NK>
 __device__ __forceinline__ void attnx_oca_fetch(const AttnArgs& p, int wi, int head, int part,
-                                                typename AttnXOcaShape<D, NK, SW>::vec (&ks)[AttnXOcaShape<D, NK, SW>::NE],
-                                                typename AttnXOcaShape<D, NK, SW>::vec (&vs)[AttnXOcaShape<D, NK, SW>::NE])
+                                                typename AttnXOcaShape<D, NK>::vec (&ks)[AttnXOcaShape<D, NK>::NE],
+                                                typename AttnXOcaShape<D, NK>::vec (&vs)[AttnXOcaShape<D, NK>::NE])
 {
-    using X = AttnXOcaShape<D, NK, SW>;
+    using X = AttnXOcaShape<D, NK>;
     using vec = typename X::vec;
     constexpr int PER_KEY = D / X::U;
     const float* Kg = p.qkv + (size_t)(p.heads + head) * p.T * D;
@@ -417,7 +412,7 @@ __device__ __forceinline__ void attnx_oca_fetch(const AttnArgs& p, int wi, int h
         vec kv{}, vv{};
         if (e < NK * PER_KEY) {
             const int kl = e / PER_KEY, d = (e - kl * PER_KEY) * X::U;
-            const int pix = attn_key_pixel<!SW>(p, wi, part * NK + kl);
+            const int pix = attn_key_pixel<true>(p, wi, part * NK + kl);
             if (pix >= 0) {
                 kv = *(const vec*)(Kg + (size_t)pix * D + d);
                 vv = *(const vec*)(Vg + (size_t)pix * D + d);
@@ -428,12 +423,12 @@ __device__ __forceinline__ void attnx_oca_fetch(const AttnArgs& p, int wi, int h
     }
 }
 
-template <int D, int NK, bool SW = false>
+template <int D, int NK>
 __device__ __forceinline__ void attnx_oca_stash(unsigned short* Kp, unsigned short* Vp,
-                                                const typename AttnXOcaShape<D, NK, SW>::vec (&ks)[AttnXOcaShape<D, NK, SW>::NE],
-                                                const typename AttnXOcaShape<D, NK, SW>::vec (&vs)[AttnXOcaShape<D, NK, SW>::NE])
+                                                const typename AttnXOcaShape<D, NK>::vec (&ks)[AttnXOcaShape<D, NK>::NE],
+                                                const typename AttnXOcaShape<D, NK>::vec (&vs)[AttnXOcaShape<D, NK>::NE])
 {
-    using X = AttnXOcaShape<D, NK, SW>;
+    using X = AttnXOcaShape<D, NK>;
     constexpr int PER_KEY = D / X::U;
 #pragma unroll
     for (int i = 0; i < X::NE; ++i) {
@@ -451,18 +446,15 @@ __device__ __forceinline__ void attnx_oca_stash(unsigned short* Kp, unsigned sho
             const int pos = vpos(k);
 #pragma unroll
             for (int j = 0; j < X::U; j += 2) {
-                unsigned k0, k1, k2, v0, v1, v2;
-                split3_pk(kv[j], kv[j + 1], k0, k1, k2);
+                unsigned k0, k1, v0, v1;
+                split2_pk(kv[j], kv[j + 1], k0, k1);
                 *(unsigned*)(Kp + 0 * X::KPL + k * X::KS + d + j) = k0;
                 *(unsigned*)(Kp + 1 * X::KPL + k * X::KS + d + j) = k1;
-                *(unsigned*)(Kp + 2 * X::KPL + k * X::KS + d + j) = k2;
-                split3_pk(vv[j], vv[j + 1], v0, v1, v2);
+                split2_pk(vv[j], vv[j + 1], v0, v1);
                 Vp[0 * X::VPL + (d + j) * X::VS + pos] = (unsigned short)v0;
                 Vp[0 * X::VPL + (d + j + 1) * X::VS + pos] = (unsigned short)(v0 >> 16);
                 Vp[1 * X::VPL + (d + j) * X::VS + pos] = (unsigned short)v1;
                 Vp[1 * X::VPL + (d + j + 1) * X::VS + pos] = (unsigned short)(v1 >> 16);
-                Vp[2 * X::VPL + (d + j) * X::VS + pos] = (unsigned short)v2;
-                Vp[2 * X::VPL + (d + j + 1) * X::VS + pos] = (unsigned short)(v2 >> 16);
             }
         }
     }
@@ -471,14 +463,14 @@ __device__ __forceinline__ void attnx_oca_stash(unsigned short* Kp, unsigned sho
 // One part's key tiles onto the running (o, mrun) of the item; SAFE as in
 // attnx_tiles (without it the base stays 0 and mrun is not used).
 template <int D, int NK, bool SAFE>
-__device__ __forceinline__ void attnx_oca_compute(const unsigned char* lds, int part, const u32x4 (&qb)[2][3],
+__device__ __forceinline__ void attnx_oca_compute(const unsigned char* lds, int part, const u32x4 (&qb)[2][2],
                                                   f32x16& o, float& mrun)
 {
     using X = AttnXOcaShape<D, NK>;
     constexpr int NKT = NK / 32;
     const unsigned short* Kp = (const unsigned short*)lds;
-    const unsigned short* Vp = Kp + 3 * X::KPL;
-    const float* Tb = (const float*)(Vp + 3 * X::VPL);
+    const unsigned short* Vp = Kp + 2 * X::KPL;
+    const float* Tb = (const float*)(Vp + 2 * X::VPL);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, in a scalar register
     const int ql = lane & 31, h = lane >> 5;
@@ -516,118 +508,32 @@ __device__ __forceinline__ void attnx_oca_compute(const unsigned char* lds, int 
         for (int st = 0; st < 2; ++st) {
             float pv[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pv[j] = fast_exp2(SAFE ? s[8 * st + j] - mrun : s[8 * st + j]);
-            u32x4 pb[3], va[3];
-            split3_x8(pv, pb);
+            for (int j = 0; j < 8; ++j) pv[j] = fast_exp2(SAFE ? s[8 * st + j] - (mrun - ATTNX_SAFE_UP) : s[8 * st + j]);
+            u32x4 pb[2], va[2];
+            split2_x8(pv, pb);
 #pragma unroll
-            for (int pl = 0; pl < 3; ++pl) va[pl] = *(const u32x4*)(vrow + pl * X::VPL + kt * 32 + 16 * st);
-            o = mfma6(va, pb, o);
+            for (int pl = 0; pl < 2; ++pl) va[pl] = *(const u32x4*)(vrow + pl * X::VPL + kt * 32 + 16 * st);
+            o = mfma3(va, pb, o);
         }
     }
 }
 
-// One part of a shifted-window item (the SW form of attnx_oca_compute): the
-// keys part * NK .. + NK - 1 of the rolled window, bias and mask as attnx_tiles.
-template <int D, int NK, bool SAFE, bool MASKED>
-__device__ __forceinline__ void attnx_swp_compute(const AttnArgs& p, const unsigned char* lds, int wi, int part,
-                                                  const u32x4 (&qb)[2][3], f32x16& o, float& mrun)
-{
-    using X = AttnXOcaShape<D, NK, true>;
-    constexpr int NKT = NK / 32;
-    static_assert(NK % 16 == 0, "parts of whole window rows");
-    const unsigned short* Kp = (const unsigned short*)lds;
-    const unsigned short* Vp = Kp + 3 * X::KPL;
-    const float* Tb = (const float*)(Vp + 3 * X::VPL);
-    const int wy = wi / p.nx, wx = wi - (wi / p.nx) * p.nx;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, in a scalar register
-    const int ql = lane & 31, h = lane >> 5;
-    const int q = wave * 32 + ql;
-    const int qy = q >> 4, qx = q & 15;
-    // the part's first key row: NK / 16 rows of 31 table entries each
-    const float* Tr = Tb + 960 - ((qy + 15) * 31 + qx + 15 - 4 * h) + part * (NK / 16) * 31;
-    const float NEG = -100.0f * HAT_LOG2E;
-    const bool mrow = MASKED && wy == p.ny - 1;
-    const bool mcol = MASKED && wx == p.nx - 1;
-    const bool r_lo = mrow && (qy & 8), r_hi = mrow && !(qy & 8);
-    const bool c_lo = mcol && (qx & 8), c_hi = mcol && !(qx & 8);
-    const float madd[2][2] = {{(r_lo || c_lo) ? NEG : 0.0f, (r_lo || c_hi) ? NEG : 0.0f},
-                              {(r_hi || c_lo) ? NEG : 0.0f, (r_hi || c_hi) ? NEG : 0.0f}};
-    const unsigned short* vrow = Vp + (ql < D ? ql : D) * X::VS + 8 * h;
-    AttnxKRows<D, X::KS, X::KPL> kr;
-    kr.init(Kp, ql, h);
-#pragma unroll 1
-    for (int kt = 0; kt < NKT; ++kt) {
-        f32x16 s;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int kl = kt * 32 + (i >> 2) * 8 + (i & 3);  // key within the part (lane half 0)
-            const int ky = kl >> 4, kx = kl & 15;
-            float b = Tr[ky * 31 + kx];
-            // the mask's row band: the key row within the window, part * NK / 16 + ky
-            if (MASKED) b += madd[((part * (NK / 16) + ky) >> 3) & 1][(kx >> 3) & 1];
-            s[i] = b;
-        }
-        s = kr.qk(kt * 32 * X::KS, qb, s);
-        if constexpr (SAFE) {
-            float mx = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-            if ((part == 0 && kt == 0) || __any(mx > mrun + 8.0f)) {  // wave-uniform
-                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-                const float mnew = fmaxf(mrun, mx);
-                const float corr = fast_exp2(mrun - mnew);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[i] *= corr;
-                mrun = mnew;
-            }
-        }
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-            float pv[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) pv[j] = fast_exp2(SAFE ? s[8 * st + j] - mrun : s[8 * st + j]);
-            u32x4 pb[3], va[3];
-            split3_x8(pv, pb);
-#pragma unroll
-            for (int pl = 0; pl < 3; ++pl) va[pl] = *(const u32x4*)(vrow + pl * X::VPL + kt * 32 + 16 * st);
-            o = mfma6(va, pb, o);
-        }
-    }
-}
-
-template <int D, int NK, bool SW = false>
+template <int D, int NK>
 __device__ __forceinline__ void attnx_oca_kernel(const AttnArgs& p, unsigned char* lds)
 {
-    using X = AttnXOcaShape<D, NK, SW>;
+    using X = AttnXOcaShape<D, NK>;
     const int wi = blockIdx.x, head = blockIdx.y;
-    // SW: the windows of the last row and column of a shifted grid carry the mask
-    const bool masked = SW && p.shift > 0 && (wi / p.nx == p.ny - 1 || wi % p.nx == p.nx - 1);  // block-uniform
-    if constexpr (SW) {
-        // the CAB's gates ride on the SW launch, in its first block, as in
-        // attnx_item_kernel
-        if (p.with_gate && wi == 0 && head == 0) {  // block-uniform
-            static_assert(4 * CAB_GATE_LDS <= X::LDS_BYTES, "the gate's scratch fits the item LDS");
-            cab_gate_body<8>(p.gate, (float*)lds);
-            __syncthreads();
-        }
-        if (p.with_se && wi == 0 && head == 0) {  // block-uniform
-            static_assert(4 * SE_GATE_LDS <= X::LDS_BYTES, "the gate's scratch fits the item LDS");
-            se_gate_body<8>(p.se, (float*)lds);
-            __syncthreads();
-        }
-    }
     unsigned short* Kp = (unsigned short*)lds;
-    unsigned short* Vp = Kp + 3 * X::KPL;
-    float* Tb = (float*)(Vp + 3 * X::VPL);
+    unsigned short* Vp = Kp + 2 * X::KPL;
+    float* Tb = (float*)(Vp + 2 * X::VPL);
     // Written once (no part's staging touches them): row D of V^T (ones in the
     // high plane), K dims 30, 31 (D = 30).
-    for (int e = threadIdx.x; e < 3 * (NK / 2); e += 512) {
+    for (int e = threadIdx.x; e < 2 * (NK / 2); e += 512) {
         const int pl = e / (NK / 2), k2 = e - pl * (NK / 2);
-        *(unsigned*)(Vp + pl * X::VPL + D * X::VS + 2 * k2) = pl == 0 ? 0x3f803f80u : 0u;
+        *(unsigned*)(Vp + pl * X::VPL + D * X::VS + 2 * k2) = pl == 0 ? 0x3c003c00u : 0u;  // f16 1.0 pairs
     }
     if (D == 30) {
-        for (int e = threadIdx.x; e < 3 * NK; e += 512) {
+        for (int e = threadIdx.x; e < 2 * NK; e += 512) {
             const int pl = e / NK, k = e - pl * NK;
             *(unsigned*)(Kp + pl * X::KPL + k * X::KS + 30) = 0u;
         }
@@ -636,14 +542,14 @@ __device__ __forceinline__ void attnx_oca_kernel(const AttnArgs& p, unsigned cha
     const int ql = lane & 31, h = lane >> 5;
     constexpr int RH = (D % 8) / 4, RR = (D / 8) * 4 + D % 4;
     typename X::vec ks[X::NE], vs[X::NE];
-    u32x4 qb[2][3];
+    u32x4 qb[2][2];
     int qpix;
     {
-        attnx_oca_fetch<D, NK, SW>(p, wi, head, 0, ks, vs);
-        AttnTableRegs<D, !SW> tr;
-        attn_table_load<D, !SW>(p, head, tr);
+        attnx_oca_fetch<D, NK>(p, wi, head, 0, ks, vs);
+        AttnTableRegs<D, true> tr;
+        attn_table_load<D, true>(p, head, tr);
         qpix = attnx_query<D>(p, wi, head, qb);
-        attn_table_store<D, !SW>(Tb, tr);
+        attn_table_store<D, true>(Tb, tr);
     }
     f32x16 o;
 #pragma unroll
@@ -653,19 +559,13 @@ __device__ __forceinline__ void attnx_oca_kernel(const AttnArgs& p, unsigned cha
 #pragma unroll 1
     for (int part = 0; part < X::NPART; ++part) {
         if (part > 0) __syncthreads();  // every read of the previous part's K and V is done
-        attnx_oca_stash<D, NK, SW>(Kp, Vp, ks, vs);
+        attnx_oca_stash<D, NK>(Kp, Vp, ks, vs);
         __syncthreads();
         // the next part's K and V in flight while this part's tiles run (the
-        // registers are free once stashed; same-box: head_dim 30 SW 356 ->
-        // 344 us, OCA 677 -> 661, head_dim 24 OCA 589 -> 585)
-        if (part + 1 < X::NPART) attnx_oca_fetch<D, NK, SW>(p, wi, head, part + 1, ks, vs);
-        if constexpr (SW) {
-            if (masked) attnx_swp_compute<D, NK, false, true>(p, lds, wi, part, qb, o, mrun);
-            else attnx_swp_compute<D, NK, false, false>(p, lds, wi, part, qb, o, mrun);
-        } else {
-            attnx_oca_compute<D, NK, false>(lds, part, qb, o, mrun);
-        }
-
+        // registers are free once stashed; same-box with the bf16 split: OCA head_dim
+        // 30 677 -> 661 us, head_dim 24 589 -> 585)
+        if (part + 1 < X::NPART) attnx_oca_fetch<D, NK>(p, wi, head, part + 1, ks, vs);
+        attnx_oca_compute<D, NK, false>(lds, part, qb, o, mrun);
     }
     // The parts are staged by the whole block, so the block redoes the item
     // with the max-subtracted softmax if any of its waves needs it.
@@ -682,16 +582,11 @@ __device__ __forceinline__ void attnx_oca_kernel(const AttnArgs& p, unsigned cha
         mrun = -INFINITY;
 #pragma unroll 1
         for (int part = 0; part < X::NPART; ++part) {
-            attnx_oca_fetch<D, NK, SW>(p, wi, head, part, ks, vs);
+            attnx_oca_fetch<D, NK>(p, wi, head, part, ks, vs);
             if (part > 0) __syncthreads();  // every read of the previous part's K and V is done
-            attnx_oca_stash<D, NK, SW>(Kp, Vp, ks, vs);
+            attnx_oca_stash<D, NK>(Kp, Vp, ks, vs);
             __syncthreads();
-            if constexpr (SW) {
-                if (masked) attnx_swp_compute<D, NK, true, true>(p, lds, wi, part, qb, o, mrun);
-                else attnx_swp_compute<D, NK, true, false>(p, lds, wi, part, qb, o, mrun);
-            } else {
-                attnx_oca_compute<D, NK, true>(lds, part, qb, o, mrun);
-            }
+            attnx_oca_compute<D, NK, true>(lds, part, qb, o, mrun);
         }
     }
     const float ltot = __shfl(o[RR], ql + 32 * RH, 64);
@@ -723,25 +618,13 @@ __device__ __forceinline__ void attnx_oca_kernel(const AttnArgs& p, unsigned cha
 ATTNX_OCA_INST(hat_attnx_oca_d24, 24, 192)
 ATTNX_OCA_INST(hat_attnx_oca_d30, 30, 96)
 
-// Shifted-window attention for head_dim 30 in two parts of 128 keys (60 KB of
-// LDS: two blocks per CU), the masked form for the windows of the last row
-// and column of a shifted grid.
-#define ATTNX_SWP_INST(NAME, D, NK)                                                                      \
-    extern "C" __global__ __launch_bounds__(512, 4) void NAME(AttnArgs p)                                \
-    {                                                                                                    \
-        static_assert(AttnXOcaShape<D, NK, true>::LDS_BYTES <= 80 * 1024, "two blocks per CU");          \
-        __shared__ __attribute__((aligned(16))) unsigned char lds[AttnXOcaShape<D, NK, true>::LDS_BYTES]; \
-        attnx_oca_kernel<D, NK, true>(p, lds);                                                           \
-    }
-
-ATTNX_SWP_INST(hat_attnx_swp_d30, 30, 64)
-
-#define ATTNX_INST(NAME, D, OCC)                                                             \
-    extern "C" __global__ __launch_bounds__(512, OCC) void NAME(AttnArgs p)                  \
+#define ATTNX_INST(NAME, D)                                                                  \
+    extern "C" __global__ __launch_bounds__(512, 4) void NAME(AttnArgs p)                    \
     {                                                                                        \
+        static_assert(AttnXShape<D>::LDS_BYTES <= 80 * 1024, "two blocks per CU");           \
         __shared__ __attribute__((aligned(16))) unsigned char lds[AttnXShape<D>::LDS_BYTES]; \
         attnx_item_kernel<D>(p, lds);                                                        \
     }
 
-ATTNX_INST(hat_attnx_sw_d24, 24, 4)
-ATTNX_INST(hat_attnx_sw_d30, 30, 2)
+ATTNX_INST(hat_attnx_sw_d24, 24)
+ATTNX_INST(hat_attnx_sw_d30, 30)

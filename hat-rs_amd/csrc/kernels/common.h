@@ -130,6 +130,60 @@ __device__ __forceinline__ f32x16 mfma6(const u32x4 (&a)[3], const u32x4 (&b)[3]
     return mfma_bf16(a[0], b[0], c);
 }
 
+// ---- split-f16 arithmetic (the F16 MFMA path at fp32 accuracy): an fp32
+// operand x as two f16 parts, x = x0 + x1 + e, x0 the round-to-nearest f16 of x
+// and x1 of what x0 leaves (exact in fp32), so |e| <= 2^-22 |x| while x1 is a
+// normal number and 2^-25 absolute below that (F16 MFMA takes subnormals as they
+// are); a product as a0 b0 + a0 b1 + a1 b0 (the term dropped is below 2^-22
+// |ab|), three MFMAs where the three-part bf16 split takes six. The operands
+// must lie inside f16's range, so the host scales every weight matrix, and the
+// activations it can bound, by powers of two (exact) and takes the scale out
+// after the accumulation. Measured against a double reference (N(0,1)
+// activations, N(0,0.02) weights scaled to 2^14, rms of the error over the rms
+// of the result): K = 144 1.45e-7 (six-product bf16: 1.64e-7, FP32 MFMA
+// 2.14e-7), K = 180 1.61e-7 (1.91e-7, 2.40e-7), K = 288 1.95e-7 (2.46e-7,
+// 3.01e-7): half the accumulator roundings outweigh the wider split. Only very
+// short products are less exact (K = 24: 9.0e-8 against 3.5e-8, FP32 MFMA
+// 9.0e-8).
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// (a, b) = p0 + p1 (+ e), each part a packed pair of f16 (a in the low half):
+// two v_cvt_pk_f16_f32 and two v_fma_mix_f32, 2 instructions a value.
+__device__ __forceinline__ void split2_pk(float a, float b, unsigned& p0, unsigned& p1)
+{
+    const f16x2 h = __builtin_convertvector((f32x2){a, b}, f16x2);
+    const float ra = __builtin_fmaf((float)h[0], -1.0f, a), rb = __builtin_fmaf((float)h[1], -1.0f, b);
+    p0 = __builtin_bit_cast(unsigned, h);
+    p1 = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){ra, rb}, f16x2));
+}
+
+// Eight consecutive fp32 values as two 8-wide f16 parts.
+__device__ __forceinline__ void split2_x8(const float (&v)[8], u32x4 (&out)[2])
+{
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        unsigned p0, p1;
+        split2_pk(v[2 * j], v[2 * j + 1], p0, p1);
+        out[0][j] = p0;
+        out[1][j] = p1;
+    }
+}
+
+// v_mfma_f32_32x32x16_f16 (the layout of mfma_bf16).
+__device__ __forceinline__ f32x16 mfma_f16(u32x4 a, u32x4 b, f32x16 c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+}
+
+__device__ __forceinline__ f32x16 mfma3(const u32x4 (&a)[2], const u32x4 (&b)[2], f32x16 c)
+{
+    c = mfma_f16(a[1], b[0], c);
+    c = mfma_f16(a[0], b[1], c);
+    return mfma_f16(a[0], b[0], c);
+}
+
 // ---- weight chunks for the split-bf16 linears: one 32-k step of up to 192
 // rows as three bf16 planes [rows][32] with swizzled k-groups (ws_mma), packed
 // on the host WC_CHUNK elements apart. A block copies chunk c + 1 into one of

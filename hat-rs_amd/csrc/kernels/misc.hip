@@ -190,3 +190,26 @@ extern "C" __global__ __launch_bounds__(256) void hat_se_gate(SeArgs p)
         p.gate[c] = 1.0f / (1.0f + __expf(-acc));
     }
 }
+
+// The largest finite magnitude of a buffer (hat_op_swmsa's input, which no norm
+// bounds). One HBM pass; the blocks meet in one atomic maximum, whose result
+// does not depend on their order.
+extern "C" __global__ __launch_bounds__(256) void hat_absmax(AbsMaxArgs p)
+{
+    __shared__ float part[4];
+    float m = 0.0f;
+    for (long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4; i < p.n; i += (long)gridDim.x * 1024) {
+        const f32x4 v = *(const f32x4*)(p.x + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float a = fabsf(v[j]);
+            m = a <= 3.402823466e38f ? fmaxf(m, a) : m;  // infinities and NaN left out
+        }
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(p.out, __float_as_uint(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]))));
+}
