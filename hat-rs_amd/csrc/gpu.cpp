@@ -1136,7 +1136,9 @@ void run_attn(hipStream_t s, const float* qkv, const float* table, float* out, c
         launch(s, name, (unsigned)std::min<long>((long)pl.nw() * heads, cus), 1, 1, 512, p);
         return;
     }
-    launch(s, name, (unsigned)pl.nw(), (unsigned)heads, 1, 512, p);
+    // the split-f16 SW kernels run the gate as a column of blocks of its own
+    const unsigned lead = f16 && (p.with_gate || p.with_se) ? 1 : 0;
+    launch(s, name, (unsigned)pl.nw() + lead, (unsigned)heads, 1, 512, p);
 }
 
 void run_ln(hipStream_t s, const float* x, float* y, const float* w, const float* b, long rows, int C)
@@ -1665,7 +1667,7 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
         const bool split = proj.wx && C == 144 && mx != mlpx_.end();  // the split tail runs
         CabGateArgs gate{};
         run_cab(stream_, cab_.at(p), a_.xn, H, W, proj.b, wt_.conv_scale, wt_.squeezed, a_.t1, a_.cab_part,
-                a_.w2g, a_.bias2, a_.gate, (unsigned short*)a_.w2gx, &gate);
+                split ? nullptr : a_.w2g, a_.bias2, a_.gate, (unsigned short*)a_.w2gx, &gate);
         gemm(lin_.at(p + ".attn.qkv"), a_.xn, C, T, a_.qkv, 0, EPI_QKV);
         attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, &gate);
         if (split) {

@@ -182,8 +182,10 @@ struct AttnArgs {
     int owin, opad;      // OCA: unfold window and padding
     int T;
     float qscale;        // head_dim^-0.5 * log2(e)
-    // with_gate: block (0, 0) of the item grid first computes the folded CAB's
-    // gate (hat_cab_gate's work), which the HAB tail after this launch needs
+    // with_gate: the launch also computes the folded CAB's gate (hat_cab_gate's
+    // work), which the HAB tail after it needs: the split-f16 SW kernels in a
+    // block of its own (the grid has one more column, the first), the FP32 ones
+    // in block (0, 0) before its item
     int with_gate;
     CabGateArgs gate;
     // with_se: the same for the unfolded CAB's squeeze-excite gate (C = 180)

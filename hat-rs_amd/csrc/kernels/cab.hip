@@ -230,13 +230,19 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 1) void hat_cab_conv1_t32
 // result does not depend on timing.
 #define CG_WAVES 16
 
-// The gate computation for a block of WAVES waves; lds: CAB_GATE_LDS floats.
-#define CAB_GATE_LDS (CAB_NSUM * CAB_CS + 9 * CAB_CC + CAB_C + 64 + CAB_C)
+// The gate computation for a block of WAVES waves; lds: CAB_GATE_LDS floats. It
+// rides on the attention launch as a block of its own (attnx.hip), so what
+// counts is its latency, which small planes would wait for: conv2's weights
+// are read once, coalesced, under the tile sums' loads, and the split chunks
+// go out eight values at a time.
+#define CAB_GATE_W2 (CAB_C * CAB_CC * 9)
+#define CAB_GATE_LDS (CAB_GATE_W2 + CAB_NSUM * CAB_CS + 9 * CAB_CC + CAB_C + 64 + CAB_C)
 template <int WAVES>
 __device__ __forceinline__ void cab_gate_body(const CabGateArgs& p, float* lds)
 {
     constexpr int NV = CAB_NSUM * CAB_CS;  // 40 sums per tile
-    float* s_sum = lds;
+    float* s_w2 = lds;
+    float* s_sum = s_w2 + CAB_GATE_W2;
     float* s_S = s_sum + NV;
     float* s_mean = s_S + 9 * CAB_CC;
     float* s_z = s_mean + CAB_C;
@@ -244,6 +250,8 @@ __device__ __forceinline__ void cab_gate_body(const CabGateArgs& p, float* lds)
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
 
+    static_assert(CAB_GATE_W2 % 4 == 0, "float4 units");
+    for (int i = tid; i < CAB_GATE_W2 / 4; i += WAVES * 64) ((f32x4*)s_w2)[i] = ((const f32x4*)p.w2)[i];
     // Tile sums: partial is value-major, so a wave reads 64 tiles per load.
     for (int v = wave; v < NV; v += WAVES) {
         const float* src = p.partial + (size_t)v * p.tiles;
@@ -274,7 +282,7 @@ __device__ __forceinline__ void cab_gate_body(const CabGateArgs& p, float* lds)
 #pragma unroll
         for (int ci = 0; ci < CAB_CC; ++ci)
 #pragma unroll
-            for (int tap = 0; tap < 9; ++tap) acc += p.w2[(c * CAB_CC + ci) * 9 + tap] * s_S[tap * CAB_CC + ci];
+            for (int tap = 0; tap < 9; ++tap) acc += s_w2[(c * CAB_CC + ci) * 9 + tap] * s_S[tap * CAB_CC + ci];
         s_mean[c] = p.b2[c] + acc * inv;
     }
     __syncthreads();
@@ -294,70 +302,73 @@ __device__ __forceinline__ void cab_gate_body(const CabGateArgs& p, float* lds)
         p.bias2[c] = p.bproj[c] + (p.cscale * g) * p.b2[c];
     }
     __syncthreads();
-    for (int i = tid; i < CAB_C * CAB_K2; i += WAVES * 64) {
-        const int c = i / CAB_K2, k = i - c * CAB_K2;
-        const int tap = k / CAB_CC, ci = k - tap * CAB_CC;
-        float v = 0.0f;
-        if (tap < 9) v = (p.cscale * s_gate[c]) * p.w2[(c * CAB_CC + ci) * 9 + tap];
-        p.w2g[i] = v;
-    }
-    // the same weights as hat_projx_cab's two weight chunks: [s][plane][c][32],
-    // row c's k-group g at slot ws_slot(c, g), k = 32 s + j, zeros elsewhere
+    // the gated weights for the FP32 tail, where it runs
+    if (p.w2g)
+        for (int i = tid; i < CAB_C * CAB_K2; i += WAVES * 64) {
+            const int c = i / CAB_K2, k = i - c * CAB_K2;
+            const int tap = k / CAB_CC, ci = k - tap * CAB_CC;
+            p.w2g[i] = tap < 9 ? (p.cscale * s_gate[c]) * s_w2[(c * CAB_CC + ci) * 9 + tap] : 0.0f;
+        }
+    // the same weights as the split tail's two weight chunks: [s][plane][c][32],
+    // row c's k-group g at slot ws_slot(c, g), k = 32 s + j, zeros from k = 54;
+    // one k-group (8 values, 16 bytes a plane) at a time
     if (p.w2gx) {
         constexpr int PLANE = CAB_C * 32;
-        for (int i = tid; i < 2 * WC_CHUNK; i += WAVES * 64) {
-            const int s = i / WC_CHUNK, r = i - s * WC_CHUNK;
-            unsigned short h = 0;
-            if (r < 3 * PLANE) {
-                const int pl = r / PLANE, c = (r - pl * PLANE) / 32, pos = r - pl * PLANE - c * 32;
-                const int j = (ws_slot(c, pos >> 3) << 3) | (pos & 7);
-                const int k = 32 * s + j, tap = k / CAB_CC, ci = k - tap * CAB_CC;
-                const float v = tap < 9 ? (p.cscale * s_gate[c]) * p.w2[(c * CAB_CC + ci) * 9 + tap] : 0.0f;
-                h = split3_part(v, pl);
+        for (int u = tid; u < 2 * CAB_C * 4; u += WAVES * 64) {
+            const int s = u / (CAB_C * 4), c = (u >> 2) - s * CAB_C, g = u & 3;
+            const float sc = p.cscale * s_gate[c];
+            float f[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int k = 32 * s + 8 * g + j, tap = k / CAB_CC, ci = k - tap * CAB_CC;
+                f[j] = tap < 9 ? sc * s_w2[(c * CAB_CC + ci) * 9 + tap] : 0.0f;
             }
-            p.w2gx[i] = h;
+            u32x4 parts[3];
+            split3_x8(f, parts);
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl)
+                *(u32x4*)(p.w2gx + (size_t)s * WC_CHUNK + pl * PLANE + c * 32 + ws_slot(c, g) * 8) = parts[pl];
         }
     }
 }
 
 // The unfolded CAB's gate (the C = 180 family; hat_arch.py:40-55, cpu.rs:
 // 940-955) for a block of WAVES waves, straight from the conv2 partial column
-// sums: wave w adds rows w, w + WAVES, ... (its lanes over the columns), the
-// waves' sums are added in wave order through LDS, then mean, squeeze + ReLU,
-// excite + sigmoid. lds: SE_GATE_LDS floats.
-#define SE_GATE_LDS (8 * 192 + 192 + 64)
+// sums: thread (r, q) adds rows r, r + R, ... of the four columns of quad q,
+// eight loads in flight (one row a wave and two loads in flight took 330 us for
+// the 2048 rows of a 512 x 512 plane, longer than the attention launch it rides
+// on), the R sums of a column are added in order through LDS, then mean,
+// squeeze + ReLU, excite + sigmoid. C <= 192, a multiple of 4. lds: SE_GATE_LDS
+// floats.
+#define SE_GATE_ROWS 16
+#define SE_GATE_LDS (SE_GATE_ROWS * 192 + 192 + 64)
 template <int WAVES>
 __device__ __forceinline__ void se_gate_body(const SeArgs& p, float* lds)
 {
-    static_assert(WAVES <= 8, "the LDS holds eight waves' sums");
-    float* s_part = lds;              // [WAVES][192]
-    float* s_mean = s_part + 8 * 192;  // [192]
-    float* s_sq = s_mean + 192;        // [64]
+    float* s_part = lds;                          // [R][192]
+    float* s_mean = s_part + SE_GATE_ROWS * 192;  // [192]
+    float* s_sq = s_mean + 192;                   // [64]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    for (int c0 = 0; c0 < p.C; c0 += 64) {
-        const int c = c0 + lane;
-        float a0 = 0.0f, a1 = 0.0f;
-        if (c < p.C) {
-            int b = wave;
-            for (; b + WAVES < p.nblk; b += 2 * WAVES) {
-                a0 += p.partial[(size_t)b * p.co_stride + c];
-                a1 += p.partial[(size_t)(b + WAVES) * p.co_stride + c];
-            }
-            if (b < p.nblk) a0 += p.partial[(size_t)b * p.co_stride + c];
-            s_part[wave * 192 + c] = a0 + a1;
-        }
+    const int nq = p.C / 4, R = min(WAVES * 64 / nq, SE_GATE_ROWS);
+    const int r = tid / nq, q = tid - r * nq;
+    if (r < R) {
+        f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+        for (int b = r; b < p.nblk; b += R) a += *(const f32x4*)(p.partial + (size_t)b * p.co_stride + 4 * q);
+        *(f32x4*)(s_part + r * 192 + 4 * q) = a;
     }
     __syncthreads();
     for (int c = tid; c < p.C; c += WAVES * 64) {
         float acc = 0.0f;
-        for (int w = 0; w < WAVES; ++w) acc += s_part[w * 192 + c];
+        for (int w = 0; w < R; ++w) acc += s_part[w * 192 + c];
         s_mean[c] = acc / p.count;
     }
     __syncthreads();
-    for (int j = tid; j < p.sq; j += WAVES * 64) {
-        float acc = p.b1[j];
-        for (int c = 0; c < p.C; ++c) acc += s_mean[c] * p.w1[(size_t)j * p.C + c];
-        s_sq[j] = acc < 0.0f ? 0.0f : acc;
+    for (int j = wave; j < p.sq; j += WAVES) {
+        float acc = 0.0f;
+        for (int c = lane; c < p.C; c += 64) acc += s_mean[c] * p.w1[(size_t)j * p.C + c];
+        acc = wave_sum(acc) + p.b1[j];
+        if (lane == 0) s_sq[j] = acc < 0.0f ? 0.0f : acc;
     }
     __syncthreads();
     for (int c = tid; c < p.C; c += WAVES * 64) {
@@ -369,6 +380,6 @@ __device__ __forceinline__ void se_gate_body(const SeArgs& p, float* lds)
 
 extern "C" __global__ __launch_bounds__(CG_WAVES * 64) void hat_cab_gate(CabGateArgs p)
 {
-    __shared__ float lds[CAB_GATE_LDS];
+    __shared__ __attribute__((aligned(16))) float lds[CAB_GATE_LDS];
     cab_gate_body<CG_WAVES>(p, lds);
 }
