@@ -110,51 +110,108 @@ std::vector<unsigned short> pack_linear_x(const float* w, int N, int K)
     return out;
 }
 
-std::vector<unsigned short> pack_linear_ws(const float* w, const float* bias, int N, int K)
+// float -> f16, round to nearest even, subnormals kept, past the range infinite
+static inline unsigned short f16_rne(float x)
 {
-    // C = 144: slices of 144 rows (q, k, v), five k-steps; C = 180: slices of
-    // 90 rows (three heads of 30) padded to 96, six k-steps
+    uint32_t u;
+    memcpy(&u, &x, 4);
+    const uint32_t sign = (u >> 16) & 0x8000u;
+    u &= 0x7fffffffu;
+    if (u >= 0x477ff000u)  // rounds to 2^16 or more, infinite or NaN
+        return (unsigned short)(sign | (u > 0x7f800000u ? 0x7e00u : 0x7c00u));
+    if (u < 0x38800000u) {  // below 2^-14: units of 2^-24, rounded by adding 1.5 * 2^23 of them
+        float a;
+        memcpy(&a, &u, 4);
+        const float r = a * 16777216.0f + 12582912.0f;
+        uint32_t v;
+        memcpy(&v, &r, 4);
+        return (unsigned short)(sign | (v - 0x4b400000u));
+    }
+    u += 0xfffu + ((u >> 13) & 1u);
+    return (unsigned short)(sign | ((u - 0x38000000u) >> 13));
+}
+static inline float f16_float(unsigned short h)
+{
+    const uint32_t e = (h >> 10) & 31u, m = h & 1023u;
+    float v;
+    if (e == 0) {
+        v = (float)m * 5.9604644775390625e-8f;  // 2^-24
+    } else {
+        const uint32_t u = e == 31 ? 0x7f800000u | (m << 13) : ((e + 112u) << 23) | (m << 13);
+        memcpy(&v, &u, 4);
+    }
+    return h & 0x8000u ? -v : v;
+}
+
+// x = h0 + h1 (+ at most 2^-22 |x|), each part the round-to-nearest f16 of what
+// the one before leaves.
+static void split2_f16(float x, unsigned short* h0, unsigned short* h1)
+{
+    const unsigned short a = f16_rne(x), b = f16_rne(x - f16_float(a));
+    *h0 = a;
+    *h1 = b;
+}
+
+// value(r, kk), r < rows, kk < 32: one 32-k step as two f16 planes [rows][32],
+// row r's k-group g at slot ws_slot(r, g).
+template <typename F>
+static void split2_step(int rows, F value, unsigned short* dst)
+{
+    for (int r = 0; r < rows; ++r)
+        for (int kk = 0; kk < 32; ++kk) {
+            unsigned short* d = dst + (size_t)r * 32 + hatk::ws_slot(r, kk / 8) * 8 + kk % 8;
+            split2_f16(value(r, kk), d, d + (size_t)rows * 32);
+        }
+}
+
+// value(r, kk), kk < 16: the packed last step of a K = 144 linear (k = 128 + kk;
+// common.h half_operand): lane group g's slots j < 4 and 4 + j hold k = 128 + 4 g
+// + j, the planes (a0 | a0) and (a1 | a1).
+template <typename F>
+static void split2_half_step(int rows, F value, unsigned short* dst)
+{
+    for (int r = 0; r < rows; ++r)
+        for (int kk = 0; kk < 16; ++kk) {
+            unsigned short* d = dst + (size_t)r * 32 + hatk::ws_slot(r, kk / 4) * 8 + kk % 4;
+            split2_f16(value(r, kk), d, d + (size_t)rows * 32);
+            d[4] = d[0];
+            d[(size_t)rows * 32 + 4] = d[(size_t)rows * 32];
+        }
+}
+
+std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const float (&ws)[3])
+{
+    // three slices, q, k and v: C = 144 of 144 rows, five k-steps; C = 180 of
+    // 180 rows padded to 192, six k-steps
     if (!((K == 144 && N == 432) || (K == 180 && N == 540)))
         throw Error("pack_linear_ws: needs the qkv shapes K = 144, N = 432 or K = 180, N = 540");
-    const int real = K == 144 ? 144 : 90, rows = K == 144 ? 144 : 96, ks_n = (K + 32) / 32;
-    const size_t chunk = (size_t)3 * rows * 32;
+    const int real = K == 144 ? 144 : 180, rows = K == 144 ? 144 : 192, ks_n = (K + 31) / 32;
+    const size_t chunk = (size_t)2 * rows * 32;
     std::vector<unsigned short> out((size_t)(N / real) * ks_n * chunk, 0);
-    if (K == 144) {
-        // four whole k-steps, then k = 128 .. 143 packed (split_half_step);
-        // the bias is the accumulators' start value (hat_gemmx_qkv reads it)
-        for (int sl = 0; sl < N / real; ++sl) {
-            for (int n = 0; n < real; ++n)
-                for (int k = 0; k < 128; ++k) {
-                    const float x = w[((size_t)sl * real + n) * K + k];
-                    const unsigned short h0 = bf16_rne(x);
-                    const float r1 = x - bf16_float(h0);
-                    const unsigned short h1 = bf16_rne(r1);
-                    const unsigned short h2 = bf16_rne(r1 - bf16_float(h1));
-                    const int s = k / 32, g = (k % 32) / 8, j = k % 8;
-                    unsigned short* d = &out[((size_t)sl * ks_n + s) * chunk + (size_t)n * 32 + hatk::ws_slot(n, g) * 8 + j];
-                    d[0] = h0;
-                    d[(size_t)rows * 32] = h1;
-                    d[(size_t)2 * rows * 32] = h2;
-                }
-            split_half_step(w + (size_t)sl * real * K, real, K, &out[((size_t)sl * ks_n + 4) * chunk]);
+    for (int sl = 0; sl < N / real; ++sl) {
+        const float f = ws[sl * real / (N / 3)];
+        for (int s = 0; s < ks_n; ++s) {
+            auto value = [&](int r, int kk) {
+                const int k = 32 * s + kk;
+                return r < real && k < K ? w[((size_t)sl * real + r) * K + k] * f : 0.0f;
+            };
+            unsigned short* dst = &out[((size_t)sl * ks_n + s) * chunk];
+            if (K == 144 && s == 4) split2_half_step(rows, value, dst);
+            else split2_step(rows, value, dst);
         }
-        return out;
     }
-    for (int n = 0; n < N; ++n)
-        for (int k = 0; k <= K; ++k) {
-            if (k == K && !bias) break;
-            const float x = k < K ? w[(size_t)n * K + k] : bias[n];  // k = K: the bias column
-            const unsigned short h0 = bf16_rne(x);
-            const float r1 = x - bf16_float(h0);
-            const unsigned short h1 = bf16_rne(r1);
-            const unsigned short h2 = bf16_rne(r1 - bf16_float(h1));
-            const int r = n % real, s = k / 32, g = (k % 32) / 8, j = k % 8;
-            unsigned short* d = &out[((size_t)(n / real) * ks_n + s) * chunk + (size_t)r * 32 + hatk::ws_slot(r, g) * 8 + j];
-            d[0] = h0;
-            d[(size_t)rows * 32] = h1;
-            d[(size_t)2 * rows * 32] = h2;
-        }
     return out;
+}
+
+double abs_max(const float* w, size_t n)
+{
+    double m = 0.0;
+    for (size_t i = 0; i < n; ++i) {
+        const double a = std::fabs((double)w[i]);
+        if (std::isnan(a)) return a;
+        m = std::max(m, a);
+    }
+    return m;
 }
 
 // fc1 output tile t, row 4g + r (lane group g, register r) -> hidden unit
@@ -573,17 +630,19 @@ void run_gemm(hipStream_t s, const DevLinear& L, const float* a, int lda, long M
     p.cscale = cscale;
     p.eps = 1e-5f;
     if (epi == EPI_QKV && L.wx && L.K == 144 && L.N == 432 && heads == 6 && hdim == 24 && lda == 144) {
-        // split-bf16 qkv (gemmx.hip): weight-stationary, groups of three blocks
+        // split-f16 qkv (gemmx.hip): weight-stationary, groups of three blocks
         static const int cus = std::max(1, Runtime::get().cu_count());
         p.w = (const float*)L.wx;
+        memcpy(p.oscale, L.oscale, sizeof p.oscale);
         launch(s, "hat_gemmx_qkv", (unsigned)(3 * gemmx_qkv_groups(cus, 3)), 1, 1, GX_THREADS, p);
         return;
     }
     if (epi == EPI_QKV && L.wx && L.K == 180 && L.N == 540 && heads == 6 && hdim == 30 && lda == 180) {
-        // the same for C = 180: groups of six blocks (96-column slices)
+        // the same for C = 180
         static const int cus = std::max(1, Runtime::get().cu_count());
         p.w = (const float*)L.wx;
-        launch(s, "hat_gemmx_qkv180", (unsigned)(6 * gemmx_qkv_groups(cus, 6)), 1, 1, GX_THREADS, p);
+        memcpy(p.oscale, L.oscale, sizeof p.oscale);
+        launch(s, "hat_gemmx_qkv180", (unsigned)(3 * gemmx_qkv_groups(cus, 3)), 1, 1, GX_THREADS, p);
         return;
     }
     int wbn = 0;
@@ -1208,7 +1267,20 @@ void GpuBackend::upload_raw(const std::string& name)
     raw_[name] = upload(wt_.t(name), ti.numel());
 }
 
-void GpuBackend::upload_linear(const std::string& name, const std::vector<float>* row_scale, float all, bool split)
+// The qkv weights for hat_gemmx_qkv*: each of q, k and v scaled into f16's range
+// (w: the linear's own weights, out[3] the results' factors, in the inverse of
+// the input's scale); sets oscale.
+static std::vector<unsigned short> split_qkv(const float* w, int N, int K, const float* out, float in, float* oscale)
+{
+    float ws[3];
+    for (int i = 0; i < 3; ++i) {
+        ws[i] = f16_scale(abs_max(w + (size_t)i * (N / 3) * K, (size_t)(N / 3) * K));
+        oscale[i] = in * out[i] / ws[i];
+    }
+    return pack_linear_ws(w, N, K, ws);
+}
+
+void GpuBackend::upload_linear(const std::string& name, const float* out, float in)
 {
     const TensorInfo& ti = wt_.info(name + ".weight");
     DevLinear L;
@@ -1216,35 +1288,53 @@ void GpuBackend::upload_linear(const std::string& name, const std::vector<float>
     L.K = (int)ti.shape[1];
     const float *w = wt_.t(name + ".weight"), *bias = wt_.t(name + ".bias");
     std::vector<float> ws, bs;
-    if (row_scale || all != 1.0f) {
+    if (out || in != 1.0f) {
         ws.assign(w, w + (size_t)L.N * L.K);
         bs.assign(bias, bias + L.N);
         for (int n = 0; n < L.N; ++n) {
-            const float f = row_scale ? (*row_scale)[n] : 1.0f;
-            for (int k = 0; k < L.K; ++k) ws[(size_t)n * L.K + k] *= f * all;
+            const float f = out ? out[n / (L.N / 3)] : 1.0f;
+            for (int k = 0; k < L.K; ++k) ws[(size_t)n * L.K + k] *= f * in;
             bs[n] *= f;
         }
-        w = ws.data();
-        bias = bs.data();
     }
-    std::vector<float> pk = pack_linear(w, L.N, L.K, &L.Kp);
+    const float *sw = ws.empty() ? w : ws.data(), *sb = bs.empty() ? bias : bs.data();
+    std::vector<float> pk = pack_linear(sw, L.N, L.K, &L.Kp);
     L.w = upload(pk.data(), pk.size());
-    L.b = upload(bias, L.N);
+    L.b = upload(sb, L.N);
     auto ends = [&](const char* t) {
         const size_t n = strlen(t);
         return name.size() >= n && name.compare(name.size() - n, n, t) == 0;
     };
-    if (split && L.K == 180 && L.N == 180 && ends("proj")) {
+    if (L.K == 180 && L.N == 180 && ends("proj")) {
         // the C = 180 projection tails (hat_projx180*)
-        std::vector<unsigned short> x = pack_linear_x180(w);
+        std::vector<unsigned short> x = pack_linear_x180(sw);
         L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
     }
-    if (split && ((L.K == 180 && L.N == 540 && ends(".qkv")) || (L.K == 144 && ((L.N == 432 && ends(".qkv")) || (L.N == 144 && ends("proj")))))) {
-        // qkv: the weight-stationary layout of hat_gemmx_qkv; proj: streamed chunks (tailx)
-        std::vector<unsigned short> x = ends(".qkv") ? pack_linear_ws(w, bias, L.N, L.K) : pack_linear_x(w, L.N, L.K);
+    if (L.K == 144 && L.N == 144 && ends("proj")) {
+        // streamed chunks (tailx)
+        std::vector<unsigned short> x = pack_linear_x(sw, L.N, L.K);
+        L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
+    }
+    if (out && ((L.K == 180 && L.N == 540) || (L.K == 144 && L.N == 432))) {
+        // qkv: the weight-stationary layout of hat_gemmx_qkv
+        std::vector<unsigned short> x = split_qkv(w, L.N, L.K, out, in, L.oscale);
         L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
     }
     lin_[name] = L;
+}
+
+void GpuBackend::upload_norm(const std::string& name)
+{
+    const int C = wt_.embed;
+    const float *w = wt_.t(name + ".weight"), *b = wt_.t(name + ".bias");
+    // the widths with split-f16 kernels behind their norms
+    const float s = C == 144 || C == 180 ? f16_scale(ln_bound(w, b, C)) : 1.0f;
+    std::vector<float> v(C);
+    for (int i = 0; i < C; ++i) v[i] = w[i] * s;
+    raw_[name + ".weight"] = upload(v.data(), C);
+    for (int i = 0; i < C; ++i) v[i] = b[i] * s;
+    raw_[name + ".bias"] = upload(v.data(), C);
+    norm_scale_[name] = s;
 }
 
 void GpuBackend::upload_attn(const std::string& qkv, const std::string& proj, const std::string& ln,
@@ -1255,9 +1345,8 @@ void GpuBackend::upload_attn(const std::string& qkv, const std::string& proj, co
                 *lb = wt_.t(ln + ".bias");
     const QkvScale s = qkv_scale(ln_linear_bound(w, b, lw, lb, 0, C, C), ln_linear_bound(w, b, lw, lb, C, 2 * C, C),
                                  ln_linear_bound(w, b, lw, lb, 2 * C, 3 * C, C), wt_.head_dim);
-    std::vector<float> rows((size_t)3 * C);
-    for (int n = 0; n < 3 * C; ++n) rows[n] = n < C ? s.q : n < 2 * C ? s.k : s.v;
-    upload_linear(qkv, &rows);
+    const float out[3] = {s.q, s.k, s.v};
+    upload_linear(qkv, out, 1.0f / norm_scale_.at(ln));
     upload_linear(proj, nullptr, 1.0f / s.v);
     attn_f16_[table] = s.ok;
 }
@@ -1293,7 +1382,7 @@ void GpuBackend::upload_mlpx(const std::string& name)
     mlpx_[name] = m;
 }
 
-void GpuBackend::upload_conv(const std::string& name, int r)
+void GpuBackend::upload_conv(const std::string& name, int r, float in)
 {
     const TensorInfo& ti = wt_.info(name + ".weight");
     DevConv C;
@@ -1301,12 +1390,18 @@ void GpuBackend::upload_conv(const std::string& name, int r)
     C.CI = (int)ti.shape[1];
     C.r = r;
     std::vector<float> bias;
-    std::vector<float> pk = pack_conv(wt_.t(name + ".weight"), wt_.t(name + ".bias"), C.CO, C.CI, r,
-                                      &bias, &C.CIp, &C.COp);
+    const float* w = wt_.t(name + ".weight");
+    std::vector<float> ws;
+    if (in != 1.0f) {
+        ws.assign(w, w + ti.numel());
+        for (float& x : ws) x *= in;
+        w = ws.data();
+    }
+    std::vector<float> pk = pack_conv(w, wt_.t(name + ".bias"), C.CO, C.CI, r, &bias, &C.CIp, &C.COp);
     C.w = upload(pk.data(), pk.size());
     C.b = upload(bias.data(), bias.size());
     if (wino_conv(C.CO, C.CI, r)) {
-        std::vector<unsigned short> wu = pack_wino(wt_.t(name + ".weight"), C.CO, C.CI, r);
+        std::vector<unsigned short> wu = pack_wino(w, C.CO, C.CI, r);
         C.wu = (unsigned short*)upload_bytes(wu.data(), wu.size() * sizeof(unsigned short));
     }
     conv_[name] = C;
@@ -1356,8 +1451,8 @@ void GpuBackend::upload_all()
         const std::string L = "layers." + std::to_string(s);
         for (int b = 0; b < wt.depths[s]; ++b) {
             const std::string p = L + ".residual_group.blocks." + std::to_string(b);
-            for (const char* n : {".norm1.weight", ".norm1.bias", ".norm2.weight", ".norm2.bias",
-                                  ".attn.relative_position_bias_table",
+            upload_norm(p + ".norm1");
+            for (const char* n : {".norm2.weight", ".norm2.bias", ".attn.relative_position_bias_table",
                                   ".conv_block.cab.3.attention.1.weight",
                                   ".conv_block.cab.3.attention.1.bias",
                                   ".conv_block.cab.3.attention.3.weight",
@@ -1367,10 +1462,13 @@ void GpuBackend::upload_all()
             upload_linear(p + ".mlp.fc1");
             upload_linear(p + ".mlp.fc2");
             upload_mlpx(p + ".mlp");
+            const float xin = 1.0f / norm_scale_.at(p + ".norm1");
             if (cab_fold_) {
                 const std::string c = p + ".conv_block.cab.";
                 for (const char* n : {"0.bias", "2.weight", "2.bias"}) upload_raw(c + n);
-                std::vector<unsigned short> w1 = pack_cab_conv1(wt.t(c + "0.weight"));
+                std::vector<float> w0(wt.t(c + "0.weight"), wt.t(c + "0.weight") + wt.info(c + "0.weight").numel());
+                for (float& x : w0) x *= xin;
+                std::vector<unsigned short> w1 = pack_cab_conv1(w0.data());
                 DevCab cb;
                 cb.w1 = (unsigned short*)upload_bytes(w1.data(), w1.size() * sizeof(unsigned short));
                 cb.b1 = raw_.at(c + "0.bias");
@@ -1382,13 +1480,13 @@ void GpuBackend::upload_all()
                 cb.bb = raw_.at(c + "3.attention.3.bias");
                 cab_[p] = cb;
             } else {
-                upload_conv(p + ".conv_block.cab.0");
+                upload_conv(p + ".conv_block.cab.0", 0, xin);
                 upload_conv(p + ".conv_block.cab.2");
             }
         }
         const std::string p = L + ".residual_group.overlap_attn";
-        for (const char* n : {".norm1.weight", ".norm1.bias", ".norm2.weight", ".norm2.bias",
-                              ".relative_position_bias_table"})
+        upload_norm(p + ".norm1");
+        for (const char* n : {".norm2.weight", ".norm2.bias", ".relative_position_bias_table"})
             upload_raw(p + n);
         upload_attn(p + ".qkv", p + ".proj", p + ".norm1", p + ".relative_position_bias_table");
         upload_linear(p + ".mlp.fc1");
@@ -2309,22 +2407,21 @@ struct OpLinear {
                 for (int k = 0; k < K; ++k) ws[(size_t)n * K + k] *= f * in;
                 bs[n] *= f;
             }
-            wt = ws.data();
-            bias = bs.data();
-            ib = ar.keep(bs);
+            ib = ar.keep(std::move(bs));
         } else {
             ib = ar.add(N, bias);
         }
+        const float* sw = ws.empty() ? wt : ws.data();
         std::vector<unsigned short> xs;
         if (sp == kQkv && ((N == 432 && K == 144) || (N == 540 && K == 180)))
-            xs = pack_linear_ws(wt, bias, N, K);
+            xs = split_qkv(wt, N, K, out, in, L.oscale);
         else if (sp == kProj && N == 144 && K == 144)
-            xs = pack_linear_x(wt, N, K);
+            xs = pack_linear_x(sw, N, K);
         else if (sp == kProj && N == 180 && K == 180)
-            xs = pack_linear_x180(wt);
+            xs = pack_linear_x180(sw);
         L.Kp = (K + 15) / 16 * 16;
         if ((split = !xs.empty())) ix = ar.keep(std::move(xs));
-        else if ((fp32 = sp != kBias)) iw = ar.keep(pack_linear(wt, N, K, &L.Kp));
+        else if ((fp32 = sp != kBias)) iw = ar.keep(pack_linear(sw, N, K, &L.Kp));
     }
     void bind(const OpArena& ar)
     {
@@ -2431,11 +2528,19 @@ void op_swmsa(const float* x, float* out, int hp, int wp, int c, int heads, int 
                                       op_linear_bound(qkv_w, qkv_b, c, 2 * c, c, mx),
                                       op_linear_bound(qkv_w, qkv_b, 2 * c, 3 * c, c, mx), D);
         const float osc[3] = {sc.q, sc.k, sc.v};
+        // x itself goes through the split: into f16's range, unless it lies there
+        // already with its ordinary values clear of the subnormals
+        float sx = 1.0f;
+        if ((mx < 4.0f || mx > 32768.0f) && (c == 144 || c == 180)) {
+            sx = f16_scale(mx);
+            ScaleArgs sa{dx, sx, (long)(T * c)};
+            if (sx != 1.0f) launch(s, "hat_scale", (unsigned)std::min<size_t>((T * c + 4095) / 4096, 512), 1, 1, 256, sa);
+        }
         // qkv as in the forward; the projection here has no residual, a form the
         // forward never runs, so it stays on the FP32 store epilogue
         OpArena wr;
         const size_t itab = wr.add(961 * (size_t)heads, table);
-        OpLinear qkv(wr, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc),
+        OpLinear qkv(wr, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc, 1.0f / sx),
             proj(wr, proj_w, proj_b, c, c, OpLinear::kNone, nullptr, 1.0f / sc.v);
         wr.commit();
         qkv.bind(wr);
@@ -2489,10 +2594,14 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
     const size_t T = (size_t)hp * wp, hid = (size_t)c * mlp_ratio;
     hipStream_t s = nullptr;  // the null stream, as in op_swmsa
     {
+        // norm1 into f16's range, as GpuBackend::upload_norm
+        const float s1 = c == 144 || c == 180 ? f16_scale(ln_bound(n1w, n1b, c)) : 1.0f;
+        std::vector<float> n1(2 * (size_t)c);
+        for (int i = 0; i < c; ++i) n1[i] = n1w[i] * s1, n1[c + i] = n1b[i] * s1;
         OpArena ar;
         const size_t ix = ar.add(T * c, x), iwork = ar.add(T * c), ixn = ar.add(T * c), iq = ar.add(3 * T * c),
-                     iao = ar.add(T * c), itab = ar.add(1521 * (size_t)heads, table), i1w = ar.add(c, n1w),
-                     i1b = ar.add(c, n1b), i2w = ar.add(c, n2w), i2b = ar.add(c, n2b);
+                     iao = ar.add(T * c), itab = ar.add(1521 * (size_t)heads, table), i1w = ar.add(c, n1.data()),
+                     i1b = ar.add(c, n1.data() + c), i2w = ar.add(c, n2w), i2b = ar.add(c, n2b);
         OpMlpX mx(ar, fc1_w, fc1_b, fc2_w, c, hid);
         const QkvScale sc = qkv_scale(ln_linear_bound(qkv_w, qkv_b, n1w, n1b, 0, c, c),
                                       ln_linear_bound(qkv_w, qkv_b, n1w, n1b, c, 2 * c, c),
@@ -2500,7 +2609,7 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
         const float osc[3] = {sc.q, sc.k, sc.v};
         // the split tails read only fc2's bias of these two
         const OpLinear::Split mlp = mx.fused ? OpLinear::kBias : OpLinear::kNone;
-        OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc),
+        OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc, 1.0f / s1),
             proj(ar, proj_w, proj_b, c, c, mx.fused ? OpLinear::kProj : OpLinear::kNone, nullptr, 1.0f / sc.v),
             fc1(ar, fc1_w, fc1_b, (int)hid, c, mlp), fc2(ar, fc2_w, fc2_b, c, (int)hid, mlp);
         const size_t ih = ar.add(mx.fused || mlp_fused(fc1.L, fc2.L) ? 1 : T * hid);

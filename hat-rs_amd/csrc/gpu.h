@@ -30,6 +30,8 @@ struct DevLinear {
     // (qkv: pack_linear_ws; projection: pack_linear_x, pack_linear_x180), or
     // null where the FP32 kernels run.
     unsigned short* wx = nullptr;
+    // qkv: what the split-f16 kernel multiplies q, k and v by (GemmArgs::oscale)
+    float oscale[3] = {1.0f, 1.0f, 1.0f};
     int N = 0, K = 0, Kp = 0;
 };
 
@@ -97,13 +99,14 @@ std::vector<float> pack_linear(const float* w, int N, int K, int* Kp);
 // leave; the fifth step (k = 128..143) packed, two parts per MFMA operand
 // (split_half_step). The tails add the bias in fp32.
 std::vector<unsigned short> pack_linear_x(const float* w, int N, int K);
-// The same split for hat_gemmx_qkv's weight-stationary slices: per slice
-// (144 rows at K = 144, 96 at 180) five or six chunks of three planes
-// [rows][32], each row's 16-byte k-groups swizzled (ws_slot), WS_CHUNK
-// elements apart. K = 144: the fifth step packed as in pack_linear_x, the bias
-// not in the chunks (the kernel starts its accumulators from it); K = 180: the
-// bias at k = 180.
-std::vector<unsigned short> pack_linear_ws(const float* w, const float* bias, int N, int K);
+// hat_gemmx_qkv's weight-stationary slices: per slice (144 rows at K = 144, 192
+// at 180) five or six chunks of two f16 planes [rows][32], each row's 16-byte
+// k-groups swizzled (ws_slot), WS_CHUNK elements apart; K = 144's fifth step
+// packed (split2_half_step). w = p0 + p1, each part the round-to-nearest f16 of
+// what the one before leaves; q's, k's and v's rows times ws[0..2] first.
+std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const float (&ws)[3]);
+// The largest |w[i]|, i < n (NaN if there is one).
+double abs_max(const float* w, size_t n);
 // The C = 144 MLP (fc1 [288][144] + b1, fc2 [144][288]) for hat_mlpx: per
 // third of the hidden layer eight weight chunks - five of fc1's 96 rows (b1
 // as their column k = 144), then three of fc2 on those units - with fc1's
@@ -253,14 +256,17 @@ private:
     float* upload(const float* src, size_t n);
     void* upload_bytes(const void* src, size_t bytes);
     void upload_raw(const std::string& name);
-    // row_scale (if set): each weight row's and bias entry's factor; all: every
-    // weight's (the bias is not touched). split: whether the split copy is made.
-    void upload_linear(const std::string& name, const std::vector<float>* row_scale = nullptr, float all = 1.0f,
-                       bool split = true);
+    // out[3]: the factors of a qkv's q, k and v outputs (weights and bias), or
+    // null; in: the factor of every weight (the inverse of its input's scale).
+    void upload_linear(const std::string& name, const float* out = nullptr, float in = 1.0f);
+    // A norm whose output feeds split-f16 kernels: its weight and bias times the
+    // power of two that takes every row it can produce to f16's range.
+    void upload_norm(const std::string& name);
+    std::map<std::string, float> norm_scale_;
     // An attention's qkv and projection behind norm `ln`, scaled for the
     // split-f16 attention where the bounds allow it (attn_f16_ of its table).
     void upload_attn(const std::string& qkv, const std::string& proj, const std::string& ln, const std::string& table);
-    void upload_conv(const std::string& name, int r = 0);
+    void upload_conv(const std::string& name, int r = 0, float in = 1.0f);  // in: as upload_linear's
     void upload_mlpx(const std::string& name);
     void ensure_plan(int h, int w);
     void free_plan();

@@ -31,7 +31,7 @@ const std::vector<std::string>& required_kernels()
         "hat_cab_gate",        "hat_convw_n9_store_ln", "hat_convw_n9_resid_ln", "hat_convwino_resid", "hat_convwino_n4_store", "hat_convwino_n8_shuffle", "hat_convwino_resid180", "hat_convwino_n4_store180",
         "hat_convwino_cab1_180", "hat_convwino_cab2_180", "hat_convw_n9_resid",
         "hat_convw_n4_store",  "hat_convw_n8_shuffle", "hat_convw_n6_resid", "hat_convw_n6_colsum", "hat_hab_tail", "hat_ocab_tail",
-        "hat_layernorm",       "hat_pre",  "hat_absmax",             "hat_colsum_reduce",  "hat_se_gate",
+        "hat_layernorm",       "hat_pre",  "hat_absmax", "hat_scale",             "hat_colsum_reduce",  "hat_se_gate",
         "hat_copy",
     };
     return k;

@@ -70,6 +70,9 @@ struct GemmArgs {
     const float* t1;     // [H*W][CAB_CS]
     const float* w2g;    // [N][CAB_K2]
     int H, W;
+    // hat_gemmx_qkv*: what takes the operands' scales out of q, k and v (the
+    // bias is in the result's scale already)
+    float oscale[3];
 };
 
 // CAB of the compress-to-6 family (HAT-S: 144 -> 6 -> 144), restated by the
@@ -278,15 +281,15 @@ constexpr int ws_slot(int r, int g) { return g ^ ((r >> 1) & 3); }
 constexpr int wx_tiles(int M) { return (M + WX_ROWS - 1) / WX_ROWS; }
 
 // The qkv linear (hat_gemmx_qkv, hat_gemmx_qkv180) keeps one column slice in
-// LDS for the whole launch: per 32-k step three bf16 planes [rows][32],
-// unpadded, each row's four 16-byte k-groups stored at slot ws_slot(row, g)
-// (so that reads of one k-group down the rows are free of bank conflicts),
-// WS_CHUNK elements apart. C = 144: three slices (q, k, v) of 144 rows, five
-// k-steps; C = 180: six slices of 96 rows (three heads of 30, rows 90..95
-// zero), six k-steps (WS_CHUNK180). Groups of NS blocks (one per slice, on one
-// XCD) walk the same 32-token subtiles: gemmx_qkv_groups(cus, NS) groups.
-#define WS_CHUNK (3 * 144 * 32)
-#define WS_CHUNK180 (3 * 96 * 32)
+// LDS for the whole launch: per 32-k step two f16 planes [rows][32], unpadded,
+// each row's four 16-byte k-groups stored at slot ws_slot(row, g) (so that reads
+// of one k-group down the rows are free of bank conflicts), WS_CHUNK elements
+// apart. Three slices, q, k and v: C = 144 of 144 rows, five k-steps; C = 180 of
+// 192 rows (180 real), six k-steps (WS_CHUNK180). Groups of NS blocks (one per
+// slice, on one XCD) walk the same subtiles of tokens: gemmx_qkv_groups(cus, NS)
+// groups.
+#define WS_CHUNK (2 * 144 * 32)
+#define WS_CHUNK180 (2 * 192 * 32)
 #define GX_THREADS 512
 constexpr int gemmx_qkv_groups(int cus, int ns) { return cus >= 8 * ns ? cus / (8 * ns) * 8 : 1; }
 
@@ -349,6 +352,13 @@ struct CopyArgs {
 struct AbsMaxArgs {
     const float* x;
     unsigned* out;
+    long n;
+};
+
+// x[i] *= s, i < n (a multiple of 4).
+struct ScaleArgs {
+    float* x;
+    float s;
     long n;
 };
 

@@ -170,6 +170,38 @@ __device__ __forceinline__ void split2_x8(const float (&v)[8], u32x4 (&out)[2])
     }
 }
 
+// v_mfma_f32_16x16x32_f16 (the layout of mfma16_bf16).
+__device__ __forceinline__ f32x4 mfma16_f16(u32x4 a, u32x4 b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+}
+
+__device__ __forceinline__ f32x4 mfma16x3h(const u32x4 (&a)[2], const u32x4 (&b)[2], f32x4 c)
+{
+    c = mfma16_f16(a[1], b[0], c);
+    c = mfma16_f16(a[0], b[1], c);
+    return mfma16_f16(a[0], b[0], c);
+}
+
+// The packed last k-step of a K = 144 linear (the host's split2_half_step): lane
+// group lg's slots j < 4 and 4 + j both hold channel 128 + 4 lg + j, the weight
+// planes (a0 | a0) and (a1 | a1), the activation operand (b0 | b1): two MFMAs
+// give the three products (and a1 b1) that three give for a whole step.
+__device__ __forceinline__ u32x4 half_operand(const f32x4& v)
+{
+    unsigned p0a, p1a, p0b, p1b;
+    split2_pk(v[0], v[1], p0a, p1a);
+    split2_pk(v[2], v[3], p0b, p1b);
+    return (u32x4){p0a, p0b, p1a, p1b};
+}
+
+__device__ __forceinline__ f32x4 mfma16x2h(const u32x4 (&a)[2], const u32x4& b, f32x4 c)
+{
+    c = mfma16_f16(a[1], b, c);
+    return mfma16_f16(a[0], b, c);
+}
+
 // v_mfma_f32_32x32x16_f16 (the layout of mfma_bf16).
 __device__ __forceinline__ f32x16 mfma_f16(u32x4 a, u32x4 b, f32x16 c)
 {

@@ -213,3 +213,9 @@ extern "C" __global__ __launch_bounds__(256) void hat_absmax(AbsMaxArgs p)
     if (threadIdx.x == 0)
         atomicMax(p.out, __float_as_uint(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]))));
 }
+
+extern "C" __global__ __launch_bounds__(256) void hat_scale(ScaleArgs p)
+{
+    for (long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4; i < p.n; i += (long)gridDim.x * 1024)
+        *(f32x4*)(p.x + i) *= p.s;
+}

@@ -297,18 +297,19 @@ int gpu_selftest(std::string* err)
                 if (lnout) check_close(k + " C " + std::to_string(C) + " layernorm", dxn.get(), wxn, 5e-5);
                 note(k + " C " + std::to_string(C) + " M " + std::to_string(M) + " K " + std::to_string(K));
                 if (ws && epi == EPI_QKV) {
-                    // the split-bf16 form on the same inputs (the last
-                    // subtile partial: 600 rows are 18.75 subtiles of 32 at
-                    // C = 144, 12.5 of 48 at C = 180), one group: its 8 waves
-                    // walk them all
-                    std::vector<unsigned short> px = pack_linear_ws(w.data(), b.data(), N, K);
+                    // the split-f16 form on the same inputs (the last
+                    // subtile partial: 600 rows are 18.75 subtiles of 32),
+                    // one group: its 8 waves walk them all; the weights scaled into f16's range
+                    const float ws[3] = {1 << 15, 1 << 16, 1 << 17};
+                    std::vector<unsigned short> px = pack_linear_ws(w.data(), N, K, ws);
                     Dev dwx(std::vector<float>((px.size() + 1) / 2)), dout2((size_t)M * N);
                     rt.h2d(dwx.p, px.data(), px.size() * sizeof(unsigned short));
                     GemmArgs px2 = p;
                     px2.w = dwx.p;
                     px2.out = dout2.p;
+                    for (int i = 0; i < 3; ++i) px2.oscale[i] = 1.0f / ws[i];
                     const char* kx = C == 144 ? "hat_gemmx_qkv" : "hat_gemmx_qkv180";
-                    launch(s, kx, C == 144 ? 3 : 6, 1, 1, GX_THREADS, px2);
+                    launch(s, kx, 3, 1, 1, GX_THREADS, px2);
                     check_close(std::string(kx) + " C " + std::to_string(C), dout2.get(), want, 3e-5);
                     note(std::string(kx) + " C " + std::to_string(C) + " M " + std::to_string(M) + " K " + std::to_string(K));
                 }
