@@ -1,5 +1,9 @@
 #include "gpu.h"
 
+#if defined(__x86_64__)
+#include <immintrin.h>
+#endif
+
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -46,70 +50,6 @@ float bf16_float(unsigned short h)
 }
 }  // namespace
 
-// Rows [N][K] of w (row stride ldw), N <= 192, as weight chunks at dst: the
-// value at (n, k) is column kbase + k, which lands in 32-k step s = (kbase +
-// k) / 32, WC_CHUNK elements apart, as three bf16 planes [N][32] (plane stride
-// N * 32) with row n's 16-byte k-groups g stored at slot ws_slot(n, g) (so that
-// reads of one k-group down the rows are free of bank conflicts): x = h0 + h1 +
-// h2, each part the RNE of what the parts before it leave; the rest stays zero.
-static void split_chunks(const float* w, int N, int K, int ldw, unsigned short* dst, int kbase = 0)
-{
-    for (int n = 0; n < N; ++n)
-        for (int k = 0; k < K; ++k) {
-            const float x = w[(size_t)n * ldw + k];
-            const unsigned short h0 = bf16_rne(x);
-            const float r1 = x - bf16_float(h0);
-            const unsigned short h1 = bf16_rne(r1);
-            const unsigned short h2 = bf16_rne(r1 - bf16_float(h1));
-            const int s = (kbase + k) / 32, kk = (kbase + k) % 32;
-            unsigned short* d = dst + (size_t)s * WC_CHUNK + (size_t)n * 32 + hatk::ws_slot(n, kk / 8) * 8 + kk % 8;
-            d[0] = h0;
-            d[(size_t)N * 32] = h1;
-            d[(size_t)2 * N * 32] = h2;
-        }
-}
-
-// The last k-step of a K = 144 split linear in the packed form (common.h
-// ws_mma_half): only k = 128 .. 143 are real, so lane group g's slots j < 4
-// hold k = 128 + 4 g + j and slots 4 + j the same k, and the three planes hold
-// the part pairs (a0 | a0), (a1 | a0), (a1 | a2): against the activation pairs
-// (b0 | b1), (b0 | b2), (b1 | b0) they give the six products of order <= 2 in
-// three MFMAs. Row n of w (ldw apart) goes to row n of the chunk at dst, whose
-// planes are N * 32 elements apart.
-static void split_half_step(const float* w, int N, int ldw, unsigned short* dst)
-{
-    for (int n = 0; n < N; ++n)
-        for (int kk = 0; kk < 16; ++kk) {
-            const float x = w[(size_t)n * ldw + 128 + kk];
-            const unsigned short h0 = bf16_rne(x);
-            const float r1 = x - bf16_float(h0);
-            const unsigned short h1 = bf16_rne(r1);
-            const unsigned short h2 = bf16_rne(r1 - bf16_float(h1));
-            const int g = kk / 4, j = kk % 4;
-            unsigned short* d = dst + (size_t)n * 32 + hatk::ws_slot(n, g) * 8 + j;
-            const size_t pl = (size_t)N * 32;
-            d[0] = h0, d[4] = h0;            // (a0 | a0)
-            d[pl] = h1, d[pl + 4] = h0;      // (a1 | a0)
-            d[2 * pl] = h1, d[2 * pl + 4] = h2;  // (a1 | a2)
-        }
-}
-
-std::vector<unsigned short> pack_linear_x(const float* w, int N, int K)
-{
-    constexpr int BN = 144;
-    if (K != 144 || N % BN != 0) throw Error("pack_linear_x: needs K = 144 and N a multiple of 144");
-    const int steps = (K + 31) / 32;
-    std::vector<unsigned short> out((size_t)(N / BN) * steps * WC_CHUNK, 0);
-    for (int sl = 0; sl < N / BN; ++sl) {
-        unsigned short* dst = &out[(size_t)sl * steps * WC_CHUNK];
-        // four whole k-steps, then k = 128 .. 143 packed (split_half_step);
-        // the tails add the bias in fp32
-        split_chunks(w + (size_t)sl * BN * K, BN, 128, K, dst);
-        split_half_step(w + (size_t)sl * BN * K, BN, K, dst + (size_t)4 * WC_CHUNK);
-    }
-    return out;
-}
-
 // float -> f16, round to nearest even, subnormals kept, past the range infinite
 static inline unsigned short f16_rne(float x)
 {
@@ -145,11 +85,32 @@ static inline float f16_float(unsigned short h)
 
 // x = h0 + h1 (+ at most 2^-22 |x|), each part the round-to-nearest f16 of what
 // the one before leaves.
-static void split2_f16(float x, unsigned short* h0, unsigned short* h1)
+static inline void split2_f16(float x, unsigned short* h0, unsigned short* h1)
 {
-    const unsigned short a = f16_rne(x), b = f16_rne(x - f16_float(a));
-    *h0 = a;
-    *h1 = b;
+    *h0 = f16_rne(x);
+    *h1 = f16_rne(x - f16_float(*h0));
+}
+
+// Eight values at once, with the conversion instructions where the host has them
+// (a few million weights are split per network, and an op splits its own on every
+// call). Both forms give the same bits.
+#if defined(__x86_64__)
+__attribute__((target("avx,f16c"))) static void split2_f16_x8_f16c(const float* x, unsigned short* h0, unsigned short* h1)
+{
+    const __m256 v = _mm256_loadu_ps(x);
+    const __m128i a = _mm256_cvtps_ph(v, _MM_FROUND_TO_NEAREST_INT);
+    const __m128i b = _mm256_cvtps_ph(_mm256_sub_ps(v, _mm256_cvtph_ps(a)), _MM_FROUND_TO_NEAREST_INT);
+    _mm_storeu_si128((__m128i*)h0, a);
+    _mm_storeu_si128((__m128i*)h1, b);
+}
+#endif
+static void split2_f16_x8(const float* x, unsigned short* h0, unsigned short* h1)
+{
+#if defined(__x86_64__)
+    static const bool f16c = __builtin_cpu_supports("avx") && __builtin_cpu_supports("f16c");
+    if (f16c) return split2_f16_x8_f16c(x, h0, h1);
+#endif
+    for (int j = 0; j < 8; ++j) split2_f16(x[j], h0 + j, h1 + j);
 }
 
 // value(r, kk), r < rows, kk < 32: one 32-k step as two f16 planes [rows][32],
@@ -158,9 +119,11 @@ template <typename F>
 static void split2_step(int rows, F value, unsigned short* dst)
 {
     for (int r = 0; r < rows; ++r)
-        for (int kk = 0; kk < 32; ++kk) {
-            unsigned short* d = dst + (size_t)r * 32 + hatk::ws_slot(r, kk / 8) * 8 + kk % 8;
-            split2_f16(value(r, kk), d, d + (size_t)rows * 32);
+        for (int g = 0; g < 4; ++g) {
+            float v[8];
+            for (int j = 0; j < 8; ++j) v[j] = value(r, 8 * g + j);
+            unsigned short* d = dst + (size_t)r * 32 + hatk::ws_slot(r, g) * 8;
+            split2_f16_x8(v, d, d + (size_t)rows * 32);
         }
 }
 
@@ -179,7 +142,7 @@ static void split2_half_step(int rows, F value, unsigned short* dst)
         }
 }
 
-std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const float (&ws)[3])
+std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const float (&ws)[3], bool fill)
 {
     // three slices, q, k and v: C = 144 of 144 rows, five k-steps; C = 180 of
     // 180 rows padded to 192, six k-steps
@@ -188,6 +151,7 @@ std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const f
     const int real = K == 144 ? 144 : 180, rows = K == 144 ? 144 : 192, ks_n = (K + 31) / 32;
     const size_t chunk = (size_t)2 * rows * 32;
     std::vector<unsigned short> out((size_t)(N / real) * ks_n * chunk, 0);
+    if (!fill) return out;
     for (int sl = 0; sl < N / real; ++sl) {
         const float f = ws[sl * real / (N / 3)];
         for (int s = 0; s < ks_n; ++s) {
@@ -205,173 +169,82 @@ std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const f
 
 double abs_max(const float* w, size_t n)
 {
-    double m = 0.0;
+    uint32_t m = 0;  // non-negative floats order as their bits do, a NaN above all
     for (size_t i = 0; i < n; ++i) {
-        const double a = std::fabs((double)w[i]);
-        if (std::isnan(a)) return a;
-        m = std::max(m, a);
+        uint32_t u;
+        memcpy(&u, w + i, 4);
+        m = std::max(m, u & 0x7fffffffu);
     }
-    return m;
+    float f;
+    memcpy(&f, &m, 4);
+    return f;
 }
 
 // fc1 output tile t, row 4g + r (lane group g, register r) -> hidden unit
-// within a 96-unit third (tailx.hip): fc2's 32-k step s then finds units
-// 32 s + 8 g .. +7 in tiles 2 s and 2 s + 1 of lane group g.
-static int mlpx_unit(int row)
+// within a part (tailx.hip): fc2's 32-k step s then finds units 32 s + 8 g ..
+// +7 in tiles 2 s and 2 s + 1 of lane group g.
+static int tailx_unit(int row)
 {
     const int t = row / 16, g = (row % 16) / 4, r = row % 4;
     return 32 * (t / 2) + 8 * g + 4 * (t % 2) + r;
 }
 
-void pack_mlp_x(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w)
-{
-    constexpr int C = 144, H = 288;
-    static_assert(3 * C * 32 <= WC_CHUNK && WC_CHUNK % 512 == 0 && H % MX_HID == 0, "chunks");
-    std::vector<float> f1((size_t)MX_HID * C), fb((size_t)MX_HID);
-    w->assign((size_t)24 * WC_CHUNK, 0);
-    for (int q = 0; q < H / MX_HID; ++q) {
-        for (int row = 0; row < MX_HID; ++row) {
-            const int u = q * MX_HID + mlpx_unit(row);
-            memcpy(&f1[(size_t)row * C], w1 + (size_t)u * C, C * sizeof(float));
-            fb[row] = b1[u];
-        }
-        unsigned short* dst = &(*w)[(size_t)(8 * q) * WC_CHUNK];
-        split_chunks(f1.data(), MX_HID, C, C, dst);
-        // b1 as fc1's column k = 144 (step 4, j = 16)
-        split_chunks(fb.data(), MX_HID, 1, 1, dst, C);
-        split_chunks(w2 + q * MX_HID, C, MX_HID, H, &(*w)[(size_t)(8 * q + 5) * WC_CHUNK]);
-    }
-}
-
-// Fused tail input position k = 32 ks + 8 g + j (ks: 32-k step, g: lane group,
-// j < 8) -> channel of x': steps 0..3 hold the lane's accumulator tiles 2 ks
-// and 2 ks + 1 (channels 32 ks + 4 g + j and 32 ks + 16 + 4 g + j - 4), step 4
-// tile 8 (128 + 4 g + j) and b1's 1 at g = 0, j = 4 (-1); -2: an empty position.
-// The device twin is habx_channel (tailx.hip).
-int mlpx_fused_channel(int k)
-{
-    const int ks = k >> 5, g = (k >> 3) & 3, j = k & 7;
-    if (ks < 4) return 32 * ks + (j < 4 ? 4 * g + j : 16 + 4 * g + (j - 4));
-    if (j < 4) return 128 + 4 * g + j;
-    return g == 0 && j == 4 ? -1 : -2;
-}
-
-void pack_mlp_xf(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w,
-                 std::vector<float>* b1x)
-{
-    // per third: fc1's steps 0..3 in the fused input order, step 4 (channels
-    // 128 .. 143, whose fused positions are 128 + 4 g + j) packed
-    // (split_half_step), b1 added in fp32 before the GELU (b1x, in the
-    // third's permuted row order), then fc2's three steps
-    constexpr int C = 144, H = 288, KF = 128;
-    std::vector<float> f1((size_t)MX_HID * KF), rows((size_t)MX_HID * C);
-    w->assign((size_t)24 * WC_CHUNK, 0);
-    b1x->assign(H, 0.0f);
-    for (int q = 0; q < H / MX_HID; ++q) {
-        for (int row = 0; row < MX_HID; ++row) {
-            const int u = q * MX_HID + mlpx_unit(row);
-            for (int k = 0; k < KF; ++k) f1[(size_t)row * KF + k] = w1[(size_t)u * C + mlpx_fused_channel(k)];
-            memcpy(&rows[(size_t)row * C], w1 + (size_t)u * C, C * sizeof(float));
-            (*b1x)[(size_t)q * MX_HID + row] = b1[u];
-        }
-        split_chunks(f1.data(), MX_HID, KF, KF, &(*w)[(size_t)(8 * q) * WC_CHUNK]);
-        split_half_step(rows.data(), MX_HID, C, &(*w)[(size_t)(8 * q + 4) * WC_CHUNK]);
-        split_chunks(w2 + q * MX_HID, C, MX_HID, H, &(*w)[(size_t)(8 * q + 5) * WC_CHUNK]);
-    }
-}
-
-// One 32-k step of `rows` weight rows (value(r, kk), kk < 32) split into three
-// bf16 planes [rows][32] in the swizzled layout of the weight-stationary
-// kernels (row r's k-group g at slot ws_slot(r, g)).
-template <typename F>
-static void split_ws_step(int rows, F value, unsigned short* dst)
-{
-    for (int r = 0; r < rows; ++r)
-        for (int kk = 0; kk < 32; ++kk) {
-            const float x = value(r, kk);
-            const unsigned short h0 = bf16_rne(x);
-            const float r1 = x - bf16_float(h0);
-            const unsigned short h1 = bf16_rne(r1);
-            const unsigned short h2 = bf16_rne(r1 - bf16_float(h1));
-            unsigned short* d = dst + (size_t)r * 32 + hatk::ws_slot(r, kk / 8) * 8 + kk % 8;
-            d[0] = h0;
-            d[(size_t)rows * 32] = h1;
-            d[(size_t)2 * rows * 32] = h2;
-        }
-}
-
-// The C = 180 projection [180][180] for hat_projx180*: six 32-k steps of 192
-// rows (180 real; the bias is added in the epilogue), MX180_SLOT apart.
-std::vector<unsigned short> pack_linear_x180(const float* w)
-{
-    constexpr int C = 180;
-    std::vector<unsigned short> out((size_t)6 * MX180_SLOT, 0);
-    for (int ks = 0; ks < 6; ++ks)
-        split_ws_step(192, [&](int n, int kk) {
-            const int k = ks * 32 + kk;
-            return n < C && k < C ? w[(size_t)n * C + k] : 0.0f;
-        }, &out[(size_t)ks * MX180_SLOT]);
-    return out;
-}
-
-// The C = 180 MLP (fc1 [360][180] + b1, fc2 [180][360]) for hat_mlpx180: per
-// part of 64 hidden units, six fc1 k-steps (rows permuted by mlpx_unit, b1 at
-// k = 180) and two fc2 k-steps (192 rows, 180 real, the part's units in
-// natural order), MX180_SLOT elements apart.
-void pack_mlp_x180(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w)
-{
-    constexpr int C = 180, H = 360, NP = 6;
-    w->assign((size_t)8 * NP * MX180_SLOT, 0);
-    for (int q = 0; q < NP; ++q) {
-        for (int ks = 0; ks < 6; ++ks)
-            split_ws_step(MX180_HID, [&](int r, int kk) {
-                const int u = q * MX180_HID + mlpx_unit(r), k = ks * 32 + kk;
-                if (u >= H) return 0.0f;
-                return k < C ? w1[(size_t)u * C + k] : (k == C ? b1[u] : 0.0f);
-            }, &(*w)[(size_t)(8 * q + ks) * MX180_SLOT]);
-        for (int st = 0; st < 2; ++st)
-            split_ws_step(192, [&](int n, int kk) {
-                const int u = q * MX180_HID + st * 32 + kk;
-                return n < C && u < H ? w2[(size_t)n * H + u] : 0.0f;
-            }, &(*w)[(size_t)(8 * q + 6 + st) * MX180_SLOT]);
-    }
-}
-
-// Fused C = 180 tail input position k = 32 ks + 8 g + j (ks < 6: 32-k step, g:
-// lane group, j < 8) -> channel of x': the lane's accumulator tiles 2 ks and
-// 2 ks + 1 (channels 32 ks + 4 g + j and 32 ks + 16 + 4 g + j - 4); -1 past
-// channel 179. The device twin is habx180_channel (tailx.hip).
-int mlpx180_fused_channel(int k)
+// fc1 input position k = 32 ks + 8 g + j (ks: 32-k step, g: lane group, j < 8) ->
+// channel of x': the lane's accumulator tiles 2 ks and 2 ks + 1 (channels 32 ks +
+// 4 g + j and 32 ks + 16 + 4 g + j - 4); -1 past channel C - 1. (C = 144's packed
+// fifth step takes channels 128 + kk in order: split2_half_step.)
+int tailx_channel(int C, int k)
 {
     const int ks = k >> 5, g = (k >> 3) & 3, j = k & 7;
     const int c = 32 * ks + (j < 4 ? 4 * g + j : 16 + 4 * g + (j - 4));
-    return c < 180 ? c : -1;
+    return c < C ? c : -1;
 }
 
-void pack_mlp_xf180(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w,
-                    std::vector<float>* b1x)
+std::vector<unsigned short> pack_tail_proj(const float* w, int C, float s, bool fill)
 {
-    // per part: fc1's six steps with rows permuted by mlpx_unit and input
-    // columns in the fused order, b1 in b1x (the same row order, added in
-    // fp32 before the GELU), then fc2's two steps as in pack_mlp_x180
-    constexpr int C = 180, H = 360, NP = 6;
-    w->assign((size_t)8 * NP * MX180_SLOT, 0);
-    b1x->assign((size_t)NP * MX180_HID, 0.0f);
+    const int rows = (C + 15) / 16 * 16, ks_n = (C + 31) / 32;
+    const size_t step = (size_t)2 * rows * 32;
+    std::vector<unsigned short> out(ks_n * step + TX_PAD, 0);
+    if (!fill) return out;
+    for (int ks = 0; ks < ks_n; ++ks) {
+        auto value = [&](int n, int kk) {
+            const int k = 32 * ks + kk;
+            return n < C && k < C ? w[(size_t)n * C + k] * s : 0.0f;
+        };
+        if (C == 144 && ks == 4) split2_half_step(rows, value, &out[ks * step]);
+        else split2_step(rows, value, &out[ks * step]);
+    }
+    return out;
+}
+
+void pack_tail_mlp(const float* w1, const float* b1, const float* w2, int C, float s1, float s2, float hs,
+                   std::vector<unsigned short>* w, std::vector<float>* b1x, bool fill)
+{
+    const int H = 2 * C, HU = tailx_hu(C), NP = (H + HU - 1) / HU, rows = (C + 15) / 16 * 16, ks_n = (C + 31) / 32;
+    const size_t step1 = (size_t)2 * HU * 32, step = (size_t)2 * rows * 32, part = ks_n * step1 + HU / 32 * step;
+    w->assign(NP * part + TX_PAD, 0);
+    b1x->assign((size_t)NP * HU, 0.0f);
+    if (!fill) return;
     for (int q = 0; q < NP; ++q) {
-        for (int r = 0; r < MX180_HID; ++r) {
-            const int u = q * MX180_HID + mlpx_unit(r);
-            if (u < H) (*b1x)[(size_t)q * MX180_HID + r] = b1[u];
+        for (int r = 0; r < HU; ++r) {
+            const int u = q * HU + tailx_unit(r);
+            if (u < H) (*b1x)[(size_t)q * HU + r] = b1[u] * hs;
         }
-        for (int ks = 0; ks < 6; ++ks)
-            split_ws_step(MX180_HID, [&](int r, int kk) {
-                const int u = q * MX180_HID + mlpx_unit(r), c = mlpx180_fused_channel(ks * 32 + kk);
-                return u < H && c >= 0 ? w1[(size_t)u * C + c] : 0.0f;
-            }, &(*w)[(size_t)(8 * q + ks) * MX180_SLOT]);
-        for (int st = 0; st < 2; ++st)
-            split_ws_step(192, [&](int n, int kk) {
-                const int u = q * MX180_HID + st * 32 + kk;
-                return n < C && u < H ? w2[(size_t)n * H + u] : 0.0f;
-            }, &(*w)[(size_t)(8 * q + 6 + st) * MX180_SLOT]);
+        for (int ks = 0; ks < ks_n; ++ks) {
+            const bool half = C == 144 && ks == 4;
+            auto value = [&](int r, int kk) {
+                const int u = q * HU + tailx_unit(r), c = half ? 128 + kk : tailx_channel(C, 32 * ks + kk);
+                return u < H && c >= 0 ? w1[(size_t)u * C + c] * s1 : 0.0f;
+            };
+            unsigned short* dst = &(*w)[q * part + ks * step1];
+            if (half) split2_half_step(HU, value, dst);
+            else split2_step(HU, value, dst);
+        }
+        for (int st = 0; st < HU / 32; ++st)
+            split2_step(rows, [&](int n, int kk) {
+                const int u = q * HU + st * 32 + kk;
+                return n < C && u < H ? w2[(size_t)n * H + u] * s2 : 0.0f;
+            }, &(*w)[q * part + ks_n * step1 + st * step]);
     }
 }
 
@@ -416,13 +289,14 @@ std::vector<float> pack_conv(const float* w, const float* b, int CO, int CI, int
 // channels (CI = 144), it is packed as the K = 144 linears' last step
 // (split_half_step): lane r + 16 g, slots j < 4 hold channel 32 kc + 4 g + j,
 // slots 4 + j the same channel, the parts as (0 | 0), (1 | 0), (1 | 2).
-std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r)
+std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r, bool fill)
 {
     if (r > 0 && CO % 16 != 0) throw Error("pack_wino: shuffled output channels must come in 16s");
     static const double G[4][3] = {{1, 0, 0}, {0.5, 0.5, 0.5}, {0.5, -0.5, 0.5}, {0, 0, 1}};
     const int NTT = (CO + 15) / 16, NKC = (CI + 31) / 32, Cf = r > 0 ? CO / (r * r) : 0;
     const bool packed = CI % 32 != 0 && CI % 32 <= 16;  // the kernels' PACK
     std::vector<unsigned short> out((size_t)NKC * 16 * NTT * 3 * 512, 0);
+    if (!fill) return out;
     for (int o2 = 0; o2 < CO; ++o2) {
         int o = o2;
         if (r > 0) {
@@ -507,13 +381,14 @@ double ln_linear_bound(const float* w, const float* b, const float* lnw, const f
     double worst = 0.0;
     for (int n = n0; n < n1; ++n) {
         const float* r = w + (size_t)n * C;
-        double sq = 0.0, off = b ? b[n] : 0.0;
-        for (int c = 0; c < C; ++c) {
-            const double x = (double)r[c] * lnw[c];
-            sq += x * x;
-            off += (double)r[c] * lnb[c];
-        }
-        const double v = std::sqrt(sq * C) + std::fabs(off);
+        double sq[4] = {}, off[4] = {b ? b[n] : 0.0};  // four chains: an op does this on every call
+        for (int c = 0; c < C; c += 4)
+            for (int i = 0; i < 4 && c + i < C; ++i) {
+                const double x = (double)r[c + i] * lnw[c + i];
+                sq[i] += x * x;
+                off[i] += (double)r[c + i] * lnb[c + i];
+            }
+        const double v = std::sqrt((sq[0] + sq[1] + sq[2] + sq[3]) * C) + std::fabs(off[0] + off[1] + off[2] + off[3]);
         if (std::isnan(v)) return v;
         worst = std::max(worst, v);
     }
@@ -544,6 +419,55 @@ QkvScale qkv_scale(double bq, double bk, double bv, int head_dim)
     s.v = f16_scale(bv);
     s.ok = true;
     return s;
+}
+
+// TailXArgs' scales.
+void tail_scales(const DevTail& t, TailXArgs* f)
+{
+    f->ps = t.ps;
+    f->pi = 1.0f / t.ps;
+    f->h1 = t.h1;
+    f->g0 = 0.3275911f * 0.70710678f / t.hs;
+    f->g1 = -0.5f * 1.4426950408889634f / (t.hs * t.hs);
+    f->ms = t.ms;
+    f->mi = 1.0f / t.ms;
+}
+
+TailPack pack_tail(const float* wp, const float* w1, const float* b1, const float* w2, const float* n2w, const float* n2b,
+                   int C, float sv, float sn, const TailCab* cab, bool fill)
+{
+    TailPack p;
+    DevTail& t = p.t;
+    t.C = C;
+    if (!fill) {
+        p.w = pack_tail_proj(wp, C, 1.0f, false);
+        pack_tail_mlp(w1, b1, w2, C, 1.0f, 1.0f, 1.0f, &p.wm, &p.b1x, false);
+        return p;
+    }
+    float sp = f16_scale(abs_max(wp, (size_t)C * C));
+    if (cab) {
+        // the projection and the gated conv2 add into the same accumulators, so
+        // ts gs = sv sp: each of the two as far from its limit as the other, and
+        // the projection's weights scaled down where the limits leave no room
+        auto limit = [](double bound) { return bound == 0.0 ? 60 : std::ilogb(f16_scale(bound)); };
+        const int lt = limit(cab->t1), lg = limit(cab->w2);
+        int spare = lt + lg - std::ilogb(sv) - std::ilogb(sp);
+        if (spare < 0) {
+            sp = std::ldexp(sp, spare);
+            spare = 0;
+        }
+        t.ts = std::ldexp(1.0f, lt - spare / 2);
+        t.gs = std::ldexp(1.0f, lg - (spare - spare / 2));
+    }
+    t.ps = sv * sp;
+    p.w = pack_tail_proj(wp, C, sp);
+    // |gelu(v)| <= |v|, and fc1 reads a norm's output
+    t.hs = f16_scale(ln_linear_bound(w1, b1, n2w, n2b, 0, 2 * C, C));
+    const float s1 = f16_scale(abs_max(w1, (size_t)2 * C * C)), s2 = f16_scale(abs_max(w2, (size_t)2 * C * C));
+    t.h1 = t.hs / (sn * s1);
+    t.ms = t.hs * s2;
+    pack_tail_mlp(w1, b1, w2, C, s1, s2, t.hs, &p.wm, &p.b1x);
+    return p;
 }
 
 // ---------------------------------------------------------------------------
@@ -722,12 +646,12 @@ void run_mlp(hipStream_t s, const DevLinear& fc1, const DevLinear& fc2, const fl
 // is not launched: its arguments go to *defer, for the attention launch to run.
 void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, const float* bproj,
              float cscale, int sq, float* t1, float* partial, float* w2g, float* bias2, float* gate,
-             unsigned short* w2gx, CabGateArgs* defer = nullptr)
+             unsigned short* w2gx, float ts, float gs, CabGateArgs* defer = nullptr)
 {
     if (H % 16 != 0 || W % 16 != 0 || H < 16 || W < 16) throw Error("CAB: plane must be 16-aligned");
     if (sq < 1 || sq > 64) throw Error("CAB: squeeze width must be 1..64");
     static const int cus = std::max(1, Runtime::get().cu_count());
-    CabConvArgs a{xn, cb.w1, cb.b1, t1, partial, H, W};
+    CabConvArgs a{xn, cb.w1, cb.b1, t1, partial, H, W, ts};
     // Persistent over the output tiles, one block of 4 waves per CU: 16 wide x
     // 32 tall when the height allows, else 16 x 16.
     const bool t32 = H % 32 == 0;
@@ -752,6 +676,8 @@ void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, con
     g.cscale = cscale;
     g.sq = sq;
     g.w2gx = w2gx;
+    g.ts = ts;
+    g.gs = gs;
     if (defer) {
         *defer = g;
         return;
@@ -810,79 +736,51 @@ void run_hab_tail(hipStream_t s, const DevLinear& proj, const DevLinear& fc1, co
     launch(s, cab ? "hat_hab_tail" : "hat_ocab_tail", (unsigned)g, 1, 1, MLP_WAVES * 64, p);
 }
 
-// The tail on split-bf16 (tailx.hip): x' = res + a . Wp^T (+ CAB: the gated
-// conv2 of t1) + bias [hat_projx(_cab)]; out = x' + MLP(norm2(x')), norm2
-// formed in the MLP kernel (+ with nw: xn = norm_next(out)) [hat_mlpx(_ln)].
-// out may alias res.
-void run_tailx(hipStream_t s, bool cab, const DevLinear& proj, const DevMlpX& mlp, const float* b2, const float* a,
-               const float* res, float* out, float* xn, const float* t1, const unsigned short* w2gx, const float* bias,
-               const float* n2w, const float* n2b, const float* nw, const float* nb, int H, int W)
+// The tail on split-f16 (tailx.hip): x' = res + a . Wp^T + bias (+ t1: the gated
+// conv2 w2gx of it on the H x W plane, C = 144; + aux * gate * cscale, C = 180);
+// out = x' + MLP(norm2(x')) (+ with nw: xn = norm_next(out)). The HAB's forms have
+// a CAB and a next norm, the OCAB's neither. out may alias res.
+struct TailCabIn {
+    const float* t1 = nullptr;
+    const unsigned short* w2gx = nullptr;
+    const float *aux = nullptr, *gate = nullptr;
+    float cscale = 0.0f;
+    int H = 0, W = 0;
+};
+void run_tailx(hipStream_t s, const DevTail& t, const float* a, const float* res, float* out, float* xn, const float* bias,
+               const float* b2, const float* n2w, const float* n2b, const float* nw, const float* nb, long M,
+               const TailCabIn& cab)
 {
-    if (!proj.wx || proj.K != 144 || proj.N != 144) throw Error("tailx: needs the pre-split 144 x 144 projection");
-    if (cab && (!t1 || !w2gx)) throw Error("tailx: the CAB form needs t1 and the gated conv2 weight chunks");
-    const long M = (long)H * W;
+    const bool hab = nw != nullptr;
+    if (hab != (t.C == 144 ? cab.t1 && cab.w2gx : cab.aux && cab.gate))
+        throw Error("tailx: the HAB's form needs its CAB and the next norm, the OCAB's has neither");
     if (M > 0x7fffffffL) throw Error("tailx: too many rows");
-    const unsigned g = (unsigned)wx_tiles((int)M);  // a block per 128-token tile
-    if (mlp.wf && cab == (nw != nullptr)) {
-        // one kernel, x' kept on the chip (the forms the network runs: the HAB's
-        // with the next norm, the OCAB's without)
-        TailXArgs f{};
-        f.a = a;
-        f.res = res;
-        f.out = out;
-        f.xn = nw ? xn : nullptr;
-        f.w = proj.wx;
-        f.wm = mlp.wf;
-        f.b1x = mlp.b1x;
-        f.bias = bias;
-        f.b2 = b2;
-        f.w2gx = w2gx;
-        f.t1 = t1;
-        f.inw = n2w;
-        f.inb = n2b;
-        f.nw = nw;
-        f.nb = nb;
-        f.M = (int)M;
-        f.H = H;
-        f.W = W;
-        f.eps = 1e-5f;
-        launch(s, cab ? "hat_habx_cab_ln" : "hat_habx", g, 1, 1, WX_THREADS, f);
-        return;
-    }
-    // the projection writes x' only: the MLP forms norm2(x') from the x'
-    // rows it reads
-    TailXArgs p{};
-    p.a = a;
-    p.res = res;
-    p.out = out;
-    p.xn = nullptr;
-    p.w = proj.wx;
-    p.bias = bias;
-    p.w2gx = w2gx;
-    p.t1 = t1;
-    p.nw = n2w;
-    p.nb = n2b;
-    p.M = (int)M;
-    p.H = H;
-    p.W = W;
-    p.eps = 1e-5f;
-    launch(s, cab ? "hat_projx_cab" : "hat_projx", g, 1, 1, WX_THREADS, p);
-    TailXArgs q{};
-    q.a = out;
-    q.res = out;
-    q.out = out;
-    q.xn = nw ? xn : nullptr;
-    q.w = mlp.w;
-    q.b2 = b2;
-    q.nw = nw;
-    q.nb = nb;
-    q.inw = n2w;
-    q.inb = n2b;
-    q.M = (int)M;
-    q.H = H;
-    q.W = W;
-    q.eps = 1e-5f;
-    launch(s, nw ? "hat_mlpx_ln" : "hat_mlpx", g, 1, 1, WX_THREADS, q);
+    TailXArgs f{};
+    f.a = a;
+    f.res = res;
+    f.out = out;
+    f.xn = hab ? xn : nullptr;
+    f.w = t.w;
+    f.wm = t.wm;
+    f.w2gx = cab.w2gx;
+    f.t1 = cab.t1;
+    f.aux = cab.aux;
+    f.gate = cab.gate;
+    f.bias = bias;
+    f.b1x = t.b1x;
+    f.b2 = b2;
+    f.inw = n2w;
+    f.inb = n2b;
+    f.nw = nw;
+    f.nb = nb;
+    f.M = (int)M;
+    f.H = cab.H;
+    f.W = cab.W;
+    f.eps = 1e-5f;
+    f.cscale = cab.cscale;
+    tail_scales(t, &f);
+    const char* name = t.C == 144 ? (hab ? "hat_habx_cab_ln" : "hat_habx") : (hab ? "hat_habx180_hab_ln" : "hat_habx180");
+    launch(s, name, (unsigned)wx_tiles((int)M), 1, 1, WX_THREADS, f);
 }
 
 // The channel-attention gate from the CAB conv's per-tile column sums:
@@ -1233,31 +1131,23 @@ void launch_wino(hipStream_t s, const char* name, unsigned tiles, unsigned ncb, 
 // ---------------------------------------------------------------------------
 // GpuBackend
 
-float* GpuBackend::upload(const float* src, size_t n)
-{
-    if (count_only_) {
-        weight_bytes_ += n * sizeof(float);
-        return nullptr;
-    }
-    Runtime& rt = Runtime::get();
-    float* d = (float*)rt.alloc(n * sizeof(float));
-    owned_.push_back(d);
-    rt.h2d(d, src, n * sizeof(float));
-    weight_bytes_ += n * sizeof(float);
-    return d;
-}
+// Weights are allocated in whole granules: the kernels that copy them to LDS do so
+// in whole loads, which may read past a tensor's end, and small ones are spread
+// over the memory channels instead of sharing a page. weight_bytes_ counts what
+// is allocated.
+static constexpr size_t kWeightGranule = 128u << 10;
+
+float* GpuBackend::upload(const float* src, size_t n) { return (float*)upload_bytes(src, n * sizeof(float)); }
 
 void* GpuBackend::upload_bytes(const void* src, size_t bytes)
 {
-    if (count_only_) {
-        weight_bytes_ += bytes;
-        return nullptr;
-    }
+    const size_t room = (bytes + kWeightGranule - 1) / kWeightGranule * kWeightGranule;
+    weight_bytes_ += room;
+    if (count_only_) return nullptr;
     Runtime& rt = Runtime::get();
-    void* d = rt.alloc(bytes);
+    void* d = rt.alloc(room);
     owned_.push_back(d);
     rt.h2d(d, src, bytes);
-    weight_bytes_ += bytes;
     return d;
 }
 
@@ -1270,55 +1160,41 @@ void GpuBackend::upload_raw(const std::string& name)
 // The qkv weights for hat_gemmx_qkv*: each of q, k and v scaled into f16's range
 // (w: the linear's own weights, out[3] the results' factors, in the inverse of
 // the input's scale); sets oscale.
-static std::vector<unsigned short> split_qkv(const float* w, int N, int K, const float* out, float in, float* oscale)
+static std::vector<unsigned short> split_qkv(const float* w, int N, int K, const float* out, float in, float* oscale,
+                                             bool fill = true)
 {
-    float ws[3];
-    for (int i = 0; i < 3; ++i) {
+    float ws[3] = {1.0f, 1.0f, 1.0f};
+    for (int i = 0; fill && i < 3; ++i) {
         ws[i] = f16_scale(abs_max(w + (size_t)i * (N / 3) * K, (size_t)(N / 3) * K));
         oscale[i] = in * out[i] / ws[i];
     }
-    return pack_linear_ws(w, N, K, ws);
+    return pack_linear_ws(w, N, K, ws, fill);
 }
 
-void GpuBackend::upload_linear(const std::string& name, const float* out, float in)
+void GpuBackend::upload_linear(const std::string& name, const float* out, float in, bool bias_only)
 {
     const TensorInfo& ti = wt_.info(name + ".weight");
     DevLinear L;
     L.N = (int)ti.shape[0];
     L.K = (int)ti.shape[1];
+    L.Kp = (L.K + 15) / 16 * 16;
     const float *w = wt_.t(name + ".weight"), *bias = wt_.t(name + ".bias");
-    std::vector<float> ws, bs;
-    if (out || in != 1.0f) {
-        ws.assign(w, w + (size_t)L.N * L.K);
-        bs.assign(bias, bias + L.N);
-        for (int n = 0; n < L.N; ++n) {
-            const float f = out ? out[n / (L.N / 3)] : 1.0f;
-            for (int k = 0; k < L.K; ++k) ws[(size_t)n * L.K + k] *= f * in;
-            bs[n] *= f;
-        }
-    }
-    const float *sw = ws.empty() ? w : ws.data(), *sb = bs.empty() ? bias : bs.data();
-    std::vector<float> pk = pack_linear(sw, L.N, L.K, &L.Kp);
-    L.w = upload(pk.data(), pk.size());
-    L.b = upload(sb, L.N);
-    auto ends = [&](const char* t) {
-        const size_t n = strlen(t);
-        return name.size() >= n && name.compare(name.size() - n, n, t) == 0;
-    };
-    if (L.K == 180 && L.N == 180 && ends("proj")) {
-        // the C = 180 projection tails (hat_projx180*)
-        std::vector<unsigned short> x = pack_linear_x180(sw);
-        L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
-    }
-    if (L.K == 144 && L.N == 144 && ends("proj")) {
-        // streamed chunks (tailx)
-        std::vector<unsigned short> x = pack_linear_x(sw, L.N, L.K);
-        L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
-    }
+    std::vector<float> bs(bias, bias + L.N);
+    if (out)
+        for (int n = 0; n < L.N; ++n) bs[n] *= out[n / (L.N / 3)];
+    L.b = upload(bs.data(), L.N);
     if (out && ((L.K == 180 && L.N == 540) || (L.K == 144 && L.N == 432))) {
         // qkv: the weight-stationary layout of hat_gemmx_qkv
-        std::vector<unsigned short> x = split_qkv(w, L.N, L.K, out, in, L.oscale);
+        std::vector<unsigned short> x = split_qkv(w, L.N, L.K, out, in, L.oscale, !count_only_);
         L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
+    } else if (!bias_only) {
+        std::vector<float> ws(w, w + (size_t)L.N * L.K);
+        for (int n = 0; n < L.N; ++n) {
+            const float f = (out ? out[n / (L.N / 3)] : 1.0f) * in;
+            for (int k = 0; k < L.K; ++k) ws[(size_t)n * L.K + k] *= f;
+        }
+        std::vector<float> pk = pack_linear(ws.data(), L.N, L.K, &L.Kp);
+        L.w = upload(pk.data(), pk.size());
     }
     lin_[name] = L;
 }
@@ -1343,43 +1219,52 @@ void GpuBackend::upload_attn(const std::string& qkv, const std::string& proj, co
     const int C = wt_.embed;
     const float *w = wt_.t(qkv + ".weight"), *b = wt_.t(qkv + ".bias"), *lw = wt_.t(ln + ".weight"),
                 *lb = wt_.t(ln + ".bias");
-    const QkvScale s = qkv_scale(ln_linear_bound(w, b, lw, lb, 0, C, C), ln_linear_bound(w, b, lw, lb, C, 2 * C, C),
-                                 ln_linear_bound(w, b, lw, lb, 2 * C, 3 * C, C), wt_.head_dim);
+    QkvScale s;
+    if (!count_only_)
+        s = qkv_scale(ln_linear_bound(w, b, lw, lb, 0, C, C), ln_linear_bound(w, b, lw, lb, C, 2 * C, C),
+                      ln_linear_bound(w, b, lw, lb, 2 * C, 3 * C, C), wt_.head_dim);
     const float out[3] = {s.q, s.k, s.v};
     upload_linear(qkv, out, 1.0f / norm_scale_.at(ln));
-    upload_linear(proj, nullptr, 1.0f / s.v);
     attn_f16_[table] = s.ok;
+    v_scale_ = s.v;
 }
 
-// The C = 144 MLP, pre-split for hat_mlpx (other widths keep the FP32 kernels).
-void GpuBackend::upload_mlpx(const std::string& name)
+void GpuBackend::upload_tail(const std::string& proj, const std::string& mlp, const std::string& norm2,
+                             const std::string& cab, const std::string& norm1)
 {
-    const TensorInfo& t1 = wt_.info(name + ".fc1.weight");
-    const TensorInfo& t2 = wt_.info(name + ".fc2.weight");
-    std::vector<unsigned short> w;
-    DevMlpX m;
-    if (t1.shape == std::vector<size_t>{288, 144} && t2.shape == std::vector<size_t>{144, 288}) {
-        pack_mlp_x(wt_.t(name + ".fc1.weight"), wt_.t(name + ".fc1.bias"), wt_.t(name + ".fc2.weight"), &w);
-        m.C = 144;
-        std::vector<unsigned short> wf;
-        std::vector<float> b1x;
-        pack_mlp_xf(wt_.t(name + ".fc1.weight"), wt_.t(name + ".fc1.bias"), wt_.t(name + ".fc2.weight"), &wf, &b1x);
-        m.wf = (unsigned short*)upload_bytes(wf.data(), wf.size() * sizeof(unsigned short));
-        m.b1x = upload(b1x.data(), b1x.size());
-    } else if (t1.shape == std::vector<size_t>{360, 180} && t2.shape == std::vector<size_t>{180, 360}) {
-        pack_mlp_x180(wt_.t(name + ".fc1.weight"), wt_.t(name + ".fc1.bias"), wt_.t(name + ".fc2.weight"), &w);
-        m.C = 180;
-        std::vector<unsigned short> wf;
-        std::vector<float> b1x;
-        pack_mlp_xf180(wt_.t(name + ".fc1.weight"), wt_.t(name + ".fc1.bias"), wt_.t(name + ".fc2.weight"), &wf,
-                       &b1x);
-        m.wf = (unsigned short*)upload_bytes(wf.data(), wf.size() * sizeof(unsigned short));
-        m.b1x = upload(b1x.data(), b1x.size());
-    } else {
-        return;
+    const size_t C = (size_t)wt_.embed;
+    upload_norm(norm2);
+    const float sn = norm_scale_.at(norm2);
+    const bool fits = (C == 144 || C == 180) && wt_.info(proj + ".weight").shape == std::vector<size_t>{C, C} &&
+                      wt_.info(mlp + ".fc1.weight").shape == std::vector<size_t>{2 * C, C} &&
+                      wt_.info(mlp + ".fc2.weight").shape == std::vector<size_t>{C, 2 * C};
+    upload_linear(proj, nullptr, 1.0f / v_scale_, fits);
+    upload_linear(mlp + ".fc1", nullptr, 1.0f / sn, fits);
+    upload_linear(mlp + ".fc2", nullptr, 1.0f, fits);
+    if (!fits) return;
+    TailCab tc{0.0, 0.0};
+    if (!cab.empty() && !count_only_) {
+        // |t1|: conv1's nine taps of norm1 rows
+        const float *w = wt_.t(cab + "0.weight"), *b = wt_.t(cab + "0.bias"), *lw = wt_.t(norm1 + ".weight"),
+                    *lb = wt_.t(norm1 + ".bias");
+        std::vector<float> row(C);
+        for (int co = 0; co < CAB_CC; ++co) {
+            double v = std::fabs((double)b[co]);
+            for (int tap = 0; tap < 9; ++tap) {
+                for (size_t ci = 0; ci < C; ++ci) row[ci] = w[(co * C + ci) * 9 + tap];
+                v += ln_linear_bound(row.data(), nullptr, lw, lb, 0, 1, (int)C);
+            }
+            tc.t1 = std::isnan(v) ? v : std::max(tc.t1, v);
+        }
+        tc.w2 = std::fabs((double)wt_.conv_scale) * abs_max(wt_.t(cab + "2.weight"), C * CAB_CC * 9);
     }
-    m.w = (unsigned short*)upload_bytes(w.data(), w.size() * sizeof(unsigned short));
-    mlpx_[name] = m;
+    TailPack p = pack_tail(wt_.t(proj + ".weight"), wt_.t(mlp + ".fc1.weight"), wt_.t(mlp + ".fc1.bias"),
+                           wt_.t(mlp + ".fc2.weight"), wt_.t(norm2 + ".weight"), wt_.t(norm2 + ".bias"), (int)C, v_scale_, sn,
+                           cab.empty() ? nullptr : &tc, !count_only_);
+    p.t.w = (unsigned short*)upload_bytes(p.w.data(), p.w.size() * sizeof(unsigned short));
+    p.t.wm = (unsigned short*)upload_bytes(p.wm.data(), p.wm.size() * sizeof(unsigned short));
+    p.t.b1x = upload(p.b1x.data(), p.b1x.size());
+    tail_[mlp] = p.t;
 }
 
 void GpuBackend::upload_conv(const std::string& name, int r, float in)
@@ -1401,7 +1286,7 @@ void GpuBackend::upload_conv(const std::string& name, int r, float in)
     C.w = upload(pk.data(), pk.size());
     C.b = upload(bias.data(), bias.size());
     if (wino_conv(C.CO, C.CI, r)) {
-        std::vector<unsigned short> wu = pack_wino(w, C.CO, C.CI, r);
+        std::vector<unsigned short> wu = pack_wino(w, C.CO, C.CI, r, !count_only_);
         C.wu = (unsigned short*)upload_bytes(wu.data(), wu.size() * sizeof(unsigned short));
     }
     conv_[name] = C;
@@ -1452,16 +1337,15 @@ void GpuBackend::upload_all()
         for (int b = 0; b < wt.depths[s]; ++b) {
             const std::string p = L + ".residual_group.blocks." + std::to_string(b);
             upload_norm(p + ".norm1");
-            for (const char* n : {".norm2.weight", ".norm2.bias", ".attn.relative_position_bias_table",
+            for (const char* n : {".attn.relative_position_bias_table",
                                   ".conv_block.cab.3.attention.1.weight",
                                   ".conv_block.cab.3.attention.1.bias",
                                   ".conv_block.cab.3.attention.3.weight",
                                   ".conv_block.cab.3.attention.3.bias"})
                 upload_raw(p + n);
             upload_attn(p + ".attn.qkv", p + ".attn.proj", p + ".norm1", p + ".attn.relative_position_bias_table");
-            upload_linear(p + ".mlp.fc1");
-            upload_linear(p + ".mlp.fc2");
-            upload_mlpx(p + ".mlp");
+            upload_tail(p + ".attn.proj", p + ".mlp", p + ".norm2", cab_fold_ ? p + ".conv_block.cab." : std::string(),
+                        p + ".norm1");
             const float xin = 1.0f / norm_scale_.at(p + ".norm1");
             if (cab_fold_) {
                 const std::string c = p + ".conv_block.cab.";
@@ -1486,12 +1370,9 @@ void GpuBackend::upload_all()
         }
         const std::string p = L + ".residual_group.overlap_attn";
         upload_norm(p + ".norm1");
-        for (const char* n : {".norm2.weight", ".norm2.bias", ".relative_position_bias_table"})
-            upload_raw(p + n);
+        upload_raw(p + ".relative_position_bias_table");
         upload_attn(p + ".qkv", p + ".proj", p + ".norm1", p + ".relative_position_bias_table");
-        upload_linear(p + ".mlp.fc1");
-        upload_linear(p + ".mlp.fc2");
-        upload_mlpx(p + ".mlp");
+        upload_tail(p + ".proj", p + ".mlp", p + ".norm2", std::string(), p + ".norm1");
         upload_conv(L + ".conv");
     }
     upload_raw("norm.weight");
@@ -1573,7 +1454,7 @@ std::vector<std::pair<float**, size_t>> GpuBackend::layout(const Weights& wt_, c
         {&a.t1, T * t1_stride},
         {&a.cab_part, cab_fold_ ? (size_t)(p.hp / 16) * (p.wp / 16) * CAB_NSUM * CAB_CS : 0},
         {&a.w2g, cab_fold_ ? C * CAB_K2 : 0},
-        {&a.w2gx, cab_fold_ ? WC_CHUNK : 0},  // 2 chunks of bf16
+        {&a.w2gx, cab_fold_ ? (size_t)CAB_W2GX : 0},
         {&a.bias2, cab_fold_ ? C : 0},
         {&a.t2, cab_fold_ ? 0 : T * C},
         {&a.partial, cab_fold_ ? 0 : nblk * C},
@@ -1634,92 +1515,6 @@ void GpuBackend::gemm(const DevLinear& L, const float* a, int lda, long M, float
 }
 
 // x = x + fc2(gelu(fc1(a_.xn))), in place; with a norm also a_.xn = norm(x).
-// The split-bf16 C = 180 projection tail: out = res + ao . Wp^T + bias (with
-// aux: + aux * gate * cscale), and with xn: xn = LN2(out) by (nw, nb).
-void run_projx180(hipStream_t s, const DevLinear& proj, const float* ao, const float* res, float* out, float* xn,
-                  const float* nw, const float* nb, const float* aux, const float* gate, float cscale, long M)
-{
-    if (!proj.wx || proj.K != 180 || proj.N != 180) throw Error("projx180: needs the pre-split 180 x 180 projection");
-    if (M > 0x7fffffffL) throw Error("projx180: too many rows");
-    TailXArgs q{};
-    q.a = ao;
-    q.res = res;
-    q.out = out;
-    q.xn = xn;
-    q.w = proj.wx;
-    q.bias = proj.b;
-    q.nw = nw;
-    q.nb = nb;
-    q.M = (int)M;
-    q.eps = 1e-5f;
-    q.aux = aux;
-    q.gate = gate;
-    q.cscale = cscale;
-    launch(s, aux ? "hat_projx180_hab" : "hat_projx180", (unsigned)wx_tiles((int)M), 1, 1, WX_THREADS, q);
-}
-
-// The split-bf16 C = 180 MLP: x = x + fc2(gelu(fc1(norm2(x)))) + b2 (+ xn =
-// LN(x)), norm2 by (n2w, n2b) formed in the kernel from the x rows.
-void run_mlpx180(hipStream_t s, const DevMlpX& m, const float* b2, const float* n2w, const float* n2b, float* x,
-                 float* xn_out, const float* nw, const float* nb, long M)
-{
-    if (m.C != 180) throw Error("mlpx180: needs the pre-split C = 180 MLP");
-    if (M > 0x7fffffffL) throw Error("mlpx180: too many rows");
-    TailXArgs q{};
-    q.a = x;
-    q.inw = n2w;
-    q.inb = n2b;
-    q.res = x;
-    q.out = x;
-    q.xn = nw ? xn_out : nullptr;
-    q.w = m.w;
-    q.b2 = b2;
-    q.nw = nw;
-    q.nb = nb;
-    q.M = (int)M;
-    q.eps = 1e-5f;
-    launch(s, nw ? "hat_mlpx180_ln" : "hat_mlpx180", (unsigned)wx_tiles((int)M), 1, 1, WX_THREADS, q);
-}
-
-// The C = 180 tail: with the fused weights and a form hat_habx180* has (the
-// HAB's with the unfolded CAB's gated conv2 output aux and the next norm, the
-// OCAB's with neither) one kernel with x' kept on the chip; otherwise the
-// projection writes x' (hat_projx180*) and the MLP forms norm2(x') from the
-// rows it reads (hat_mlpx180*). out may alias res.
-void run_tailx180(hipStream_t s, const DevLinear& proj, const DevMlpX& mlp, const float* b2, const float* ao,
-                  const float* res, float* out, float* xn, const float* n2w, const float* n2b, const float* aux,
-                  const float* gate, float cscale, const float* nw, const float* nb, long M)
-{
-    if (!proj.wx || proj.K != 180 || proj.N != 180 || mlp.C != 180)
-        throw Error("tailx180: needs the pre-split C = 180 projection and MLP");
-    if (M > 0x7fffffffL) throw Error("tailx180: too many rows");
-    if (mlp.wf && mlp.b1x && (aux != nullptr) == (nw != nullptr)) {
-        TailXArgs f{};
-        f.a = ao;
-        f.res = res;
-        f.out = out;
-        f.xn = nw ? xn : nullptr;
-        f.w = proj.wx;
-        f.wm = mlp.wf;
-        f.b1x = mlp.b1x;
-        f.bias = proj.b;
-        f.b2 = b2;
-        f.aux = aux;
-        f.gate = gate;
-        f.cscale = cscale;
-        f.inw = n2w;
-        f.inb = n2b;
-        f.nw = nw;
-        f.nb = nb;
-        f.M = (int)M;
-        f.eps = 1e-5f;
-        launch(s, aux ? "hat_habx180_hab_ln" : "hat_habx180", (unsigned)wx_tiles((int)M), 1, 1, WX_THREADS, f);
-        return;
-    }
-    run_projx180(s, proj, ao, res, out, nullptr, n2w, n2b, aux, gate, cscale, M);
-    run_mlpx180(s, mlp, b2, n2w, n2b, out, xn, nw, nb, M);
-}
-
 void GpuBackend::mlp(const std::string& prefix, float* x, int epi, const std::string& norm)
 {
     GemmEpilogue e;
@@ -1761,18 +1556,24 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
         // CAB, folded: conv1 + GELU here, the gate inside the attention
         // launch (its first block), conv2 inside the tail's projection.
         const DevLinear& proj = lin_.at(p + ".attn.proj");
-        auto mx = mlpx_.find(p + ".mlp");
-        const bool split = proj.wx && C == 144 && mx != mlpx_.end();  // the split tail runs
+        auto tl = tail_.find(p + ".mlp");
+        const bool split = tl != tail_.end();  // the split tail runs
         CabGateArgs gate{};
         run_cab(stream_, cab_.at(p), a_.xn, H, W, proj.b, wt_.conv_scale, wt_.squeezed, a_.t1, a_.cab_part,
-                split ? nullptr : a_.w2g, a_.bias2, a_.gate, (unsigned short*)a_.w2gx, &gate);
+                split ? nullptr : a_.w2g, a_.bias2, a_.gate, (unsigned short*)a_.w2gx,
+                split ? tl->second.ts : 1.0f, split ? tl->second.gs : 1.0f, &gate);
         gemm(lin_.at(p + ".attn.qkv"), a_.xn, C, T, a_.qkv, 0, EPI_QKV);
         attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, &gate);
         if (split) {
-            // split-bf16: proj + gated conv2 + shortcut + norm2, then the MLP + next norm1
-            run_tailx(stream_, true, proj, mx->second, lin_.at(p + ".mlp.fc2").b, a_.ao, x_in, x_out, a_.xn, a_.t1,
-                      (const unsigned short*)a_.w2gx, a_.bias2, raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"),
-                      raw_.at(next_norm + ".weight"), raw_.at(next_norm + ".bias"), H, W);
+            // proj + gated conv2 + shortcut, norm2, the MLP + next norm1
+            TailCabIn cab;
+            cab.t1 = a_.t1;
+            cab.w2gx = (const unsigned short*)a_.w2gx;
+            cab.H = H;
+            cab.W = W;
+            run_tailx(stream_, tl->second, a_.ao, x_in, x_out, a_.xn, a_.bias2, lin_.at(p + ".mlp.fc2").b,
+                      raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), raw_.at(next_norm + ".weight"),
+                      raw_.at(next_norm + ".bias"), T, cab);
             return;
         }
         run_hab_tail(stream_, proj, lin_.at(p + ".mlp.fc1"), lin_.at(p + ".mlp.fc2"), a_.ao, x_in, x_out, a_.xn, a_.t1,
@@ -1796,14 +1597,16 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
     gemm(lin_.at(p + ".attn.qkv"), a_.xn, C, T, a_.qkv, 0, EPI_QKV);
     attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, nullptr, &se);
     const DevLinear& proj = lin_.at(p + ".attn.proj");
-    auto mx = mlpx_.find(p + ".mlp");
-    if (proj.wx && C == 180 && mx != mlpx_.end() && mx->second.C == 180) {
-        // split-bf16: projection + gated conv branch + shortcut, norm2, the
-        // MLP + residual + next norm
-        run_tailx180(stream_, proj, mx->second, lin_.at(p + ".mlp.fc2").b, a_.ao, x_in, x_out, a_.xn,
-                     raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), a_.t2, a_.gate, wt_.conv_scale,
-                     next_norm.empty() ? nullptr : raw_.at(next_norm + ".weight"),
-                     next_norm.empty() ? nullptr : raw_.at(next_norm + ".bias"), T);
+    auto tl = tail_.find(p + ".mlp");
+    if (tl != tail_.end() && C == 180) {
+        // projection + gated conv branch + shortcut, norm2, the MLP + residual + next norm
+        TailCabIn cab;
+        cab.aux = a_.t2;
+        cab.gate = a_.gate;
+        cab.cscale = wt_.conv_scale;
+        run_tailx(stream_, tl->second, a_.ao, x_in, x_out, a_.xn, proj.b, lin_.at(p + ".mlp.fc2").b,
+                  raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), raw_.at(next_norm + ".weight"),
+                  raw_.at(next_norm + ".bias"), T, cab);
         return;
     }
     gemm(proj, a_.ao, C, T, x_out, C, EPI_HAB_LN, x_in, a_.t2, a_.gate, a_.xn, p + ".norm2");
@@ -1821,11 +1624,10 @@ void GpuBackend::ocab(int stage, float* x)
     attention(p + ".relative_position_bias_table", true, 0);
     const DevLinear& proj = lin_.at(p + ".proj");
     const DevLinear &fc1 = lin_.at(p + ".mlp.fc1"), &fc2 = lin_.at(p + ".mlp.fc2");
-    auto mx = mlpx_.find(p + ".mlp");
-    if (proj.wx && C == 144 && mx != mlpx_.end()) {
-        // split-bf16: projection + shortcut + norm2, then the MLP + residual
-        run_tailx(stream_, false, proj, mx->second, fc2.b, a_.ao, x, x, a_.xn, nullptr, nullptr, proj.b,
-                  raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), nullptr, nullptr, plan_.hp, plan_.wp);
+    auto tl = tail_.find(p + ".mlp");
+    if (tl != tail_.end()) {
+        run_tailx(stream_, tl->second, a_.ao, x, x, nullptr, proj.b, fc2.b, raw_.at(p + ".norm2.weight"),
+                  raw_.at(p + ".norm2.bias"), nullptr, nullptr, T, TailCabIn{});
         return;
     }
     if (hab_tail_fits(proj, fc1, fc2)) {
@@ -1833,11 +1635,6 @@ void GpuBackend::ocab(int stage, float* x)
         run_hab_tail(stream_, proj, fc1, fc2, a_.ao, x, x, nullptr, nullptr,
                      nullptr, proj.b, raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), nullptr, nullptr,
                      plan_.hp, plan_.wp);
-        return;
-    }
-    if (proj.wx && C == 180 && mx != mlpx_.end() && mx->second.C == 180) {
-        run_tailx180(stream_, proj, mx->second, fc2.b, a_.ao, x, x, nullptr, raw_.at(p + ".norm2.weight"),
-                     raw_.at(p + ".norm2.bias"), nullptr, nullptr, 0.0f, nullptr, nullptr, T);
         return;
     }
     gemm(proj, a_.ao, C, T, x, C, EPI_RESID_LN, x, nullptr, nullptr, a_.xn, p + ".norm2");
@@ -2383,45 +2180,36 @@ private:
 };
 
 // A linear of the op entry points, packed as the backend packs it
-// (upload_linear): for the shapes a split-bf16 kernel takes (the qkv of 144 /
-// 180 channels, the 144 / 180 projection) the split weights, so that an op runs
-// the forward's kernels; for the others (and with kBias, where only the bias is
-// read, neither) the FP32 rows.
+// (upload_linear, which explains out and in): a qkv of 144 or 180 channels as
+// hat_gemmx_qkv takes it, so that an op runs the forward's kernels, others as
+// FP32 rows; with kBias only the bias (a split tail holds the weights).
 struct OpLinear {
-    enum Split { kNone, kQkv, kProj, kBias };
+    enum Form { kNone, kQkv, kBias };
     DevLinear L;
     size_t iw = 0, ib = 0, ix = 0;
     bool fp32 = false, split = false;
-    // out, in: as GpuBackend::upload_linear's
-    OpLinear(OpArena& ar, const float* wt, const float* bias, int N, int K, Split sp = kNone, const float* out = nullptr,
+    OpLinear(OpArena& ar, const float* wt, const float* bias, int N, int K, Form form = kNone, const float* out = nullptr,
              float in = 1.0f)
     {
         L.N = N;
         L.K = K;
-        std::vector<float> ws, bs;
-        if (out || in != 1.0f) {
-            ws.assign(wt, wt + (size_t)N * K);
-            bs.assign(bias, bias + N);
-            for (int n = 0; n < N; ++n) {
-                const float f = out ? out[n / (N / 3)] : 1.0f;
-                for (int k = 0; k < K; ++k) ws[(size_t)n * K + k] *= f * in;
-                bs[n] *= f;
-            }
-            ib = ar.keep(std::move(bs));
-        } else {
-            ib = ar.add(N, bias);
-        }
-        const float* sw = ws.empty() ? wt : ws.data();
-        std::vector<unsigned short> xs;
-        if (sp == kQkv && ((N == 432 && K == 144) || (N == 540 && K == 180)))
-            xs = split_qkv(wt, N, K, out, in, L.oscale);
-        else if (sp == kProj && N == 144 && K == 144)
-            xs = pack_linear_x(sw, N, K);
-        else if (sp == kProj && N == 180 && K == 180)
-            xs = pack_linear_x180(sw);
         L.Kp = (K + 15) / 16 * 16;
-        if ((split = !xs.empty())) ix = ar.keep(std::move(xs));
-        else if ((fp32 = sp != kBias)) iw = ar.keep(pack_linear(sw, N, K, &L.Kp));
+        std::vector<float> bs(bias, bias + N);
+        if (out)
+            for (int n = 0; n < N; ++n) bs[n] *= out[n / (N / 3)];
+        ib = ar.keep(std::move(bs));
+        if (form == kQkv && ((N == 432 && K == 144) || (N == 540 && K == 180))) {
+            split = true;
+            ix = ar.keep(split_qkv(wt, N, K, out, in, L.oscale));
+        } else if (form != kBias) {
+            fp32 = true;
+            std::vector<float> ws(wt, wt + (size_t)N * K);
+            for (int n = 0; n < N; ++n) {
+                const float f = (out ? out[n / (N / 3)] : 1.0f) * in;
+                for (int k = 0; k < K; ++k) ws[(size_t)n * K + k] *= f;
+            }
+            iw = ar.keep(pack_linear(ws.data(), N, K, &L.Kp));
+        }
     }
     void bind(const OpArena& ar)
     {
@@ -2431,29 +2219,21 @@ struct OpLinear {
     }
 };
 
-// An op's MLP pre-split for the fused tails (hat_habx, hat_habx180), as
-// upload_mlpx packs it; other shapes (fused false) run the FP32 kernels.
-struct OpMlpX {
-    DevMlpX m;
-    size_t iwf = 0, ib1 = 0;
-    bool fused = false;
-    OpMlpX(OpArena& ar, const float* w1, const float* b1, const float* w2, int c, size_t hid)
+// An op's projection and MLP for the split tail, as upload_tail packs them.
+struct OpTail {
+    DevTail t;
+    size_t iw, iwm, ib1;
+    OpTail(OpArena& ar, TailPack p) : t(p.t)
     {
-        std::vector<unsigned short> wf;
-        std::vector<float> b1x;
-        if (c == 144 && hid == 288) pack_mlp_xf(w1, b1, w2, &wf, &b1x);
-        else if (c == 180 && hid == 360) pack_mlp_xf180(w1, b1, w2, &wf, &b1x);
-        else return;
-        fused = true;
-        m.C = c;
-        iwf = ar.keep(std::move(wf));
-        ib1 = ar.keep(std::move(b1x));
+        iw = ar.keep(std::move(p.w));
+        iwm = ar.keep(std::move(p.wm));
+        ib1 = ar.keep(std::move(p.b1x));
     }
     void bind(const OpArena& ar)
     {
-        if (!fused) return;
-        m.wf = (unsigned short*)ar.ptr(iwf);
-        m.b1x = ar.ptr(ib1);
+        t.w = (unsigned short*)ar.ptr(iw);
+        t.wm = (unsigned short*)ar.ptr(iwm);
+        t.b1x = ar.ptr(ib1);
     }
 };
 
@@ -2462,9 +2242,10 @@ double op_linear_bound(const float* w, const float* b, int n0, int n1, int K, do
 {
     double worst = 0.0;
     for (int n = n0; n < n1; ++n) {
-        double v = 0.0;
-        for (int k = 0; k < K; ++k) v += std::fabs((double)w[(size_t)n * K + k]);
-        v = v * mx + std::fabs((double)b[n]);
+        double l1[4] = {};
+        for (int k = 0; k < K; k += 4)
+            for (int i = 0; i < 4 && k + i < K; ++i) l1[i] += std::fabs((double)w[(size_t)n * K + k + i]);
+        const double v = (l1[0] + l1[1] + l1[2] + l1[3]) * mx + std::fabs((double)b[n]);
         if (std::isnan(v)) return v;
         worst = std::max(worst, v);
     }
@@ -2594,27 +2375,33 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
     const size_t T = (size_t)hp * wp, hid = (size_t)c * mlp_ratio;
     hipStream_t s = nullptr;  // the null stream, as in op_swmsa
     {
-        // norm1 into f16's range, as GpuBackend::upload_norm
-        const float s1 = c == 144 || c == 180 ? f16_scale(ln_bound(n1w, n1b, c)) : 1.0f;
-        std::vector<float> n1(2 * (size_t)c);
-        for (int i = 0; i < c; ++i) n1[i] = n1w[i] * s1, n1[c + i] = n1b[i] * s1;
+        // the split tail's shapes; the norms into f16's range where split-f16
+        // kernels read them, as GpuBackend::upload_norm
+        const bool wide = c == 144 || c == 180, fits = wide && hid == 2 * (size_t)c;
+        const float s1 = wide ? f16_scale(ln_bound(n1w, n1b, c)) : 1.0f,
+                    s2 = fits ? f16_scale(ln_bound(n2w, n2b, c)) : 1.0f;
+        std::vector<float> n1(2 * (size_t)c), n2(2 * (size_t)c);
+        for (int i = 0; i < c; ++i) {
+            n1[i] = n1w[i] * s1, n1[c + i] = n1b[i] * s1;
+            n2[i] = n2w[i] * s2, n2[c + i] = n2b[i] * s2;
+        }
         OpArena ar;
         const size_t ix = ar.add(T * c, x), iwork = ar.add(T * c), ixn = ar.add(T * c), iq = ar.add(3 * T * c),
                      iao = ar.add(T * c), itab = ar.add(1521 * (size_t)heads, table), i1w = ar.add(c, n1.data()),
-                     i1b = ar.add(c, n1.data() + c), i2w = ar.add(c, n2w), i2b = ar.add(c, n2b);
-        OpMlpX mx(ar, fc1_w, fc1_b, fc2_w, c, hid);
+                     i1b = ar.add(c, n1.data() + c), i2w = ar.add(c, n2.data()), i2b = ar.add(c, n2.data() + c);
         const QkvScale sc = qkv_scale(ln_linear_bound(qkv_w, qkv_b, n1w, n1b, 0, c, c),
                                       ln_linear_bound(qkv_w, qkv_b, n1w, n1b, c, 2 * c, c),
                                       ln_linear_bound(qkv_w, qkv_b, n1w, n1b, 2 * c, 3 * c, c), D);
         const float osc[3] = {sc.q, sc.k, sc.v};
-        // the split tails read only fc2's bias of these two
-        const OpLinear::Split mlp = mx.fused ? OpLinear::kBias : OpLinear::kNone;
+        std::unique_ptr<OpTail> tail;
+        if (fits) tail.reset(new OpTail(ar, pack_tail(proj_w, fc1_w, fc1_b, fc2_w, n2w, n2b, c, sc.v, s2, nullptr)));
+        const OpLinear::Form form = fits ? OpLinear::kBias : OpLinear::kNone;
         OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc, 1.0f / s1),
-            proj(ar, proj_w, proj_b, c, c, mx.fused ? OpLinear::kProj : OpLinear::kNone, nullptr, 1.0f / sc.v),
-            fc1(ar, fc1_w, fc1_b, (int)hid, c, mlp), fc2(ar, fc2_w, fc2_b, c, (int)hid, mlp);
-        const size_t ih = ar.add(mx.fused || mlp_fused(fc1.L, fc2.L) ? 1 : T * hid);
+            proj(ar, proj_w, proj_b, c, c, form, nullptr, 1.0f / sc.v), fc1(ar, fc1_w, fc1_b, (int)hid, c, form),
+            fc2(ar, fc2_w, fc2_b, c, (int)hid, form);
+        const size_t ih = ar.add(fits || mlp_fused(fc1.L, fc2.L) ? 1 : T * hid);
         ar.commit();
-        mx.bind(ar);
+        if (tail) tail->bind(ar);
         for (OpLinear* l : {&qkv, &proj, &fc1, &fc2}) l->bind(ar);
         float *dx = ar.ptr(ix), *dwork = ar.ptr(iwork), *dxn = ar.ptr(ixn), *dq = ar.ptr(iq), *dao = ar.ptr(iao),
               *dtab = ar.ptr(itab), *d1w = ar.ptr(i1w), *d1b = ar.ptr(i1b), *d2w = ar.ptr(i2w), *d2b = ar.ptr(i2b);
@@ -2630,12 +2417,9 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
             run_ln(s, dx, dxn, d1w, d1b, (long)T, c);
             run_gemm(s, qkv.L, dxn, c, (long)T, dq, 0, EPI_QKV, none, heads, D, 0.f);
             run_attn(s, dq, dtab, dao, pl, heads, D, true, 0, sc.ok);
-            if (mx.fused && c == 144) {
-                run_tailx(s, false, proj.L, mx.m, fc2.L.b, dao, dx, dwork, dxn, nullptr, nullptr, proj.L.b, d2w, d2b,
-                          nullptr, nullptr, hp, wp);
-            } else if (mx.fused) {
-                run_tailx180(s, proj.L, mx.m, fc2.L.b, dao, dx, dwork, nullptr, d2w, d2b, nullptr, nullptr, 0.f,
-                             nullptr, nullptr, (long)T);
+            if (tail) {
+                run_tailx(s, tail->t, dao, dx, dwork, nullptr, proj.L.b, fc2.L.b, d2w, d2b, nullptr, nullptr, (long)T,
+                          TailCabIn{});
             } else {
                 run_gemm(s, proj.L, dao, c, (long)T, dwork, c, EPI_RESID_LN, resid_ln, heads, D, 0.f);
                 run_mlp(s, fc1.L, fc2.L, dxn, (long)T, dwork, dwork, EPI_RESID, none, ar.ptr(ih));

@@ -26,9 +26,8 @@ public:
 struct DevLinear {
     float* w = nullptr;  // [N][Kp]
     float* b = nullptr;  // [N]
-    // The same weights split into three bf16 parts for the split-bf16 kernels
-    // (qkv: pack_linear_ws; projection: pack_linear_x, pack_linear_x180), or
-    // null where the FP32 kernels run.
+    // qkv: the same weights split for hat_gemmx_qkv* (pack_linear_ws), or null
+    // where the FP32 kernels run (and w is null where they do not).
     unsigned short* wx = nullptr;
     // qkv: what the split-f16 kernel multiplies q, k and v by (GemmArgs::oscale)
     float oscale[3] = {1.0f, 1.0f, 1.0f};
@@ -53,12 +52,15 @@ struct DevCab {
 // hat_cab_conv1's A-operand layout (CX_WPACK elements).
 std::vector<unsigned short> pack_cab_conv1(const float* w);
 
-// hat_mlpx's weights: the packed slices and b1 in fc1's row order.
-struct DevMlpX {
-    unsigned short* w = nullptr;  // C = 144: 24 weight chunks (pack_mlp_x); 180: 48 (pack_mlp_x180)
-    unsigned short* wf = nullptr;  // the same in the fused tail's input order (pack_mlp_xf, pack_mlp_xf180)
-    float* b1x = nullptr;          // fc1's bias in the fused tail's row order (pack_mlp_xf, pack_mlp_xf180)
-    int C = 144;
+// A block's second half on split-f16 (tailx.hip): the projection's and the MLP's
+// packed steps, fc1's bias in the parts' row order, and the scales (TailXArgs).
+struct DevTail {
+    unsigned short* w = nullptr;
+    unsigned short* wm = nullptr;
+    float* b1x = nullptr;
+    int C = 0;  // 144 or 180
+    float ps = 1.0f, h1 = 1.0f, hs = 1.0f, ms = 1.0f;  // hs: the hidden units' scale
+    float ts = 1.0f, gs = 1.0f;                        // folded CAB: t1's and w2gx's scales (ps = ts gs)
 };
 
 struct DevConv {
@@ -91,57 +93,45 @@ struct QkvScale {
 };
 QkvScale qkv_scale(double bq, double bk, double bv, int head_dim);
 
-// Host-side repacking (also used by the selftest and the op entry points).
+// Host-side repacking (also used by the selftest and the op entry points). fill:
+// false leaves zeros, for the counting pass that needs only the sizes.
 std::vector<float> pack_linear(const float* w, int N, int K, int* Kp);
-// [N][144] -> per 144-row slice, five weight chunks (one per 32-k step) of
-// three bf16 planes [144][32] (k-groups swizzled as in pack_linear_ws): w =
-// p0 + p1 + p2, each part the round-to-nearest bf16 of what the earlier ones
-// leave; the fifth step (k = 128..143) packed, two parts per MFMA operand
-// (split_half_step). The tails add the bias in fp32.
-std::vector<unsigned short> pack_linear_x(const float* w, int N, int K);
 // hat_gemmx_qkv's weight-stationary slices: per slice (144 rows at K = 144, 192
 // at 180) five or six chunks of two f16 planes [rows][32], each row's 16-byte
 // k-groups swizzled (ws_slot), WS_CHUNK elements apart; K = 144's fifth step
 // packed (split2_half_step). w = p0 + p1, each part the round-to-nearest f16 of
 // what the one before leaves; q's, k's and v's rows times ws[0..2] first.
-std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const float (&ws)[3]);
+std::vector<unsigned short> pack_linear_ws(const float* w, int N, int K, const float (&ws)[3], bool fill = true);
 // The largest |w[i]|, i < n (NaN if there is one).
 double abs_max(const float* w, size_t n);
-// The C = 144 MLP (fc1 [288][144] + b1, fc2 [144][288]) for hat_mlpx: per
-// third of the hidden layer eight weight chunks - five of fc1's 96 rows (b1
-// as their column k = 144), then three of fc2 on those units - with fc1's
-// rows in the order that leaves its output in fc2's operand layout
-// (tailx.hip).
-void pack_mlp_x(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w);
-// The same for the fused tails (hat_habx*), whose fc1 reads x' in the order a
-// lane holds the projection's accumulators: input position k = 32 ks + 8 g + j
-// of steps 0..3 is channel mlpx_fused_channel(k), step 4 (channels 128 ..
-// 143) is packed as the K = 144 linears' last step, and b1 comes back in b1x
-// (the thirds' permuted row order), added to fc1's output in fp32.
-void pack_mlp_xf(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w,
-                 std::vector<float>* b1x);
-int mlpx_fused_channel(int k);
-// The C = 180 projection [180][180] for hat_projx180*: six chunks (one per
-// 32-k step, k 180..191 zero) of three bf16 planes [192][32] (rows 180..191
-// zero), k-groups swizzled as in pack_linear_ws, MX180_SLOT elements apart;
-// the bias stays FP32 (added in the epilogue).
-std::vector<unsigned short> pack_linear_x180(const float* w);
-// The C = 180 MLP (fc1 [360][180] + b1, fc2 [180][360]) for hat_mlpx180: per
-// part of MX180_HID hidden units six fc1 chunks (64 permuted rows, b1 as
-// their column k = 180) then two fc2 chunks (192 rows), 48 chunks in all.
-void pack_mlp_x180(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w);
-// The same for the fused C = 180 tails (hat_habx180*), whose fc1 reads x' in
-// the order a lane holds the projection's accumulators: input position k =
-// 32 ks + 8 g + j is channel mlpx180_fused_channel(k) (zero where that is -1),
-// and b1 comes back in b1x (the parts' permuted row order), added to fc1's
-// output in fp32.
-void pack_mlp_xf180(const float* w1, const float* b1, const float* w2, std::vector<unsigned short>* w,
-                    std::vector<float>* b1x);
-int mlpx180_fused_channel(int k);
+// The tails' steps (tailx.hip), every weight times a scale and split into two f16
+// parts; both arrays end in TX_PAD zeros. The projection [C][C]: its k-steps. The
+// MLP (fc1 [2C][C] + b1, fc2 [C][2C]): per part of tailx_hu(C) units fc1's k-steps
+// (the unit rows in tailx_unit's order, column k the channel tailx_channel(C, k))
+// and fc2's, fc1 times s1 and fc2 times s2; b1 times hs in the parts' row order.
+std::vector<unsigned short> pack_tail_proj(const float* w, int C, float s, bool fill = true);
+void pack_tail_mlp(const float* w1, const float* b1, const float* w2, int C, float s1, float s2, float hs,
+                   std::vector<unsigned short>* w, std::vector<float>* b1x, bool fill = true);
+int tailx_channel(int C, int k);
+// The scales and packed weights of a tail whose attention output comes times sv
+// and norm2 (n2w, n2b unscaled) times sn; cab (if set): the folded CAB's bound of
+// |t1| and largest |cscale * conv2 weight|, which share the projection's scale.
+struct TailPack {
+    std::vector<unsigned short> w, wm;
+    std::vector<float> b1x;
+    DevTail t;  // the scales; no device pointers
+};
+struct TailCab {
+    double t1, w2;
+};
+void tail_scales(const DevTail& t, hatk::TailXArgs* f);
+TailPack pack_tail(const float* wp, const float* w1, const float* b1, const float* w2, const float* n2w, const float* n2b,
+                   int C, float sv, float sn, const TailCab* cab, bool fill = true);
+
 // Winograd U = G g G^T of a 3x3 conv [CO][CI][3][3] (formed in double), split
 // into three bf16 parts in the layout convwino.hip streams:
 // [32-channel chunk][point][16-channel tile][part][lane][8].
-std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r);
+std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r, bool fill = true);
 std::vector<float> pack_conv(const float* w, const float* b, int CO, int CI, int r,
                              std::vector<float>* bias_out, int* CIp, int* COp);
 // A Winograd conv kernel (convwino.hip) over `tiles` 8 x 16 tiles in `ncb`
@@ -204,7 +194,7 @@ private:
     std::map<std::string, DevLinear> lin_;
     std::map<std::string, DevConv> conv_;
     std::map<std::string, DevCab> cab_;
-    std::map<std::string, DevMlpX> mlpx_;  // C = 144 MLPs (blocks and OCABs) for hat_mlpx
+    std::map<std::string, DevTail> tail_;  // by MLP name: blocks and OCABs that run tailx.hip
     std::map<std::string, bool> attn_f16_;  // by bias table name: the split-f16 attention runs
     bool cab_fold_ = false;  // the C = 144, 6-channel CAB runs folded
     std::vector<void*> owned_;
@@ -257,8 +247,9 @@ private:
     void* upload_bytes(const void* src, size_t bytes);
     void upload_raw(const std::string& name);
     // out[3]: the factors of a qkv's q, k and v outputs (weights and bias), or
-    // null; in: the factor of every weight (the inverse of its input's scale).
-    void upload_linear(const std::string& name, const float* out = nullptr, float in = 1.0f);
+    // null; in: the factor of every weight (the inverse of its input's scale);
+    // bias_only: the weights go up elsewhere (upload_tail).
+    void upload_linear(const std::string& name, const float* out = nullptr, float in = 1.0f, bool bias_only = false);
     // A norm whose output feeds split-f16 kernels: its weight and bias times the
     // power of two that takes every row it can produce to f16's range.
     void upload_norm(const std::string& name);
@@ -267,7 +258,11 @@ private:
     // split-f16 attention where the bounds allow it (attn_f16_ of its table).
     void upload_attn(const std::string& qkv, const std::string& proj, const std::string& ln, const std::string& table);
     void upload_conv(const std::string& name, int r = 0, float in = 1.0f);  // in: as upload_linear's
-    void upload_mlpx(const std::string& name);
+    // the split-f16 tail of a block, where its shapes have one (upload_attn first;
+    // conv: the folded CAB's prefix, or empty)
+    void upload_tail(const std::string& proj, const std::string& mlp, const std::string& norm2, const std::string& cab,
+                     const std::string& norm1);
+    float v_scale_ = 1.0f;  // of the attention uploaded last
     void ensure_plan(int h, int w);
     void free_plan();
     // With bands: the output's row bands [y0, y1) in the order they are

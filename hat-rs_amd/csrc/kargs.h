@@ -86,15 +86,18 @@ struct GemmArgs {
 // tile nt (2 x 32 rows, row tap*6 + co, rows 54.. zero) and part (3), the
 // 32x32x16 A operand of each lane (row l % 32, channels 16 ks + 8 (l / 32) .. +7)
 #define CX_WPACK (9 * 2 * 3 * 64 * 8)
+// floats of the gated conv2 weights' buffer (CabGateArgs::w2gx: 9216 used)
+#define CAB_W2GX 20480
 #define CAB_NSUM 5           // per-tile sums: whole tile, row 0, row H-1, col 0, col W-1
 
 struct CabConvArgs {
     const float* xn;     // [H*W][144]
     const unsigned short* w;  // [9][2][3][64][8] bf16: step ks, row tile nt, part, lane (CX_WPACK)
     const float* bias;   // [6]
-    float* t1;           // [H*W][8]: gelu(conv1(xn))
-    float* partial;      // [CAB_NSUM * 8][tiles] (value-major)
+    float* t1;           // [H*W][8]: ts * gelu(conv1(xn))
+    float* partial;      // [CAB_NSUM * 8][tiles] (value-major), of t1 as stored
     int H, W;            // multiples of 16
+    float ts;            // t1's scale (a power of two: the split tail's range)
 };
 
 struct CabGateArgs {
@@ -108,12 +111,13 @@ struct CabGateArgs {
     const float* wb;     // excite [144][sq]
     const float* bb;     // [144]
     const float* bproj;  // attention projection bias [144]
-    float* w2g;          // out (if set): cscale * gate[c] * conv2 weight, [144][CAB_K2] (k = tap*6 + ci)
+    float* w2g;          // out (if set): cscale * gate[c] * conv2 weight / ts, [144][CAB_K2] (k = tap*6 + ci)
     float* bias2;        // out: bproj + cscale * gate * b2, [144]
     float* gate;         // out: the gate itself [144]
     float cscale;
     int sq;
-    unsigned short* w2gx;  // out (if set): w2g as 2 weight chunks [3][144][32] (swizzled) for hat_projx_cab
+    unsigned short* w2gx;  // out (if set): w2g * gs as the split tail's two steps, [2][144][32] each (ws_slot)
+    float ts, gs;        // t1's scale; w2gx's scale (powers of two)
 };
 
 // Implicit-GEMM 3x3 convolution, stride 1, zero padding 1, NHWC.
@@ -246,17 +250,12 @@ struct HabTailArgs {
     int ldw1, ldw2;
 };
 
-// The C = 144 HAB / OCAB tail on split-bf16 MFMA as two kernels (tailx.hip):
-// hat_projx(_cab): out = x' = res + a . Wp^T (+ nb(t1) . W2g^T) + bias,
-//                  xn = LN(x') with nw / nb;
-// hat_mlpx(_ln):   out = res + fc2(gelu(fc1(a))) + b2 (+ xn = LN(out)).
-// Weight chunks of the split-bf16 tails (tailx.hip): one 32-k step of up to
-// 192 rows as three bf16 planes [rows][32], each row's four 16-byte k-groups g
-// stored at slot ws_slot(row, g) (ws_mma), WC_CHUNK elements apart (zeros after
-// the planes). A chunk is copied as loads of 1 KB, the same number from every
-// wave of a block: 144 rows take 27 (28 to share them out evenly), 96 rows 18
-// (20), 192 rows 36.
-#define WC_CHUNK 20480  // 40 x 512 >= 3 x 192 x 32
+// The HAB / OCAB tails on split-f16 MFMA (tailx.hip). Their weights are arrays
+// of 32-k steps, each step two f16 planes [rows][32] with row r's four 16-byte
+// k-groups g at slot ws_slot(r, g) (ws_mma2), copied to LDS as loads of 1 KB,
+// the same number from every wave of a block; the arrays end in TX_PAD elements
+// that those loads may read.
+#define TX_PAD 4096
 // The slot of row r's 16-byte k-group g in a 64-byte row of those planes. An
 // MFMA fragment read has lane i take rows r0 + i at one k-group, 16 bytes a
 // lane, and the LDS serves such reads 8 consecutive lanes at a time over its
@@ -264,17 +263,11 @@ struct HabTailArgs {
 // (r >> 1) & 3 gives the four row pairs of every 8 lanes four distinct slots
 // and the reads have no bank conflicts without padding (measured: none).
 constexpr int ws_slot(int r, int g) { return g ^ ((r >> 1) & 3); }
-// The MLP walks the hidden layer in thirds of MX_HID units: per third five
-// fc1 chunks (96 permuted rows, k = input channel) then three fc2 chunks (144
-// rows, k = the third's hidden units), 24 chunks in all.
-#define MX_HID 96
-// The C = 180 MLP (hat_mlpx180*) walks its 360 hidden units (384 with 24
-// zero units) in six parts of MX180_HID: per part six fc1 chunks (64 permuted
-// rows, k = input channel, b1 at k = 180) and two fc2 chunks (192 rows, 180
-// real, k = the part's units), 48 chunks in the swizzled [rows][32] layout of
-// the weight-stationary kernels, MX180_SLOT elements apart.
-#define MX180_HID 64
-#define MX180_SLOT (3 * 192 * 32)
+// The MLP walks the hidden layer in parts of tailx_hu units (C = 144: 288 in
+// three of 96; 180: 360 in twelve of 32, the last 24 of 384 zero): per part fc1's
+// k-steps (that many rows, permuted, the columns in the order a lane holds x'),
+// then fc2's (C rows in 16s, k = the part's units).
+constexpr int tailx_hu(int C) { return C == 144 ? 96 : 32; }
 // Their launch geometry (tailx): blocks of 4 waves, one 128-token row tile a block.
 #define WX_THREADS 256
 #define WX_ROWS 128
@@ -294,34 +287,28 @@ constexpr int wx_tiles(int M) { return (M + WX_ROWS - 1) / WX_ROWS; }
 constexpr int gemmx_qkv_groups(int cus, int ns) { return cus >= 8 * ns ? cus / (8 * ns) * 8 : 1; }
 
 struct TailXArgs {
-    const float* a;            // projx: attention output; mlpx (C = 144): x' rows, normed in the kernel by
-                               // (inw, inb); mlpx180: LN2(x') rows
-    const float* res;          // projx: block input; mlpx: x'
-    float* out;                // [M][144] (may alias res)
-    float* xn;                 // projx: LN2(x') when non-null; mlpx (LN): the next norm1 (may alias a)
-    const unsigned short* w;   // weight chunks (projx: 5, mlpx: 24)
-    const float* bias;         // projx: bias2 or the projection bias (mlpx: b1 is in its chunks)
-    const float* b2;           // mlpx: fc2 bias
-    const unsigned short* w2gx;  // projx_cab: the gate-scaled conv2 weights as 2 chunks (k = tap*6 + ci)
-    const float* t1;           // projx_cab: [M][CAB_CS] CAB conv1 output
-    const float* nw;
-    const float* nb;
-    int M, H, W;               // rows = the H x W plane
-    float eps;
-    // hat_projx180_hab (the unfolded CAB of the C = 180 family): out = x +
-    // proj + bias + aux * gate * cscale (aux: conv2's output [M][180])
-    const float* aux;
-    const float* gate;
-    float cscale;
-    // hat_mlpx(_ln): norm2's weight and bias, applied to the x' rows of a
-    const float* inw;
+    const float* a;             // [M][C] attention output, in v's scale
+    const float* res;           // [M][C] block input
+    float* out;                 // [M][C] (may alias res)
+    float* xn;                  // [M][C] the next norm of out (LN forms)
+    const unsigned short* w;    // the projection's steps
+    const unsigned short* wm;   // the MLP's steps, part by part
+    const unsigned short* w2gx; // CAB: the gate-scaled conv2 weights as 2 steps (k = tap*6 + ci)
+    const float* t1;            // CAB: [M][CAB_CS] CAB conv1 output (scaled)
+    const float* aux;           // HAB at C = 180: conv2's output [M][C]
+    const float* gate;          // and its gate [C]
+    const float* bias;          // projection bias (CAB: bias2)
+    const float* b1x;           // fc1's bias times the hidden scale, in the parts' row order
+    const float* b2;            // fc2's bias
+    const float* inw;           // norm2 (scaled)
     const float* inb;
-    // hat_habx*: the MLP's 24 weight chunks in the fused input order (w holds
-    // the projection's)
-    const unsigned short* wm;
-    // hat_habx*: fc1's bias in the thirds' permuted row order (added to fc1's
-    // output before the GELU)
-    const float* b1x;
+    const float* nw;            // the next norm
+    const float* nb;
+    int M, H, W;                // rows = the H x W plane (CAB)
+    float eps, cscale;
+    float ps, pi;               // the projection accumulators' scale and its inverse
+    float h1, g0, g1;           // fc1's accumulators to scaled hidden units; gelu_scaled's constants
+    float ms, mi;               // the output accumulators' scale and its inverse
 };
 
 struct LnArgs {

@@ -171,7 +171,7 @@ __device__ __forceinline__ void cab_conv1_body(const CabConvArgs& p)
                     }
                 }
 #pragma unroll
-            for (int co = 0; co < CAB_CC; ++co) v[r][co] = gelu(v[r][co]);
+            for (int co = 0; co < CAB_CC; ++co) v[r][co] = gelu(v[r][co]) * p.ts;
             float* dst = p.t1 + ((size_t)(y0 + oy) * W + x0 + ox) * CAB_CS;
             *(float4*)dst = make_float4(v[r][0], v[r][1], v[r][2], v[r][3]);
             *(float4*)(dst + 4) = make_float4(v[r][4], v[r][5], 0.f, 0.f);
@@ -276,7 +276,7 @@ __device__ __forceinline__ void cab_gate_body(const CabGateArgs& p, float* lds)
         s_S[tid] = s;
     }
     __syncthreads();
-    const float inv = 1.0f / ((float)H * (float)W);
+    const float inv = 1.0f / ((float)H * (float)W * p.ts);
     for (int c = tid; c < CAB_C; c += WAVES * 64) {
         float acc = 0.0f;
 #pragma unroll
@@ -307,27 +307,27 @@ __device__ __forceinline__ void cab_gate_body(const CabGateArgs& p, float* lds)
         for (int i = tid; i < CAB_C * CAB_K2; i += WAVES * 64) {
             const int c = i / CAB_K2, k = i - c * CAB_K2;
             const int tap = k / CAB_CC, ci = k - tap * CAB_CC;
-            p.w2g[i] = tap < 9 ? (p.cscale * s_gate[c]) * s_w2[(c * CAB_CC + ci) * 9 + tap] : 0.0f;
+            p.w2g[i] = tap < 9 ? (p.cscale * s_gate[c]) * s_w2[(c * CAB_CC + ci) * 9 + tap] / p.ts : 0.0f;
         }
-    // the same weights as the split tail's two weight chunks: [s][plane][c][32],
+    // the same weights as the split tail's two weight steps: [s][plane][c][32],
     // row c's k-group g at slot ws_slot(c, g), k = 32 s + j, zeros from k = 54;
     // one k-group (8 values, 16 bytes a plane) at a time
     if (p.w2gx) {
         constexpr int PLANE = CAB_C * 32;
         for (int u = tid; u < 2 * CAB_C * 4; u += WAVES * 64) {
             const int s = u / (CAB_C * 4), c = (u >> 2) - s * CAB_C, g = u & 3;
-            const float sc = p.cscale * s_gate[c];
+            const float sc = p.cscale * s_gate[c] * p.gs;
             float f[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int k = 32 * s + 8 * g + j, tap = k / CAB_CC, ci = k - tap * CAB_CC;
                 f[j] = tap < 9 ? sc * s_w2[(c * CAB_CC + ci) * 9 + tap] : 0.0f;
             }
-            u32x4 parts[3];
-            split3_x8(f, parts);
+            u32x4 parts[2];
+            split2_x8(f, parts);
 #pragma unroll
-            for (int pl = 0; pl < 3; ++pl)
-                *(u32x4*)(p.w2gx + (size_t)s * WC_CHUNK + pl * PLANE + c * 32 + ws_slot(c, g) * 8) = parts[pl];
+            for (int pl = 0; pl < 2; ++pl)
+                *(u32x4*)(p.w2gx + (size_t)(2 * s + pl) * PLANE + c * 32 + ws_slot(c, g) * 8) = parts[pl];
         }
     }
 }

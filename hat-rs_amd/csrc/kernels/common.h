@@ -216,12 +216,11 @@ __device__ __forceinline__ f32x16 mfma3(const u32x4 (&a)[2], const u32x4 (&b)[2]
     return mfma_f16(a[0], b[0], c);
 }
 
-// ---- weight chunks for the split-bf16 linears: one 32-k step of up to 192
-// rows as three bf16 planes [rows][32] with swizzled k-groups (ws_mma), packed
-// on the host WC_CHUNK elements apart. A block copies chunk c + 1 into one of
-// two LDS buffers while its waves multiply chunk c out of the other.
+// ---- weight steps for the split-f16 linears: one 32-k step of up to 192 rows
+// as two f16 planes [rows][32] with swizzled k-groups (ws_mma2), packed on the
+// host.
 
-// The NL loads (1 KB each) of one chunk into an LDS buffer, NL / WAVES from
+// The NL loads (1 KB each) of one stage into an LDS buffer, NL / WAVES from
 // every wave: wave w issues loads w, w + WAVES, ...; lane l of a load writes
 // 16 bytes at the load's LDS base + 16 l. Straight-line code: as a loop, the
 // per-load scalar bookkeeping (M0, the address, the counter and the branch)
@@ -231,7 +230,7 @@ __device__ __forceinline__ f32x16 mfma3(const u32x4 (&a)[2], const u32x4 (&b)[2]
 template <int NL, int WAVES>
 __device__ __forceinline__ void wc_issue(unsigned short* dst, const unsigned short* src, int wave, int lane)
 {
-    static_assert(NL % WAVES == 0 && NL * 512 <= WC_CHUNK, "whole loads per wave, within a chunk");
+    static_assert(NL % WAVES == 0, "whole loads per wave");
     const unsigned loff = (unsigned)lane * 16;  // the lane's bytes within a load: one VGPR for every load
 #pragma unroll
     for (int j = 0; j < NL / WAVES; ++j) {
@@ -242,32 +241,31 @@ __device__ __forceinline__ void wc_issue(unsigned short* dst, const unsigned sho
     }
 }
 
-// acc[mt][nt] += W[rows 16 nt .. +15] . xb[mt] for one chunk in the swizzled
-// layout of the weight-stationary kernels:
-// three planes [ROWS][32] (plane stride ROWS * 32), row r's four 16-byte
-// k-groups g stored at slot ws_slot(r, g), so that the fragment reads down the
-// rows at one k-group are free of bank conflicts without padding (a 192-row
-// chunk fits TX_BUF). HALF: the packed last step of a K = 144 linear (xb from
-// half_operands, three MFMAs per tile).
+// acc[mt][nt] += W[rows 16 nt .. +15] . xb[mt] for one step in the swizzled
+// layout of the weight-stationary kernels: two planes [ROWS][32] (plane stride
+// ROWS * 32), row r's four 16-byte k-groups g stored at slot ws_slot(r, g), so
+// that the fragment reads down the rows at one k-group are free of bank
+// conflicts without padding. HALF: the packed last step of a K = 144 linear
+// (xb[mt][0] from half_operand, two MFMAs a tile).
 template <int NT, int ROWS, bool HALF = false>
-__device__ __forceinline__ void ws_mma(const unsigned short* Ws, int lr, int lg, const u32x4 (&xb)[2][3],
-                                       f32x4 (&acc)[2][NT])
+__device__ __forceinline__ void ws_mma2(const unsigned short* Ws, int lr, int lg, const u32x4 (&xb)[2][2],
+                                        f32x4 (&acc)[2][NT])
 {
     const unsigned short* wr = Ws + lr * 32 + (hatk::ws_slot(lr, lg) * 8);
-    u32x4 wa[2][3];
+    u32x4 wa[2][2];
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl) wa[0][pl] = *(const u32x4*)(wr + pl * ROWS * 32);
+    for (int pl = 0; pl < 2; ++pl) wa[0][pl] = *(const u32x4*)(wr + pl * ROWS * 32);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         __builtin_amdgcn_sched_barrier(0);
         if (nt + 1 < NT) {
 #pragma unroll
-            for (int pl = 0; pl < 3; ++pl)
+            for (int pl = 0; pl < 2; ++pl)
                 wa[(nt + 1) & 1][pl] = *(const u32x4*)(wr + (nt + 1) * 16 * 32 + pl * ROWS * 32);
         }
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
-            acc[mt][nt] = HALF ? mfma16x3(wa[nt & 1], xb[mt], acc[mt][nt]) : mfma16x6(wa[nt & 1], xb[mt], acc[mt][nt]);
+            acc[mt][nt] = HALF ? mfma16x2h(wa[nt & 1], xb[mt][0], acc[mt][nt]) : mfma16x3h(wa[nt & 1], xb[mt], acc[mt][nt]);
     }
 }
 
@@ -297,6 +295,20 @@ __device__ __forceinline__ float gelu(float v)
     return __builtin_fmaf(-av, (q * t) * e, fmaxf(v, 0.0f));
 }
 
+// s GELU(v) from V = s v for a power of two s > 0: gelu's form with s in its
+// constants, g0 = 0.3275911 / (sqrt2 s), g1 = -log2(e) / (2 s^2).
+__device__ __forceinline__ float gelu_scaled(float V, float g0, float g1)
+{
+    const float av = fabsf(V);
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(g0, av, 1.0f));
+    float q = __builtin_fmaf(0.5f * 1.061405429f, t, 0.5f * -1.453152027f);
+    q = __builtin_fmaf(q, t, 0.5f * 1.421413741f);
+    q = __builtin_fmaf(q, t, 0.5f * -0.284496736f);
+    q = __builtin_fmaf(q, t, 0.5f * 0.254829592f);
+    const float e = fast_exp2((V * V) * g1);
+    return __builtin_fmaf(-av, (q * t) * e, fmaxf(V, 0.0f));
+}
+
 // 1 KB of zeros in global memory, never written (and not const, so the
 // compiler cannot fold loads from it). Loads that fall outside an operand -
 // rows past M, padding channels, taps outside the plane, padding slots of the
@@ -305,9 +317,6 @@ __device__ __forceinline__ float gelu(float v)
 // later waits drain every load; zeroing the value after the load makes it wait
 // for that load at once.
 __device__ __attribute__((aligned(16))) float hat_zero_row[256] = {};
-
-// A 1 then zeros: the activation of a bias column (see WcRows::load_b).
-__device__ __attribute__((aligned(16))) float hat_one_row[4] = {1.0f, 0.0f, 0.0f, 0.0f};
 
 // Where stores of rows past the end of an output go, so that a wave issues
 // the same number of stores whatever the row count (never read).

@@ -45,9 +45,7 @@
 #define GX_WAVES 8
 
 // This wave's 16 MT token rows of a [M][K] plane, 8 values at k = 32 ks + 8 lg
-// per token, for the B operand: zeros past M and past k = K, with load_b the
-// 1 at k = K that multiplies the bias column (read from hat_one_row like the
-// rest, so that nothing waits for the loads here).
+// per token, for the B operand: zeros past M and past k = K.
 template <int K, int MT = 2>
 struct WcRows {
     static_assert(K % 4 == 0, "float4 units");
@@ -62,7 +60,6 @@ struct WcRows {
             rows[mt] = base + (size_t)(alive[mt] ? m : 0) * K;
         }
     }
-    // zeros from k = K on (for a bias added elsewhere)
     __device__ __forceinline__ void load(int ks, int lg, f32x4 (&dst)[MT][2]) const
     {
         const int k0 = ks * 32 + lg * 8;
@@ -77,29 +74,7 @@ struct WcRows {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) dst[mt][0] = load_or_zero(rows[mt] + 128 + 4 * lg, alive[mt]);
     }
-    __device__ __forceinline__ void load_b(int ks, int lg, f32x4 (&dst)[MT][2]) const
-    {
-        const int k0 = ks * 32 + lg * 8;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int kq = k0 + 4 * j;
-                dst[mt][j] = *(const f32x4*)(alive[mt] && kq < K ? rows[mt] + kq : (kq == K ? hat_one_row : hat_zero_row));
-            }
-    }
 };
-
-template <int MT>
-__device__ __forceinline__ void split_pre(const f32x4 (&pre)[MT][2], u32x4 (&xb)[MT][3])
-{
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const float f[8] = {pre[mt][0][0], pre[mt][0][1], pre[mt][0][2], pre[mt][0][3],
-                            pre[mt][1][0], pre[mt][1][1], pre[mt][1][2], pre[mt][1][3]};
-        split3_x8(f, xb[mt]);
-    }
-}
 
 template <int MT>
 __device__ __forceinline__ void split_pre2(const f32x4 (&pre)[MT][2], u32x4 (&xb)[MT][2])

@@ -376,181 +376,82 @@ int gpu_selftest(std::string* err)
             check_close(std::string(k), dx.get(), want, 5e-5);
             if (epi == EPI_RESID_LN) check_close(std::string(k) + " layernorm", da.get(), wxn, 5e-5);
             note(std::string(k) + " C " + std::to_string(C) + " M 600 (in place)");
-            if (C == 180) {
-                // the split-bf16 form, in place the same way, 5 tiles of 128
-                // (the last partial): its fc1 input is norm2 (n2w, n2b) of the
-                // residual rows, formed in the kernel; against double
-                std::vector<float> n2w = rng.vec(C, 1.0f), n2b = rng.vec(C, 0.1f);
-                std::vector<unsigned short> mw;
-                pack_mlp_x180(w1.data(), b1.data(), w2.data(), &mw);
-                Dev dx2(res), dxn2((size_t)M * C), dn2w(n2w), dn2b(n2b), dmw((mw.size() + 1) / 2);
-                Runtime::get().h2d(dmw.p, mw.data(), mw.size() * sizeof(unsigned short));
-                TailXArgs q{};
-                q.a = dx2.p;
-                q.inw = dn2w.p;
-                q.inb = dn2b.p;
-                q.res = dx2.p;
-                q.out = dx2.p;
-                q.xn = epi == EPI_RESID_LN ? dxn2.p : nullptr;
-                q.w = (const unsigned short*)dmw.p;
-                q.b2 = db2.p;
-                q.nw = dnw.p;
-                q.nb = dnb.p;
-                q.M = M;
-                q.eps = 1e-5f;
-                const char* kx = epi == EPI_RESID_LN ? "hat_mlpx180_ln" : "hat_mlpx180";
-                launch(s, kx, (unsigned)wx_tiles(M), 1, 1, WX_THREADS, q);
-                std::vector<double> want2((size_t)M * C), wxn2((size_t)M * C), y(C);
-                for (int m = 0; m < M; ++m) {
-                    const float* r = &res[(size_t)m * C];
-                    double mu = 0, va = 0;
-                    for (int c = 0; c < C; ++c) mu += r[c];
-                    mu /= C;
-                    for (int c = 0; c < C; ++c) va += (r[c] - mu) * (r[c] - mu);
-                    va /= C;
-                    for (int c = 0; c < C; ++c) y[c] = (r[c] - mu) / std::sqrt(va + 1e-5) * n2w[c] + n2b[c];
-                    for (int j = 0; j < H; ++j) {
-                        double v = b1[j];
-                        for (int c = 0; c < C; ++c) v += y[c] * w1[(size_t)j * C + c];
-                        hid[j] = gelu_d(v);
-                    }
-                    double mean = 0, var = 0;
-                    for (int n = 0; n < C; ++n) {
-                        double v = b2[n];
-                        for (int j = 0; j < H; ++j) v += hid[j] * w2[(size_t)n * H + j];
-                        want2[(size_t)m * C + n] = r[n] + v;
-                        mean += want2[(size_t)m * C + n];
-                    }
-                    mean /= C;
-                    for (int n = 0; n < C; ++n) var += (want2[(size_t)m * C + n] - mean) * (want2[(size_t)m * C + n] - mean);
-                    var /= C;
-                    for (int n = 0; n < C; ++n)
-                        wxn2[(size_t)m * C + n] = (want2[(size_t)m * C + n] - mean) / std::sqrt(var + 1e-5) * nw[n] + nb[n];
-                }
-                check_close(kx, dx2.get(), want2, 5e-5);
-                if (epi == EPI_RESID_LN) check_close(std::string(kx) + " layernorm", dxn2.get(), wxn2, 5e-5);
-                note(std::string(kx) + " C 180 M 600 (split-bf16 with norm2 in the kernel, in place) vs double");
-            }
         }
 
-        // ---- the split-bf16 C = 180 projection tails against double: out =
-        // res + a . Wp^T + b (+ aux * gate * cscale), xn = LN(out), in place
-        // over the residual, 600 rows (the last tile partial).
+        // ---- the split-f16 C = 180 tails against double, in place over the
+        // residual, 600 rows (the last tile partial): HAB form (gated conv2
+        // output + next norm) and OCAB form (neither), the attention output and
+        // norm2 scaled as the forward scales them.
         for (int hab : {1, 0}) {
-            const int M = 600, C = 180;
-            const float cscale = 0.01f;
-            std::vector<float> a = rng.vec((size_t)M * C, 1.0f), w = rng.vec((size_t)C * C, 0.08f),
-                               b = rng.vec(C, 0.1f), res = rng.vec((size_t)M * C, 1.0f), aux = rng.vec((size_t)M * C, 1.0f),
-                               gate = rng.vec(C, 1.0f), nw = rng.vec(C, 1.0f), nb = rng.vec(C, 0.1f);
-            std::vector<unsigned short> wx = pack_linear_x180(w.data());
-            Dev da(a), db(b), dx(res), daux(aux), dg(gate), dnw(nw), dnb(nb), dxn((size_t)M * C), dw((wx.size() + 1) / 2);
-            Runtime::get().h2d(dw.p, wx.data(), wx.size() * sizeof(unsigned short));
-            TailXArgs q{};
-            q.a = da.p;
-            q.res = dx.p;
-            q.out = dx.p;
-            q.xn = dxn.p;
-            q.w = (const unsigned short*)dw.p;
-            q.bias = db.p;
-            q.nw = dnw.p;
-            q.nb = dnb.p;
-            q.M = M;
-            q.eps = 1e-5f;
-            q.aux = hab ? daux.p : nullptr;
-            q.gate = hab ? dg.p : nullptr;
-            q.cscale = cscale;
-            const char* k = hab ? "hat_projx180_hab" : "hat_projx180";
-            launch(s, k, (unsigned)wx_tiles(M), 1, 1, WX_THREADS, q);
-            std::vector<double> want((size_t)M * C), wxn((size_t)M * C);
-            for (int m = 0; m < M; ++m) {
-                double mean = 0, var = 0;
-                for (int n = 0; n < C; ++n) {
-                    double v = b[n];
-                    for (int c = 0; c < C; ++c) v += (double)a[(size_t)m * C + c] * w[(size_t)n * C + c];
-                    v += res[(size_t)m * C + n];
-                    if (hab) v += (double)aux[(size_t)m * C + n] * gate[n] * cscale;
-                    want[(size_t)m * C + n] = v;
-                    mean += v / C;
-                }
-                for (int n = 0; n < C; ++n) var += (want[(size_t)m * C + n] - mean) * (want[(size_t)m * C + n] - mean) / C;
-                for (int n = 0; n < C; ++n)
-                    wxn[(size_t)m * C + n] = (want[(size_t)m * C + n] - mean) / std::sqrt(var + 1e-5) * nw[n] + nb[n];
-            }
-            check_close(k, dx.get(), want, 3e-5);
-            check_close(std::string(k) + " layernorm", dxn.get(), wxn, 5e-5);
-            note(std::string(k) + " C 180 M 600 (split-bf16, in place)");
-        }
-
-        // ---- the fused C = 180 tails (x' on the chip) against the two
-        // kernels above on the same inputs, in place over the residual, 600
-        // rows (the last tile partial): HAB form (gated conv2 output + next
-        // norm) and OCAB form (neither).
-        for (int hab : {1, 0}) {
-            const int M = 600, C = 180, H = 360;
-            const float cscale = 0.01f;
+            const int M = 600, C = 180, Hd = 360;
+            const float cscale = 0.01f, sv = 64.0f, sn = 512.0f;
             std::vector<float> a = rng.vec((size_t)M * C, 1.0f), wp = rng.vec((size_t)C * C, 0.08f),
                                bp = rng.vec(C, 0.1f), res = rng.vec((size_t)M * C, 1.0f),
                                aux = rng.vec((size_t)M * C, 1.0f), gate = rng.vec(C, 1.0f),
-                               n2w = rng.vec(C, 1.0f), n2b = rng.vec(C, 0.1f), w1 = rng.vec((size_t)H * C, 0.08f),
-                               b1 = rng.vec(H, 0.1f), w2 = rng.vec((size_t)C * H, 0.05f), b2 = rng.vec(C, 0.1f),
+                               n2w = rng.vec(C, 1.0f), n2b = rng.vec(C, 0.1f), w1 = rng.vec((size_t)Hd * C, 0.08f),
+                               b1 = rng.vec(Hd, 0.1f), w2 = rng.vec((size_t)C * Hd, 0.05f), b2 = rng.vec(C, 0.1f),
                                nw = rng.vec(C, 1.0f), nb = rng.vec(C, 0.1f);
-            std::vector<unsigned short> pwx = pack_linear_x180(wp.data()), mw, mwf;
-            std::vector<float> mb1x;
-            pack_mlp_x180(w1.data(), b1.data(), w2.data(), &mw);
-            pack_mlp_xf180(w1.data(), b1.data(), w2.data(), &mwf, &mb1x);
-            Dev da(a), dbp(bp), daux(aux), dg(gate), dn2w(n2w), dn2b(n2b), db2(b2), dnw(nw), dnb(nb), dmb1x(mb1x),
-                dx2(res), dxn2((size_t)M * C), dxf(res), dxnf((size_t)M * C), dpw((pwx.size() + 1) / 2),
-                dmw((mw.size() + 1) / 2), dmwf((mwf.size() + 1) / 2);
-            Runtime::get().h2d(dpw.p, pwx.data(), pwx.size() * sizeof(unsigned short));
-            Runtime::get().h2d(dmw.p, mw.data(), mw.size() * sizeof(unsigned short));
-            Runtime::get().h2d(dmwf.p, mwf.data(), mwf.size() * sizeof(unsigned short));
-            TailXArgs q{};
-            q.a = da.p;
-            q.res = dx2.p;
-            q.out = dx2.p;
-            q.w = (const unsigned short*)dpw.p;
-            q.bias = dbp.p;
-            q.M = M;
-            q.eps = 1e-5f;
-            q.aux = hab ? daux.p : nullptr;
-            q.gate = hab ? dg.p : nullptr;
-            q.cscale = cscale;
-            launch(s, hab ? "hat_projx180_hab" : "hat_projx180", (unsigned)wx_tiles(M), 1, 1, WX_THREADS, q);
-            TailXArgs m2{};
-            m2.a = dx2.p;
-            m2.inw = dn2w.p;
-            m2.inb = dn2b.p;
-            m2.res = dx2.p;
-            m2.out = dx2.p;
-            m2.xn = hab ? dxn2.p : nullptr;
-            m2.w = (const unsigned short*)dmw.p;
-            m2.b2 = db2.p;
-            m2.nw = hab ? dnw.p : nullptr;
-            m2.nb = hab ? dnb.p : nullptr;
-            m2.M = M;
-            m2.eps = 1e-5f;
-            launch(s, hab ? "hat_mlpx180_ln" : "hat_mlpx180", (unsigned)wx_tiles(M), 1, 1, WX_THREADS, m2);
-            TailXArgs f = q;
-            f.res = dxf.p;
-            f.out = dxf.p;
-            f.xn = hab ? dxnf.p : nullptr;
-            f.wm = (const unsigned short*)dmwf.p;
-            f.b1x = dmb1x.p;
+            TailPack tp = pack_tail(wp.data(), w1.data(), b1.data(), w2.data(), n2w.data(), n2b.data(), C, sv, sn, nullptr);
+            std::vector<float> as(a), n2ws(n2w), n2bs(n2b);
+            for (float& x : as) x *= sv;
+            for (float& x : n2ws) x *= sn;
+            for (float& x : n2bs) x *= sn;
+            Dev da(as), dbp(bp), daux(aux), dg(gate), dn2w(n2ws), dn2b(n2bs), db2(b2), dnw(nw), dnb(nb), db1x(tp.b1x), dx(res),
+                dxn((size_t)M * C), dw((tp.w.size() + 1) / 2), dwm((tp.wm.size() + 1) / 2);
+            Runtime::get().h2d(dw.p, tp.w.data(), tp.w.size() * sizeof(unsigned short));
+            Runtime::get().h2d(dwm.p, tp.wm.data(), tp.wm.size() * sizeof(unsigned short));
+            TailXArgs f{};
+            f.a = da.p;
+            f.res = dx.p;
+            f.out = dx.p;
+            f.xn = hab ? dxn.p : nullptr;
+            f.w = (const unsigned short*)dw.p;
+            f.wm = (const unsigned short*)dwm.p;
+            f.bias = dbp.p;
+            f.b1x = db1x.p;
             f.b2 = db2.p;
             f.inw = dn2w.p;
             f.inb = dn2b.p;
             f.nw = hab ? dnw.p : nullptr;
             f.nb = hab ? dnb.p : nullptr;
+            f.aux = hab ? daux.p : nullptr;
+            f.gate = hab ? dg.p : nullptr;
+            f.cscale = cscale;
+            f.M = M;
+            f.eps = 1e-5f;
+            tail_scales(tp.t, &f);
             const char* k = hab ? "hat_habx180_hab_ln" : "hat_habx180";
             launch(s, k, (unsigned)wx_tiles(M), 1, 1, WX_THREADS, f);
-            const std::vector<float> two = dx2.get();
-            check_close(k, dxf.get(), std::vector<double>(two.begin(), two.end()), 2e-5);
-            if (hab) {
-                const std::vector<float> twon = dxn2.get();
-                check_close(std::string(k) + " next norm", dxnf.get(), std::vector<double>(twon.begin(), twon.end()),
-                            2e-5);
+            std::vector<double> want((size_t)M * C), wxn((size_t)M * C), x(C), y(C), hid(Hd);
+            auto norm = [&](const double* v, const std::vector<float>& w, const std::vector<float>& b, double* o) {
+                double mean = 0, var = 0;
+                for (int c = 0; c < C; ++c) mean += v[c] / C;
+                for (int c = 0; c < C; ++c) var += (v[c] - mean) * (v[c] - mean) / C;
+                for (int c = 0; c < C; ++c) o[c] = (v[c] - mean) / std::sqrt(var + 1e-5) * w[c] + b[c];
+            };
+            for (int m = 0; m < M; ++m) {
+                const size_t o = (size_t)m * C;
+                for (int n = 0; n < C; ++n) {
+                    x[n] = (double)res[o + n] + bp[n];
+                    for (int c = 0; c < C; ++c) x[n] += (double)a[o + c] * wp[(size_t)n * C + c];
+                    if (hab) x[n] += (double)aux[o + n] * gate[n] * cscale;
+                }
+                norm(x.data(), n2w, n2b, y.data());
+                for (int j = 0; j < Hd; ++j) {
+                    double v = b1[j];
+                    for (int c = 0; c < C; ++c) v += y[c] * w1[(size_t)j * C + c];
+                    hid[j] = gelu_d(v);
+                }
+                for (int n = 0; n < C; ++n) {
+                    double v = x[n] + b2[n];
+                    for (int j = 0; j < Hd; ++j) v += hid[j] * w2[(size_t)n * Hd + j];
+                    want[o + n] = v;
+                }
+                norm(&want[o], nw, nb, &wxn[o]);
             }
-            note(std::string(k) + " (fused split-bf16 C 180 tail, M 600, in place) vs the two-kernel path");
+            check_close(k, dx.get(), want, 5e-5);
+            if (hab) check_close(std::string(k) + " next norm", dxn.get(), wxn, 5e-5);
+            note(std::string(k) + " (split-f16 C 180 tail, M 600, in place) vs double");
         }
 
         // ---- folded CAB (144 -> 6 -> 144) against the unfolded computation:
@@ -573,10 +474,10 @@ int gpu_selftest(std::string* err)
             const int tiles = (H / 16) * (W / 16);
             Dev dxn(xn), dw1(w1p.size() / 2), db1(b1), dw2(w2), db2(b2), dwa(wa), dba(ba), dwb(wb), dbb(bb), dao(ao),
                 dwp(wpp), dbp(bp), dres(res), dnw(nw), dnb(nb), dt1((size_t)T * CAB_CS),
-                dpart((size_t)tiles * CAB_NSUM * CAB_CS), dw2g((size_t)C * CAB_K2), dw2gx(WC_CHUNK), dbias2(C), dgate(C),
+                dpart((size_t)tiles * CAB_NSUM * CAB_CS), dw2g((size_t)C * CAB_K2), dw2gx(2 * C * 32), dbias2(C), dgate(C),
                 dout((size_t)T * C), dxo((size_t)T * C);
             Runtime::get().h2d(dw1.p, w1p.data(), w1p.size() * sizeof(unsigned short));
-            CabConvArgs ca{dxn.p, (const unsigned short*)dw1.p, db1.p, dt1.p, dpart.p, H, W};
+            CabConvArgs ca{dxn.p, (const unsigned short*)dw1.p, db1.p, dt1.p, dpart.p, H, W, 1.0f};
             launch(s, "hat_cab_conv1", 2, 1, 1, 256, ca);
             CabGateArgs ga{};
             ga.partial = dpart.p;
@@ -597,6 +498,8 @@ int gpu_selftest(std::string* err)
             ga.cscale = cscale;
             ga.sq = sq;
             ga.w2gx = (unsigned short*)dw2gx.p;
+            ga.ts = 1.0f;
+            ga.gs = 1.0f;
             launch(s, "hat_cab_gate", 1, 1, 1, 1024, ga);
             GemmArgs gp{};
             gp.a = dao.p;
@@ -689,7 +592,7 @@ int gpu_selftest(std::string* err)
                 const int tiles32 = (H / 32) * (W / 16);
                 Dev dt1b((size_t)T * CAB_CS), dpartb((size_t)tiles32 * CAB_NSUM * CAB_CS), dw2gb((size_t)C * CAB_K2),
                     dbias2b(C), dgateb(C);
-                CabConvArgs cb2{dxn.p, (const unsigned short*)dw1.p, db1.p, dt1b.p, dpartb.p, H, W};
+                CabConvArgs cb2{dxn.p, (const unsigned short*)dw1.p, db1.p, dt1b.p, dpartb.p, H, W, 1.0f};
                 launch(s, "hat_cab_conv1_t32", 2, 1, 1, 256, cb2);
                 CabGateArgs gb = ga;
                 gb.partial = dpartb.p;
@@ -807,116 +710,72 @@ int gpu_selftest(std::string* err)
                 check_close("hat_ocab_tail", dout_o.get(), std::vector<double>(r2.begin(), r2.end()), 2e-5);
                 note("hat_ocab_tail (proj + norm2 + MLP) vs the two-kernel path");
 
-                // The split-bf16 tails (tailx.hip) on the same inputs, in place
-                // as the forward runs them (out over the block input, the next
-                // norm over norm2's rows); 12 row tiles of 128.
-                std::vector<unsigned short> pwx = pack_linear_x(wp.data(), C, C), mwx, mwf;
-                std::vector<float> mb1x;
-                pack_mlp_x(f1.data(), fb1.data(), f2.data(), &mwx);
-                pack_mlp_xf(f1.data(), fb1.data(), f2.data(), &mwf, &mb1x);
-                Dev dmb1x(mb1x);
-                Dev dpwx(std::vector<float>((pwx.size() + 1) / 2)), dmwx(std::vector<float>((mwx.size() + 1) / 2)),
-                    dmwf(std::vector<float>((mwf.size() + 1) / 2)), dout_x(res), dxn_x((size_t)T * C),
-                    dout_f(res), dxn_f((size_t)T * C);
-                Runtime::get().h2d(dpwx.p, pwx.data(), pwx.size() * sizeof(unsigned short));
-                Runtime::get().h2d(dmwx.p, mwx.data(), mwx.size() * sizeof(unsigned short));
-                Runtime::get().h2d(dmwf.p, mwf.data(), mwf.size() * sizeof(unsigned short));
-                TailXArgs xa{};
-                xa.a = dao.p;
-                xa.res = dout_x.p;
-                xa.out = dout_x.p;
-                xa.xn = dxn_x.p;
-                xa.w = (const unsigned short*)dpwx.p;
-                xa.bias = dbias2.p;
-                xa.w2gx = (const unsigned short*)dw2gx.p;
-                xa.t1 = dt1.p;
-                xa.nw = dnw.p;
-                xa.nb = dnb.p;
-                xa.M = T;
-                xa.H = H;
-                xa.W = W;
-                xa.eps = 1e-5f;
-                launch(s, "hat_projx_cab", (unsigned)wx_tiles(T), 1, 1, WX_THREADS, xa);
-                check_close("hat_projx_cab", dout_x.get(), want, 5e-5);
-                check_close("hat_projx_cab layernorm", dxn_x.get(), wxn, 5e-5);
-                note("hat_projx_cab (split-bf16 proj + folded conv2 + norm2) vs double");
-                TailXArgs xm{};
-                xm.a = dout_x.p;  // x': the kernel forms norm2 from it
-                xm.inw = dnw.p;
-                xm.inb = dnb.p;
-                xm.res = dout_x.p;
-                xm.out = dout_x.p;
-                xm.xn = dxn_x.p;
-                xm.w = (const unsigned short*)dmwx.p;
-                xm.b2 = dfb2.p;
-                xm.nw = dmw.p;
-                xm.nb = dmb.p;
-                xm.M = T;
-                xm.H = H;
-                xm.W = W;
-                xm.eps = 1e-5f;
-                launch(s, "hat_mlpx_ln", (unsigned)wx_tiles(T), 1, 1, WX_THREADS, xm);
-                check_close("hat_mlpx_ln", dout_x.get(), std::vector<double>(ro.begin(), ro.end()), 2e-5);
-                check_close("hat_mlpx_ln next norm", dxn_x.get(), std::vector<double>(rx.begin(), rx.end()), 2e-5);
-                note("hat_mlpx_ln (split-bf16 MLP + norm) vs the two-kernel path");
-                // The fused tail (x' on the chip) on the same inputs, in place,
-                // against the same references.
-                TailXArgs xf = xa;
+                // The split-f16 tails (tailx.hip) on the same inputs, in place as
+                // the forward runs them (out over the block input); 12 row tiles
+                // of 128. conv1 and the gate run again with the scales the tail
+                // asks for (t1 and the gated weights times powers of two).
+                const TailCab tc{8.0, 0.01};
+                TailPack xt = pack_tail(wp.data(), f1.data(), fb1.data(), f2.data(), nw.data(), nb.data(), C, 1.0f, 1.0f, &tc);
+                Dev dpw((xt.w.size() + 1) / 2), dpm((xt.wm.size() + 1) / 2), db1x(xt.b1x), dt1x((size_t)T * CAB_CS),
+                    dpartx((size_t)tiles * CAB_NSUM * CAB_CS), dbias2x(C), dgatex(C), dout_f(res), dxn_f((size_t)T * C);
+                Runtime::get().h2d(dpw.p, xt.w.data(), xt.w.size() * sizeof(unsigned short));
+                Runtime::get().h2d(dpm.p, xt.wm.data(), xt.wm.size() * sizeof(unsigned short));
+                CabConvArgs cx{dxn.p, (const unsigned short*)dw1.p, db1.p, dt1x.p, dpartx.p, H, W, xt.t.ts};
+                launch(s, "hat_cab_conv1", 2, 1, 1, 256, cx);
+                CabGateArgs gx = ga;
+                gx.partial = dpartx.p;
+                gx.t1 = dt1x.p;
+                gx.w2g = nullptr;
+                gx.bias2 = dbias2x.p;
+                gx.gate = dgatex.p;
+                gx.ts = xt.t.ts;
+                gx.gs = xt.t.gs;
+                launch(s, "hat_cab_gate", 1, 1, 1, 1024, gx);
+                check_close("hat_cab_gate gate (scaled t1)", dgatex.get(), gate, 2e-6);
+                TailXArgs xf{};
+                xf.a = dao.p;
                 xf.res = dout_f.p;
                 xf.out = dout_f.p;
                 xf.xn = dxn_f.p;
-                xf.wm = (const unsigned short*)dmwf.p;
-                xf.b1x = dmb1x.p;
+                xf.w = (const unsigned short*)dpw.p;
+                xf.wm = (const unsigned short*)dpm.p;
+                xf.w2gx = (const unsigned short*)dw2gx.p;
+                xf.t1 = dt1x.p;
+                xf.bias = dbias2x.p;
+                xf.b1x = db1x.p;
                 xf.b2 = dfb2.p;
                 xf.inw = dnw.p;
                 xf.inb = dnb.p;
                 xf.nw = dmw.p;
                 xf.nb = dmb.p;
+                xf.M = T;
+                xf.H = H;
+                xf.W = W;
+                xf.eps = 1e-5f;
+                tail_scales(xt.t, &xf);
                 launch(s, "hat_habx_cab_ln", (unsigned)wx_tiles(T), 1, 1, WX_THREADS, xf);
                 check_close("hat_habx_cab_ln", dout_f.get(), std::vector<double>(ro.begin(), ro.end()), 2e-5);
                 check_close("hat_habx_cab_ln next norm", dxn_f.get(), std::vector<double>(rx.begin(), rx.end()), 2e-5);
-                note("hat_habx_cab_ln (fused split-bf16 proj + conv2 + MLP + norm) vs the two-kernel path");
+                note("hat_habx_cab_ln (split-f16 proj + conv2 + MLP + norm) vs the two-kernel path");
                 // The OCAB form over a partial last tile: rows from Mo on stay
                 // the block input.
                 const int Mo = T - 100;
-                Dev dout_ox(res), dxn_ox((size_t)T * C);
-                TailXArgs xo = xa;
-                xo.res = dout_ox.p;
-                xo.out = dout_ox.p;
-                xo.xn = dxn_ox.p;
-                xo.bias = dbp.p;
-                xo.w2gx = nullptr;
-                xo.t1 = nullptr;
-                xo.M = Mo;
-                launch(s, "hat_projx", (unsigned)wx_tiles(Mo), 1, 1, WX_THREADS, xo);
-                TailXArgs xo2 = xm;
-                xo2.a = dout_ox.p;
-                xo2.res = dout_ox.p;
-                xo2.out = dout_ox.p;
-                xo2.xn = nullptr;
-                xo2.nw = nullptr;
-                xo2.nb = nullptr;
-                xo2.M = Mo;
-                launch(s, "hat_mlpx", (unsigned)wx_tiles(Mo), 1, 1, WX_THREADS, xo2);
                 std::vector<double> wo(r2.begin(), r2.end());
                 for (size_t i = (size_t)Mo * C; i < wo.size(); ++i) wo[i] = res[i];
-                check_close("hat_projx + hat_mlpx", dout_ox.get(), wo, 2e-5);
-                note("hat_projx + hat_mlpx (split-bf16 OCAB tail, partial tile) vs the two-kernel path");
                 Dev dout_of(res);
-                TailXArgs xof = xo;
+                TailXArgs xof = xf;
                 xof.res = dout_of.p;
                 xof.out = dout_of.p;
                 xof.xn = nullptr;
-                xof.wm = (const unsigned short*)dmwf.p;
-                xof.b1x = dmb1x.p;
-                xof.b2 = dfb2.p;
-                xof.inw = dnw.p;
-                xof.inb = dnb.p;
+                xof.w2gx = nullptr;
+                xof.t1 = nullptr;
+                xof.bias = dbp.p;
                 xof.nw = nullptr;
                 xof.nb = nullptr;
+                xof.M = Mo;
                 launch(s, "hat_habx", (unsigned)wx_tiles(Mo), 1, 1, WX_THREADS, xof);
                 check_close("hat_habx", dout_of.get(), wo, 2e-5);
-                note("hat_habx (fused split-bf16 OCAB tail, partial tile) vs the two-kernel path");
+                note("hat_habx (split-f16 OCAB tail, partial tile) vs the two-kernel path");
             }
         }
 
