@@ -344,9 +344,9 @@ static bool wino_conv(int CO, int CI, int r)
            (r == 0 && CI == 180 && CO == 60) || (r == 0 && CI == 60 && CO == 180);
 }
 
-// conv1 [6][144][3][3] as the split A operands of hat_cab_conv1* (CX_WPACK):
-// row r = tap * 6 + co (rows 54..63 zero), each weight as three bf16 parts.
-std::vector<unsigned short> pack_cab_conv1(const float* w)
+// conv1 [6][144][3][3] as the split A operands of hat_cab_conv1 (CX_WPACK):
+// row r = tap * 6 + co (rows 54..63 zero), each weight times sw as two f16 parts.
+std::vector<unsigned short> pack_cab_conv1(const float* w, float sw)
 {
     std::vector<unsigned short> out(CX_WPACK, 0);
     for (int ks = 0; ks < 9; ++ks)
@@ -356,16 +356,18 @@ std::vector<unsigned short> pack_cab_conv1(const float* w)
                     const int r = nt * 32 + lane % 32, ci = ks * 16 + 8 * (lane / 32) + j;
                     if (r >= 9 * CAB_CC) continue;
                     const int tap = r / CAB_CC, co = r % CAB_CC;
-                    const float x = w[((size_t)co * CAB_C + ci) * 9 + tap];
-                    const unsigned short h0 = bf16_rne(x);
-                    const float r1 = x - bf16_float(h0);
-                    const unsigned short h1 = bf16_rne(r1);
-                    const unsigned short h2 = bf16_rne(r1 - bf16_float(h1));
-                    const unsigned short parts[3] = {h0, h1, h2};
-                    for (int part = 0; part < 3; ++part)
-                        out[((size_t)((ks * 2 + nt) * 3 + part) * 64 + lane) * 8 + j] = parts[part];
+                    unsigned short* d = &out[((size_t)((ks * 2 + nt) * 2) * 64 + lane) * 8 + j];
+                    split2_f16(w[((size_t)co * CAB_C + ci) * 9 + tap] * sw, d, d + 64 * 8);
                 }
     return out;
+}
+
+void cab_scales(float ts, float oscale, CabConvArgs* a)
+{
+    a->ts = ts;
+    a->oinv = ts * oscale;
+    a->g0 = 0.3275911f * 0.70710678f / ts;
+    a->g1 = -0.5f * 1.4426950408889634f / (ts * ts);
 }
 
 float f16_scale(double bound)
@@ -651,12 +653,18 @@ void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, con
     if (H % 16 != 0 || W % 16 != 0 || H < 16 || W < 16) throw Error("CAB: plane must be 16-aligned");
     if (sq < 1 || sq > 64) throw Error("CAB: squeeze width must be 1..64");
     static const int cus = std::max(1, Runtime::get().cu_count());
-    CabConvArgs a{xn, cb.w1, cb.b1, t1, partial, H, W, ts};
-    // Persistent over the output tiles, one block of 4 waves per CU: 16 wide x
-    // 32 tall when the height allows, else 16 x 16.
-    const bool t32 = H % 32 == 0;
-    const int tiles = (H / (t32 ? 32 : 16)) * (W / 16);
-    launch(s, t32 ? "hat_cab_conv1_t32" : "hat_cab_conv1", (unsigned)std::min(tiles, cus), 1, 1, 256, a);
+    CabConvArgs a{};
+    a.xn = xn;
+    a.w = cb.w1;
+    a.bias = cb.b1;
+    a.t1 = t1;
+    a.partial = partial;
+    a.H = H;
+    a.W = W;
+    cab_scales(ts, cb.oscale, &a);
+    // Persistent over the 16 x 16 output tiles, two blocks of 4 waves per CU.
+    const int tiles = (H / 16) * (W / 16);
+    launch(s, "hat_cab_conv1", (unsigned)std::min(tiles, 2 * cus), 1, 1, 256, a);
     CabGateArgs g{};
     g.partial = partial;
     g.t1 = t1;
@@ -1350,10 +1358,11 @@ void GpuBackend::upload_all()
             if (cab_fold_) {
                 const std::string c = p + ".conv_block.cab.";
                 for (const char* n : {"0.bias", "2.weight", "2.bias"}) upload_raw(c + n);
-                std::vector<float> w0(wt.t(c + "0.weight"), wt.t(c + "0.weight") + wt.info(c + "0.weight").numel());
-                for (float& x : w0) x *= xin;
-                std::vector<unsigned short> w1 = pack_cab_conv1(w0.data());
+                const float* w0 = wt.t(c + "0.weight");
+                const float sw = f16_scale(abs_max(w0, wt.info(c + "0.weight").numel()));
+                std::vector<unsigned short> w1 = pack_cab_conv1(w0, sw);
                 DevCab cb;
+                cb.oscale = xin / sw;
                 cb.w1 = (unsigned short*)upload_bytes(w1.data(), w1.size() * sizeof(unsigned short));
                 cb.b1 = raw_.at(c + "0.bias");
                 cb.w2 = raw_.at(c + "2.weight");

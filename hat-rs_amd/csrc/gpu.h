@@ -37,7 +37,8 @@ struct DevLinear {
 // The CAB of the compress-to-6 family, in the folded form (conv1 per-tap
 // weights; conv2 and the channel attention as raw tensors for the gate kernel).
 struct DevCab {
-    unsigned short* w1 = nullptr;  // conv1 split for hat_cab_conv1* (CX_WPACK bf16)
+    unsigned short* w1 = nullptr;  // conv1 split for hat_cab_conv1 (CX_WPACK f16)
+    float oscale = 1.0f;           // 1 over norm1's scale and the weights'
     float* b1 = nullptr;  // [6]
     float* w2 = nullptr;  // [144][6][3][3]
     float* b2 = nullptr;  // [144]
@@ -48,9 +49,11 @@ struct DevCab {
 };
 
 // conv1 weight [6][144][3][3] -> 64 rows of 144 (row tap*6 + co holds
-// w[co][:][tap], rows 54..63 zero), each weight as three bf16 parts in
+// w[co][:][tap], rows 54..63 zero), each weight times sw and as two f16 parts in
 // hat_cab_conv1's A-operand layout (CX_WPACK elements).
-std::vector<unsigned short> pack_cab_conv1(const float* w);
+std::vector<unsigned short> pack_cab_conv1(const float* w, float sw);
+// CabConvArgs' scales: t1's, and oscale as DevCab's.
+void cab_scales(float ts, float oscale, hatk::CabConvArgs* a);
 
 // A block's second half on split-f16 (tailx.hip): the projection's and the MLP's
 // packed steps, fc1's bias in the parts' row order, and the scales (TailXArgs).

@@ -82,22 +82,24 @@ struct GemmArgs {
 #define CAB_CC 6             // compressed channels
 #define CAB_CS 8             // t1 channel stride (channels 6, 7 are zero)
 #define CAB_K2 56            // 9 taps x 6 channels (k = tap*6 + ci), 2 zero: 3 x 16 + 8
-// conv1's weights split for hat_cab_conv1*: per 16-channel step ks (9), row
-// tile nt (2 x 32 rows, row tap*6 + co, rows 54.. zero) and part (3), the
+// conv1's weights split for hat_cab_conv1: per 16-channel step ks (9), row
+// tile nt (2 x 32 rows, row tap*6 + co, rows 54.. zero) and part (2), the
 // 32x32x16 A operand of each lane (row l % 32, channels 16 ks + 8 (l / 32) .. +7)
-#define CX_WPACK (9 * 2 * 3 * 64 * 8)
+#define CX_WPACK (9 * 2 * 2 * 64 * 8)
 // floats of the gated conv2 weights' buffer (CabGateArgs::w2gx: 9216 used)
 #define CAB_W2GX 20480
 #define CAB_NSUM 5           // per-tile sums: whole tile, row 0, row H-1, col 0, col W-1
 
 struct CabConvArgs {
     const float* xn;     // [H*W][144]
-    const unsigned short* w;  // [9][2][3][64][8] bf16: step ks, row tile nt, part, lane (CX_WPACK)
+    const unsigned short* w;  // [9][2][2][64][8] f16: step ks, row tile nt, part, lane (CX_WPACK)
     const float* bias;   // [6]
     float* t1;           // [H*W][8]: ts * gelu(conv1(xn))
     float* partial;      // [CAB_NSUM * 8][tiles] (value-major), of t1 as stored
     int H, W;            // multiples of 16
     float ts;            // t1's scale (a power of two: the split tail's range)
+    float oinv;          // ts over xn's scale and the weights'
+    float g0, g1;        // gelu_scaled's constants for ts
 };
 
 struct CabGateArgs {

@@ -20,64 +20,58 @@
 using namespace hatk;
 
 // ---------------------------------------------------------------------------
-// conv1 (144 -> 6, 3x3, zero padding) + GELU on split-bf16 MFMA, one 16-wide,
-// TY-tall output tile at a time: persistent over the tiles, one block of four
-// waves per CU.
+// conv1 (144 -> 6, 3x3, zero padding) + GELU on split-f16 MFMA, one 16 x 16
+// output tile at a time: persistent over the tiles, two blocks of four waves
+// per CU.
 //
-// Per-tap products: for each pixel q of the tile's 18 x (TY+2) halo,
-// P[q][tap*6+co] = sum_ci xn[q][ci] * w[co][ci][tap] is a 144-deep product with
-// 54 outputs (padded to 64): v_mfma_f32_32x32x16_bf16 with the 64 weight rows as
-// A (two tiles of 32) and 32 halo pixels as B, nine 16-channel steps, every fp32
-// operand as three bf16 parts and every product as the six terms of order <= 2
-// (the arithmetic of the split-bf16 attention, as accurate as FP32 MFMA). The
-// conv output at p is then the sum over the 9 taps of P[p + d(tap)][tap*6 + co],
-// read from LDS in fp32. The split weights (216 registers a lane) stay in
-// registers for the whole kernel, which takes the register file of one wave per
-// SIMD. Each wave streams its 32-pixel halo tiles (TY = 32: 612 pixels in 20
-// tiles, five a wave; TY = 16: 324 in 11), loading the next tile's 144 channels
-// step by step while this one's MFMAs run, across the output tiles too: the
-// barriers here wait for LDS only, so those loads stay in flight through them.
+// Per-tap products: for each pixel q of the tile's 18 x 18 halo, P[q][tap*6+co]
+// = sum_ci xn[q][ci] * w[co][ci][tap] is a 144-deep product with 54 outputs
+// (padded to 64): v_mfma_f32_32x32x16_f16 with the 64 weight rows as A (two
+// tiles of 32) and 32 halo pixels as B, nine 16-channel steps, every fp32
+// operand as two f16 parts and every product as three terms (common.h; norm1
+// leaves xn in f16's range, the host scales the weights, p.oinv takes both
+// out). The conv output at p is then the sum over the 9 taps of P[p +
+// d(tap)][tap*6 + co], read from LDS in fp32.
+//
+// The split weights (144 registers a lane) stay in registers for the whole
+// kernel, and the rows are read CX_RING steps ahead, across halo tiles and
+// output tiles: the barriers here wait for LDS only, so those loads stay in
+// flight through them. That leaves two waves a SIMD (256 registers), so that
+// one block's taps, GELU and stores run beside the other's MFMAs; the bf16
+// split's 216 weight registers left one, in 16 x 32 tiles. HAT-S 512 x 512: 53.3
+// -> 50.5 us (151 MB: 27 us at the copy kernel's rate; issue and the rows'
+// latency bound it), 64 x 64, whose 16 tiles are as many blocks: 22.8 -> 12.0.
 #define CX_WAVES 4
-#define CX_HS 18  // halo width
-#define CX_PS 60  // LDS row stride of P (56 written, 54 used): a b128 phase's 16 rows on distinct banks
+#define CX_HS 18                               // halo width and height
+#define CX_HP (CX_HS * CX_HS)                  // halo pixels
+#define CX_PT ((CX_HP + 31) / 32)              // 32-pixel halo tiles
+#define CX_NPW ((CX_PT + CX_WAVES - 1) / CX_WAVES)  // per wave (past CX_PT: zeros, not stored)
+#define CX_PS 60    // LDS row stride of P (56 written, 54 used): a b128 phase's 16 rows on distinct banks
+#define CX_RING 3   // 16-channel steps of rows in flight
 
-template <int TY>
-struct Cx1Shape {
-    static constexpr int HY = TY + 2;
-    static constexpr int HP = CX_HS * HY;      // halo pixels
-    static constexpr int PT = (HP + 31) / 32;  // 32-pixel halo tiles
-    static constexpr int NPW = (PT + CX_WAVES - 1) / CX_WAVES;  // per wave (past PT: zeros, not stored)
-    static constexpr int NPX = TY / 16;        // output pixels per thread
-    static_assert(16 * TY == CX_WAVES * 64 * NPX, "whole pixels per thread");
-};
-
-template <int TY>
-__device__ __forceinline__ void cab_conv1_body(const CabConvArgs& p)
+extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(CabConvArgs p)
 {
-    using S = Cx1Shape<TY>;
-    __shared__ __attribute__((aligned(16))) float Ps[S::HP * CX_PS];
+    __shared__ __attribute__((aligned(16))) float Ps[CX_HP * CX_PS];
     __shared__ float red[CX_WAVES][CAB_NSUM * CAB_CC];
+    static_assert(16 * 16 == CX_WAVES * 64, "one pixel per thread");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in a scalar register
     const int pl = lane & 31, h = lane >> 5;
     const int H = p.H, W = p.W;
     const int ntx = W / 16;
-    const int ntiles = ntx * (H / TY);
+    const int ntiles = ntx * (H / 16);
 
     // The split weights go through LDS (the P region, free until the first
     // halo tile's stores) once per block, then into every wave's registers.
     constexpr int NWU = CX_WPACK / 8, WIT = (NWU + CX_WAVES * 64 - 1) / (CX_WAVES * 64);  // 16-byte units
-    static_assert(NWU * 16 <= S::HP * CX_PS * 4, "the weights fit the P region");
+    static_assert(NWU % (CX_WAVES * 64) == 0 && NWU * 16 <= CX_HP * CX_PS * 4, "whole rounds; the weights fit the P region");
     u32x4 stage[WIT];
 #pragma unroll
-    for (int i = 0; i < WIT; ++i) {
-        const int e = min(tid + i * CX_WAVES * 64, NWU - 1);  // the last units again past the end
-        stage[i] = ((const u32x4*)p.w)[e];
-    }
+    for (int i = 0; i < WIT; ++i) stage[i] = ((const u32x4*)p.w)[tid + i * CX_WAVES * 64];
     float bias[CAB_CC];
 #pragma unroll
-    for (int co = 0; co < CAB_CC; ++co) bias[co] = p.bias[co];
+    for (int co = 0; co < CAB_CC; ++co) bias[co] = p.bias[co] * p.ts;
 
     // The lane's input row (channels 8h.. of each 16-channel step) for halo
     // tile i of output tile tl; hat_zero_row outside the plane, past the halo
@@ -86,59 +80,62 @@ __device__ __forceinline__ void cab_conv1_body(const CabConvArgs& p)
         const int ty = tl / ntx, tx = tl - ty * ntx;
         const int hi = (wave + CX_WAVES * i) * 32 + pl;
         const int hy = hi / CX_HS, hx = hi - hy * CX_HS;
-        const int gy = ty * TY - 1 + hy, gx = tx * 16 - 1 + hx;
-        const bool valid = tl < ntiles && hi < S::HP && gy >= 0 && gy < H && gx >= 0 && gx < W;
+        const int gy = ty * 16 - 1 + hy, gx = tx * 16 - 1 + hx;
+        const bool valid = tl < ntiles && hi < CX_HP && gy >= 0 && gy < H && gx >= 0 && gx < W;
         return valid ? p.xn + (size_t)(gy * W + gx) * CAB_C + 8 * h : hat_zero_row;
     };
-    f32x4 xr[9][2];
-    {
-        const float* first = src_of(blockIdx.x, 0);
+    // row steps in flight: step t of an output tile (halo tile t / 9, channels
+    // 16 (t % 9) ..) in slot t % CX_RING
+    f32x4 xr[CX_RING][2];
+    const float* cur = src_of(blockIdx.x, 0);
 #pragma unroll
-        for (int ks = 0; ks < 9; ++ks) {
-            xr[ks][0] = *(const f32x4*)(first + ks * 16);
-            xr[ks][1] = *(const f32x4*)(first + ks * 16 + 4);
-        }
+    for (int t = 0; t < CX_RING; ++t) {
+        xr[t][0] = *(const f32x4*)(cur + t * 16);
+        xr[t][1] = *(const f32x4*)(cur + t * 16 + 4);
     }
 #pragma unroll
-    for (int i = 0; i < WIT; ++i) ((u32x4*)Ps)[min(tid + i * CX_WAVES * 64, NWU - 1)] = stage[i];
+    for (int i = 0; i < WIT; ++i) ((u32x4*)Ps)[tid + i * CX_WAVES * 64] = stage[i];
     lds_barrier();
-    u32x4 wr[9][2][3];
+    u32x4 wr[9][2][2];
 #pragma unroll
     for (int ks = 0; ks < 9; ++ks)
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-            for (int part = 0; part < 3; ++part)
-                wr[ks][nt][part] = ((const u32x4*)Ps)[((ks * 2 + nt) * 3 + part) * 64 + lane];
+            for (int part = 0; part < 2; ++part)
+                wr[ks][nt][part] = ((const u32x4*)Ps)[((ks * 2 + nt) * 2 + part) * 64 + lane];
     lds_barrier();  // every wave has its weights before P is written
 
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         const int ty = tile / ntx, tx = tile - ty * ntx;
-        const int y0 = ty * TY, x0 = tx * 16;
+        const int y0 = ty * 16, x0 = tx * 16;
         // unrolled: with no back-edge here, the compiler's waits for the rows
         // read ahead are exact
 #pragma unroll
-        for (int i = 0; i < S::NPW; ++i) {
-            const float* nxt = i + 1 < S::NPW ? src_of(tile, i + 1) : src_of(tile + gridDim.x, 0);
+        for (int i = 0; i < CX_NPW; ++i) {
+            const float* nxt = i + 1 < CX_NPW ? src_of(tile, i + 1) : src_of(tile + gridDim.x, 0);
             f32x16 acc[2];
 #pragma unroll
             for (int j = 0; j < 16; ++j) acc[0][j] = acc[1][j] = 0.0f;
 #pragma unroll
             for (int ks = 0; ks < 9; ++ks) {
-                const float f[8] = {xr[ks][0][0], xr[ks][0][1], xr[ks][0][2], xr[ks][0][3],
-                                    xr[ks][1][0], xr[ks][1][1], xr[ks][1][2], xr[ks][1][3]};
-                u32x4 xb[3];
-                split3_x8(f, xb);
-                xr[ks][0] = *(const f32x4*)(nxt + ks * 16);  // step ks of the next halo tile
-                xr[ks][1] = *(const f32x4*)(nxt + ks * 16 + 4);
+                const int slot = (9 * i + ks) % CX_RING, ahead = ks + CX_RING;
+                const float f[8] = {xr[slot][0][0], xr[slot][0][1], xr[slot][0][2], xr[slot][0][3],
+                                    xr[slot][1][0], xr[slot][1][1], xr[slot][1][2], xr[slot][1][3]};
+                u32x4 xb[2];
+                split2_x8(f, xb);
+                const float* src = ahead < 9 ? cur + ahead * 16 : nxt + (ahead - 9) * 16;
+                xr[slot][0] = *(const f32x4*)src;
+                xr[slot][1] = *(const f32x4*)(src + 4);
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) acc[nt] = mfma6(wr[ks][nt], xb, acc[nt]);
+                for (int nt = 0; nt < 2; ++nt) acc[nt] = mfma3(wr[ks][nt], xb, acc[nt]);
                 __builtin_amdgcn_sched_barrier(0);  // the loads stay in their step
             }
+            cur = nxt;
             // lane (pl, h) holds P[hi][32 nt + 8 g + 4 h .. +3] in acc[nt][4g .. 4g+3];
             // columns 56.. (nt = 1, g = 3) are not stored
             const int hi = (wave + CX_WAVES * i) * 32 + pl;
-            if (hi < S::HP) {
+            if (hi < CX_HP) {
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
@@ -147,54 +144,57 @@ __device__ __forceinline__ void cab_conv1_body(const CabConvArgs& p)
                             (f32x4){acc[nt][4 * g], acc[nt][4 * g + 1], acc[nt][4 * g + 2], acc[nt][4 * g + 3]};
             }
         }
+        // the next output tile's first steps into slots 0 .. CX_RING - 1
+        {
+            f32x4 nx[CX_RING][2];
+#pragma unroll
+            for (int t = 0; t < CX_RING; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) nx[t][j] = xr[(9 * CX_NPW + t) % CX_RING][j];
+#pragma unroll
+            for (int t = 0; t < CX_RING; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) xr[t][j] = nx[t][j];
+        }
         lds_barrier();  // P complete
 
-        // The 9 taps from the halo products, NPX output pixels per thread
-        // (rows oy, oy + 16).
-        const int ox = tid & 15;
-        float v[S::NPX][CAB_CC];
+        // The 9 taps from the halo products, one output pixel per thread.
+        const int ox = tid & 15, oy = tid >> 4;
+        float v[CAB_CC];
 #pragma unroll
-        for (int r = 0; r < S::NPX; ++r) {
-            const int oy = (tid >> 4) + 16 * r;
+        for (int co = 0; co < CAB_CC; ++co) v[co] = 0.0f;
 #pragma unroll
-            for (int co = 0; co < CAB_CC; ++co) v[r][co] = bias[co];
+        for (int ky = 0; ky < 3; ++ky)
 #pragma unroll
-            for (int ky = 0; ky < 3; ++ky)
+            for (int kx = 0; kx < 3; ++kx) {
+                const float* q = Ps + ((oy + ky) * CX_HS + ox + kx) * CX_PS + (ky * 3 + kx) * CAB_CC;
 #pragma unroll
-                for (int kx = 0; kx < 3; ++kx) {
-                    const float* q = Ps + ((oy + ky) * CX_HS + ox + kx) * CX_PS + (ky * 3 + kx) * CAB_CC;
-#pragma unroll
-                    for (int j = 0; j < CAB_CC / 2; ++j) {
-                        const float2 t = *(const float2*)(q + 2 * j);
-                        v[r][2 * j] += t.x;
-                        v[r][2 * j + 1] += t.y;
-                    }
+                for (int j = 0; j < CAB_CC / 2; ++j) {
+                    const float2 t = *(const float2*)(q + 2 * j);
+                    v[2 * j] += t.x;
+                    v[2 * j + 1] += t.y;
                 }
+            }
 #pragma unroll
-            for (int co = 0; co < CAB_CC; ++co) v[r][co] = gelu(v[r][co]) * p.ts;
+        for (int co = 0; co < CAB_CC; ++co) v[co] = gelu_scaled(__builtin_fmaf(v[co], p.oinv, bias[co]), p.g0, p.g1);
+        {
             float* dst = p.t1 + ((size_t)(y0 + oy) * W + x0 + ox) * CAB_CS;
-            *(float4*)dst = make_float4(v[r][0], v[r][1], v[r][2], v[r][3]);
-            *(float4*)(dst + 4) = make_float4(v[r][4], v[r][5], 0.f, 0.f);
+            *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
+            *(float4*)(dst + 4) = make_float4(v[4], v[5], 0.f, 0.f);
         }
 
         // Per-tile sums: the tile, and its pixels on row 0, row H-1, col 0,
         // col W-1 - only tiles on the plane's border have any of the latter.
-        // A thread adds its pixels in row order, then the wave tree.
-        const bool border = y0 == 0 || y0 + TY == H || x0 == 0 || x0 + 16 == W;  // tile-uniform
+        const bool border = y0 == 0 || y0 + 16 == H || x0 == 0 || x0 + 16 == W;  // tile-uniform
 #pragma unroll
         for (int l = 0; l < CAB_NSUM; ++l) {
             if (l > 0 && !border) break;
 #pragma unroll
             for (int co = 0; co < CAB_CC; ++co) {
-                float s = 0.0f;
-#pragma unroll
-                for (int r = 0; r < S::NPX; ++r) {
-                    const int gy = y0 + (tid >> 4) + 16 * r, gx = x0 + ox;
-                    const bool on = l == 0 || (l == 1 && gy == 0) || (l == 2 && gy == H - 1) ||
-                                    (l == 3 && gx == 0) || (l == 4 && gx == W - 1);
-                    s += on ? v[r][co] : 0.0f;
-                }
-                s = wave_sum_dpp(s);
+                const int gy = y0 + oy, gx = x0 + ox;
+                const bool on = l == 0 || (l == 1 && gy == 0) || (l == 2 && gy == H - 1) || (l == 3 && gx == 0) ||
+                                (l == 4 && gx == W - 1);
+                const float s = wave_sum_dpp(on ? v[co] : 0.0f);
                 if (lane == 0) red[wave][l * CAB_CC + co] = s;
             }
         }
@@ -213,15 +213,6 @@ __device__ __forceinline__ void cab_conv1_body(const CabConvArgs& p)
         // and red above precedes it.
         lds_barrier();
     }
-}
-
-extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 1) void hat_cab_conv1(CabConvArgs p)
-{
-    cab_conv1_body<16>(p);
-}
-extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 1) void hat_cab_conv1_t32(CabConvArgs p)
-{
-    cab_conv1_body<32>(p);
 }
 
 // ---------------------------------------------------------------------------
