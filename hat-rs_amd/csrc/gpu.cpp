@@ -31,24 +31,6 @@ std::vector<float> pack_linear(const float* w, int N, int K, int* Kp)
     return out;
 }
 
-namespace {
-// float -> bf16, round to nearest even (NaN kept a NaN)
-unsigned short bf16_rne(float x)
-{
-    uint32_t u;
-    memcpy(&u, &x, 4);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
-float bf16_float(unsigned short h)
-{
-    const uint32_t u = (uint32_t)h << 16;
-    float f;
-    memcpy(&f, &u, 4);
-    return f;
-}
-}  // namespace
 
 // float -> f16, round to nearest even, subnormals kept, past the range infinite
 static inline unsigned short f16_rne(float x)
@@ -281,22 +263,24 @@ std::vector<float> pack_conv(const float* w, const float* b, int CO, int CI, int
 
 // [CO][CI][3][3] -> the Winograd F(2x2, 3x3) weights U[xi] = G g G^T of the
 // hat_convwino_* kernels, G = [1 0 0; 1/2 1/2 1/2; 1/2 -1/2 1/2; 0 0 1],
-// formed in double, rounded to fp32 and split into three bf16 parts, arranged
-// [kc][xi][nt][part][lane][8]: lane r + 16 g of (kc, xi, nt) holds part `part`
-// of U[xi][16 nt + r][32 kc + 8 g .. +7]; channels past CO and CI are zero
-// (CO padded to 16s, CI to 32s). With r > 0 the output channels are permuted
-// as pack_conv permutes them. When the last chunk holds at most 16 real
+// formed in double, rounded to fp32, scaled into f16's range and split into two
+// f16 parts, arranged [kc][xi][nt][part][lane][8]: lane r + 16 g of (kc, xi, nt)
+// holds part `part` of U[xi][16 nt + r][32 kc + 8 g .. +7]; channels past CO and CI
+// are zero (CO padded to 16s, CI to 32s). With r > 0 the output channels are
+// permuted as pack_conv permutes them. When the last chunk holds at most 16 real
 // channels (CI = 144), it is packed as the K = 144 linears' last step
-// (split_half_step): lane r + 16 g, slots j < 4 hold channel 32 kc + 4 g + j,
-// slots 4 + j the same channel, the parts as (0 | 0), (1 | 0), (1 | 2).
-std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r, bool fill)
+// (split2_half_step): lane r + 16 g, slots j < 4 hold channel 32 kc + 4 g + j,
+// slots 4 + j the same channel and part.
+std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r, float* uinv, bool fill)
 {
     if (r > 0 && CO % 16 != 0) throw Error("pack_wino: shuffled output channels must come in 16s");
     static const double G[4][3] = {{1, 0, 0}, {0.5, 0.5, 0.5}, {0.5, -0.5, 0.5}, {0, 0, 1}};
     const int NTT = (CO + 15) / 16, NKC = (CI + 31) / 32, Cf = r > 0 ? CO / (r * r) : 0;
     const bool packed = CI % 32 != 0 && CI % 32 <= 16;  // the kernels' PACK
-    std::vector<unsigned short> out((size_t)NKC * 16 * NTT * 3 * 512, 0);
+    std::vector<unsigned short> out((size_t)NKC * 16 * NTT * 2 * 512, 0);
+    *uinv = 1.0f;
     if (!fill) return out;
+    std::vector<float> U((size_t)CO * CI * 16);
     for (int o2 = 0; o2 < CO; ++o2) {
         int o = o2;
         if (r > 0) {
@@ -305,33 +289,33 @@ std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r, boo
         }
         for (int ci = 0; ci < CI; ++ci) {
             const float* g = w + ((size_t)o * CI + ci) * 9;
+            double t[4][3];  // G g
+            for (int i = 0; i < 4; ++i)
+                for (int b = 0; b < 3; ++b) {
+                    double u = 0.0;
+                    for (int a = 0; a < 3; ++a) u += G[i][a] * (double)g[a * 3 + b];
+                    t[i][b] = u;
+                }
             for (int i = 0; i < 4; ++i)
                 for (int j = 0; j < 4; ++j) {
                     double u = 0.0;
-                    for (int a = 0; a < 3; ++a)
-                        for (int b = 0; b < 3; ++b) u += G[i][a] * (double)g[a * 3 + b] * G[j][b];
-                    const float x = (float)u;
-                    const unsigned short h0 = bf16_rne(x);
-                    const float r1 = x - bf16_float(h0);
-                    const unsigned short h1 = bf16_rne(r1);
-                    const unsigned short h2 = bf16_rne(r1 - bf16_float(h1));
-                    const int xi = 4 * i + j, kc = ci / 32, c32 = ci % 32, nt = o2 / 16, rr = o2 % 16;
-                    if (packed && kc == NKC - 1) {
-                        const int lane = rr + 16 * (c32 / 4);
-                        const size_t at = ((((size_t)kc * 16 + xi) * NTT + nt) * 3 * 64 + lane) * 8 + c32 % 4;
-                        out[at] = h0, out[at + 4] = h0;
-                        out[at + 512] = h1, out[at + 512 + 4] = h0;
-                        out[at + 1024] = h1, out[at + 1024 + 4] = h2;
-                        continue;
-                    }
-                    const int lane = rr + 16 * (c32 / 8);
-                    const size_t at = ((((size_t)kc * 16 + xi) * NTT + nt) * 3 * 64 + lane) * 8 + c32 % 8;
-                    out[at] = h0;
-                    out[at + 512] = h1;
-                    out[at + 1024] = h2;
+                    for (int b = 0; b < 3; ++b) u += t[i][b] * G[j][b];
+                    U[((size_t)o2 * CI + ci) * 16 + 4 * i + j] = (float)u;
                 }
         }
     }
+    const float su = f16_scale(abs_max(U.data(), U.size()));
+    *uinv = 1.0f / su;
+    for (int o2 = 0; o2 < CO; ++o2)
+        for (int ci = 0; ci < CI; ++ci)
+            for (int xi = 0; xi < 16; ++xi) {
+                const int kc = ci / 32, c32 = ci % 32, nt = o2 / 16, rr = o2 % 16;
+                const bool half = packed && kc == NKC - 1;
+                const int lane = rr + 16 * (half ? c32 / 4 : c32 / 8);
+                const size_t at = ((((size_t)kc * 16 + xi) * NTT + nt) * 2 * 64 + lane) * 8 + (half ? c32 % 4 : c32 % 8);
+                split2_f16(U[((size_t)o2 * CI + ci) * 16 + xi] * su, &out[at], &out[at + 512]);
+                if (half) out[at + 4] = out[at], out[at + 512 + 4] = out[at + 512];
+            }
     return out;
 }
 
@@ -757,7 +741,7 @@ struct TailCabIn {
 };
 void run_tailx(hipStream_t s, const DevTail& t, const float* a, const float* res, float* out, float* xn, const float* bias,
                const float* b2, const float* n2w, const float* n2b, const float* nw, const float* nb, long M,
-               const TailCabIn& cab)
+               const TailCabIn& cab, Amax* out_max = nullptr)
 {
     const bool hab = nw != nullptr;
     if (hab != (t.C == 144 ? cab.t1 && cab.w2gx : cab.aux && cab.gate))
@@ -787,6 +771,10 @@ void run_tailx(hipStream_t s, const DevTail& t, const float* a, const float* res
     f.eps = 1e-5f;
     f.cscale = cab.cscale;
     tail_scales(t, &f);
+    if (out_max && !hab) {
+        f.amax_out = out_max->slot;
+        out_max->filled = true;
+    }
     const char* name = t.C == 144 ? (hab ? "hat_habx_cab_ln" : "hat_habx") : (hab ? "hat_habx180_hab_ln" : "hat_habx180");
     launch(s, name, (unsigned)wx_tiles((int)M), 1, 1, WX_THREADS, f);
 }
@@ -849,6 +837,26 @@ int colsum_rows(int CO, int H, int W, int co_stride)
     return colsum_wide(CO, H, W, co_stride) ? (W / 16) * (H / 16) : (W / 16) * (H / 8);
 }
 
+// The Winograd kernels' scales: V's from the host, or (in_max) of the input's
+// largest magnitude, found here over its n floats where no kernel has left it.
+void wino_scales(hipStream_t s, const DevConv& C, long n, Amax* in_max, Amax* out_max, ConvArgs* p)
+{
+    p->uinv = C.uinv;
+    p->vs = C.vs;
+    if (in_max) {
+        if (!in_max->filled) {
+            AbsMaxArgs a{p->in, in_max->slot, n};
+            launch(s, "hat_absmax", (unsigned)std::min<long>((n + 4095) / 4096, 2048), 1, 1, 256, a);
+            in_max->filled = true;
+        }
+        p->amax = in_max->slot;
+    }
+    if (out_max) {
+        p->amax_out = out_max->slot;
+        out_max->filled = true;
+    }
+}
+
 // [band_r0, band_r1): with band_r1 >= 0, only that band of tile rows is
 // launched (the host-memory forward's head): 8 input rows of the Winograd
 // upsample conv (hat_convwino_n8_shuffle), 16 output rows of conv_last
@@ -856,7 +864,8 @@ int colsum_rows(int CO, int H, int W, int co_stride)
 // doubles the rows. Other convs are always whole planes.
 void run_conv(hipStream_t s, const DevConv& C, const float* in, int cin_stride, int H, int W,
               float* out, int co_stride, int epi, int act, const float* res, float* partial,
-              int crop_h, int crop_w, float img_range, const float* mean, int band_r0, int band_r1)
+              int crop_h, int crop_w, float img_range, const float* mean, int band_r0, int band_r1, Amax* in_max,
+              Amax* out_max, float os)
 {
     if (H % 8 != 0 || W % 16 != 0) throw Error("conv: plane must be a multiple of 8x16");
     const bool band = band_r1 >= 0;
@@ -932,7 +941,11 @@ void run_conv(hipStream_t s, const DevConv& C, const float* in, int cin_stride, 
     // conv_before_upsample and the x2 upsample convs by Winograd F(2x2, 3x3):
     // 8 x 16 output tiles, 32-bit element offsets into both planes
     p.wu = C.wu;
-    auto wino = [&](const char* name, unsigned tiles, unsigned ncb) { launch_wino(s, name, tiles, ncb, p); };
+    p.os = os;
+    auto wino = [&](const char* name, unsigned tiles, unsigned ncb) {
+        wino_scales(s, C, (long)H * W * cin_stride, in_max, out_max, &p);
+        launch_wino(s, name, tiles, ncb, p);
+    };
     const size_t rr = C.r > 0 ? (size_t)C.r * C.r : 1;
     if (C.wu && H % 16 == 0 && W % 16 == 0 && cin_stride % 4 == 0 && cin_stride >= C.CI &&
         (size_t)H * W * cin_stride < ((size_t)1 << 31) && (size_t)H * W * rr * co_stride < ((size_t)1 << 31)) {
@@ -1004,7 +1017,8 @@ bool convw_fits(const DevConv& C) { return C.r == 0 && C.CO == 144 && C.COp == 1
 void run_ln(hipStream_t s, const float* x, float* y, const float* w, const float* b, long rows, int C);
 
 void run_convw(hipStream_t s, const DevConv& C, const float* in, int cin_stride, int H, int W,
-               float* out, int epi, const float* res, float* xn, const float* nw, const float* nb)
+               float* out, int epi, const float* res, float* xn, const float* nw, const float* nb, Amax* in_max,
+               Amax* out_max)
 {
     if (!convw_fits(C)) throw Error("convw: needs 144 output channels");
     if (H % 16 != 0 || W % 16 != 0) throw Error("convw: plane must be 16-aligned");
@@ -1042,6 +1056,7 @@ void run_convw(hipStream_t s, const DevConv& C, const float* in, int cin_stride,
     if (C.wu && C.CI == 144 && (epi == EPI_RESID_LN || epi == EPI_RESID) && H % 8 == 0 &&
         (size_t)H * W * cin_stride < ((size_t)1 << 31)) {
         if (in == out) throw Error("convw: the output must not overlap the input");
+        wino_scales(s, C, (long)H * W * cin_stride, in_max, out_max, &p);
         launch_wino(s, "hat_convwino_resid", (unsigned)((W / 16) * (H / 8)), 1, p);
         if (epi == EPI_RESID_LN) run_ln(s, out, xn, nw, nb, (long)H * W, C.CO);
         return;
@@ -1237,6 +1252,26 @@ void GpuBackend::upload_attn(const std::string& qkv, const std::string& proj, co
     v_scale_ = s.v;
 }
 
+double GpuBackend::cab_t1_bound(const std::string& cab, const std::string& norm1) const
+{
+    // conv1's nine taps of norm1 rows, and |gelu(v)| <= |v|
+    const size_t C = (size_t)wt_.embed;
+    const float *w = wt_.t(cab + "0.weight"), *b = wt_.t(cab + "0.bias"), *lw = wt_.t(norm1 + ".weight"),
+                *lb = wt_.t(norm1 + ".bias");
+    std::vector<float> row(C);
+    double worst = 0.0;
+    for (int co = 0; co < wt_.compressed; ++co) {
+        double v = std::fabs((double)b[co]);
+        for (int tap = 0; tap < 9; ++tap) {
+            for (size_t ci = 0; ci < C; ++ci) row[ci] = w[(co * C + ci) * 9 + tap];
+            v += ln_linear_bound(row.data(), nullptr, lw, lb, 0, 1, (int)C);
+        }
+        if (std::isnan(v)) return v;
+        worst = std::max(worst, v);
+    }
+    return worst;
+}
+
 void GpuBackend::upload_tail(const std::string& proj, const std::string& mlp, const std::string& norm2,
                              const std::string& cab, const std::string& norm1)
 {
@@ -1252,18 +1287,7 @@ void GpuBackend::upload_tail(const std::string& proj, const std::string& mlp, co
     if (!fits) return;
     TailCab tc{0.0, 0.0};
     if (!cab.empty() && !count_only_) {
-        // |t1|: conv1's nine taps of norm1 rows
-        const float *w = wt_.t(cab + "0.weight"), *b = wt_.t(cab + "0.bias"), *lw = wt_.t(norm1 + ".weight"),
-                    *lb = wt_.t(norm1 + ".bias");
-        std::vector<float> row(C);
-        for (int co = 0; co < CAB_CC; ++co) {
-            double v = std::fabs((double)b[co]);
-            for (int tap = 0; tap < 9; ++tap) {
-                for (size_t ci = 0; ci < C; ++ci) row[ci] = w[(co * C + ci) * 9 + tap];
-                v += ln_linear_bound(row.data(), nullptr, lw, lb, 0, 1, (int)C);
-            }
-            tc.t1 = std::isnan(v) ? v : std::max(tc.t1, v);
-        }
+        tc.t1 = cab_t1_bound(cab, norm1);
         tc.w2 = std::fabs((double)wt_.conv_scale) * abs_max(wt_.t(cab + "2.weight"), C * CAB_CC * 9);
     }
     TailPack p = pack_tail(wt_.t(proj + ".weight"), wt_.t(mlp + ".fc1.weight"), wt_.t(mlp + ".fc1.bias"),
@@ -1275,7 +1299,7 @@ void GpuBackend::upload_tail(const std::string& proj, const std::string& mlp, co
     tail_[mlp] = p.t;
 }
 
-void GpuBackend::upload_conv(const std::string& name, int r, float in)
+void GpuBackend::upload_conv(const std::string& name, int r, float in, double bound)
 {
     const TensorInfo& ti = wt_.info(name + ".weight");
     DevConv C;
@@ -1294,7 +1318,8 @@ void GpuBackend::upload_conv(const std::string& name, int r, float in)
     C.w = upload(pk.data(), pk.size());
     C.b = upload(bias.data(), bias.size());
     if (wino_conv(C.CO, C.CI, r)) {
-        std::vector<unsigned short> wu = pack_wino(w, C.CO, C.CI, r, !count_only_);
+        std::vector<unsigned short> wu = pack_wino(w, C.CO, C.CI, r, &C.uinv, !count_only_);
+        C.vs = f16_scale(4.0 * bound);  // |B^T d B| <= 4 max|d|
         C.wu = (unsigned short*)upload_bytes(wu.data(), wu.size() * sizeof(unsigned short));
     }
     conv_[name] = C;
@@ -1373,8 +1398,13 @@ void GpuBackend::upload_all()
                 cb.bb = raw_.at(c + "3.attention.3.bias");
                 cab_[p] = cb;
             } else {
-                upload_conv(p + ".conv_block.cab.0", 0, xin);
-                upload_conv(p + ".conv_block.cab.2");
+                // norm1's rows are below 2^15 as stored (upload_norm); conv1
+                // leaves t1 scaled for conv2's transform
+                const float ts = wino_conv(wt.embed, wt.compressed, 0) && !count_only_
+                                     ? f16_scale(4.0 * cab_t1_bound(p + ".conv_block.cab.", p + ".norm1")) : 1.0f;
+                t1_scale_[p] = ts;
+                upload_conv(p + ".conv_block.cab.0", 0, xin, 32768.0);
+                upload_conv(p + ".conv_block.cab.2", 0, 1.0f / ts, 8192.0);
             }
         }
         const std::string p = L + ".residual_group.overlap_attn";
@@ -1386,7 +1416,7 @@ void GpuBackend::upload_all()
     }
     upload_raw("norm.weight");
     upload_raw("norm.bias");
-    upload_conv("conv_after_body");
+    upload_conv("conv_after_body", 0, 1.0f, ln_bound(wt.t("norm.weight"), wt.t("norm.bias"), wt.embed));
     upload_conv("conv_before_upsample.0");
     const auto blocks = wt.up_blocks();
     for (size_t b = 0; b < blocks.size(); ++b)
@@ -1465,6 +1495,8 @@ std::vector<std::pair<float**, size_t>> GpuBackend::layout(const Weights& wt_, c
         {&a.w2g, cab_fold_ ? C * CAB_K2 : 0},
         {&a.w2gx, cab_fold_ ? (size_t)CAB_W2GX : 0},
         {&a.bias2, cab_fold_ ? C : 0},
+        // (the folded CAB's are in w2gx's buffer: magnitude_slots)
+        {&a.amax, cab_fold_ ? 0 : (size_t)AMAX_SLOTS * AMAX_WORDS},
         {&a.t2, cab_fold_ ? 0 : T * C},
         {&a.partial, cab_fold_ ? 0 : nblk * C},
         {&a.red, cab_fold_ ? 0 : (nblk + 31) / 32 * C},
@@ -1538,10 +1570,10 @@ void GpuBackend::mlp(const std::string& prefix, float* x, int epi, const std::st
 
 void GpuBackend::conv(const DevConv& C, const float* in, int cin_stride, int H, int W, float* out,
                       int co_stride, int epi, int act, const float* res, float* partial,
-                      int crop_h, int crop_w, int band_r0, int band_r1)
+                      int crop_h, int crop_w, int band_r0, int band_r1, Amax* in_max, Amax* out_max, float os)
 {
     run_conv(stream_, C, in, cin_stride, H, W, out, co_stride, epi, act, res, partial, crop_h,
-             crop_w, wt_.img_range, wt_.mean, band_r0, band_r1);
+             crop_w, wt_.img_range, wt_.mean, band_r0, band_r1, in_max, out_max, os);
 }
 
 void GpuBackend::attention(const std::string& table, bool oca, int shift, const CabGateArgs* gate,
@@ -1591,7 +1623,8 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
         return;
     }
     // CAB: conv3x3 -> GELU -> conv3x3 (+ per-tile channel sums) -> gate.
-    conv(conv_.at(p + ".conv_block.cab.0"), a_.xn, C, H, W, a_.t1, t1_stride_, CEPI_STORE, 1);
+    conv(conv_.at(p + ".conv_block.cab.0"), a_.xn, C, H, W, a_.t1, t1_stride_, CEPI_STORE, 1, nullptr,
+         nullptr, 0, 0, 0, -1, nullptr, nullptr, t1_scale_.at(p));
     conv(conv_.at(p + ".conv_block.cab.2"), a_.t1, t1_stride_, H, W, a_.t2, C, CEPI_COLSUM, 0, nullptr,
          a_.partial);
     // The gate: computed by the attention launch's first block where it fits.
@@ -1624,7 +1657,7 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
 
 // OCAB.forward (hat_arch.py:392-438; cpu.rs:1170-1198): x = proj(attn) + x;
 // x = x + mlp(norm2 x). On entry a_.xn holds norm1(x).
-void GpuBackend::ocab(int stage, float* x)
+void GpuBackend::ocab(int stage, float* x, Amax* out_max)
 {
     const std::string p = "layers." + std::to_string(stage) + ".residual_group.overlap_attn";
     const long T = plan_.tokens();
@@ -1636,7 +1669,7 @@ void GpuBackend::ocab(int stage, float* x)
     auto tl = tail_.find(p + ".mlp");
     if (tl != tail_.end()) {
         run_tailx(stream_, tl->second, a_.ao, x, x, nullptr, proj.b, fc2.b, raw_.at(p + ".norm2.weight"),
-                  raw_.at(p + ".norm2.bias"), nullptr, nullptr, T, TailCabIn{});
+                  raw_.at(p + ".norm2.bias"), nullptr, nullptr, T, TailCabIn{}, out_max);
         return;
     }
     if (hab_tail_fits(proj, fc1, fc2)) {
@@ -1715,12 +1748,20 @@ void GpuBackend::forward_noalloc(int h, int w, const float* d_in, float* d_out)
     nblk_conv2_ = saved_nblk;
 }
 
+unsigned* GpuBackend::magnitude_slots(int i) const
+{
+    static_assert(CAB_W2GX >= CAB_W2GX_USED + AMAX_SLOTS * AMAX_WORDS, "the slots fit behind the gated weights");
+    unsigned* base = (unsigned*)(cab_fold_ ? a_.w2gx + CAB_W2GX_USED : a_.amax);
+    return base + (size_t)i * AMAX_WORDS;
+}
+
 // The forward on the current plan's buffers (a_, plan_).
 void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std::vector<std::pair<int, int>>* bands)
 {
     const long T = plan_.tokens();
     const int C = wt_.embed, H = plan_.hp, W = plan_.wp;
-    PreArgs pa{d_in, a_.x0, h, w, H, W, 4, wt_.mean[0], wt_.mean[1], wt_.mean[2], wt_.img_range};
+    PreArgs pa{d_in, a_.x0, h, w, H, W, 4, wt_.mean[0], wt_.mean[1], wt_.mean[2], wt_.img_range,
+               magnitude_slots(0)};
     launch(stream_, "hat_pre", (unsigned)((T + 255) / 256), 1, 1, 256, pa);
     const DevConv& cf = conv_.at("conv_first");
     // With 144 channels the trunk convs carry the LayerNorm that follows them.
@@ -1749,7 +1790,7 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
                1, 256, p);
     } else if (fused) {
         run_convw(stream_, cf, a_.x0, 4, H, W, a_.body, EPI_STORE_LN, nullptr, a_.xa,
-                  raw_.at("patch_embed.norm.weight"), raw_.at("patch_embed.norm.bias"));
+                  raw_.at("patch_embed.norm.weight"), raw_.at("patch_embed.norm.bias"), nullptr, nullptr);
     } else {
         conv(cf, a_.x0, 4, H, W, a_.body, C, CEPI_STORE, 0);
         layernorm(a_.body, a_.xa, "patch_embed.norm", T);
@@ -1768,7 +1809,9 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
                                          : L + "overlap_attn.norm1";
             hab((int)s, b, b == 0 ? a_.xa : a_.xb, a_.xb, next);
         }
-        ocab((int)s, a_.xb);
+        // the stage's conv needs its input's range (no norm comes between)
+        Amax xmax{magnitude_slots((int)s), false};
+        ocab((int)s, a_.xb, &xmax);
         const DevConv& rc = conv_.at("layers." + std::to_string(s) + ".conv");
         if (fused) {
             // x = conv(blocks) + x, then the next stage's norm1 or the final
@@ -1776,27 +1819,33 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
             const std::string nn = s + 1 < S ? "layers." + std::to_string(s + 1) + ".residual_group.blocks.0.norm1"
                                              : std::string("norm");
             run_convw(stream_, rc, a_.xb, C, H, W, a_.xa, EPI_RESID_LN, a_.xa, a_.xn, raw_.at(nn + ".weight"),
-                      raw_.at(nn + ".bias"));
+                      raw_.at(nn + ".bias"), &xmax, nullptr);
         } else {
-            conv(rc, a_.xb, C, H, W, a_.xa, C, CEPI_RESID, 0, a_.xa);
+            conv(rc, a_.xb, C, H, W, a_.xa, C, CEPI_RESID, 0, a_.xa, nullptr, 0, 0, 0, -1, &xmax);
         }
     }
+    // the head's planes: conv_after_body's output, then each conv's
+    Amax hmax{magnitude_slots(AMAX_HEAD), false};
     if (fused) {
         run_convw(stream_, conv_.at("conv_after_body"), a_.xn, C, H, W, a_.xa, EPI_RESID, a_.body, nullptr,
-                  nullptr, nullptr);
+                  nullptr, nullptr, nullptr, &hmax);
     } else {
         layernorm(a_.xa, a_.xb, "norm", T);
-        conv(conv_.at("conv_after_body"), a_.xb, C, H, W, a_.xa, C, CEPI_RESID, 0, a_.body);
+        conv(conv_.at("conv_after_body"), a_.xb, C, H, W, a_.xa, C, CEPI_RESID, 0, a_.body, nullptr, 0, 0, 0, -1, nullptr,
+             &hmax);
     }
     // Head (gpu.rs:622-653): conv + LeakyReLU, [conv + PixelShuffle] per block, conv_last.
     const int feat = wt_.head_feat;
-    conv(conv_.at("conv_before_upsample.0"), a_.xa, C, H, W, a_.head0, feat, CEPI_STORE, 2);
+    Amax cmax{magnitude_slots(AMAX_HEAD + 1), false};  // of cur
+    conv(conv_.at("conv_before_upsample.0"), a_.xa, C, H, W, a_.head0, feat, CEPI_STORE, 2, nullptr, nullptr, 0, 0, 0, -1,
+         &hmax, &cmax);
     float* cur = a_.head0;
     float* nxt = a_.head1;
     int hh = H, ww = W;
     const auto blocks = wt_.up_blocks();
     const DevConv& last = conv_.at("conv_last");
     const int oh = h * wt_.scale, ow = w * wt_.scale;
+    if (blocks.size() + AMAX_HEAD + 2 > AMAX_SLOTS || S > AMAX_HEAD) throw Error("forward: too many stages or upsample convs");
     for (size_t b = 0; b < blocks.size(); ++b) {
         const DevConv& up = conv_.at("upsample." + std::to_string(2 * b));
         if (bands && b + 1 == blocks.size() && head_bands_fit(up, last, hh, ww, feat)) {
@@ -1813,11 +1862,11 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
             const int nb = (int)bnd.size() - 1;
             if (nb > (int)band_ev_.size()) throw Error("forward: too many output bands");
             bands->clear();
-            conv(up, cur, feat, hh, ww, nxt, feat, CEPI_SHUFFLE, 0, nullptr, nullptr, 0, 0, bnd[0], bnd[1]);
+            conv(up, cur, feat, hh, ww, nxt, feat, CEPI_SHUFFLE, 0, nullptr, nullptr, 0, 0, bnd[0], bnd[1], &cmax);
             for (int k = 0; k < nb; ++k) {
                 if (k + 1 < nb)
                     conv(up, cur, feat, hh, ww, nxt, feat, CEPI_SHUFFLE, 0, nullptr, nullptr, 0, 0, bnd[k + 1],
-                         bnd[k + 2]);
+                         bnd[k + 2], &cmax);
                 conv(last, nxt, feat, 2 * hh, 2 * ww, d_out, 0, CEPI_FINAL, 0, nullptr, nullptr, oh, ow, bnd[k],
                      bnd[k + 1]);
                 Runtime::get().check(Runtime::get().api().EventRecord(band_ev_[k], stream_), "hipEventRecord");
@@ -1825,7 +1874,10 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
             }
             return;
         }
-        conv(up, cur, feat, hh, ww, nxt, feat, CEPI_SHUFFLE, 0);
+        Amax nmax{magnitude_slots(AMAX_HEAD + 2 + (int)b), false};
+        conv(up, cur, feat, hh, ww, nxt, feat, CEPI_SHUFFLE, 0, nullptr, nullptr, 0, 0, 0, -1, &cmax,
+             b + 1 < blocks.size() ? &nmax : nullptr);
+        cmax = nmax;
         hh *= blocks[b].first;
         ww *= blocks[b].first;
         std::swap(cur, nxt);
@@ -2305,15 +2357,16 @@ void op_swmsa(const float* x, float* out, int hp, int wp, int c, int heads, int 
         // the planes first, and the input's largest finite |x|, which is what
         // bounds q, k and v here (no norm comes before them)
         OpArena ar;
-        const float zero = 0.0f;
+        const std::vector<float> zero(AMAX_WORDS, 0.0f);
         const size_t ix = ar.add(T * c, x), iq = ar.add(3 * T * c), iao = ar.add(T * c), iout = ar.add(T * c),
-                     imax = ar.add(1, &zero);
+                     imax = ar.add(AMAX_WORDS, zero.data());
         ar.commit();
         float *dx = ar.ptr(ix), *dq = ar.ptr(iq), *dao = ar.ptr(iao), *dout = ar.ptr(iout);
         AbsMaxArgs am{dx, (unsigned*)ar.ptr(imax), (long)(T * c)};
         launch(s, "hat_absmax", (unsigned)std::min<size_t>((T * c + 4095) / 4096, 512), 1, 1, 256, am);
-        float mx = 0.0f;
-        rt.d2h(&mx, ar.ptr(imax), sizeof mx);
+        float lanes[AMAX_WORDS], mx = 0.0f;
+        rt.d2h(lanes, ar.ptr(imax), sizeof lanes);
+        for (float v : lanes) mx = std::max(mx, v);
         const QkvScale sc = qkv_scale(op_linear_bound(qkv_w, qkv_b, 0, c, c, mx),
                                       op_linear_bound(qkv_w, qkv_b, c, 2 * c, c, mx),
                                       op_linear_bound(qkv_w, qkv_b, 2 * c, 3 * c, c, mx), D);

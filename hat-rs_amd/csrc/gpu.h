@@ -70,6 +70,8 @@ struct DevConv {
     float* w = nullptr;  // [CIp/16][9][COp][16]
     float* b = nullptr;  // [COp]
     unsigned short* wu = nullptr;  // convs with a Winograd kernel: split U (pack_wino)
+    float uinv = 1.0f;             // takes U's scale out
+    float vs = 1.0f;               // V's scale where the host knows it
     int CI = 0, CIp = 0, CO = 0, COp = 0, r = 0;
 };
 
@@ -131,10 +133,16 @@ void tail_scales(const DevTail& t, hatk::TailXArgs* f);
 TailPack pack_tail(const float* wp, const float* w1, const float* b1, const float* w2, const float* n2w, const float* n2b,
                    int C, float sv, float sn, const TailCab* cab, bool fill = true);
 
-// Winograd U = G g G^T of a 3x3 conv [CO][CI][3][3] (formed in double), split
-// into three bf16 parts in the layout convwino.hip streams:
-// [32-channel chunk][point][16-channel tile][part][lane][8].
-std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r, bool fill = true);
+// Winograd U = G g G^T of a 3x3 conv [CO][CI][3][3] (formed in double), times the
+// power of two 1 / *uinv and split into two f16 parts in the layout convwino.hip
+// streams: [32-channel chunk][point][16-channel tile][part][lane][8].
+std::vector<unsigned short> pack_wino(const float* w, int CO, int CI, int r, float* uinv, bool fill = true);
+// A plane's largest magnitude on the device (ConvArgs::amax), and whether a kernel
+// of this forward has left it there.
+struct Amax {
+    unsigned* slot = nullptr;
+    bool filled = false;
+};
 std::vector<float> pack_conv(const float* w, const float* b, int CO, int CI, int r,
                              std::vector<float>* bias_out, int* CIp, int* COp);
 // A Winograd conv kernel (convwino.hip) over `tiles` 8 x 16 tiles in `ncb`
@@ -210,7 +218,7 @@ private:
         float *x0 = nullptr, *body = nullptr, *xa = nullptr, *xb = nullptr, *xn = nullptr, *t1 = nullptr,
               *t2 = nullptr, *partial = nullptr, *red = nullptr, *gate = nullptr, *qkv = nullptr, *ao = nullptr,
               *hidden = nullptr, *head0 = nullptr, *head1 = nullptr, *din = nullptr, *dout = nullptr,
-              *cab_part = nullptr, *w2g = nullptr, *w2gx = nullptr, *bias2 = nullptr;
+              *cab_part = nullptr, *w2g = nullptr, *w2gx = nullptr, *bias2 = nullptr, *amax = nullptr;
     };
     // Each buffer of plan p and its size in floats (0: not used by this
     // network); host_io adds the staging buffers of the host-memory forward.
@@ -260,7 +268,12 @@ private:
     // An attention's qkv and projection behind norm `ln`, scaled for the
     // split-f16 attention where the bounds allow it (attn_f16_ of its table).
     void upload_attn(const std::string& qkv, const std::string& proj, const std::string& ln, const std::string& table);
-    void upload_conv(const std::string& name, int r = 0, float in = 1.0f);  // in: as upload_linear's
+    // in: as upload_linear's; bound: of the input's |x| as the kernel reads it, or 0
+    // where only the device can know (Amax)
+    void upload_conv(const std::string& name, int r = 0, float in = 1.0f, double bound = 0.0);
+    // what |t1| (the CAB's conv1 output) cannot exceed behind norm1
+    double cab_t1_bound(const std::string& cab, const std::string& norm1) const;
+    std::map<std::string, float> t1_scale_;  // by block: the unfolded CAB's t1
     // the split-f16 tail of a block, where its shapes have one (upload_attn first;
     // conv: the folded CAB's prefix, or empty)
     void upload_tail(const std::string& proj, const std::string& mlp, const std::string& norm2, const std::string& cab,
@@ -281,12 +294,14 @@ private:
               float* xn = nullptr, const std::string& norm = "");
     void conv(const DevConv& C, const float* in, int cin_stride, int H, int W, float* out,
               int co_stride, int epi, int act, const float* res = nullptr, float* partial = nullptr,
-              int crop_h = 0, int crop_w = 0, int band_r0 = 0, int band_r1 = -1);
+              int crop_h = 0, int crop_w = 0, int band_r0 = 0, int band_r1 = -1, Amax* in_max = nullptr,
+              Amax* out_max = nullptr, float os = 1.0f);
     void attention(const std::string& table, bool oca, int shift, const hatk::CabGateArgs* gate = nullptr,
                    const hatk::SeArgs* se = nullptr);
     void mlp(const std::string& prefix, float* x, int epi, const std::string& norm);
     void hab(int stage, int block, float* x_in, float* x_out, const std::string& next_norm);
-    void ocab(int stage, float* x);
+    void ocab(int stage, float* x, Amax* out_max);
+    unsigned* magnitude_slots(int i) const;  // the current plan's i-th
 };
 
 // Isolated ops on host buffers (cfg2 / cfg3 of the benchmark plan). Each

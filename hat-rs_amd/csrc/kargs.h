@@ -86,8 +86,10 @@ struct GemmArgs {
 // tile nt (2 x 32 rows, row tap*6 + co, rows 54.. zero) and part (2), the
 // 32x32x16 A operand of each lane (row l % 32, channels 16 ks + 8 (l / 32) .. +7)
 #define CX_WPACK (9 * 2 * 2 * 64 * 8)
-// floats of the gated conv2 weights' buffer (CabGateArgs::w2gx: 9216 used)
+// floats of the gated conv2 weights' buffer: CabGateArgs::w2gx, then the forward's
+// magnitude slots (AMAX_SLOTS)
 #define CAB_W2GX 20480
+#define CAB_W2GX_USED (2 * CAB_C * 32)
 #define CAB_NSUM 5           // per-tile sums: whole tile, row 0, row H-1, col 0, col W-1
 
 struct CabConvArgs {
@@ -151,8 +153,8 @@ struct ConvArgs {
     const float* nw;
     const float* nb;
     float eps;
-    // hat_convwino_*: Winograd F(2x2,3x3) weights U = G g G^T split into three
-    // bf16 parts, arranged [kc][xi 16][nt][part 3][lane 64][8] (lane r + 16 g:
+    // hat_convwino_*: Winograd F(2x2,3x3) weights U = G g G^T, scaled by 1 / uinv
+    // and split into two f16 parts, arranged [kc][xi 16][nt][part 2][lane 64][8] (lane r + 16 g:
     // co 16 nt + r, ci 32 kc + 8 g .. +7; channels padded to 16s and 32s)
     const unsigned short* wu;
     // hat_convwino_* and hat_conv_last3 launched over a band of tile rows (the
@@ -161,6 +163,12 @@ struct ConvArgs {
     // hat_convwino_*: the launch's virtual blocks (tiles x column blocks),
     // walked by a grid of at most one block per CU; 0: one per block
     int nblk;
+    // hat_convwino_*: V's scale, a power of two, from the host (vs) or from the
+    // input's largest magnitude (amax, its bits); where to leave the output's
+    // (amax_out, null: nowhere); the scale of a GELU output (os)
+    float uinv, vs, os;
+    const unsigned* amax;
+    unsigned* amax_out;
 };
 
 // Squeeze-excite gate: gate[c] = sigmoid(b2 + W2 relu(b1 + W1 mean)).
@@ -311,6 +319,7 @@ struct TailXArgs {
     float ps, pi;               // the projection accumulators' scale and its inverse
     float h1, g0, g1;           // fc1's accumulators to scaled hidden units; gelu_scaled's constants
     float ms, mi;               // the output accumulators' scale and its inverse
+    unsigned* amax_out;         // OCAB: out's largest finite magnitude (if set)
 };
 
 struct LnArgs {
@@ -322,11 +331,23 @@ struct LnArgs {
     float eps;
 };
 
+// A forward's magnitude slots: the bits of the largest finite |x| of the planes
+// that no norm bounds and a Winograd conv reads (ConvArgs::amax): per stage its
+// last block's output, then the head's planes. At most 32 stages. A slot is
+// AMAX_LANES words AMAX_STRIDE apart (64 bytes), whose maximum it is: one a XCD, so
+// that a kernel's blocks do not all meet in one word.
+#define AMAX_SLOTS 64
+#define AMAX_HEAD 40
+#define AMAX_LANES 8
+#define AMAX_STRIDE 16
+#define AMAX_WORDS (AMAX_LANES * AMAX_STRIDE)
+
 struct PreArgs {
     const float* in;     // [3][h][w]
     float* out;          // [hp][wp][cstride], channels >= 3 zeroed
     int h, w, hp, wp, cstride;
     float m0, m1, m2, range;
+    unsigned* amax;      // [AMAX_SLOTS][AMAX_WORDS], zeroed (if set)
 };
 
 // dst[i] = src[i] for n4 float4 (16-byte aligned buffers).
@@ -336,8 +357,8 @@ struct CopyArgs {
     long n4;
 };
 
-// out[0] = max(out[0], bits of the largest finite |x[i]|), i < n (a multiple of
-// 4): the bits of non-negative floats order as unsigned integers do.
+// The largest finite |x[i]|, i < n (a multiple of 4), into a magnitude slot
+// (AMAX_SLOTS) that holds zeros.
 struct AbsMaxArgs {
     const float* x;
     unsigned* out;

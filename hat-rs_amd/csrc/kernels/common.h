@@ -350,6 +350,37 @@ __device__ __forceinline__ float wave_sum(float v)
     return v;
 }
 
+// max(m, |v|), infinities and NaN left out.
+__device__ __forceinline__ float finite_max(float m, float v)
+{
+    const float a = fabsf(v);
+    return a <= 3.402823466e38f ? fmaxf(m, a) : m;
+}
+
+// A plane's largest magnitude (kargs.h AMAX_LANES): the block's, by an LDS maximum
+// over its waves and one atomic into the lane of its XCD, blockIdx.x & 7. (An atomic a
+// wave into one word took 70 us of the 64-channel conv at 512 x 512.) The bits of
+// non-negative floats order as unsigned integers do, and a maximum does not depend
+// on the order. lds: zeroed before an earlier barrier; every thread of the block
+// calls this.
+__device__ __forceinline__ void block_amax(unsigned* out, unsigned* lds, float m)
+{
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(lds, __float_as_uint(m));
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(out + (blockIdx.x % AMAX_LANES) * AMAX_STRIDE, *lds);
+}
+
+// The magnitude (its bits) that block_amax left.
+__device__ __forceinline__ unsigned read_amax(const unsigned* p)
+{
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < AMAX_LANES; ++i) m = max(m, p[i * AMAX_STRIDE]);
+    return m;
+}
+
 // The wave's sum in registers alone (DPP, no LDS round trips), wave-uniform:
 // pairs, quads, 8 (half-row mirror), 16 (row mirror), then row 0 into row 1
 // and row 2 into row 3 (row_bcast:15), rows 0-1 into row 3 (row_bcast:31);

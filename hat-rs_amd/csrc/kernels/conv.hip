@@ -123,7 +123,7 @@ __device__ __forceinline__ void conv_body(const ConvArgs& p)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 v[j] = acc[mt][nt][j] + (co + j < p.COp ? p.bias[co + j] : 0.0f);
-                if (p.act == 1) v[j] = gelu(v[j]);
+                if (p.act == 1) v[j] = gelu(v[j]) * p.os;
                 else if (p.act == 2) v[j] = v[j] < 0.0f ? v[j] * 0.01f : v[j];
             }
             if (!live || co >= p.CO) continue;

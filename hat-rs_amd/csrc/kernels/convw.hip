@@ -224,7 +224,7 @@ __device__ __forceinline__ void convw_body(const ConvArgs& p)
                         for (int j = 0; j < 4; ++j) v[j] = v[j] < 0.0f ? v[j] * 0.01f : v[j];
                     } else if (p.act == 1) {
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) v[j] = gelu(v[j]);
+                        for (int j = 0; j < 4; ++j) v[j] = gelu(v[j]) * p.os;
                     }
                     *(float4*)(p.out + ((size_t)y * W + x) * p.co_stride + co) = make_float4(v[0], v[1], v[2], v[3]);
                 } else {

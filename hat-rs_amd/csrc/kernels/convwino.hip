@@ -30,10 +30,12 @@
 // the current tile's epilogue). Wave w computes the two transform
 // points xi = 2w, 2w + 1 (B^T row i = w / 2, columns j = 2 (w % 2) + {0, 1}),
 // accumulating M[xi] (co 16 NT x tile 32) in 16 NT registers per lane (144
-// for the trunk convs), on split-bf16 MFMA (v_mfma_f32_16x16x32_bf16, each
-// fp32 operand as three bf16 parts and each product as the six terms of
-// order <= 2, as accurate as FP32 MFMA; the split-bf16 attention explains the
-// arithmetic). Input channels go in chunks of 32: the chunk's 10 x 18 halo
+// for the trunk convs), on split-f16 MFMA (v_mfma_f32_16x16x32_f16, each fp32
+// operand as two f16 parts and each product as three terms; common.h states the
+// accuracy). V comes into f16's range by a power of two: the host's (p.vs) where
+// a norm bounds the input, else one of the input's largest magnitude, which the
+// kernel that wrote it left in p.amax; U by the host's; the epilogue takes both
+// out. Input channels go in chunks of 32: the chunk's 10 x 18 halo
 // patch is staged in LDS (global_load_lds, double-buffered, channel-quad-major);
 // each lane forms V for its (tile, eight channels) from the patch, splits it
 // and feeds it to the MFMAs as the B operand. U (pre-transformed and split on
@@ -41,6 +43,12 @@
 // streams from global memory as the A operand, two or three steps ahead of its
 // MFMAs (a ring of three or four registers sets, whichever divides the 2 NT
 // steps of a chunk; three ahead measured up to 2% faster than two at NT = 4).
+//
+// What bounds it: the main loop's issue time, then the epilogue, which nothing
+// overlaps (one block a CU). Measured against the six-product bf16 split: the 144
+// trunk conv 363.5 -> 291.4 us, conv_before_upsample 177.9 -> 155.4, the upsample
+// convs 712 -> 604.5 (mean of the two; HAT-S 512 x 512); at 180 channels (HAT 512)
+// trunk 580 -> 490, CAB conv1 237 -> 201, conv2 231 -> 193.
 //
 // Epilogue, per 16-channel slice: the waves write their M slices to LDS, then
 // each thread forms the 2x2 outputs of one (tile, channel) from the 16 points.
@@ -79,19 +87,21 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
     static_assert(NTT % NT == 0 && 16 * NTT >= CO && 16 * (NTT - 1) < CO, "the column blocks cover CO");
     static_assert(32 * NKC >= CI && 32 * (NKC - 1) < CI && CI % 4 == 0, "the 32-channel chunks cover CI");
     // PACK: the last chunk holds at most 16 real channels (CI = 144), so it is
-    // packed as the K = 144 linears' last step (common.h half_operands, the
+    // packed as the K = 144 linears' last step (common.h half_operand, the
     // host's pack_wino): each lane forms V for four channels (quad lg), and
-    // three MFMAs per step give the six products.
+    // two MFMAs per step give the three products.
     constexpr bool PACK = CI % 32 != 0 && CI % 32 <= 16;
     __shared__ __attribute__((aligned(16))) float Pb0[WG_SLOTS * 4];
     __shared__ __attribute__((aligned(16))) float Pb1[WG_SLOTS * 4];
     __shared__ __attribute__((aligned(16))) float Ms0[16 * 32 * WG_MS];
     __shared__ __attribute__((aligned(16))) float Ms1[16 * 32 * WG_MS];
     __shared__ __attribute__((aligned(16))) float Cs[16 * NT];
+    __shared__ unsigned big;  // block_amax's
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
+    if (tid == 0) big = 0;
     const int lr = lane & 15;
     const int lg = lane >> 4;
     const int H = p.H, W = p.W;
@@ -157,21 +167,31 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
         }
     };
 
-    // U, split on the host and arranged [kc][xi][nt][part][lane][8] bf16: lane
+    // U, split on the host and arranged [kc][xi][nt][part][lane][8] f16: lane
     // (r, g) of step (e, nt) holds part `part` of U[2w + e][16 nt + r][32 kc +
     // 8 g .. +7], the MFMA A operand.
-    const unsigned short* ubase = p.wu + ((size_t)(2 * wave) * NTT + NT * cb) * 3 * 512 + lane * 8;
-    struct U3 {
-        u32x4 v[3];
+    const unsigned short* ubase = p.wu + ((size_t)(2 * wave) * NTT + NT * cb) * 2 * 512 + lane * 8;
+    struct U2 {
+        u32x4 v[2];
     };
-    auto ldu = [&](int kc, int t) -> U3 {
+    auto ldu = [&](int kc, int t) -> U2 {
         const int e = t / NT, nt = t - e * NT;
-        const unsigned short* u = ubase + ((size_t)(kc * 16 + e) * NTT + nt) * 3 * 512;
-        U3 r;
+        const unsigned short* u = ubase + ((size_t)(kc * 16 + e) * NTT + nt) * 2 * 512;
+        U2 r;
 #pragma unroll
-        for (int part = 0; part < 3; ++part) r.v[part] = *(const u32x4*)(u + part * 512);
+        for (int part = 0; part < 2; ++part) r.v[part] = *(const u32x4*)(u + part * 512);
         return r;
     };
+
+    // V's scale, and what takes it and U's out of the sums
+    float vs = p.vs;
+    if (p.amax) {
+        // |V| <= 4 max|d| < 2^(e + 3): to below 2^15 (e bounded: zeros and the
+        // smallest numbers need no more)
+        const int e = max((int)(read_amax(p.amax) >> 23) - 127, -60);
+        vs = __uint_as_float((unsigned)(12 - e + 127) << 23);
+    }
+    const float oinv = p.uinv / vs;
 
     // The lane's B^T row / column pattern: R(col) = d[ra][col] + sr d[rb][col],
     // V[2w] = R(cA) - R(cB), V[2w+1] = R(cC) + sc R(cD).
@@ -205,7 +225,7 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
     // slot t % RING lines up across chunks)
     constexpr int RING = (2 * NT) % 3 == 0 ? 3 : 4;
     static_assert((2 * NT) % RING == 0 && 2 * NT >= RING, "the ring lines up across chunks");
-    U3 ur[RING];
+    U2 ur[RING];
     fetch(0, CInt<0>{});
 #pragma unroll
     for (int t = 0; t < RING - 1; ++t) ur[t] = ldu(0, t);
@@ -226,7 +246,7 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
         constexpr bool HALF = PACK && LAST;
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            u32x4 vb[2][3];
+            u32x4 vb[2][2];
 #pragma unroll
             for (int nt2 = 0; nt2 < 2; ++nt2) {
                 float f[8];
@@ -239,10 +259,10 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
                     const f32x4 r1 = *(const f32x4*)(P + uoff[c1][0]) + sr * *(const f32x4*)(P + uoff[c1][1]);
                     const f32x4 v = e == 0 ? r0 - r1 : r0 + sc * r1;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) f[4 * hq + j] = v[j];
+                    for (int j = 0; j < 4; ++j) f[4 * hq + j] = v[j] * vs;
                 }
-                if (HALF) half_operands((f32x4){f[0], f[1], f[2], f[3]}, vb[nt2]);
-                else split3_x8(f, vb[nt2]);
+                if (HALF) vb[nt2][0] = half_operand((f32x4){f[0], f[1], f[2], f[3]});
+                else split2_x8(f, vb[nt2]);
             }
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
@@ -250,8 +270,8 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
                 if (!LAST && t == 0) fetch(kc + 1, CInt<Q ^ 1>{});
 #pragma unroll
                 for (int nt2 = 0; nt2 < 2; ++nt2)
-                    acc[e][nt][nt2] = HALF ? mfma16x3(ur[t % RING].v, vb[nt2], acc[e][nt][nt2])
-                                           : mfma16x6(ur[t % RING].v, vb[nt2], acc[e][nt][nt2]);
+                    acc[e][nt][nt2] = HALF ? mfma16x2h(ur[t % RING].v, vb[nt2][0], acc[e][nt][nt2])
+                                           : mfma16x3h(ur[t % RING].v, vb[nt2], acc[e][nt][nt2]);
                 // step t + RING - 1's load into the slot step t - 1's MFMAs
                 // have read
                 {
@@ -265,11 +285,11 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
             __builtin_amdgcn_s_waitcnt(0);
         } else {
             // The next chunk's patch copies landed: they were issued at step 0,
-            // before this chunk's 6 NT U loads, and the memory counter
-            // completes in order, so vmcnt(6 NT) covers them while the U loads
+            // before this chunk's 4 NT U loads, and the memory counter
+            // completes in order, so vmcnt(4 NT) covers them while the U loads
             // for the next chunk's first steps stay in flight under its V
             // transform.
-            constexpr int VM = 6 * NT;
+            constexpr int VM = 4 * NT;
             static_assert(VM <= 63, "the 6-bit vmcnt field");
             __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (15 << 8));
         }
@@ -354,10 +374,10 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
                 t1[i] = m[4 * i + 1] - m[4 * i + 2] - m[4 * i + 3];
             }
             const float bias = Cs[nt * 16 + ec];
-            y[nt][0] += (t0[0] + t0[1] + t0[2]) + bias;
-            y[nt][1] += (t1[0] + t1[1] + t1[2]) + bias;
-            y[nt][2] += (t0[1] - t0[2] - t0[3]) + bias;
-            y[nt][3] += (t1[1] - t1[2] - t1[3]) + bias;
+            y[nt][0] += __builtin_fmaf(t0[0] + t0[1] + t0[2], oinv, bias);
+            y[nt][1] += __builtin_fmaf(t1[0] + t1[1] + t1[2], oinv, bias);
+            y[nt][2] += __builtin_fmaf(t0[1] - t0[2] - t0[3], oinv, bias);
+            y[nt][3] += __builtin_fmaf(t1[1] - t1[2] - t1[3], oinv, bias);
         };
 #pragma unroll
         for (int nt = 0; nt + 1 < NT; nt += 2) {
@@ -366,6 +386,19 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
         }
         if constexpr (NT % 2 == 1) out_slice(NT - 1, CInt<0>{});
 
+        if constexpr (HEAD != CEPI_COLSUM) {
+            // the output's largest finite magnitude, for the conv that reads it
+            // (LeakyReLU only shrinks it)
+            if (p.amax_out) {
+                float m = 0.0f;
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (!PADCO || ocb + 16 * nt < CO) m = finite_max(m, y[nt][q]);
+                block_amax(p.amax_out, &big, m);
+            }
+        }
         if constexpr (HEAD >= 0) {
             // Channel o = 16 NT cb + 16 nt + c of pixel (y, x): CEPI_STORE and
             // CEPI_COLSUM write it there (CEPI_STORE after p.act); CEPI_SHUFFLE
@@ -381,7 +414,7 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
                     float v = y[nt][q];
                     if (HEAD == CEPI_STORE || HEAD == CEPI_COLSUM) {
                         if (HEAD == CEPI_STORE && p.act == 2) v = v < 0.0f ? v * 0.01f : v;
-                        if (HEAD == CEPI_STORE && p.act == 1) v = gelu(v);
+                        if (HEAD == CEPI_STORE && p.act == 1) v = gelu(v) * p.os;
                         p.out[(yy * W + xx) * p.co_stride + o] = v;
                     } else {
                         const int r = p.r, Cf = p.CO / (r * r);

@@ -110,6 +110,8 @@ extern "C" __global__ __launch_bounds__(256) void hat_layernorm(LnArgs p)
 extern "C" __global__ __launch_bounds__(256) void hat_pre(PreArgs p)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
+    if (p.amax)  // the forward's magnitude slots
+        for (int j = i; j < AMAX_SLOTS * AMAX_WORDS; j += gridDim.x * 256) p.amax[j] = 0;
     if (i >= p.hp * p.wp) return;
     const int y = i / p.wp, x = i - (i / p.wp) * p.wp;
     const int sy = y < p.h - 1 ? y : p.h - 1;
@@ -191,27 +193,21 @@ extern "C" __global__ __launch_bounds__(256) void hat_se_gate(SeArgs p)
     }
 }
 
-// The largest finite magnitude of a buffer (hat_op_swmsa's input, which no norm
-// bounds). One HBM pass; the blocks meet in one atomic maximum, whose result
-// does not depend on their order.
+// The largest finite magnitude of a plane that no norm bounds and no kernel has
+// measured (hat_op_swmsa's input; the Winograd convs' where the FP32 tail wrote
+// it). One HBM pass.
 extern "C" __global__ __launch_bounds__(256) void hat_absmax(AbsMaxArgs p)
 {
-    __shared__ float part[4];
+    __shared__ unsigned big;
+    if (threadIdx.x == 0) big = 0;
+    __syncthreads();
     float m = 0.0f;
     for (long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4; i < p.n; i += (long)gridDim.x * 1024) {
         const f32x4 v = *(const f32x4*)(p.x + i);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float a = fabsf(v[j]);
-            m = a <= 3.402823466e38f ? fmaxf(m, a) : m;  // infinities and NaN left out
-        }
+        for (int j = 0; j < 4; ++j) m = finite_max(m, v[j]);
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0)
-        atomicMax(p.out, __float_as_uint(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]))));
+    block_amax(p.out, &big, m);
 }
 
 extern "C" __global__ __launch_bounds__(256) void hat_scale(ScaleArgs p)

@@ -94,13 +94,15 @@ __device__ __forceinline__ float2 tx_row_stats(const f32x4 (&v)[(C + 15) / 16], 
     return make_float2(mean, 1.0f / sqrtf(q / (float)C + eps));
 }
 
-// v = acc * mi + b2 (Cs); out = v; with xn: xn = LN(v) by (nw, nb) = (Cs + 16 NT,
+// v = acc * mi + b2 (Cs); out = v (amax_out: its largest magnitude too); with xn: xn = LN(v) by (nw, nb) = (Cs + 16 NT,
 // Cs + 32 NT) (Cs zero past C).
 template <int C>
 __device__ __forceinline__ void tx_store_rows(const f32x4 (&acc)[2][(C + 15) / 16], const float* Cs, float mi, int mbase,
-                                              int M, int lr, int lg, float eps, float* out, float* xn)
+                                              int M, int lr, int lg, float eps, float* out, float* xn,
+                                              unsigned* amax_out, unsigned* lds)
 {
     constexpr int NT = (C + 15) / 16;
+    float big = 0.0f;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
         const int m = mbase + mt * 16 + lr;
@@ -114,6 +116,12 @@ __device__ __forceinline__ void tx_store_rows(const f32x4 (&acc)[2][(C + 15) / 1
         float2 st = make_float2(0.f, 0.f);
         if (xn) st = tx_row_stats<C>(v, lg, eps);
         if (m >= M) continue;
+        if (amax_out) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) big = finite_max(big, v[nt][j]);  // zeros past C
+        }
         float* orow = out + (size_t)m * C + lg * 4;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
@@ -131,6 +139,7 @@ __device__ __forceinline__ void tx_store_rows(const f32x4 (&acc)[2][(C + 15) / 1
             }
         }
     }
+    if (amax_out) block_amax(amax_out, lds, big);
 }
 
 // The shape of a tail kernel: NT channel tiles, KS 32-k steps over the channels
@@ -172,11 +181,13 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
     __shared__ __attribute__((aligned(16))) float Cp[(HAB ? 2 : 1) * 16 * NT];  // the projection's bias (HAB: and gate * cscale)
     __shared__ __attribute__((aligned(16))) float Cn[2 * 16 * NT];              // norm2 w, b
     __shared__ __attribute__((aligned(16))) float Cs[3 * 16 * NT];              // b2, next norm w, b (all zero past C)
+    __shared__ unsigned big;                                                    // block_amax's
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in a scalar register
     const int lr = lane & 15, lg = lane >> 4;
     const int M = p.M;
     if ((int)blockIdx.x * TX_ROWS >= M) return;  // whole block, before any barrier
+    if (tid == 0) big = 0;
 
     // n loads of a stage into buffer `par`
     auto issue = [&](auto nlv, auto parv, const unsigned short* src) {
@@ -438,7 +449,7 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
         if constexpr (F2 > 1) fc2_stage(CInt<F1 + 1>{});
         static_assert(F1 <= 2 && F2 <= 2, "the stages above");
     }
-    tx_store_rows<C>(acc, Cs, p.mi, mbase, M, lr, lg, p.eps, p.out, LN ? p.xn : nullptr);
+    tx_store_rows<C>(acc, Cs, p.mi, mbase, M, lr, lg, p.eps, p.out, LN ? p.xn : nullptr, LN ? nullptr : p.amax_out, &big);
 }
 
 extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx_cab_ln(TailXArgs p)

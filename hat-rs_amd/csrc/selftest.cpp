@@ -5,6 +5,7 @@
 // use the reference's own geometry formulas (plan.rs: window_index with the
 // roll, unfold_index, the calculate_mask bands, rpi_sa, rpi_oca) rather than
 // the kernels' folded forms, so an addressing shortcut that is wrong fails here.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -788,7 +789,8 @@ int gpu_selftest(std::string* err)
                 int CIp = 0, COp = 0;
                 std::vector<float> pk = pack_conv(w.data(), b.data(), CO, c.CI, 0, &bias, &CIp, &COp);
                 Dev din(in), dw(pk), db(bias), dres(res), dnw(nw), dnb(nb), dxn((size_t)HW * CO);
-                const std::vector<unsigned short> wux = c.wino ? pack_wino(w.data(), CO, c.CI, 0)
+                float uinv = 1.0f;
+                const std::vector<unsigned short> wux = c.wino ? pack_wino(w.data(), CO, c.CI, 0, &uinv)
                                                                : std::vector<unsigned short>(8, 0);
                 Dev dwu((wux.size() + 1) / 2);
                 Runtime::get().h2d(dwu.p, wux.data(), wux.size() * sizeof(unsigned short));
@@ -811,6 +813,8 @@ int gpu_selftest(std::string* err)
                 p.nb = dnb.p;
                 p.eps = 1e-5f;
                 p.wu = (const unsigned short*)dwu.p;
+                p.uinv = uinv;
+                p.vs = 4096.0f;  // |V| <= 4 max|x| <= 4
                 if (c.wino) launch_wino(s, c.k, (W / 16) * (H / 8), 1, p, 5);  // persistent ones over 5 blocks
                 else launch(s, c.k, (W / 16) * (H / 16), 1, 1, c.waves * 64, p);  // convw and conv_first: 16 x 16
                 std::vector<double> want((size_t)HW * CO), wxn((size_t)HW * CO);
@@ -882,6 +886,7 @@ int gpu_selftest(std::string* err)
             C.r = cc.r;
             const float mean[3] = {0.4488f, 0.4371f, 0.4040f};
             ConvArgs p{};
+            p.os = 1.0f;
             p.in = din.p;
             p.w = dw.p;
             p.bias = db.p;
@@ -1012,17 +1017,33 @@ int gpu_selftest(std::string* err)
                                                                                       : nullptr;
             if (wino) {
                 const int ncb = cc.CO == 256 ? 2 : cc.CO == 180 ? 2 : 1;
-                const std::vector<unsigned short> wux = pack_wino(w.data(), cc.CO, cc.CI, cc.r);
+                const std::vector<unsigned short> wux = pack_wino(w.data(), cc.CO, cc.CI, cc.r, &p.uinv);
                 Dev dwu((wux.size() + 1) / 2), dout4(out_n), dpart4((size_t)nblk * cc.CO);
                 Runtime::get().h2d(dwu.p, wux.data(), wux.size() * sizeof(unsigned short));
                 p.out = dout4.p;
                 p.partial = dpart4.p;
                 p.wu = (const unsigned short*)dwu.p;
+                // V's scale from the input's largest magnitude, and the output's
+                // left for the next conv
+                Dev dmax(std::vector<float>(2 * AMAX_WORDS, 0.0f));
+                AbsMaxArgs am{p.in, (unsigned*)dmax.p, (long)H * W * p.cin_stride};
+                launch(s, "hat_absmax", 3, 1, 1, 256, am);
+                p.amax = (const unsigned*)dmax.p;
+                p.amax_out = (unsigned*)dmax.p + AMAX_WORDS;
                 // the persistent kernels over 5 ncb blocks (2 or 3 of the 12 tiles
                 // each, the next tile's patch fetched under an epilogue)
                 launch_wino(s, wino, (W / 16) * (H / 8), ncb, p, 5 * ncb);
                 p.nblk = 0;
+                p.amax = nullptr;
+                p.amax_out = nullptr;
                 check_close(std::string(wino) + " " + cc.what, dout4.get(), want, 5e-5);
+                if (cc.epi != CEPI_COLSUM && cc.act == 0) {
+                    double big = 0.0;
+                    for (double v : want) big = std::max(big, std::fabs(v));
+                    const std::vector<float> lanes = dmax.get();
+                    const float got = *std::max_element(lanes.begin() + AMAX_WORDS, lanes.end());
+                    check_close(std::string(wino) + " output maximum", {got}, {big}, 5e-5);
+                }
                 if (cc.epi == CEPI_COLSUM) {
                     // one partial row per 8x16 tile
                     std::vector<double> ps((size_t)nblk * cc.CO, 0.0);
@@ -1074,7 +1095,7 @@ int gpu_selftest(std::string* err)
             const int h = 21, w = 35, hp = 32, wp = 48;
             std::vector<float> in = rng.vec((size_t)3 * h * w, 1.0f);
             Dev din(in), dout((size_t)hp * wp * 4);
-            PreArgs p{din.p, dout.p, h, w, hp, wp, 4, 0.4488f, 0.4371f, 0.4040f, 1.0f};
+            PreArgs p{din.p, dout.p, h, w, hp, wp, 4, 0.4488f, 0.4371f, 0.4040f, 1.0f, nullptr};
             launch(s, "hat_pre", (hp * wp + 255) / 256, 1, 1, 256, p);
             std::vector<float> got = dout.get();
             const float m[3] = {0.4488f, 0.4371f, 0.4040f};
