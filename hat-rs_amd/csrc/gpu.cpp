@@ -205,7 +205,7 @@ void pack_tail_mlp(const float* w1, const float* b1, const float* w2, int C, flo
     const int H = 2 * C, HU = tailx_hu(C), NP = (H + HU - 1) / HU, rows = (C + 15) / 16 * 16, ks_n = (C + 31) / 32;
     const size_t step1 = (size_t)2 * HU * 32, step = (size_t)2 * rows * 32, part = ks_n * step1 + HU / 32 * step;
     w->assign(NP * part + TX_PAD, 0);
-    b1x->assign((size_t)NP * HU, 0.0f);
+    b1x->assign(TX_B1, 0.0f);
     if (!fill) return;
     for (int q = 0; q < NP; ++q) {
         for (int r = 0; r < HU; ++r) {
@@ -775,8 +775,17 @@ void run_tailx(hipStream_t s, const DevTail& t, const float* a, const float* res
         f.amax_out = out_max->slot;
         out_max->filled = true;
     }
-    const char* name = t.C == 144 ? (hab ? "hat_habx_cab_ln" : "hat_habx") : (hab ? "hat_habx180_hab_ln" : "hat_habx180");
-    launch(s, name, (unsigned)wx_tiles((int)M), 1, 1, WX_THREADS, f);
+    static const int cus = std::max(1, Runtime::get().cu_count());
+    // One 64-token block a CU at most: there the larger blocks would leave half the
+    // CUs idle, and past it two rounds of small ones take as long as one of large
+    // (hat_habx_cab_ln at 4096 / 16384 / 65536 tokens: 34.2 / 37.5 / 66.1 us in
+    // 128-token blocks, 23.3 / 27.6 / 98.8 in 64; C = 180: 45.0 / 49.8 / 99.1 and
+    // 30.7 / 38.8 / 145.3).
+    const bool small = wx_tiles((int)M, WX_ROWS_S) <= cus;
+    const char* name = t.C == 144 ? (hab ? (small ? "hat_habx_cab_ln_s" : "hat_habx_cab_ln") : small ? "hat_habx_s" : "hat_habx")
+                                  : hab ? (small ? "hat_habx180_hab_ln_s" : "hat_habx180_hab_ln")
+                                        : small ? "hat_habx180_s" : "hat_habx180";
+    launch(s, name, (unsigned)wx_tiles((int)M, small ? WX_ROWS_S : WX_ROWS), 1, 1, WX_THREADS, f);
 }
 
 // The channel-attention gate from the CAB conv's per-tile column sums:

@@ -278,10 +278,14 @@ constexpr int ws_slot(int r, int g) { return g ^ ((r >> 1) & 3); }
 // k-steps (that many rows, permuted, the columns in the order a lane holds x'),
 // then fc2's (C rows in 16s, k = the part's units).
 constexpr int tailx_hu(int C) { return C == 144 ? 96 : 32; }
-// Their launch geometry (tailx): blocks of 4 waves, one 128-token row tile a block.
+// fc1's bias (b1x), padded to the whole loads that copy it.
+#define TX_B1 1024
+// Their launch geometry (tailx): blocks of 4 waves, one row tile of 128 tokens a
+// block; 64 in the small planes' kernels (_s).
 #define WX_THREADS 256
 #define WX_ROWS 128
-constexpr int wx_tiles(int M) { return (M + WX_ROWS - 1) / WX_ROWS; }
+#define WX_ROWS_S 64
+constexpr int wx_tiles(int M, int rows = WX_ROWS) { return (M + rows - 1) / rows; }
 
 // The qkv linear (hat_gemmx_qkv, hat_gemmx_qkv180) keeps one column slice in
 // LDS for the whole launch: per 32-k step two f16 planes [rows][32], unpadded,

@@ -247,25 +247,30 @@ __device__ __forceinline__ void wc_issue(unsigned short* dst, const unsigned sho
 // that the fragment reads down the rows at one k-group are free of bank
 // conflicts without padding. HALF: the packed last step of a K = 144 linear
 // (xb[mt][0] from half_operand, two MFMAs a tile).
-template <int NT, int ROWS, bool HALF = false>
-__device__ __forceinline__ void ws_mma2(const unsigned short* Ws, int lr, int lg, const u32x4 (&xb)[2][2],
-                                        f32x4 (&acc)[2][NT])
+template <int NT, int ROWS, bool HALF = false, int MT = 2>
+__device__ __forceinline__ void ws_mma2(const unsigned short* Ws, int lr, int lg, const u32x4 (&xb)[MT][2],
+                                        f32x4 (&acc)[MT][NT])
 {
     const unsigned short* wr = Ws + lr * 32 + (hatk::ws_slot(lr, lg) * 8);
-    u32x4 wa[2][2];
+    // one tile ahead; with one token tile a wave (half the MFMAs a fragment) two
+    constexpr int A = MT == 1 ? 2 : 1;
+    u32x4 wa[A + 1][2];
 #pragma unroll
-    for (int pl = 0; pl < 2; ++pl) wa[0][pl] = *(const u32x4*)(wr + pl * ROWS * 32);
+    for (int t = 0; t < A && t < NT; ++t)
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl) wa[t][pl] = *(const u32x4*)(wr + t * 16 * 32 + pl * ROWS * 32);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         __builtin_amdgcn_sched_barrier(0);
-        if (nt + 1 < NT) {
+        if (nt + A < NT) {
 #pragma unroll
             for (int pl = 0; pl < 2; ++pl)
-                wa[(nt + 1) & 1][pl] = *(const u32x4*)(wr + (nt + 1) * 16 * 32 + pl * ROWS * 32);
+                wa[(nt + A) % (A + 1)][pl] = *(const u32x4*)(wr + (nt + A) * 16 * 32 + pl * ROWS * 32);
         }
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-            acc[mt][nt] = HALF ? mfma16x2h(wa[nt & 1], xb[mt][0], acc[mt][nt]) : mfma16x3h(wa[nt & 1], xb[mt], acc[mt][nt]);
+        for (int mt = 0; mt < MT; ++mt)
+            acc[mt][nt] = HALF ? mfma16x2h(wa[nt % (A + 1)], xb[mt][0], acc[mt][nt])
+                               : mfma16x3h(wa[nt % (A + 1)], xb[mt], acc[mt][nt]);
     }
 }
 

@@ -26,7 +26,8 @@
 // output's accumulators hold p.ms times the result. Every scale comes out in a
 // multiply-add that adds a bias.
 //
-// A block of 4 waves takes one 128-token row tile, 32 tokens a wave (each weight
+// A block of 4 waves takes one 128-token row tile (64 on small planes, see the
+// instances below), 32 tokens a wave (each weight
 // fragment read from LDS feeds two 16-token MFMA tiles), and streams its weights
 // through two LDS buffers a stage at a time: stage s + 1 in flight while stage
 // s's MFMAs run, a stage as many 32-k steps as a buffer holds (C = 144: two of
@@ -57,7 +58,6 @@
 // Included after gemmx.hip (WcRows, split_pre2).
 
 #define TX_WAVES 4
-#define TX_ROWS (TX_WAVES * 32)
 
 // Row statistics of a token over its C channels (C = 144: 36 per lane, 180:
 // 45; NT = ceil(C / 16) tiles of which the last holds C % 16 real channels in
@@ -96,15 +96,15 @@ __device__ __forceinline__ float2 tx_row_stats(const f32x4 (&v)[(C + 15) / 16], 
 
 // v = acc * mi + b2 (Cs); out = v (amax_out: its largest magnitude too); with xn: xn = LN(v) by (nw, nb) = (Cs + 16 NT,
 // Cs + 32 NT) (Cs zero past C).
-template <int C>
-__device__ __forceinline__ void tx_store_rows(const f32x4 (&acc)[2][(C + 15) / 16], const float* Cs, float mi, int mbase,
+template <int C, int MT>
+__device__ __forceinline__ void tx_store_rows(const f32x4 (&acc)[MT][(C + 15) / 16], const float* Cs, float mi, int mbase,
                                               int M, int lr, int lg, float eps, float* out, float* xn,
                                               unsigned* amax_out, unsigned* lds)
 {
     constexpr int NT = (C + 15) / 16;
     float big = 0.0f;
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
+    for (int mt = 0; mt < MT; ++mt) {
         const int m = mbase + mt * 16 + lr;
         f32x4 v[NT];
 #pragma unroll
@@ -163,72 +163,131 @@ struct TailXShape {
     static_assert(HU % 32 == 0 && TX_PAD >= TX_WAVES * 512, "whole fc2 steps; padding for the last loads");
 };
 
-template <int C, bool CAB, bool HAB, bool LN>
+// MT: 16-token tiles a wave (the block's row tile is 64 MT tokens); NB: stage
+// buffers, NB - 1 stages in flight.
+template <int C, bool CAB, bool HAB, bool LN, int MT, int NB>
 __device__ __forceinline__ void habx_body(const TailXArgs& p)
 {
     using S = TailXShape<C>;
-    constexpr int NT = S::NT, KS = S::KS, HT = S::HT;
-    // the projection's stages: its own steps, then (CAB) one of conv2's two
-    constexpr int NPS = S::ceil_div(KS, S::SP) + (CAB ? 1 : 0);
-    constexpr int PB = NPS & 1;  // the MLP's first stage's buffer
+    constexpr int NT = S::NT, KS = S::KS, HT = S::HT, D = NB - 1;
+    // the projection's stages: its own steps, then (CAB) one of conv2's two;
+    // then F1 + F2 a part. Stage i is in buffer i % NB.
+    constexpr int OWN = S::ceil_div(KS, S::SP), NPS = OWN + (CAB ? 1 : 0);
     static_assert(!CAB || S::SP == 2, "conv2's two steps are one stage");
-    constexpr int F1 = S::ceil_div(KS, S::S1), F2 = S::ceil_div(S::K2, S::S2);
-    static_assert((F1 + F2) % 2 == 0, "a part leaves the buffers' parity as it was");
-    // the two stage buffers as two LDS objects, so that the compiler sees that
-    // reads of one need not wait for the copy into the other
+    constexpr int F1 = S::ceil_div(KS, S::S1), F2 = S::ceil_div(S::K2, S::S2), NF = F1 + F2;
+    // the parts are walked UQ at a time, after which the buffers line up again
+    constexpr int UQ = NF % NB == 0 ? 1 : NB / NF;
+    static_assert(NF * UQ % NB == 0 && S::NP % UQ == 0 && D <= NPS && D <= NF * UQ, "whole rounds of the buffers");
+    static_assert(NB == 2 || NB == 4, "the buffers below");
+    // with more than one stage in flight nothing but the stages' copies may be
+    // loaded between the waits: the projection's operands all come first
+    constexpr bool UP = NB > 2;
+    // the stage buffers as LDS objects of their own, so that the compiler sees
+    // that reads of one need not wait for the copy into another
     __shared__ __attribute__((aligned(16))) unsigned short Ws0[S::BUF];
     __shared__ __attribute__((aligned(16))) unsigned short Ws1[S::BUF];
-    __shared__ __attribute__((aligned(16))) float Cp[(HAB ? 2 : 1) * 16 * NT];  // the projection's bias (HAB: and gate * cscale)
-    __shared__ __attribute__((aligned(16))) float Cn[2 * 16 * NT];              // norm2 w, b
-    __shared__ __attribute__((aligned(16))) float Cs[3 * 16 * NT];              // b2, next norm w, b (all zero past C)
+    __shared__ __attribute__((aligned(16))) unsigned short Ws2[NB > 2 ? S::BUF : 8];
+    __shared__ __attribute__((aligned(16))) unsigned short Ws3[NB > 2 ? S::BUF : 8];
+    // rows of 16 NT constants (zeros past C): the projection's bias, norm2 w, b,
+    // b2, next norm w, b (LN), gate * cscale (HAB); and fc1's bias (b1x), by the
+    // stages' kind of copy, so that its reads wait for no other copy
+    constexpr int CROWS = 4 + (LN ? 2 : 0) + (HAB ? 1 : 0), GATE = CROWS - 1;
+    __shared__ __attribute__((aligned(16))) float Cc[CROWS * 16 * NT];
+    constexpr int NB1 = S::loads(2 * S::NP * S::HU);
+    static_assert(NB1 * 256 <= TX_B1, "whole loads");
+    __shared__ __attribute__((aligned(16))) float Cb[NB1 * 256];
+    const float* const Cn = Cc + 16 * NT;
+    const float* const Cs = Cc + 3 * 16 * NT;
     __shared__ unsigned big;                                                    // block_amax's
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in a scalar register
     const int lr = lane & 15, lg = lane >> 4;
     const int M = p.M;
-    if ((int)blockIdx.x * TX_ROWS >= M) return;  // whole block, before any barrier
+    constexpr int ROWS = TX_WAVES * 16 * MT;
+    if ((int)blockIdx.x * ROWS >= M) return;  // whole block, before any barrier
     if (tid == 0) big = 0;
+    unsigned* const amax_out = LN ? nullptr : p.amax_out;
+    const float ms = p.ms, mi = p.mi;
 
-    // n loads of a stage into buffer `par`
-    auto issue = [&](auto nlv, auto parv, const unsigned short* src) {
-        wc_issue<decltype(nlv)::value, TX_WAVES>(decltype(parv)::value ? Ws1 : Ws0, src, wave, lane);
+    auto buffer = [&](auto iv) -> unsigned short* {
+        constexpr int b = decltype(iv)::value % NB;
+        return b == 0 ? Ws0 : b == 1 ? Ws1 : b == 2 ? Ws2 : Ws3;
     };
-    // the loads of the step range [k0, ...) of a projection stage: at most SP
-    auto issue_proj = [&](auto sv) {
-        constexpr int s = decltype(sv)::value;
-        constexpr int own = S::ceil_div(KS, S::SP);
-        if constexpr (s < own) {
-            constexpr int n = (KS - s * S::SP < S::SP ? KS - s * S::SP : S::SP) * S::STEP;
-            issue(CInt<S::loads(n)>{}, CInt<(s & 1)>{}, p.w + (size_t)s * S::SP * S::STEP);
-        } else if constexpr (CAB && s == own) {
-            issue(CInt<S::loads(2 * S::STEP)>{}, CInt<(s & 1)>{}, p.w2gx);
+    // a wave's loads of stage i; i counts the projection's stages, then the
+    // stages of one part (NPS + s)
+    auto stage_loads = [](int i) constexpr {
+        int n = 0;
+        if (i < OWN) n = (KS - i * S::SP < S::SP ? KS - i * S::SP : S::SP) * S::STEP;
+        else if (i < NPS) n = 2 * S::STEP;
+        else {
+            const int s = (i - NPS) % NF, t = s - F1;
+            n = s < F1 ? (KS - s * S::S1 < S::S1 ? KS - s * S::S1 : S::S1) * S::STEP1
+                       : (S::K2 - t * S::S2 < S::S2 ? S::K2 - t * S::S2 : S::S2) * S::STEP;
+        }
+        return S::loads(n) / TX_WAVES;
+    };
+    // issue stage i: for i >= NPS stage (i - NPS) % NF of part q + (i - NPS) / NF
+    auto issue = [&](auto iv, int q) {
+        constexpr int i = decltype(iv)::value;
+        const unsigned short* src;
+        if constexpr (i < OWN) {
+            src = p.w + (size_t)i * S::SP * S::STEP;
+        } else if constexpr (i < NPS) {
+            src = p.w2gx;
         } else {
-            issue(CInt<S::NL1>{}, CInt<PB>{}, p.wm);  // the MLP's first stage
+            constexpr int s = (i - NPS) % NF, t = s - F1;
+            q += (i - NPS) / NF;
+            // past the last part: nothing, or (UP) the last part's again, so that
+            // the counts of stage_begin hold to the end
+            if constexpr (UP) q = q < S::NP ? q : S::NP - 1;
+            else if (q >= S::NP) return;
+            src = p.wm + (size_t)q * S::PART + (s < F1 ? (size_t)s * S::S1 * S::STEP1
+                                                       : (size_t)KS * S::STEP1 + (size_t)t * S::S2 * S::STEP);
+        }
+        wc_issue<stage_loads(i) * TX_WAVES, TX_WAVES>(buffer(iv), src, wave, lane);
+    };
+    // Stage i begins: its loads have landed (everything issued before those of
+    // the D - 1 stages after it), for every wave, and every wave is done with the
+    // stage before, whose buffer stage i + D goes to. Near the end fewer are in
+    // flight than counted, so the last part waits for everything.
+    auto stage_begin = [&](auto iv) {
+        constexpr int i = decltype(iv)::value;
+        if constexpr (NB == 2) {
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+        } else {
+            constexpr int n = stage_loads(i + 1) + stage_loads(i + 2);
+            static_assert(D == 3 && n < 64, "the vmcnt field");
+            __builtin_amdgcn_s_waitcnt(wc_vmcnt(n));
+            asm volatile("s_barrier" ::: "memory");
         }
     };
-    auto stage_begin = [&] {
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of the stage (and its operands) have landed
-        __syncthreads();                // everyone's have, and everyone is done with the stage before
-    };
 
-    issue_proj(CInt<0>{});
-    for (int i = tid; i < (HAB ? 2 : 1) * 16 * NT; i += TX_WAVES * 64) {
-        const int part = i / (16 * NT), c = i - part * 16 * NT;
-        Cp[i] = c >= C ? 0.0f : part == 0 ? p.bias[c] : p.gate[c] * p.cscale;
-    }
-    for (int i = tid; i < 2 * 16 * NT; i += TX_WAVES * 64) {
-        const int part = i / (16 * NT), c = i - part * 16 * NT;
-        Cn[i] = c >= C ? 0.0f : part == 0 ? p.inw[c] : p.inb[c];
-    }
-    for (int i = tid; i < 3 * 16 * NT; i += TX_WAVES * 64) {
-        const int part = i / (16 * NT), c = i - part * 16 * NT;
-        Cs[i] = c >= C ? 0.0f : part == 0 ? p.b2[c] : LN ? (part == 1 ? p.nw[c] : p.nb[c]) : 0.0f;
-    }
-    const int mbase = blockIdx.x * TX_ROWS + wave * 32;
-    // acc = the block input's rows in the projection's scale (zeros past M, C)
-    f32x4 acc[2][NT];
+    issue(CInt<0>{}, 0);
+    wc_issue<NB1, TX_WAVES>((unsigned short*)Cb, (const unsigned short*)p.b1x, wave, lane);
+    // all constants in flight together with the rows below; into LDS after them
+    constexpr int NCV = S::ceil_div(CROWS * 16 * NT, TX_WAVES * 64);
+    float cv[NCV];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
+    for (int k = 0; k < NCV; ++k) {
+        const int i = tid + k * TX_WAVES * 64, r = i / (16 * NT), c = i - r * 16 * NT;
+        const float* src = r == 0 ? p.bias : r == 1 ? p.inw : r == 2 ? p.inb : r == 3 ? p.b2 : HAB && r == GATE ? p.gate
+                           : r == 4 ? p.nw : p.nb;
+        cv[k] = *(c < C && r < CROWS ? src + c : hat_zero_row);
+        if (HAB && r == GATE) cv[k] *= p.cscale;
+    }
+    auto put_constants = [&] {
+#pragma unroll
+        for (int k = 0; k < NCV; ++k) {
+            const int i = tid + k * TX_WAVES * 64;
+            if (i < CROWS * 16 * NT) Cc[i] = cv[k];
+        }
+    };
+    const int mbase = blockIdx.x * ROWS + wave * 16 * MT;
+    // acc = the block input's rows in the projection's scale (zeros past M, C)
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
         const int m = mbase + mt * 16 + lr;
         const float* row = p.res + (size_t)(m < M ? m : 0) * C + lg * 4;
 #pragma unroll
@@ -236,10 +295,10 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
     }
     // HAB: conv2's output rows, added (times gate * cscale) to the block input
     // here, where registers are free, rather than to x' (52 registers spilled)
-    f32x4 aux[HAB ? 2 : 1][HAB ? NT : 1];
+    f32x4 aux[HAB ? MT : 1][HAB ? NT : 1];
     if constexpr (HAB) {
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
+        for (int mt = 0; mt < MT; ++mt) {
             const int m = mbase + mt * 16 + lr;
             const float* row = p.aux + (size_t)(m < M ? m : 0) * C + lg * 4;
 #pragma unroll
@@ -249,26 +308,27 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
 
     // ---- the projection: acc = ps (x + ao . Wp^T (+ nb(t1) . W2g^T))
     {
-        WcRows<C> ar;
+        WcRows<C, MT> ar;
         ar.init(p.a, mbase, M, lr);
-        // ao's rows: one stage ahead
-        f32x4 y[2][S::SP][2][2];
+        // ao's rows: one stage ahead, or (UP) all of them
+        constexpr int NY = UP ? NPS : 2;
+        f32x4 y[NY][S::SP][MT][2];
         auto load_rows = [&](auto sv) {
             constexpr int s = decltype(sv)::value;
 #pragma unroll
             for (int i = 0; i < S::SP; ++i) {
                 const int ks = s * S::SP + i;
                 if (ks >= KS) break;
-                if (S::HALF && ks == KS - 1) ar.load_half(lg, y[s & 1][i]);
-                else ar.load(ks, lg, y[s & 1][i]);
+                if (S::HALF && ks == KS - 1) ar.load_half(lg, y[s % NY][i]);
+                else ar.load(ks, lg, y[s % NY][i]);
             }
         };
         // conv2's B operand for its k-step s: the 3x3 neighbourhood of t1 at
         // this lane's tokens, k = 32 s + 8 lg + j = tap*6 + ci (pairs of
         // channels; taps outside the plane and k >= 54 read zeros)
-        auto gather_t1 = [&](int s, f32x4 (&dst)[2][2]) {
+        auto gather_t1 = [&](int s, f32x4 (&dst)[MT][2]) {
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt) {
+            for (int mt = 0; mt < MT; ++mt) {
                 const int m = mbase + mt * 16 + lr;
                 const bool alive = m < M;
                 const int yq = m / p.W, xq = m - yq * p.W;
@@ -285,19 +345,37 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
             }
         };
         load_rows(CInt<0>{});
+        if constexpr (!UP) put_constants();
+        if constexpr (UP) {
+            load_rows(CInt<1>{});
+            load_rows(CInt<2>{});
+            if constexpr (OWN > 3) {
+                load_rows(CInt<3>{});
+                load_rows(CInt<4>{});
+                load_rows(CInt<5>{});
+            }
+            if constexpr (CAB) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) gather_t1(i, y[OWN % NY][i]);
+            }
+            put_constants();
+            // none of those loads may sink below the copies
+            __builtin_amdgcn_sched_barrier(0);
+            issue(CInt<1>{}, 0);
+            issue(CInt<2>{}, 0);
+        }
         auto proj_stage = [&](auto sv) {
             constexpr int s = decltype(sv)::value;
-            constexpr int own = S::ceil_div(KS, S::SP);
-            const unsigned short* W = s & 1 ? Ws1 : Ws0;
-            stage_begin();
-            issue_proj(CInt<s + 1>{});
+            const unsigned short* W = buffer(sv);
+            stage_begin(sv);
+            issue(CInt<s + D>{}, 0);
             if constexpr (s == 0) {
 #pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
+                for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt) {
                         if constexpr (HAB) {
-                            const f32x4 g4 = *(const f32x4*)(Cp + 16 * NT + nt * 16 + lg * 4);
+                            const f32x4 g4 = *(const f32x4*)(Cc + GATE * 16 * NT + nt * 16 + lg * 4);
 #pragma unroll
                             for (int j = 0; j < 4; ++j)
                                 acc[mt][nt][j] = __builtin_fmaf(aux[mt][nt][j], g4[j], acc[mt][nt][j]);
@@ -305,22 +383,22 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
                         acc[mt][nt] *= p.ps;
                     }
             }
-            if constexpr (s + 1 < own) load_rows(CInt<s + 1>{});
-            else if constexpr (CAB && s + 1 == own) {
+            if constexpr (!UP && s + 1 < OWN) load_rows(CInt<s + 1>{});
+            else if constexpr (!UP && CAB && s + 1 == OWN) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) gather_t1(i, y[(s + 1) & 1][i]);
+                for (int i = 0; i < 2; ++i) gather_t1(i, y[(s + 1) % NY][i]);
             }
 #pragma unroll
             for (int i = 0; i < S::SP; ++i) {
                 const int ks = s * S::SP + i;
-                if (s < own && ks >= KS) break;
-                u32x4 xb[2][2];
-                if (S::HALF && s < own && ks == KS - 1) {
+                if (s < OWN && ks >= KS) break;
+                u32x4 xb[MT][2];
+                if (S::HALF && s < OWN && ks == KS - 1) {
 #pragma unroll
-                    for (int mt = 0; mt < 2; ++mt) xb[mt][0] = half_operand(y[s & 1][i][mt][0]);
+                    for (int mt = 0; mt < MT; ++mt) xb[mt][0] = half_operand(y[s % NY][i][mt][0]);
                     ws_mma2<NT, S::ROWS, true>(W + i * S::STEP, lr, lg, xb, acc);
                 } else {
-                    split_pre2(y[s & 1][i], xb);
+                    split_pre2(y[s % NY][i], xb);
                     ws_mma2<NT, S::ROWS>(W + i * S::STEP, lr, lg, xb, acc);
                 }
             }
@@ -333,16 +411,16 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
             proj_stage(CInt<4>{});
             proj_stage(CInt<5>{});
         }
-        static_assert(NPS <= 6 && NPS != 5, "the stages above");
+        static_assert(NPS <= 6 && NPS != 5 && (OWN == 3 || OWN == 6), "the stages above");
     }
     // x' = acc / ps + bias, then norm2 of it split into fc1's operands yb, and
     // acc = ms x'
-    u32x4 yb[2][KS][2];
+    u32x4 yb[MT][KS][2];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
+    for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const f32x4 b4 = *(const f32x4*)(Cp + nt * 16 + lg * 4);
+            const f32x4 b4 = *(const f32x4*)(Cc + nt * 16 + lg * 4);
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[mt][nt][j] = __builtin_fmaf(acc[mt][nt][j], p.pi, b4[j]);
         }
@@ -367,104 +445,101 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
             }
         }
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] *= p.ms;
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] *= ms;
         __builtin_amdgcn_sched_barrier(0);
     }
 
     // ---- the MLP, part by part: fc1 from yb, GELU, fc2 onto acc
+    auto fc1_stage = [&](auto iv, int q, f32x4 (&h)[MT][HT]) {
+        constexpr int s = (decltype(iv)::value - NPS) % NF;
+        const unsigned short* W = buffer(iv);
+        stage_begin(iv);
+        issue(CInt<decltype(iv)::value + D>{}, q);
+        if constexpr (s == 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int nt = 0; nt < HT; ++nt) h[mt][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int i = 0; i < S::S1; ++i) {
+            const int ks = s * S::S1 + i;
+            if (ks >= KS) break;
+            u32x4 xb[MT][2];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) xb[mt][0] = yb[mt][ks][0], xb[mt][1] = yb[mt][ks][1];
+            if (S::HALF && ks == KS - 1) ws_mma2<HT, S::HU, true>(W + i * S::STEP1, lr, lg, xb, h);
+            else ws_mma2<HT, S::HU>(W + i * S::STEP1, lr, lg, xb, h);
+        }
+    };
+    auto fc2_stage = [&](auto iv, int q, f32x4 (&h)[MT][HT]) {
+        constexpr int r = decltype(iv)::value - NPS, t = r % NF - F1;
+        const unsigned short* W = buffer(iv);
+        stage_begin(iv);
+        issue(CInt<decltype(iv)::value + D>{}, q);
+        if constexpr (t == 0) {
+            // the hidden units in their scale: + b1, GELU (b1x in the part's
+            // packed row order)
+#pragma unroll
+            for (int nt = 0; nt < HT; ++nt) {
+                const f32x4 b = *(const f32x4*)(Cb + (q + r / NF) * S::HU + 16 * nt + 4 * lg);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        h[mt][nt][j] = gelu_scaled(__builtin_fmaf(h[mt][nt][j], p.h1, b[j]), p.g0, p.g1);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < S::S2; ++i) {
+            const int k2 = t * S::S2 + i;
+            if (k2 >= S::K2) break;
+            u32x4 xb[MT][2];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const f32x4 a = h[mt][2 * k2], b = h[mt][2 * k2 + 1];
+                const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+                split2_x8(f, xb[mt]);
+            }
+            ws_mma2<NT, S::ROWS>(W + i * S::STEP, lr, lg, xb, acc);
+        }
+    };
+    static_assert(F1 <= 2 && F2 <= 2 && UQ <= 2, "the stages below");
 #pragma unroll 1
-    for (int q = 0; q < S::NP; ++q) {
-        const unsigned short* wq = p.wm + (size_t)q * S::PART;
-        f32x4 h[2][HT];
-#pragma unroll
-        for (int nt = 0; nt < HT; ++nt) h[0][nt] = h[1][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        // stage s of the part in buffer (PB + s) & 1; the one after the part's
-        // last is the next part's first (after the last part: none)
-        auto next = [&](auto sv) {
-            constexpr int s = decltype(sv)::value;
-            constexpr int par = (PB + s) & 1;
-            if constexpr (s < F1) {
-                constexpr int n = (KS - s * S::S1 < S::S1 ? KS - s * S::S1 : S::S1) * S::STEP1;
-                issue(CInt<S::loads(n)>{}, CInt<par>{}, wq + (size_t)s * S::S1 * S::STEP1);
-            } else if constexpr (s < F1 + F2) {
-                constexpr int t = s - F1;
-                constexpr int n = (S::K2 - t * S::S2 < S::S2 ? S::K2 - t * S::S2 : S::S2) * S::STEP;
-                issue(CInt<S::loads(n)>{}, CInt<par>{}, wq + (size_t)KS * S::STEP1 + (size_t)t * S::S2 * S::STEP);
-            } else if (q + 1 < S::NP) {
-                issue(CInt<S::NL1>{}, CInt<par>{}, wq + S::PART);
-            }
-        };
-        auto fc1_stage = [&](auto sv) {
-            constexpr int s = decltype(sv)::value;
-            const unsigned short* W = (PB + s) & 1 ? Ws1 : Ws0;
-            stage_begin();
-            next(CInt<s + 1>{});
-#pragma unroll
-            for (int i = 0; i < S::S1; ++i) {
-                const int ks = s * S::S1 + i;
-                if (ks >= KS) break;
-                u32x4 xb[2][2];
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt) xb[mt][0] = yb[mt][ks][0], xb[mt][1] = yb[mt][ks][1];
-                if (S::HALF && ks == KS - 1) ws_mma2<HT, S::HU, true>(W + i * S::STEP1, lr, lg, xb, h);
-                else ws_mma2<HT, S::HU>(W + i * S::STEP1, lr, lg, xb, h);
-            }
-        };
-        auto fc2_stage = [&](auto sv) {
-            constexpr int s = decltype(sv)::value;
-            constexpr int t = s - F1;
-            const unsigned short* W = (PB + s) & 1 ? Ws1 : Ws0;
-            stage_begin();
-            next(CInt<s + 1>{});
-            if constexpr (t == 0) {
-                // the hidden units in their scale: + b1, GELU (b1x in the
-                // part's packed row order)
-#pragma unroll
-                for (int nt = 0; nt < HT; ++nt) {
-                    const f32x4 b = *(const f32x4*)(p.b1x + q * S::HU + 16 * nt + 4 * lg);
-#pragma unroll
-                    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            h[mt][nt][j] = gelu_scaled(__builtin_fmaf(h[mt][nt][j], p.h1, b[j]), p.g0, p.g1);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < S::S2; ++i) {
-                const int k2 = t * S::S2 + i;
-                if (k2 >= S::K2) break;
-                u32x4 xb[2][2];
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt) {
-                    const f32x4 a = h[mt][2 * k2], b = h[mt][2 * k2 + 1];
-                    const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-                    split2_x8(f, xb[mt]);
-                }
-                ws_mma2<NT, S::ROWS>(W + i * S::STEP, lr, lg, xb, acc);
-            }
-        };
-        fc1_stage(CInt<0>{});
-        if constexpr (F1 > 1) fc1_stage(CInt<1>{});
-        fc2_stage(CInt<F1>{});
-        if constexpr (F2 > 1) fc2_stage(CInt<F1 + 1>{});
-        static_assert(F1 <= 2 && F2 <= 2, "the stages above");
+    for (int q = 0; q < S::NP; q += UQ) {
+        f32x4 h[MT][HT];
+        fc1_stage(CInt<NPS>{}, q, h);
+        if constexpr (F1 > 1) fc1_stage(CInt<NPS + 1>{}, q, h);
+        fc2_stage(CInt<NPS + F1>{}, q, h);
+        if constexpr (F2 > 1) fc2_stage(CInt<NPS + F1 + 1>{}, q, h);
+        if constexpr (UQ > 1) {
+            fc1_stage(CInt<NPS + NF>{}, q, h);
+            if constexpr (F1 > 1) fc1_stage(CInt<NPS + NF + 1>{}, q, h);
+            fc2_stage(CInt<NPS + NF + F1>{}, q, h);
+            if constexpr (F2 > 1) fc2_stage(CInt<NPS + NF + F1 + 1>{}, q, h);
+        }
     }
-    tx_store_rows<C>(acc, Cs, p.mi, mbase, M, lr, lg, p.eps, p.out, LN ? p.xn : nullptr, LN ? nullptr : p.amax_out, &big);
+    if constexpr (UP) __builtin_amdgcn_s_waitcnt(wc_vmcnt(0));  // no copy outlives the block
+    tx_store_rows<C>(acc, Cs, mi, mbase, M, lr, lg, p.eps, p.out, LN ? p.xn : nullptr, amax_out, &big);
 }
 
-extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx_cab_ln(TailXArgs p)
-{
-    habx_body<144, true, false, true>(p);
-}
-extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx(TailXArgs p)
-{
-    habx_body<144, false, false, false>(p);
-}
-extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx180_hab_ln(TailXArgs p)
-{
-    habx_body<180, false, true, true>(p);
-}
-extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx180(TailXArgs p)
-{
-    habx_body<180, false, false, false>(p);
-}
+// Large planes: 128-token row tiles, two blocks a CU, one stage in flight. Small
+// planes (_s, at most one such block a CU: run_tailx): 64-token tiles, one block a
+// CU. With one wave a SIMD nothing hides a wave's own latencies, so a wave has half
+// the work, three stages are in flight and the projection's operands are all loaded
+// first. The wave's issue bounds it, not the weights' latency: a second launch on
+// the same, cached weights takes as long. 64 x 64 tokens: hat_habx_cab_ln 34.2 ->
+// 23.3 us, hat_habx180_hab_ln 45.0 -> 30.7; 128 x 128: 37.5 -> 27.6, 49.8 -> 38.8.
+#define TX_INST(NAME, C, CAB, HAB, LN)                                                  \
+    extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void NAME(TailXArgs p)    \
+    {                                                                                   \
+        habx_body<C, CAB, HAB, LN, 2, 2>(p);                                            \
+    }                                                                                   \
+    extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 1) void NAME##_s(TailXArgs p) \
+    {                                                                                   \
+        habx_body<C, CAB, HAB, LN, 1, 4>(p);                                            \
+    }
+TX_INST(hat_habx_cab_ln, 144, true, false, true)
+TX_INST(hat_habx, 144, false, false, false)
+TX_INST(hat_habx180_hab_ln, 180, false, true, true)
+TX_INST(hat_habx180, 180, false, false, false)

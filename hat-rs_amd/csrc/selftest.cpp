@@ -397,15 +397,12 @@ int gpu_selftest(std::string* err)
             for (float& x : as) x *= sv;
             for (float& x : n2ws) x *= sn;
             for (float& x : n2bs) x *= sn;
-            Dev da(as), dbp(bp), daux(aux), dg(gate), dn2w(n2ws), dn2b(n2bs), db2(b2), dnw(nw), dnb(nb), db1x(tp.b1x), dx(res),
-                dxn((size_t)M * C), dw((tp.w.size() + 1) / 2), dwm((tp.wm.size() + 1) / 2);
+            Dev da(as), dbp(bp), daux(aux), dg(gate), dn2w(n2ws), dn2b(n2bs), db2(b2), dnw(nw), dnb(nb), db1x(tp.b1x),
+                dw((tp.w.size() + 1) / 2), dwm((tp.wm.size() + 1) / 2);
             Runtime::get().h2d(dw.p, tp.w.data(), tp.w.size() * sizeof(unsigned short));
             Runtime::get().h2d(dwm.p, tp.wm.data(), tp.wm.size() * sizeof(unsigned short));
             TailXArgs f{};
             f.a = da.p;
-            f.res = dx.p;
-            f.out = dx.p;
-            f.xn = hab ? dxn.p : nullptr;
             f.w = (const unsigned short*)dw.p;
             f.wm = (const unsigned short*)dwm.p;
             f.bias = dbp.p;
@@ -421,8 +418,6 @@ int gpu_selftest(std::string* err)
             f.M = M;
             f.eps = 1e-5f;
             tail_scales(tp.t, &f);
-            const char* k = hab ? "hat_habx180_hab_ln" : "hat_habx180";
-            launch(s, k, (unsigned)wx_tiles(M), 1, 1, WX_THREADS, f);
             std::vector<double> want((size_t)M * C), wxn((size_t)M * C), x(C), y(C), hid(Hd);
             auto norm = [&](const double* v, const std::vector<float>& w, const std::vector<float>& b, double* o) {
                 double mean = 0, var = 0;
@@ -450,9 +445,17 @@ int gpu_selftest(std::string* err)
                 }
                 norm(&want[o], nw, nb, &wxn[o]);
             }
-            check_close(k, dx.get(), want, 5e-5);
-            if (hab) check_close(std::string(k) + " next norm", dxn.get(), wxn, 5e-5);
-            note(std::string(k) + " (split-f16 C 180 tail, M 600, in place) vs double");
+            for (bool small : {false, true}) {
+                Dev dx(res), dxn((size_t)M * C);
+                f.res = dx.p;
+                f.out = dx.p;
+                f.xn = hab ? dxn.p : nullptr;
+                const std::string k = std::string(hab ? "hat_habx180_hab_ln" : "hat_habx180") + (small ? "_s" : "");
+                launch(s, k.c_str(), (unsigned)wx_tiles(M, small ? WX_ROWS_S : WX_ROWS), 1, 1, WX_THREADS, f);
+                check_close(k, dx.get(), want, 5e-5);
+                if (hab) check_close(k + " next norm", dxn.get(), wxn, 5e-5);
+                note(k + " (split-f16 C 180 tail, M 600, in place) vs double");
+            }
         }
 
         // ---- folded CAB (144 -> 6 -> 144) against the unfolded computation:
@@ -699,7 +702,7 @@ int gpu_selftest(std::string* err)
                 const TailCab tc{8.0, 0.01};
                 TailPack xt = pack_tail(wp.data(), f1.data(), fb1.data(), f2.data(), nw.data(), nb.data(), C, 1.0f, 1.0f, &tc);
                 Dev dpw((xt.w.size() + 1) / 2), dpm((xt.wm.size() + 1) / 2), db1x(xt.b1x), dt1x((size_t)T * CAB_CS),
-                    dpartx((size_t)tiles * CAB_NSUM * CAB_CS), dbias2x(C), dgatex(C), dout_f(res), dxn_f((size_t)T * C);
+                    dpartx((size_t)tiles * CAB_NSUM * CAB_CS), dbias2x(C), dgatex(C);
                 Runtime::get().h2d(dpw.p, xt.w.data(), xt.w.size() * sizeof(unsigned short));
                 Runtime::get().h2d(dpm.p, xt.wm.data(), xt.wm.size() * sizeof(unsigned short));
                 CabConvArgs cx = ca;
@@ -719,9 +722,6 @@ int gpu_selftest(std::string* err)
                 check_close("hat_cab_gate gate (scaled t1)", dgatex.get(), gate, 2e-6);
                 TailXArgs xf{};
                 xf.a = dao.p;
-                xf.res = dout_f.p;
-                xf.out = dout_f.p;
-                xf.xn = dxn_f.p;
                 xf.w = (const unsigned short*)dpw.p;
                 xf.wm = (const unsigned short*)dpm.p;
                 xf.w2gx = (const unsigned short*)dw2gx.p;
@@ -738,29 +738,36 @@ int gpu_selftest(std::string* err)
                 xf.W = W;
                 xf.eps = 1e-5f;
                 tail_scales(xt.t, &xf);
-                launch(s, "hat_habx_cab_ln", (unsigned)wx_tiles(T), 1, 1, WX_THREADS, xf);
-                check_close("hat_habx_cab_ln", dout_f.get(), std::vector<double>(ro.begin(), ro.end()), 2e-5);
-                check_close("hat_habx_cab_ln next norm", dxn_f.get(), std::vector<double>(rx.begin(), rx.end()), 2e-5);
-                note("hat_habx_cab_ln (split-f16 proj + conv2 + MLP + norm) vs the two-kernel path");
                 // The OCAB form over a partial last tile: rows from Mo on stay
                 // the block input.
                 const int Mo = T - 100;
                 std::vector<double> wo(r2.begin(), r2.end());
                 for (size_t i = (size_t)Mo * C; i < wo.size(); ++i) wo[i] = res[i];
-                Dev dout_of(res);
-                TailXArgs xof = xf;
-                xof.res = dout_of.p;
-                xof.out = dout_of.p;
-                xof.xn = nullptr;
-                xof.w2gx = nullptr;
-                xof.t1 = nullptr;
-                xof.bias = dbp.p;
-                xof.nw = nullptr;
-                xof.nb = nullptr;
-                xof.M = Mo;
-                launch(s, "hat_habx", (unsigned)wx_tiles(Mo), 1, 1, WX_THREADS, xof);
-                check_close("hat_habx", dout_of.get(), wo, 2e-5);
-                note("hat_habx (split-f16 OCAB tail, partial tile) vs the two-kernel path");
+                for (bool small : {false, true}) {
+                    const std::string sfx = small ? "_s" : "";
+                    const int rows = small ? WX_ROWS_S : WX_ROWS;
+                    Dev dout_f(res), dxn_f((size_t)T * C), dout_of(res);
+                    xf.res = dout_f.p;
+                    xf.out = dout_f.p;
+                    xf.xn = dxn_f.p;
+                    launch(s, ("hat_habx_cab_ln" + sfx).c_str(), (unsigned)wx_tiles(T, rows), 1, 1, WX_THREADS, xf);
+                    check_close("hat_habx_cab_ln" + sfx, dout_f.get(), std::vector<double>(ro.begin(), ro.end()), 2e-5);
+                    check_close("hat_habx_cab_ln" + sfx + " next norm", dxn_f.get(), std::vector<double>(rx.begin(), rx.end()), 2e-5);
+                    note("hat_habx_cab_ln" + sfx + " (split-f16 proj + conv2 + MLP + norm) vs the two-kernel path");
+                    TailXArgs xof = xf;
+                    xof.res = dout_of.p;
+                    xof.out = dout_of.p;
+                    xof.xn = nullptr;
+                    xof.w2gx = nullptr;
+                    xof.t1 = nullptr;
+                    xof.bias = dbp.p;
+                    xof.nw = nullptr;
+                    xof.nb = nullptr;
+                    xof.M = Mo;
+                    launch(s, ("hat_habx" + sfx).c_str(), (unsigned)wx_tiles(Mo, rows), 1, 1, WX_THREADS, xof);
+                    check_close("hat_habx" + sfx, dout_of.get(), wo, 2e-5);
+                    note("hat_habx" + sfx + " (split-f16 OCAB tail, partial tile) vs the two-kernel path");
+                }
             }
         }
 
