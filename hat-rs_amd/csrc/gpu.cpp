@@ -505,7 +505,27 @@ struct GemmEpilogue {
     float* xn = nullptr;          // LayerNorm output of the result rows
     const float* nw = nullptr;
     const float* nb = nullptr;
+    // EPI_QKV: the CAB's conv1 in the same launch (qkv_takes_cab1): C = 144, 180
+    const CabConvArgs* cab = nullptr;
+    const ConvArgs* conv1 = nullptr;
 };
+
+// Does the CAB's conv1, `tiles` blocks of it (rounded up to whole rounds of the
+// XCDs), ride on this qkv linear's launch? They are independent and, on a small
+// plane, each a fraction of the chip for about the latency of one tile: together
+// they take as long as the longer. Up to half the CUs; above, qkv's blocks (a CU
+// each) become too few and the conv's run best two a CU. A forward, in two launches
+// and in one: HAT-S 16 x 16 2.24 and 2.01 ms, 64 x 64 2.40 and 2.16, 128 x 128 3.24
+// and 2.97, 176 x 176 (121 tiles) 4.95 and 4.80, but 192 x 192 (144) 6.18 and 6.22,
+// 224 x 224 7.0 and 8.4; HAT 64 x 64 3.69 and 3.30, 112 x 112 4.79 and 4.73, 128 x 128
+// (128 tiles) 5.33 and 4.91.
+int qkv_conv1_blocks(int tiles) { return (tiles + 7) / 8 * 8; }
+bool qkv_takes_cab1(const DevLinear& L, int heads, int hdim, int tiles)
+{
+    static const int cus = std::max(1, Runtime::get().cu_count());
+    return L.wx && heads == 6 && qkv_conv1_blocks(tiles) <= cus / 2 &&
+           ((L.K == 144 && L.N == 432 && hdim == 24) || (L.K == 180 && L.N == 540 && hdim == 30));
+}
 
 void run_gemm(hipStream_t s, const DevLinear& L, const float* a, int lda, long M, float* out,
               int ldo, int epi, const GemmEpilogue& e, int heads, int hdim, float cscale)
@@ -544,6 +564,11 @@ void run_gemm(hipStream_t s, const DevLinear& L, const float* a, int lda, long M
         static const int cus = std::max(1, Runtime::get().cu_count());
         p.w = (const float*)L.wx;
         memcpy(p.oscale, L.oscale, sizeof p.oscale);
+        if (e.cab) {
+            QkvCabArgs q{p, *e.cab, qkv_conv1_blocks(e.cab->H / 16 * (e.cab->W / 16))};
+            launch(s, "hat_qkv_cab1", (unsigned)(q.nconv + 3 * gemmx_qkv_groups(cus - q.nconv, 3)), 1, 1, GX_THREADS, q);
+            return;
+        }
         launch(s, "hat_gemmx_qkv", (unsigned)(3 * gemmx_qkv_groups(cus, 3)), 1, 1, GX_THREADS, p);
         return;
     }
@@ -552,9 +577,16 @@ void run_gemm(hipStream_t s, const DevLinear& L, const float* a, int lda, long M
         static const int cus = std::max(1, Runtime::get().cu_count());
         p.w = (const float*)L.wx;
         memcpy(p.oscale, L.oscale, sizeof p.oscale);
+        if (e.conv1) {
+            QkvConvArgs q{p, *e.conv1, 0, e.conv1->H / 8 * (e.conv1->W / 16)};
+            q.nconv = qkv_conv1_blocks(q.ntile);
+            launch(s, "hat_qkv_cab1_180", (unsigned)(q.nconv + 3 * gemmx_qkv_groups(cus - q.nconv, 3)), 1, 1, GX_THREADS, q);
+            return;
+        }
         launch(s, "hat_gemmx_qkv180", (unsigned)(3 * gemmx_qkv_groups(cus, 3)), 1, 1, GX_THREADS, p);
         return;
     }
+    if (e.cab || e.conv1) throw Error("GEMM: this shape takes no CAB conv");
     int wbn = 0;
     if (const char* ws = gemm_ws_kernel(L, epi, &wbn)) {
         // One block per CU (its 85 or 150 KB weight slice fills the LDS); the
@@ -630,9 +662,10 @@ void run_mlp(hipStream_t s, const DevLinear& fc1, const DevLinear& fc2, const fl
 // the gate and the gate-scaled conv2 weights (w2g) and combined bias (bias2 =
 // bproj + cscale * gate * b2) for the projection GEMM. With `defer`, the gate
 // is not launched: its arguments go to *defer, for the attention launch to run.
+// With `conv_defer`, nor is conv1 (for the qkv linear's launch).
 void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, const float* bproj,
              float cscale, int sq, float* t1, float* partial, float* w2g, float* bias2, float* gate,
-             unsigned short* w2gx, float ts, float gs, CabGateArgs* defer = nullptr)
+             unsigned short* w2gx, float ts, float gs, CabGateArgs* defer, CabConvArgs* conv_defer)
 {
     if (H % 16 != 0 || W % 16 != 0 || H < 16 || W < 16) throw Error("CAB: plane must be 16-aligned");
     if (sq < 1 || sq > 64) throw Error("CAB: squeeze width must be 1..64");
@@ -648,7 +681,9 @@ void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, con
     cab_scales(ts, cb.oscale, &a);
     // Persistent over the 16 x 16 output tiles, two blocks of 4 waves per CU.
     const int tiles = (H / 16) * (W / 16);
-    launch(s, "hat_cab_conv1", (unsigned)std::min(tiles, 2 * cus), 1, 1, 256, a);
+    if (conv_defer && !defer) throw Error("CAB: the gate needs conv1's sums");
+    if (conv_defer) *conv_defer = a;
+    else launch(s, "hat_cab_conv1", (unsigned)std::min(tiles, 2 * cus), 1, 1, 256, a);
     CabGateArgs g{};
     g.partial = partial;
     g.t1 = t1;
@@ -870,11 +905,12 @@ void wino_scales(hipStream_t s, const DevConv& C, long n, Amax* in_max, Amax* ou
 // launched (the host-memory forward's head): 8 input rows of the Winograd
 // upsample conv (hat_convwino_n8_shuffle), 16 output rows of conv_last
 // (hat_conv_last3), the same band indices for the two since the shuffle
-// doubles the rows. Other convs are always whole planes.
+// doubles the rows. Other convs are always whole planes. With `defer`, the C = 180
+// CAB's conv1 is not launched: its arguments go to *defer (the qkv linear's launch).
 void run_conv(hipStream_t s, const DevConv& C, const float* in, int cin_stride, int H, int W,
               float* out, int co_stride, int epi, int act, const float* res, float* partial,
               int crop_h, int crop_w, float img_range, const float* mean, int band_r0, int band_r1, Amax* in_max,
-              Amax* out_max, float os)
+              Amax* out_max, float os, ConvArgs* defer = nullptr)
 {
     if (H % 8 != 0 || W % 16 != 0) throw Error("conv: plane must be a multiple of 8x16");
     const bool band = band_r1 >= 0;
@@ -980,6 +1016,11 @@ void run_conv(hipStream_t s, const DevConv& C, const float* in, int cin_stride, 
             return;
         }
         if (epi == CEPI_STORE && act == 1 && C.CO == 60 && C.CI == 180 && co_stride >= 60) {
+            if (defer) {
+                wino_scales(s, C, (long)H * W * cin_stride, in_max, out_max, &p);
+                *defer = p;
+                return;
+            }
             wino("hat_convwino_cab1_180", tiles, 1);
             return;
         }
@@ -993,6 +1034,7 @@ void run_conv(hipStream_t s, const DevConv& C, const float* in, int cin_stride, 
             return;
         }
     }
+    if (defer) throw Error("conv: only the C = 180 CAB's conv1 rides on another launch");
     if (band && !(epi == CEPI_FINAL && C.CO == 3 && C.CI == 64 && C.CIp == 64 && cin_stride >= 64))
         throw Error("conv: only the Winograd upsample conv and conv_last run in bands");
     if (wide) {
@@ -1609,10 +1651,15 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
         auto tl = tail_.find(p + ".mlp");
         const bool split = tl != tail_.end();  // the split tail runs
         CabGateArgs gate{};
+        CabConvArgs conv1{};
+        const DevLinear& qkv = lin_.at(p + ".attn.qkv");
+        const bool with = qkv_takes_cab1(qkv, wt_.heads, wt_.head_dim, H / 16 * (W / 16));  // conv1 in qkv's launch
         run_cab(stream_, cab_.at(p), a_.xn, H, W, proj.b, wt_.conv_scale, wt_.squeezed, a_.t1, a_.cab_part,
                 split ? nullptr : a_.w2g, a_.bias2, a_.gate, (unsigned short*)a_.w2gx,
-                split ? tl->second.ts : 1.0f, split ? tl->second.gs : 1.0f, &gate);
-        gemm(lin_.at(p + ".attn.qkv"), a_.xn, C, T, a_.qkv, 0, EPI_QKV);
+                split ? tl->second.ts : 1.0f, split ? tl->second.gs : 1.0f, &gate, with ? &conv1 : nullptr);
+        GemmEpilogue e;
+        e.cab = with ? &conv1 : nullptr;
+        run_gemm(stream_, qkv, a_.xn, C, T, a_.qkv, 0, EPI_QKV, e, wt_.heads, wt_.head_dim, wt_.conv_scale);
         attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, &gate);
         if (split) {
             // proj + gated conv2 + shortcut, norm2, the MLP + next norm1
@@ -1631,9 +1678,20 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
                      raw_.at(next_norm + ".weight"), raw_.at(next_norm + ".bias"), H, W);
         return;
     }
-    // CAB: conv3x3 -> GELU -> conv3x3 (+ per-tile channel sums) -> gate.
-    conv(conv_.at(p + ".conv_block.cab.0"), a_.xn, C, H, W, a_.t1, t1_stride_, CEPI_STORE, 1, nullptr,
-         nullptr, 0, 0, 0, -1, nullptr, nullptr, t1_scale_.at(p));
+    // CAB: conv3x3 -> GELU -> conv3x3 (+ per-tile channel sums) -> gate; on small
+    // planes the first conv in the qkv linear's launch.
+    const DevLinear& qkv = lin_.at(p + ".attn.qkv");
+    const DevConv& conv1 = conv_.at(p + ".conv_block.cab.0");
+    const bool with = conv1.wu && conv1.CI == 180 && conv1.CO == 60 && t1_stride_ >= 60 && (size_t)T * C < ((size_t)1 << 31) &&
+                      qkv_takes_cab1(qkv, wt_.heads, wt_.head_dim, H / 8 * (W / 16));
+    ConvArgs c1{};
+    run_conv(stream_, conv1, a_.xn, C, H, W, a_.t1, t1_stride_, CEPI_STORE, 1, nullptr, nullptr, 0, 0, wt_.img_range,
+             wt_.mean, 0, -1, nullptr, nullptr, t1_scale_.at(p), with ? &c1 : nullptr);
+    if (with) {
+        GemmEpilogue e;
+        e.conv1 = &c1;
+        run_gemm(stream_, qkv, a_.xn, C, T, a_.qkv, 0, EPI_QKV, e, wt_.heads, wt_.head_dim, wt_.conv_scale);
+    }
     conv(conv_.at(p + ".conv_block.cab.2"), a_.t1, t1_stride_, H, W, a_.t2, C, CEPI_COLSUM, 0, nullptr,
          a_.partial);
     // The gate: computed by the attention launch's first block where it fits.
@@ -1645,7 +1703,7 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
            raw_.at(p + ".conv_block.cab.3.attention.3.bias"), wt_.squeezed, a_.gate, &se);
     // Window attention, the roll and the partition folded into its addressing;
     // proj's epilogue adds the shortcut and the gated conv branch, then norm2.
-    gemm(lin_.at(p + ".attn.qkv"), a_.xn, C, T, a_.qkv, 0, EPI_QKV);
+    if (!with) gemm(qkv, a_.xn, C, T, a_.qkv, 0, EPI_QKV);
     attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, nullptr, &se);
     const DevLinear& proj = lin_.at(p + ".attn.proj");
     auto tl = tail_.find(p + ".mlp");

@@ -300,6 +300,21 @@ constexpr int wx_tiles(int M, int rows = WX_ROWS) { return (M + rows - 1) / rows
 #define GX_THREADS 512
 constexpr int gemmx_qkv_groups(int cus, int ns) { return cus >= 8 * ns ? cus / (8 * ns) * 8 : 1; }
 
+// hat_qkv_cab1: blocks 0 .. nconv - 1 (a multiple of 8, at least a tile each) run
+// the CAB's conv1, the others the qkv linear.
+struct QkvCabArgs {
+    GemmArgs g;
+    CabConvArgs c;
+    int nconv;
+};
+
+// hat_qkv_cab1_180: the same; conv1 is a Winograd conv of ntile tiles.
+struct QkvConvArgs {
+    GemmArgs g;
+    ConvArgs c;
+    int nconv, ntile;
+};
+
 struct TailXArgs {
     const float* a;             // [M][C] attention output, in v's scale
     const float* res;           // [M][C] block input

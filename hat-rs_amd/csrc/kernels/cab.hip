@@ -22,7 +22,7 @@ using namespace hatk;
 // ---------------------------------------------------------------------------
 // conv1 (144 -> 6, 3x3, zero padding) + GELU on split-f16 MFMA, one 16 x 16
 // output tile at a time: persistent over the tiles, two blocks of four waves
-// per CU.
+// per CU (on small planes in the qkv linear's launch, blocks of eight: gemmx.hip).
 //
 // Per-tap products: for each pixel q of the tile's 18 x 18 halo, P[q][tap*6+co]
 // = sum_ci xn[q][ci] * w[co][ci][tap] is a 144-deep product with 54 outputs
@@ -45,15 +45,16 @@ using namespace hatk;
 #define CX_HS 18                               // halo width and height
 #define CX_HP (CX_HS * CX_HS)                  // halo pixels
 #define CX_PT ((CX_HP + 31) / 32)              // 32-pixel halo tiles
-#define CX_NPW ((CX_PT + CX_WAVES - 1) / CX_WAVES)  // per wave (past CX_PT: zeros, not stored)
 #define CX_PS 60    // LDS row stride of P (56 written, 54 used): a b128 phase's 16 rows on distinct banks
 #define CX_RING 3   // 16-channel steps of rows in flight
 
-extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(CabConvArgs p)
+// block: of nblk; WAVES: 4 or 8, of which the first four take the taps (one pixel
+// per thread). Ps: CX_HP * CX_PS floats, red: 4 * CAB_NSUM * CAB_CC.
+template <int WAVES>
+__device__ __forceinline__ void cab_conv1_body(const CabConvArgs& p, float* Ps, float* red, int block, int nblk)
 {
-    __shared__ __attribute__((aligned(16))) float Ps[CX_HP * CX_PS];
-    __shared__ float red[CX_WAVES][CAB_NSUM * CAB_CC];
-    static_assert(16 * 16 == CX_WAVES * 64, "one pixel per thread");
+    constexpr int NPW = (CX_PT + WAVES - 1) / WAVES;  // halo tiles a wave (past CX_PT: zeros, not stored)
+    static_assert(WAVES % 4 == 0, "a pixel a thread of the first four waves");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in a scalar register
@@ -64,11 +65,14 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
 
     // The split weights go through LDS (the P region, free until the first
     // halo tile's stores) once per block, then into every wave's registers.
-    constexpr int NWU = CX_WPACK / 8, WIT = (NWU + CX_WAVES * 64 - 1) / (CX_WAVES * 64);  // 16-byte units
-    static_assert(NWU % (CX_WAVES * 64) == 0 && NWU * 16 <= CX_HP * CX_PS * 4, "whole rounds; the weights fit the P region");
+    constexpr int NWU = CX_WPACK / 8, WIT = (NWU + WAVES * 64 - 1) / (WAVES * 64);  // 16-byte units
+    static_assert(NWU * 16 <= CX_HP * CX_PS * 4, "the weights fit the P region");
     u32x4 stage[WIT];
 #pragma unroll
-    for (int i = 0; i < WIT; ++i) stage[i] = ((const u32x4*)p.w)[tid + i * CX_WAVES * 64];
+    for (int i = 0; i < WIT; ++i) {
+        const int u = tid + i * WAVES * 64;
+        stage[i] = ((const u32x4*)p.w)[NWU % (WAVES * 64) == 0 || u < NWU ? u : NWU - 1];
+    }
     float bias[CAB_CC];
 #pragma unroll
     for (int co = 0; co < CAB_CC; ++co) bias[co] = p.bias[co] * p.ts;
@@ -78,7 +82,7 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
     // and past the last tile, so that the loads are issued on every path.
     auto src_of = [&](int tl, int i) -> const float* {
         const int ty = tl / ntx, tx = tl - ty * ntx;
-        const int hi = (wave + CX_WAVES * i) * 32 + pl;
+        const int hi = (wave + WAVES * i) * 32 + pl;
         const int hy = hi / CX_HS, hx = hi - hy * CX_HS;
         const int gy = ty * 16 - 1 + hy, gx = tx * 16 - 1 + hx;
         const bool valid = tl < ntiles && hi < CX_HP && gy >= 0 && gy < H && gx >= 0 && gx < W;
@@ -87,14 +91,17 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
     // row steps in flight: step t of an output tile (halo tile t / 9, channels
     // 16 (t % 9) ..) in slot t % CX_RING
     f32x4 xr[CX_RING][2];
-    const float* cur = src_of(blockIdx.x, 0);
+    const float* cur = src_of(block, 0);
 #pragma unroll
     for (int t = 0; t < CX_RING; ++t) {
         xr[t][0] = *(const f32x4*)(cur + t * 16);
         xr[t][1] = *(const f32x4*)(cur + t * 16 + 4);
     }
 #pragma unroll
-    for (int i = 0; i < WIT; ++i) ((u32x4*)Ps)[tid + i * CX_WAVES * 64] = stage[i];
+    for (int i = 0; i < WIT; ++i) {
+        const int u = tid + i * WAVES * 64;
+        if (NWU % (WAVES * 64) == 0 || u < NWU) ((u32x4*)Ps)[u] = stage[i];
+    }
     lds_barrier();
     u32x4 wr[9][2][2];
 #pragma unroll
@@ -106,14 +113,14 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
                 wr[ks][nt][part] = ((const u32x4*)Ps)[((ks * 2 + nt) * 2 + part) * 64 + lane];
     lds_barrier();  // every wave has its weights before P is written
 
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    for (int tile = block; tile < ntiles; tile += nblk) {
         const int ty = tile / ntx, tx = tile - ty * ntx;
         const int y0 = ty * 16, x0 = tx * 16;
         // unrolled: with no back-edge here, the compiler's waits for the rows
         // read ahead are exact
 #pragma unroll
-        for (int i = 0; i < CX_NPW; ++i) {
-            const float* nxt = i + 1 < CX_NPW ? src_of(tile, i + 1) : src_of(tile + gridDim.x, 0);
+        for (int i = 0; i < NPW; ++i) {
+            const float* nxt = i + 1 < NPW ? src_of(tile, i + 1) : src_of(tile + nblk, 0);
             f32x16 acc[2];
 #pragma unroll
             for (int j = 0; j < 16; ++j) acc[0][j] = acc[1][j] = 0.0f;
@@ -134,7 +141,7 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
             cur = nxt;
             // lane (pl, h) holds P[hi][32 nt + 8 g + 4 h .. +3] in acc[nt][4g .. 4g+3];
             // columns 56.. (nt = 1, g = 3) are not stored
-            const int hi = (wave + CX_WAVES * i) * 32 + pl;
+            const int hi = (wave + WAVES * i) * 32 + pl;
             if (hi < CX_HP) {
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt)
@@ -150,7 +157,7 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
 #pragma unroll
             for (int t = 0; t < CX_RING; ++t)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) nx[t][j] = xr[(9 * CX_NPW + t) % CX_RING][j];
+                for (int j = 0; j < 2; ++j) nx[t][j] = xr[(9 * NPW + t) % CX_RING][j];
 #pragma unroll
             for (int t = 0; t < CX_RING; ++t)
 #pragma unroll
@@ -159,43 +166,45 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
         lds_barrier();  // P complete
 
         // The 9 taps from the halo products, one output pixel per thread.
-        const int ox = tid & 15, oy = tid >> 4;
-        float v[CAB_CC];
-#pragma unroll
-        for (int co = 0; co < CAB_CC; ++co) v[co] = 0.0f;
-#pragma unroll
-        for (int ky = 0; ky < 3; ++ky)
-#pragma unroll
-            for (int kx = 0; kx < 3; ++kx) {
-                const float* q = Ps + ((oy + ky) * CX_HS + ox + kx) * CX_PS + (ky * 3 + kx) * CAB_CC;
-#pragma unroll
-                for (int j = 0; j < CAB_CC / 2; ++j) {
-                    const float2 t = *(const float2*)(q + 2 * j);
-                    v[2 * j] += t.x;
-                    v[2 * j + 1] += t.y;
-                }
-            }
-#pragma unroll
-        for (int co = 0; co < CAB_CC; ++co) v[co] = gelu_scaled(__builtin_fmaf(v[co], p.oinv, bias[co]), p.g0, p.g1);
-        {
-            float* dst = p.t1 + ((size_t)(y0 + oy) * W + x0 + ox) * CAB_CS;
-            *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
-            *(float4*)(dst + 4) = make_float4(v[4], v[5], 0.f, 0.f);
-        }
-
-        // Per-tile sums: the tile, and its pixels on row 0, row H-1, col 0,
-        // col W-1 - only tiles on the plane's border have any of the latter.
         const bool border = y0 == 0 || y0 + 16 == H || x0 == 0 || x0 + 16 == W;  // tile-uniform
+        if (WAVES == 4 || wave < 4) {
+            const int ox = tid & 15, oy = tid >> 4;
+            float v[CAB_CC];
 #pragma unroll
-        for (int l = 0; l < CAB_NSUM; ++l) {
-            if (l > 0 && !border) break;
+            for (int co = 0; co < CAB_CC; ++co) v[co] = 0.0f;
 #pragma unroll
-            for (int co = 0; co < CAB_CC; ++co) {
-                const int gy = y0 + oy, gx = x0 + ox;
-                const bool on = l == 0 || (l == 1 && gy == 0) || (l == 2 && gy == H - 1) || (l == 3 && gx == 0) ||
-                                (l == 4 && gx == W - 1);
-                const float s = wave_sum_dpp(on ? v[co] : 0.0f);
-                if (lane == 0) red[wave][l * CAB_CC + co] = s;
+            for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+                for (int kx = 0; kx < 3; ++kx) {
+                    const float* q = Ps + ((oy + ky) * CX_HS + ox + kx) * CX_PS + (ky * 3 + kx) * CAB_CC;
+#pragma unroll
+                    for (int j = 0; j < CAB_CC / 2; ++j) {
+                        const float2 t = *(const float2*)(q + 2 * j);
+                        v[2 * j] += t.x;
+                        v[2 * j + 1] += t.y;
+                    }
+                }
+#pragma unroll
+            for (int co = 0; co < CAB_CC; ++co) v[co] = gelu_scaled(__builtin_fmaf(v[co], p.oinv, bias[co]), p.g0, p.g1);
+            {
+                float* dst = p.t1 + ((size_t)(y0 + oy) * W + x0 + ox) * CAB_CS;
+                *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
+                *(float4*)(dst + 4) = make_float4(v[4], v[5], 0.f, 0.f);
+            }
+
+            // Per-tile sums: the tile, and its pixels on row 0, row H-1, col 0,
+            // col W-1 - only tiles on the plane's border have any of the latter.
+#pragma unroll
+            for (int l = 0; l < CAB_NSUM; ++l) {
+                if (l > 0 && !border) break;
+#pragma unroll
+                for (int co = 0; co < CAB_CC; ++co) {
+                    const int gy = y0 + oy, gx = x0 + ox;
+                    const bool on = l == 0 || (l == 1 && gy == 0) || (l == 2 && gy == H - 1) || (l == 3 && gx == 0) ||
+                                    (l == 4 && gx == W - 1);
+                    const float s = wave_sum_dpp(on ? v[co] : 0.0f);
+                    if (lane == 0) red[wave * CAB_NSUM * CAB_CC + l * CAB_CC + co] = s;
+                }
             }
         }
         lds_barrier();
@@ -205,7 +214,7 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
             if (co < CAB_CC && (l == 0 || border)) {
                 const int k = l * CAB_CC + co;
 #pragma unroll
-                for (int w = 0; w < CX_WAVES; ++w) s += red[w][k];  // waves in order
+                for (int w = 0; w < 4; ++w) s += red[w * CAB_NSUM * CAB_CC + k];  // waves in order
             }
             p.partial[(size_t)tid * ntiles + tile] = s;  // value-major: [40][tiles]
         }
@@ -213,6 +222,13 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
         // and red above precedes it.
         lds_barrier();
     }
+}
+
+extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(CabConvArgs p)
+{
+    __shared__ __attribute__((aligned(16))) float Ps[CX_HP * CX_PS];
+    __shared__ float red[4 * CAB_NSUM * CAB_CC];
+    cab_conv1_body<CX_WAVES>(p, Ps, red, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------

@@ -71,8 +71,11 @@
 // LeakyReLU 0.01); CEPI_SHUFFLE writes into the shuffled plane (channels
 // pre-permuted as for the direct convs); CEPI_COLSUM stores and leaves the
 // 8 x 16 tile's column sums, one partial row per tile.
-template <int NT, int NTT, int NKC, int CI, int CO, int HEAD>
-__device__ __forceinline__ void convwino_body(const ConvArgs& p)
+// EXT: in a launch shared with another kernel's blocks, as block `blk` of nblk and
+// with the LDS that both use.
+__shared__ __attribute__((aligned(16))) float wg_shared[(6 * WS_CHUNK180 * 2 + GX_WAVES * 16 * gx_stage_stride(30) * 4) / 4 + 192];
+template <int NT, int NTT, int NKC, int CI, int CO, int HEAD, bool EXT = false>
+__device__ __forceinline__ void convwino_body(const ConvArgs& p, int blk = 0, int nblk = 0)
 {
     // Persistent over tiles only for the column-sum epilogue (CAB conv2 60 ->
     // 180: two input chunks, a six-slice epilogue and the sums), where fetching
@@ -91,17 +94,26 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
     // host's pack_wino): each lane forms V for four channels (quad lg), and
     // two MFMAs per step give the three products.
     constexpr bool PACK = CI % 32 != 0 && CI % 32 <= 16;
-    __shared__ __attribute__((aligned(16))) float Pb0[WG_SLOTS * 4];
-    __shared__ __attribute__((aligned(16))) float Pb1[WG_SLOTS * 4];
-    __shared__ __attribute__((aligned(16))) float Ms0[16 * 32 * WG_MS];
-    __shared__ __attribute__((aligned(16))) float Ms1[16 * 32 * WG_MS];
-    __shared__ __attribute__((aligned(16))) float Cs[16 * NT];
-    __shared__ unsigned big;  // block_amax's
+    // objects of their own, so that the compiler sees that reads of one patch
+    // buffer need not wait for the copy into the other (EXT: not seen)
+    __shared__ __attribute__((aligned(16))) float own_pb0[EXT ? 4 : WG_SLOTS * 4];
+    __shared__ __attribute__((aligned(16))) float own_pb1[EXT ? 4 : WG_SLOTS * 4];
+    __shared__ __attribute__((aligned(16))) float own_ms0[EXT ? 4 : 16 * 32 * WG_MS];
+    __shared__ __attribute__((aligned(16))) float own_ms1[EXT ? 4 : 16 * 32 * WG_MS];
+    __shared__ __attribute__((aligned(16))) float own_cs[EXT ? 4 : 16 * NT];
+    __shared__ unsigned own_big[4];  // block_amax's
+    // (by name, not through pointers: those cost the NT = 9 kernel 29 more spills)
+#define Pb0 (EXT ? wg_shared : own_pb0)
+#define Pb1 (EXT ? wg_shared + WG_SLOTS * 4 : own_pb1)
+#define Ms0 (EXT ? wg_shared + 2 * WG_SLOTS * 4 : own_ms0)
+#define Ms1 (EXT ? wg_shared + 2 * WG_SLOTS * 4 + 16 * 32 * WG_MS : own_ms1)
+#define Cs (EXT ? wg_shared + 2 * WG_SLOTS * 4 + 2 * 16 * 32 * WG_MS : own_cs)
+#define big (EXT ? (unsigned*)wg_shared + 2 * WG_SLOTS * 4 + 2 * 16 * 32 * WG_MS + 16 * NT : own_big)
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    if (tid == 0) big = 0;
+    if (tid == 0) *big = 0;
     const int lr = lane & 15;
     const int lg = lane >> 4;
     const int H = p.H, W = p.W;
@@ -113,8 +125,8 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
     // a multiple of NCB). A tile's column blocks are consecutive virtual
     // blocks, so they read its patch from L2 at about the same time.
     constexpr int NCB = NTT / NT;
-    const int nvb = PERSIST && p.nblk > 0 ? p.nblk : (int)gridDim.x;
-    int vb = (int)blockIdx.x;
+    const int nvb = PERSIST && p.nblk > 0 ? p.nblk : EXT ? nblk : (int)gridDim.x;
+    int vb = EXT ? blk : (int)blockIdx.x;
     const int cb = vb % NCB;
     int tile, y0, x0;
     auto set_tile = [&](int v) {
@@ -323,7 +335,7 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
         // The next tile's first patch chunk, in flight under this tile's epilogue:
         // the last chunk ended at a barrier, so no wave still reads the patch
         // buffers, and the epilogue uses Ms0 / Ms1 only.
-        const int vn = vb + (int)gridDim.x;
+        const int vn = vb + (EXT ? nblk : (int)gridDim.x);
         const bool more = PERSIST && vn < nvb;  // block-uniform
         if (more) {
             const int nt_tile = p.tile0 + vn / NCB;
@@ -396,7 +408,7 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
                         if (!PADCO || ocb + 16 * nt < CO) m = finite_max(m, y[nt][q]);
-                block_amax(p.amax_out, &big, m);
+                block_amax(p.amax_out, big, m);
             }
         }
         if constexpr (HEAD >= 0) {
@@ -467,6 +479,12 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p)
         __syncthreads();
     }  // the block's tiles
 }
+#undef Pb0
+#undef Pb1
+#undef Ms0
+#undef Ms1
+#undef Cs
+#undef big
 
 extern "C" __global__ __launch_bounds__(512) void hat_convwino_resid(ConvArgs p)
 {
@@ -500,4 +518,22 @@ extern "C" __global__ __launch_bounds__(512) void hat_convwino_cab1_180(ConvArgs
 extern "C" __global__ __launch_bounds__(512) void hat_convwino_cab2_180(ConvArgs p)
 {
     convwino_body<6, 12, 2, 60, 180, CEPI_COLSUM>(p);
+}
+
+// Small planes, C = 180: the CAB's conv1 and the qkv linear in one launch, as
+// hat_qkv_cab1 (gemmx.hip); the first nconv blocks are conv1's, ntile of them a
+// tile each. Both parts are one block a CU (131 and 164 KB of LDS, overlaid; conv1
+// loses the compiler's knowledge of which buffer a copy goes to, about 1 us).
+// 64 x 64: 21.2 us + 14.3 -> 22.5; 128 x 128: 25.0 + 22.3 -> 34.3.
+extern "C" __global__ __launch_bounds__(512, 1) void hat_qkv_cab1_180(QkvConvArgs p)
+{
+    constexpr int WB = 6 * WS_CHUNK180 * 2, QB = GX_WAVES * 16 * gx_stage_stride(30) * 4;  // bytes
+    unsigned char* lds = (unsigned char*)wg_shared;
+    if ((int)blockIdx.x < p.nconv) {
+        if ((int)blockIdx.x >= p.ntile) return;
+        convwino_body<4, 4, 6, 180, 60, CEPI_STORE, true>(p.c, (int)blockIdx.x, p.ntile);
+    } else {
+        gemmx_qkv_body<180, 12, 3, 30, 6, 2>(p.g, (unsigned short*)lds, (float*)(lds + WB), (float*)(lds + WB + QB),
+                                             (int)blockIdx.x - p.nconv, (int)gridDim.x - p.nconv);
+    }
 }

@@ -97,7 +97,8 @@ constexpr int gx_stage_stride(int hd) { return hd == 24 ? 48 : 30; }
 // tiles, so MT sets the LDS bytes per MFMA).
 // K = 144 (HALF): the last step packed (half_operand, mfma16x2h).
 template <int K, int NT, int NS, int HD, int NH, int MT>
-__device__ __forceinline__ void gemmx_qkv_body(const GemmArgs& p, unsigned short* Wsl, float* Qs, float* Bs)
+__device__ __forceinline__ void gemmx_qkv_body(const GemmArgs& p, unsigned short* Wsl, float* Qs, float* Bs, int block,
+                                               int nblk)
 {
     constexpr bool HALF = K == 144;
     constexpr int KS = (K + 31) / 32;             // 32-k steps (the packed one included)
@@ -115,15 +116,15 @@ __device__ __forceinline__ void gemmx_qkv_body(const GemmArgs& p, unsigned short
     const int M = p.M;
     // block -> (group, slice): with a multiple of 8 groups, blocks b, b + 8,
     // ..., b + 8 (NS - 1) (one XCD) are one group's slices
-    const int G = gridDim.x / NS;
+    const int G = nblk / NS;
     int grp, sl;
     if (G % 8 == 0) {
-        const int i = blockIdx.x >> 3;
+        const int i = block >> 3;
         sl = i % NS;
-        grp = (i / NS) * 8 + (blockIdx.x & 7);
+        grp = (i / NS) * 8 + (block & 7);
     } else {
-        sl = blockIdx.x / G;
-        grp = blockIdx.x - sl * G;
+        sl = block / G;
+        grp = block - sl * G;
     }
     {
         const unsigned short* src = (const unsigned short*)p.w + (size_t)sl * KS * CHUNK;
@@ -288,7 +289,25 @@ extern "C" __global__ __launch_bounds__(GX_WAVES * 64, 1) void hat_gemmx_qkv(Gem
     __shared__ __attribute__((aligned(16))) unsigned short Wsl[5 * WS_CHUNK];  // the slice
     __shared__ __attribute__((aligned(16))) float Qs[GX_WAVES * 16 * gx_stage_stride(24)];  // per-wave staging
     __shared__ __attribute__((aligned(16))) float Bs[144];  // the slice's bias
-    gemmx_qkv_body<144, 9, 3, 24, 6, 2>(p, Wsl, Qs, Bs);
+    gemmx_qkv_body<144, 9, 3, 24, 6, 2>(p, Wsl, Qs, Bs, (int)blockIdx.x, (int)gridDim.x);
+}
+
+// Small planes: the CAB's conv1 and the qkv linear read the same rows and neither
+// fills the chip, so the first nconv blocks (a multiple of 8, so that the groups
+// keep to their XCDs) are conv1's, a 16 x 16 tile each, and the others qkv's. conv1
+// takes the block's eight waves (eleven 32-pixel halo tiles, two a wave instead of
+// three). 64 x 64: 12.3 us + 9.8 -> 13.2; 128 x 128: 12.8 + 13.3 -> 15.9.
+extern "C" __global__ __launch_bounds__(GX_WAVES * 64, 1) void hat_qkv_cab1(QkvCabArgs p)
+{
+    constexpr int WB = 5 * WS_CHUNK * 2, QB = GX_WAVES * 16 * gx_stage_stride(24) * 4;  // bytes
+    constexpr int PB = CX_HP * CX_PS * 4, RB = 4 * CAB_NSUM * CAB_CC * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[WB + QB + 144 * 4 > PB + RB ? WB + QB + 144 * 4 : PB + RB];
+    if ((int)blockIdx.x < p.nconv) {
+        cab_conv1_body<GX_WAVES>(p.c, (float*)lds, (float*)(lds + PB), (int)blockIdx.x, p.nconv);
+    } else {
+        gemmx_qkv_body<144, 9, 3, 24, 6, 2>(p.g, (unsigned short*)lds, (float*)(lds + WB), (float*)(lds + WB + QB),
+                                            (int)blockIdx.x - p.nconv, (int)gridDim.x - p.nconv);
+    }
 }
 
 extern "C" __global__ __launch_bounds__(GX_WAVES * 64, 1) void hat_gemmx_qkv180(GemmArgs p)
@@ -296,5 +315,5 @@ extern "C" __global__ __launch_bounds__(GX_WAVES * 64, 1) void hat_gemmx_qkv180(
     __shared__ __attribute__((aligned(16))) unsigned short Wsl[6 * WS_CHUNK180];  // the slice
     __shared__ __attribute__((aligned(16))) float Qs[GX_WAVES * 16 * gx_stage_stride(30)];  // per-wave staging
     __shared__ __attribute__((aligned(16))) float Bs[192];  // the slice's bias
-    gemmx_qkv_body<180, 12, 3, 30, 6, 2>(p, Wsl, Qs, Bs);
+    gemmx_qkv_body<180, 12, 3, 30, 6, 2>(p, Wsl, Qs, Bs, (int)blockIdx.x, (int)gridDim.x);
 }
