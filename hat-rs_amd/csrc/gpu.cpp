@@ -578,7 +578,10 @@ void run_gemm(hipStream_t s, const DevLinear& L, const float* a, int lda, long M
         p.w = (const float*)L.wx;
         memcpy(p.oscale, L.oscale, sizeof p.oscale);
         if (e.conv1) {
-            QkvConvArgs q{p, *e.conv1, 0, e.conv1->H / 8 * (e.conv1->W / 16)};
+            const int tiles = e.conv1->H / 8 * (e.conv1->W / 16);
+            QkvConvArgs q{p, *e.conv1, 0, tiles, 1};
+            // as two column blocks a tile while those fit as well (64 x 64: 23.2 -> 18.8 us)
+            if (qkv_conv1_blocks(2 * tiles) <= cus / 2) q.ntile = 2 * tiles, q.ncb = 2;
             q.nconv = qkv_conv1_blocks(q.ntile);
             launch(s, "hat_qkv_cab1_180", (unsigned)(q.nconv + 3 * gemmx_qkv_groups(cus - q.nconv, 3)), 1, 1, GX_THREADS, q);
             return;
@@ -901,6 +904,19 @@ void wino_scales(hipStream_t s, const DevConv& C, long n, Amax* in_max, Amax* ou
     }
 }
 
+// A Winograd conv, in its small planes' form while those blocks are one round of the
+// CUs: the trunk convs at 64 x 64 32.9 -> 17.6 us (C = 144) and 27.1 -> 21.2 (180),
+// cab2_180 14.8 -> 12.0, n4_store 18.9 -> 14.8; past one round the repeated V costs
+// more than the wider spread gives (128 x 128: resid180 36.0 and 41.5 us, cab2_180 18.8
+// and 21.0, the upsample conv at 128 x 128 24 and 24.9).
+void launch_wino_for(hipStream_t s, const char* name, unsigned tiles, unsigned ncb, ConvArgs& p)
+{
+    static const unsigned cus = (unsigned)std::max(1, Runtime::get().cu_count());
+    const WinoSmall k = convwino_small(name);
+    if ((size_t)tiles * k.ncb <= cus) launch_wino(s, k.name.c_str(), tiles, k.ncb, p);
+    else launch_wino(s, name, tiles, ncb, p);
+}
+
 // [band_r0, band_r1): with band_r1 >= 0, only that band of tile rows is
 // launched (the host-memory forward's head): 8 input rows of the Winograd
 // upsample conv (hat_convwino_n8_shuffle), 16 output rows of conv_last
@@ -989,7 +1005,7 @@ void run_conv(hipStream_t s, const DevConv& C, const float* in, int cin_stride, 
     p.os = os;
     auto wino = [&](const char* name, unsigned tiles, unsigned ncb) {
         wino_scales(s, C, (long)H * W * cin_stride, in_max, out_max, &p);
-        launch_wino(s, name, tiles, ncb, p);
+        launch_wino_for(s, name, tiles, ncb, p);
     };
     const size_t rr = C.r > 0 ? (size_t)C.r * C.r : 1;
     if (C.wu && H % 16 == 0 && W % 16 == 0 && cin_stride % 4 == 0 && cin_stride >= C.CI &&
@@ -1108,7 +1124,7 @@ void run_convw(hipStream_t s, const DevConv& C, const float* in, int cin_stride,
         (size_t)H * W * cin_stride < ((size_t)1 << 31)) {
         if (in == out) throw Error("convw: the output must not overlap the input");
         wino_scales(s, C, (long)H * W * cin_stride, in_max, out_max, &p);
-        launch_wino(s, "hat_convwino_resid", (unsigned)((W / 16) * (H / 8)), 1, p);
+        launch_wino_for(s, "hat_convwino_resid", (unsigned)((W / 16) * (H / 8)), 1, p);
         if (epi == EPI_RESID_LN) run_ln(s, out, xn, nw, nb, (long)H * W, C.CO);
         return;
     }
@@ -1186,7 +1202,16 @@ void run_ln(hipStream_t s, const float* x, float* y, const float* w, const float
 bool convwino_persistent(const std::string& name)
 {
     // convwino.hip: the column-sum kernel (the CAB's conv2 at C = 180)
-    return name == "hat_convwino_cab2_180";
+    return name == "hat_convwino_cab2_180" || name == "hat_convwino_cab2_180_s";
+}
+
+WinoSmall convwino_small(const std::string& name)
+{
+    const unsigned ncb = name == "hat_convwino_resid" ? 3
+                         : name == "hat_convwino_resid180" || name == "hat_convwino_cab2_180" || name == "hat_convwino_n8_shuffle"
+                             ? 4
+                             : 2;
+    return {name + "_s", ncb};
 }
 
 void launch_wino(hipStream_t s, const char* name, unsigned tiles, unsigned ncb, ConvArgs& p, unsigned max_blocks)

@@ -152,6 +152,12 @@ std::vector<float> pack_conv(const float* w, const float* b, int CO, int CI, int
 // each walking the virtual blocks blockIdx.x + i gridDim.x and fetching its
 // next tile's first patch chunk under the current tile's epilogue; the others
 // take one block a tile.
+// The kernel's form for small planes: its name and column blocks.
+struct WinoSmall {
+    std::string name;
+    unsigned ncb;
+};
+WinoSmall convwino_small(const std::string& name);
 bool convwino_persistent(const std::string& name);
 void launch_wino(hipStream_t s, const char* name, unsigned tiles, unsigned ncb, hatk::ConvArgs& p,
                  unsigned max_blocks = 0);

@@ -17,7 +17,9 @@ const std::vector<std::string>& required_kernels()
     static const std::vector<std::string> k = {
         "hat_attn_sw_d24",     "hat_attn_sw_d30",     "hat_attn_oca_d24",   "hat_attn_oca_d30",
         "hat_attnx_sw_d24",    "hat_attnx_sw_d30",    "hat_attnx_oca_d24",  "hat_attnx_oca_d30",
-        "hat_gemmx_qkv", "hat_gemmx_qkv180", "hat_qkv_cab1", "hat_qkv_cab1_180", "hat_habx_cab_ln", "hat_habx", "hat_habx180_hab_ln", "hat_habx180",
+        "hat_gemmx_qkv", "hat_gemmx_qkv180", "hat_qkv_cab1", "hat_qkv_cab1_180", "hat_convwino_resid_s", "hat_convwino_n4_store_s",
+        "hat_convwino_n8_shuffle_s", "hat_convwino_resid180_s", "hat_convwino_n4_store180_s", "hat_convwino_cab1_180_s",
+        "hat_convwino_cab2_180_s", "hat_habx_cab_ln", "hat_habx", "hat_habx180_hab_ln", "hat_habx180",
         "hat_habx_cab_ln_s", "hat_habx_s", "hat_habx180_hab_ln_s", "hat_habx180_s",
         "hat_conv_first_ln144", "hat_conv_first_ln180",
         "hat_conv_n1_store",   "hat_conv_n3_store",   "hat_conv_n4_store",  "hat_conv_n3_resid",

@@ -312,7 +312,8 @@ struct QkvCabArgs {
 struct QkvConvArgs {
     GemmArgs g;
     ConvArgs c;
-    int nconv, ntile;
+    int nconv, ntile;  // ntile: tiles times ncb
+    int ncb;           // conv1's column blocks: 1, or 2 of 32 channels
 };
 
 struct TailXArgs {

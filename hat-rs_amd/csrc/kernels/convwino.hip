@@ -234,8 +234,9 @@ __device__ __forceinline__ void convwino_body(const ConvArgs& p, int blk = 0, in
     f32x4 acc[2][NT][2];
 
     // U loads RING - 1 steps ahead (2 NT steps a chunk, a multiple of RING, so
-    // slot t % RING lines up across chunks)
-    constexpr int RING = (2 * NT) % 3 == 0 ? 3 : 4;
+    // slot t % RING lines up across chunks); narrow blocks have registers for a
+    // whole chunk's and little else to hide them under
+    constexpr int RING = NT <= 3 ? 2 * NT : (2 * NT) % 3 == 0 ? 3 : 4;
     static_assert((2 * NT) % RING == 0 && 2 * NT >= RING, "the ring lines up across chunks");
     U2 ur[RING];
     fetch(0, CInt<0>{});
@@ -520,6 +521,38 @@ extern "C" __global__ __launch_bounds__(512) void hat_convwino_cab2_180(ConvArgs
     convwino_body<6, 12, 2, 60, 180, CEPI_COLSUM>(p);
 }
 
+// Small planes (_s): narrower column blocks, so that a plane whose tiles are a
+// fraction of the chip runs on more of it; each forms the tiles' V again, and a
+// whole chunk's U is in flight. Where and what it gives: launch_wino_for.
+extern "C" __global__ __launch_bounds__(512) void hat_convwino_resid_s(ConvArgs p)
+{
+    convwino_body<3, 9, 5, 144, 144, -1>(p);
+}
+extern "C" __global__ __launch_bounds__(512) void hat_convwino_n4_store_s(ConvArgs p)
+{
+    convwino_body<2, 4, 5, 144, 64, CEPI_STORE>(p);
+}
+extern "C" __global__ __launch_bounds__(512) void hat_convwino_n8_shuffle_s(ConvArgs p)
+{
+    convwino_body<4, 16, 2, 64, 256, CEPI_SHUFFLE>(p);
+}
+extern "C" __global__ __launch_bounds__(512) void hat_convwino_resid180_s(ConvArgs p)
+{
+    convwino_body<3, 12, 6, 180, 180, -1>(p);
+}
+extern "C" __global__ __launch_bounds__(512) void hat_convwino_n4_store180_s(ConvArgs p)
+{
+    convwino_body<2, 4, 6, 180, 64, CEPI_STORE>(p);
+}
+extern "C" __global__ __launch_bounds__(512) void hat_convwino_cab1_180_s(ConvArgs p)
+{
+    convwino_body<2, 4, 6, 180, 60, CEPI_STORE>(p);
+}
+extern "C" __global__ __launch_bounds__(512) void hat_convwino_cab2_180_s(ConvArgs p)
+{
+    convwino_body<3, 12, 2, 60, 180, CEPI_COLSUM>(p);
+}
+
 // Small planes, C = 180: the CAB's conv1 and the qkv linear in one launch, as
 // hat_qkv_cab1 (gemmx.hip); the first nconv blocks are conv1's, ntile of them a
 // tile each. Both parts are one block a CU (131 and 164 KB of LDS, overlaid; conv1
@@ -531,7 +564,8 @@ extern "C" __global__ __launch_bounds__(512, 1) void hat_qkv_cab1_180(QkvConvArg
     unsigned char* lds = (unsigned char*)wg_shared;
     if ((int)blockIdx.x < p.nconv) {
         if ((int)blockIdx.x >= p.ntile) return;
-        convwino_body<4, 4, 6, 180, 60, CEPI_STORE, true>(p.c, (int)blockIdx.x, p.ntile);
+        if (p.ncb == 2) convwino_body<2, 4, 6, 180, 60, CEPI_STORE, true>(p.c, (int)blockIdx.x, p.ntile);
+        else convwino_body<4, 4, 6, 180, 60, CEPI_STORE, true>(p.c, (int)blockIdx.x, p.ntile);
     } else {
         gemmx_qkv_body<180, 12, 3, 30, 6, 2>(p.g, (unsigned short*)lds, (float*)(lds + WB), (float*)(lds + WB + QB),
                                              (int)blockIdx.x - p.nconv, (int)gridDim.x - p.nconv);

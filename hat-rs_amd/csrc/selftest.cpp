@@ -777,13 +777,14 @@ int gpu_selftest(std::string* err)
         {
             // wino: the Winograd F(2x2, 3x3) kernels (8 x 16 tiles, 512 threads)
             // the conv_first kernels (convfirst.hip): 16 x 16 tiles, 4 waves
-            struct WCase { int CI, cin_stride, CO, epi; const char* k; int waves; bool wino; };
-            const WCase wc[] = {{144, 144, 144, EPI_RESID_LN, "hat_convw_n9_resid_ln", CONVW_WAVES_N9_RESID_LN, false},
-                                {3, 4, 144, EPI_STORE_LN, "hat_convw_n9_store_ln", CONVW_WAVES_N9_STORE_LN, false},
-                                {3, 4, 144, EPI_STORE_LN, "hat_conv_first_ln144", 4, false},
-                                {3, 4, 180, EPI_STORE_LN, "hat_conv_first_ln180", 4, false},
-                                {144, 144, 144, EPI_RESID, "hat_convw_n9_resid", CONVW_WAVES_N9_RESID, false},
-                                {144, 144, 144, EPI_RESID, "hat_convwino_resid", 8, true}};
+            struct WCase { int CI, cin_stride, CO, epi; const char* k; int waves; bool wino, small; };
+            const WCase wc[] = {{144, 144, 144, EPI_RESID_LN, "hat_convw_n9_resid_ln", CONVW_WAVES_N9_RESID_LN, false, false},
+                                {3, 4, 144, EPI_STORE_LN, "hat_convw_n9_store_ln", CONVW_WAVES_N9_STORE_LN, false, false},
+                                {3, 4, 144, EPI_STORE_LN, "hat_conv_first_ln144", 4, false, false},
+                                {3, 4, 180, EPI_STORE_LN, "hat_conv_first_ln180", 4, false, false},
+                                {144, 144, 144, EPI_RESID, "hat_convw_n9_resid", CONVW_WAVES_N9_RESID, false, false},
+                                {144, 144, 144, EPI_RESID, "hat_convwino_resid", 8, true, false},
+                                {144, 144, 144, EPI_RESID, "hat_convwino_resid_s", 8, true, true}};
             for (const WCase& c : wc) {
                 const int H = 32, W = 48, HW = H * W, CO = c.CO;
                 std::vector<float> in((size_t)HW * c.cin_stride, 0.0f);
@@ -822,7 +823,7 @@ int gpu_selftest(std::string* err)
                 p.wu = (const unsigned short*)dwu.p;
                 p.uinv = uinv;
                 p.vs = 4096.0f;  // |V| <= 4 max|x| <= 4
-                if (c.wino) launch_wino(s, c.k, (W / 16) * (H / 8), 1, p, 5);  // persistent ones over 5 blocks
+                if (c.wino) launch_wino(s, c.k, (W / 16) * (H / 8), c.small ? convwino_small("hat_convwino_resid").ncb : 1, p);
                 else launch(s, c.k, (W / 16) * (H / 16), 1, 1, c.waves * 64, p);  // convw and conv_first: 16 x 16
                 std::vector<double> want((size_t)HW * CO), wxn((size_t)HW * CO);
                 for (int y = 0; y < H; ++y)
@@ -1023,45 +1024,47 @@ int gpu_selftest(std::string* err)
                                : cc.epi == CEPI_RESID && cc.CI == 180 && cc.CO == 180 ? "hat_convwino_resid180"
                                                                                       : nullptr;
             if (wino) {
-                const int ncb = cc.CO == 256 ? 2 : cc.CO == 180 ? 2 : 1;
+                const unsigned ncb = cc.CO == 256 ? 2 : cc.CO == 180 ? 2 : 1;
                 const std::vector<unsigned short> wux = pack_wino(w.data(), cc.CO, cc.CI, cc.r, &p.uinv);
-                Dev dwu((wux.size() + 1) / 2), dout4(out_n), dpart4((size_t)nblk * cc.CO);
-                Runtime::get().h2d(dwu.p, wux.data(), wux.size() * sizeof(unsigned short));
-                p.out = dout4.p;
-                p.partial = dpart4.p;
-                p.wu = (const unsigned short*)dwu.p;
-                // V's scale from the input's largest magnitude, and the output's
-                // left for the next conv
-                Dev dmax(std::vector<float>(2 * AMAX_WORDS, 0.0f));
-                AbsMaxArgs am{p.in, (unsigned*)dmax.p, (long)H * W * p.cin_stride};
-                launch(s, "hat_absmax", 3, 1, 1, 256, am);
-                p.amax = (const unsigned*)dmax.p;
-                p.amax_out = (unsigned*)dmax.p + AMAX_WORDS;
-                // the persistent kernels over 5 ncb blocks (2 or 3 of the 12 tiles
-                // each, the next tile's patch fetched under an epilogue)
-                launch_wino(s, wino, (W / 16) * (H / 8), ncb, p, 5 * ncb);
-                p.nblk = 0;
-                p.amax = nullptr;
-                p.amax_out = nullptr;
-                check_close(std::string(wino) + " " + cc.what, dout4.get(), want, 5e-5);
-                if (cc.epi != CEPI_COLSUM && cc.act == 0) {
-                    double big = 0.0;
-                    for (double v : want) big = std::max(big, std::fabs(v));
-                    const std::vector<float> lanes = dmax.get();
-                    const float got = *std::max_element(lanes.begin() + AMAX_WORDS, lanes.end());
-                    check_close(std::string(wino) + " output maximum", {got}, {big}, 5e-5);
+                for (const WinoSmall& k : {WinoSmall{wino, ncb}, convwino_small(wino)}) {
+                    Dev dwu((wux.size() + 1) / 2), dout4(out_n), dpart4((size_t)nblk * cc.CO);
+                    Runtime::get().h2d(dwu.p, wux.data(), wux.size() * sizeof(unsigned short));
+                    p.out = dout4.p;
+                    p.partial = dpart4.p;
+                    p.wu = (const unsigned short*)dwu.p;
+                    // V's scale from the input's largest magnitude, and the output's
+                    // left for the next conv
+                    Dev dmax(std::vector<float>(2 * AMAX_WORDS, 0.0f));
+                    AbsMaxArgs am{p.in, (unsigned*)dmax.p, (long)H * W * p.cin_stride};
+                    launch(s, "hat_absmax", 3, 1, 1, 256, am);
+                    p.amax = (const unsigned*)dmax.p;
+                    p.amax_out = (unsigned*)dmax.p + AMAX_WORDS;
+                    // the persistent kernels over 5 ncb blocks (2 or 3 of the 12 tiles
+                    // each, the next tile's patch fetched under an epilogue)
+                    launch_wino(s, k.name.c_str(), (W / 16) * (H / 8), k.ncb, p, 5 * k.ncb);
+                    p.nblk = 0;
+                    p.amax = nullptr;
+                    p.amax_out = nullptr;
+                    check_close(k.name + " " + cc.what, dout4.get(), want, 5e-5);
+                    if (cc.epi != CEPI_COLSUM && cc.act == 0) {
+                        double big = 0.0;
+                        for (double v : want) big = std::max(big, std::fabs(v));
+                        const std::vector<float> lanes = dmax.get();
+                        const float got = *std::max_element(lanes.begin() + AMAX_WORDS, lanes.end());
+                        check_close(k.name + " output maximum", {got}, {big}, 5e-5);
+                    }
+                    if (cc.epi == CEPI_COLSUM) {
+                        // one partial row per 8x16 tile
+                        std::vector<double> ps((size_t)nblk * cc.CO, 0.0);
+                        for (int y = 0; y < H; ++y)
+                            for (int x = 0; x < W; ++x) {
+                                const int blk = (y / 8) * (W / 16) + x / 16;
+                                for (int o = 0; o < cc.CO; ++o) ps[(size_t)blk * cc.CO + o] += full[((size_t)y * W + x) * cc.CO + o];
+                            }
+                        check_close(k.name + " partial sums", dpart4.get(), ps, 5e-4);
+                    }
+                    note(k.name + "  " + cc.what + "  32x48");
                 }
-                if (cc.epi == CEPI_COLSUM) {
-                    // one partial row per 8x16 tile
-                    std::vector<double> ps((size_t)nblk * cc.CO, 0.0);
-                    for (int y = 0; y < H; ++y)
-                        for (int x = 0; x < W; ++x) {
-                            const int blk = (y / 8) * (W / 16) + x / 16;
-                            for (int o = 0; o < cc.CO; ++o) ps[(size_t)blk * cc.CO + o] += full[((size_t)y * W + x) * cc.CO + o];
-                        }
-                    check_close(std::string(wino) + " partial sums", dpart4.get(), ps, 5e-4);
-                }
-                note(std::string(wino) + "  " + cc.what + "  32x48");
             }
             // conv_last by per-tap products: 16 x 32 tiles, so W = 48 leaves a
             // half tile whose pixels past W are zero halo and are not stored.
