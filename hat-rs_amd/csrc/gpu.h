@@ -186,7 +186,7 @@ public:
     // h x w forward (gpu.rs:78-290 footprint_floats), computed without a device.
     static size_t plan_bytes(const Weights& wt, int h, int w, bool host_io);
     // Device bytes the weight upload of a backend over `wt` allocates (the
-    // packed FP32 tensors and their split-bf16 copies), computed without a
+    // packed FP32 tensors and their split copies), computed without a
     // device by running the upload's packers in a counting pass; cached in wt.
     static size_t device_weight_bytes(const Weights& wt);
     static bool cab_folded(const Weights& wt);

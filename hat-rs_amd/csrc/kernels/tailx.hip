@@ -530,16 +530,11 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
 // first. The wave's issue bounds it, not the weights' latency: a second launch on
 // the same, cached weights takes as long. 64 x 64 tokens: hat_habx_cab_ln 34.2 ->
 // 23.3 us, hat_habx180_hab_ln 45.0 -> 30.7; 128 x 128: 37.5 -> 27.6, 49.8 -> 38.8.
-#define TX_INST(NAME, C, CAB, HAB, LN)                                                  \
-    extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void NAME(TailXArgs p)    \
-    {                                                                                   \
-        habx_body<C, CAB, HAB, LN, 2, 2>(p);                                            \
-    }                                                                                   \
-    extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 1) void NAME##_s(TailXArgs p) \
-    {                                                                                   \
-        habx_body<C, CAB, HAB, LN, 1, 4>(p);                                            \
-    }
-TX_INST(hat_habx_cab_ln, 144, true, false, true)
-TX_INST(hat_habx, 144, false, false, false)
-TX_INST(hat_habx180_hab_ln, 180, false, true, true)
-TX_INST(hat_habx180, 180, false, false, false)
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx_cab_ln(TailXArgs p) { habx_body<144, true, false, true, 2, 2>(p); }
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 1) void hat_habx_cab_ln_s(TailXArgs p) { habx_body<144, true, false, true, 1, 4>(p); }
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx(TailXArgs p) { habx_body<144, false, false, false, 2, 2>(p); }
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 1) void hat_habx_s(TailXArgs p) { habx_body<144, false, false, false, 1, 4>(p); }
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx180_hab_ln(TailXArgs p) { habx_body<180, false, true, true, 2, 2>(p); }
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 1) void hat_habx180_hab_ln_s(TailXArgs p) { habx_body<180, false, true, true, 1, 4>(p); }
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 2) void hat_habx180(TailXArgs p) { habx_body<180, false, false, false, 2, 2>(p); }
+extern "C" __global__ __launch_bounds__(TX_WAVES * 64, 1) void hat_habx180_s(TailXArgs p) { habx_body<180, false, false, false, 1, 4>(p); }
