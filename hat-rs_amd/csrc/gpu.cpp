@@ -590,6 +590,7 @@ void run_gemm(hipStream_t s, const DevLinear& L, const float* a, int lda, long M
         return;
     }
     if (e.cab || e.conv1) throw Error("GEMM: this shape takes no CAB conv");
+    if (!L.w) throw Error("GEMM: the FP32 weights were not uploaded");
     int wbn = 0;
     if (const char* ws = gemm_ws_kernel(L, epi, &wbn)) {
         // One block per CU (its 85 or 150 KB weight slice fills the LDS); the
@@ -626,6 +627,7 @@ void run_mlp(hipStream_t s, const DevLinear& fc1, const DevLinear& fc2, const fl
     const bool c144 = mlp_c144(fc1, fc2);
     if (mlp_fused(fc1, fc2)) {
         if (M > 0x7fffffffL) throw Error("MLP: too many rows");
+        if (!fc1.w || !fc2.w) throw Error("MLP: the FP32 weights were not uploaded");
         MlpArgs p{};
         p.a = a;
         p.w1 = fc1.w;
@@ -733,6 +735,7 @@ void run_hab_tail(hipStream_t s, const DevLinear& proj, const DevLinear& fc1, co
     const bool cab = t1 != nullptr;
     if (cab && (!w2g || !xn || !nw || !nb)) throw Error("HAB tail: the CAB form needs w2g and the next norm");
     if (!hab_tail_fits(proj, fc1, fc2)) throw Error("HAB tail: needs the 144 x 144 projection and 144 -> 288 -> 144 MLP");
+    if (!proj.w || !fc1.w || !fc2.w) throw Error("HAB tail: the FP32 weights were not uploaded");
     const long M = (long)H * W;
     if (M > 0x7fffffffL) throw Error("HAB tail: too many rows");
     HabTailArgs p{};
@@ -1282,10 +1285,12 @@ void GpuBackend::upload_linear(const std::string& name, const float* out, float 
     if (out)
         for (int n = 0; n < L.N; ++n) bs[n] *= out[n / (L.N / 3)];
     L.b = upload(bs.data(), L.N);
+    bool split = false;
     if (out && ((L.K == 180 && L.N == 540) || (L.K == 144 && L.N == 432))) {
         // qkv: the weight-stationary layout of hat_gemmx_qkv
         std::vector<unsigned short> x = split_qkv(w, L.N, L.K, out, in, L.oscale, !count_only_);
         L.wx = (unsigned short*)upload_bytes(x.data(), x.size() * sizeof(unsigned short));
+        split = true;
     } else if (!bias_only) {
         std::vector<float> ws(w, w + (size_t)L.N * L.K);
         for (int n = 0; n < L.N; ++n) {
@@ -1295,6 +1300,7 @@ void GpuBackend::upload_linear(const std::string& name, const float* out, float 
         std::vector<float> pk = pack_linear(ws.data(), L.N, L.K, &L.Kp);
         L.w = upload(pk.data(), pk.size());
     }
+    L.rows = !split && !bias_only;
     lin_[name] = L;
 }
 
@@ -1349,18 +1355,16 @@ double GpuBackend::cab_t1_bound(const std::string& cab, const std::string& norm1
 }
 
 void GpuBackend::upload_tail(const std::string& proj, const std::string& mlp, const std::string& norm2,
-                             const std::string& cab, const std::string& norm1)
+                             const std::string& cab, const std::string& norm1, bool ocab)
 {
     const size_t C = (size_t)wt_.embed;
     upload_norm(norm2);
     const float sn = norm_scale_.at(norm2);
-    const bool fits = (C == 144 || C == 180) && wt_.info(proj + ".weight").shape == std::vector<size_t>{C, C} &&
-                      wt_.info(mlp + ".fc1.weight").shape == std::vector<size_t>{2 * C, C} &&
-                      wt_.info(mlp + ".fc2.weight").shape == std::vector<size_t>{C, 2 * C};
-    upload_linear(proj, nullptr, 1.0f / v_scale_, fits);
-    upload_linear(mlp + ".fc1", nullptr, 1.0f / sn, fits);
-    upload_linear(mlp + ".fc2", nullptr, 1.0f, fits);
-    if (!fits) return;
+    const bool tail = tail_runs(wt_, ocab);
+    upload_linear(proj, nullptr, 1.0f / v_scale_, tail);
+    upload_linear(mlp + ".fc1", nullptr, 1.0f / sn, tail);
+    upload_linear(mlp + ".fc2", nullptr, 1.0f, tail);
+    if (!tail) return;
     TailCab tc{0.0, 0.0};
     if (!cab.empty() && !count_only_) {
         tc.t1 = cab_t1_bound(cab, norm1);
@@ -1399,6 +1403,32 @@ void GpuBackend::upload_conv(const std::string& name, int r, float in, double bo
         C.wu = (unsigned short*)upload_bytes(wu.data(), wu.size() * sizeof(unsigned short));
     }
     conv_[name] = C;
+}
+
+// Which blocks' second half runs tailx.hip: C = 180, and at C = 144 the OCAB and
+// the HAB with the folded CAB (there is no 144-channel tail for conv2's output).
+// The others run the projection and the MLP as FP32 linears.
+bool GpuBackend::tail_runs(const Weights& wt, bool ocab)
+{
+    return wt.mlp_ratio == 2 && (wt.embed == 180 || (wt.embed == 144 && (ocab || cab_folded(wt))));
+}
+
+// Every linear that a block reads as FP32 rows has them (upload_all).
+void GpuBackend::check_linears() const
+{
+    auto need = [&](const std::string& proj, const std::string& mlp, bool ocab) {
+        if (tail_runs(wt_, ocab)) return;
+        for (const std::string& n : {proj, mlp + ".fc1", mlp + ".fc2"})
+            if (!lin_.at(n).rows) throw Error("upload: " + n + " was left out, and its block reads it");
+    };
+    for (size_t s = 0; s < wt_.depths.size(); ++s) {
+        const std::string L = "layers." + std::to_string(s) + ".residual_group.";
+        for (int b = 0; b < wt_.depths[s]; ++b) {
+            const std::string p = L + "blocks." + std::to_string(b);
+            need(p + ".attn.proj", p + ".mlp", false);
+        }
+        need(L + "overlap_attn.proj", L + "overlap_attn.mlp", true);
+    }
 }
 
 // Gpu::new (gpu.rs:372-386): bring up the runtime, then upload every tensor.
@@ -1454,7 +1484,7 @@ void GpuBackend::upload_all()
                 upload_raw(p + n);
             upload_attn(p + ".attn.qkv", p + ".attn.proj", p + ".norm1", p + ".attn.relative_position_bias_table");
             upload_tail(p + ".attn.proj", p + ".mlp", p + ".norm2", cab_fold_ ? p + ".conv_block.cab." : std::string(),
-                        p + ".norm1");
+                        p + ".norm1", false);
             const float xin = 1.0f / norm_scale_.at(p + ".norm1");
             if (cab_fold_) {
                 const std::string c = p + ".conv_block.cab.";
@@ -1487,7 +1517,7 @@ void GpuBackend::upload_all()
         upload_norm(p + ".norm1");
         upload_raw(p + ".relative_position_bias_table");
         upload_attn(p + ".qkv", p + ".proj", p + ".norm1", p + ".relative_position_bias_table");
-        upload_tail(p + ".proj", p + ".mlp", p + ".norm2", std::string(), p + ".norm1");
+        upload_tail(p + ".proj", p + ".mlp", p + ".norm2", std::string(), p + ".norm1", true);
         upload_conv(L + ".conv");
     }
     upload_raw("norm.weight");
@@ -1498,6 +1528,7 @@ void GpuBackend::upload_all()
     for (size_t b = 0; b < blocks.size(); ++b)
         upload_conv("upsample." + std::to_string(2 * b), blocks[b].first);
     upload_conv("conv_last");
+    check_linears();
 }
 
 GpuBackend::~GpuBackend()
@@ -1674,7 +1705,7 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
         // launch (its first block), conv2 inside the tail's projection.
         const DevLinear& proj = lin_.at(p + ".attn.proj");
         auto tl = tail_.find(p + ".mlp");
-        const bool split = tl != tail_.end();  // the split tail runs
+        const bool split = tail_runs(wt_, false);
         CabGateArgs gate{};
         CabConvArgs conv1{};
         const DevLinear& qkv = lin_.at(p + ".attn.qkv");
@@ -1731,14 +1762,13 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
     if (!with) gemm(qkv, a_.xn, C, T, a_.qkv, 0, EPI_QKV);
     attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, nullptr, &se);
     const DevLinear& proj = lin_.at(p + ".attn.proj");
-    auto tl = tail_.find(p + ".mlp");
-    if (tl != tail_.end() && C == 180) {
+    if (tail_runs(wt_, false)) {
         // projection + gated conv branch + shortcut, norm2, the MLP + residual + next norm
         TailCabIn cab;
         cab.aux = a_.t2;
         cab.gate = a_.gate;
         cab.cscale = wt_.conv_scale;
-        run_tailx(stream_, tl->second, a_.ao, x_in, x_out, a_.xn, proj.b, lin_.at(p + ".mlp.fc2").b,
+        run_tailx(stream_, tail_.at(p + ".mlp"), a_.ao, x_in, x_out, a_.xn, proj.b, lin_.at(p + ".mlp.fc2").b,
                   raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), raw_.at(next_norm + ".weight"),
                   raw_.at(next_norm + ".bias"), T, cab);
         return;
@@ -1758,9 +1788,8 @@ void GpuBackend::ocab(int stage, float* x, Amax* out_max)
     attention(p + ".relative_position_bias_table", true, 0);
     const DevLinear& proj = lin_.at(p + ".proj");
     const DevLinear &fc1 = lin_.at(p + ".mlp.fc1"), &fc2 = lin_.at(p + ".mlp.fc2");
-    auto tl = tail_.find(p + ".mlp");
-    if (tl != tail_.end()) {
-        run_tailx(stream_, tl->second, a_.ao, x, x, nullptr, proj.b, fc2.b, raw_.at(p + ".norm2.weight"),
+    if (tail_runs(wt_, true)) {
+        run_tailx(stream_, tail_.at(p + ".mlp"), a_.ao, x, x, nullptr, proj.b, fc2.b, raw_.at(p + ".norm2.weight"),
                   raw_.at(p + ".norm2.bias"), nullptr, nullptr, T, TailCabIn{}, out_max);
         return;
     }

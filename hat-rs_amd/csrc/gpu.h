@@ -24,7 +24,8 @@ public:
 };
 
 struct DevLinear {
-    float* w = nullptr;  // [N][Kp]
+    float* w = nullptr;  // [N][Kp], or null where the split kernels hold the weights
+    bool rows = false;   // w is set (in the counting pass: would be)
     float* b = nullptr;  // [N]
     // qkv: the same weights split for hat_gemmx_qkv* (pack_linear_ws), or null
     // where the FP32 kernels run (and w is null where they do not).
@@ -190,6 +191,7 @@ public:
     // device by running the upload's packers in a counting pass; cached in wt.
     static size_t device_weight_bytes(const Weights& wt);
     static bool cab_folded(const Weights& wt);
+    static bool tail_runs(const Weights& wt, bool ocab);
     // HAB.forward of one block (gpu.rs:469-520 `hab`) on a window-multiple
     // hp x wp plane: host x, out token-major [hp*wp][embed]; with the block's
     // shift and mask when it is odd. iters > 0: *ms = mean device time of the
@@ -280,10 +282,12 @@ private:
     // what |t1| (the CAB's conv1 output) cannot exceed behind norm1
     double cab_t1_bound(const std::string& cab, const std::string& norm1) const;
     std::map<std::string, float> t1_scale_;  // by block: the unfolded CAB's t1
-    // the split-f16 tail of a block, where its shapes have one (upload_attn first;
-    // conv: the folded CAB's prefix, or empty)
+    // a block's norm2, projection and MLP: the split-f16 tail where it runs
+    // (tail_runs), else FP32 rows (upload_attn first; cab: the folded CAB's prefix,
+    // or empty)
     void upload_tail(const std::string& proj, const std::string& mlp, const std::string& norm2, const std::string& cab,
-                     const std::string& norm1);
+                     const std::string& norm1, bool ocab);
+    void check_linears() const;
     float v_scale_ = 1.0f;  // of the attention uploaded last
     void ensure_plan(int h, int w);
     void free_plan();
