@@ -395,6 +395,7 @@ double ln_bound(const float* lnw, const float* lnb, int C)
 QkvScale qkv_scale(double bq, double bk, double bv, int head_dim)
 {
     QkvScale s;
+    s.v = f16_scale(bv);  // whichever attention runs: the split tail reads its output
     bq *= 1.4426950408889634 / std::sqrt((double)head_dim);  // the kernels split q times this
     if (!std::isfinite(bq) || !std::isfinite(bk) || !std::isfinite(bv)) return s;
     int a = 0;
@@ -402,7 +403,6 @@ QkvScale qkv_scale(double bq, double bk, double bv, int head_dim)
     if (std::abs(a) > 60 || std::ldexp(bq, a) > 32768.0 || std::ldexp(bk, -a) > 32768.0) return s;
     s.q = std::ldexp(1.0f, a);
     s.k = std::ldexp(1.0f, -a);
-    s.v = f16_scale(bv);
     s.ok = true;
     return s;
 }

@@ -92,7 +92,8 @@ double ln_bound(const float* lnw, const float* lnb, int C);
 // The scales of an attention's q, k and v rows (folded into the qkv weights):
 // q and k by inverse powers of two that balance their bounds, so that the scores
 // do not change, v by its own (the projection's weights take it out). ok: the
-// balanced bounds fit; otherwise the FP32 kernels run and every scale is 1.
+// balanced bounds fit; otherwise the FP32 attention runs on q and k as they are.
+// It is linear in v, which keeps its scale: the tail behind it splits its output.
 struct QkvScale {
     float q = 1.0f, k = 1.0f, v = 1.0f;
     bool ok = false;
@@ -273,8 +274,8 @@ private:
     // power of two that takes every row it can produce to f16's range.
     void upload_norm(const std::string& name);
     std::map<std::string, float> norm_scale_;
-    // An attention's qkv and projection behind norm `ln`, scaled for the
-    // split-f16 attention where the bounds allow it (attn_f16_ of its table).
+    // An attention's qkv and projection behind norm `ln`, scaled (qkv_scale);
+    // attn_f16_ of its table: whether the split-f16 attention runs.
     void upload_attn(const std::string& qkv, const std::string& proj, const std::string& ln, const std::string& table);
     // in: as upload_linear's; bound: of the input's |x| as the kernel reads it, or 0
     // where only the device can know (Amax)

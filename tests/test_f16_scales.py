@@ -1,0 +1,95 @@
+"""The powers of two that bring operands into f16's range, where the values are far
+from 1 or the attention's q and k admit none (the FP32 attention then runs before the
+split-f16 tail)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from checkpoint_edit import edited
+from conftest import OP_TOL, make_weights
+
+HEADS = 6
+
+
+class _QkvScale(C.Structure):
+    _fields_ = [("q", C.c_float), ("k", C.c_float), ("v", C.c_float), ("ok", C.c_bool)]
+
+
+def _qkv_scale(bq, bk, bv, head_dim):
+    import hat_amd as hl
+    f = hl.lib()._ZN3hat9qkv_scaleEdddi  # hat::qkv_scale(double, double, double, int)
+    f.restype, f.argtypes = _QkvScale, [C.c_double, C.c_double, C.c_double, C.c_int]
+    return f(bq, bk, bv, head_dim)
+
+
+@pytest.mark.parametrize("bq,bk,ok", [(10.0, 10.0, True), (1e6, 1e6, False), (1e30, 1e-30, False),
+                                      (float("inf"), 1.0, False)])
+@pytest.mark.parametrize("bv", [1e-6, 1.0, 1e5])
+def test_v_is_scaled_whatever_becomes_of_q_and_k(bq, bk, ok, bv):
+    """v feeds the split tail whichever attention runs."""
+    s = _qkv_scale(bq, bk, bv, 24)
+    assert s.ok == ok and (ok or s.q == s.k == 1.0)
+    assert 2.0 ** 14 <= bv * s.v <= 2.0 ** 15
+
+
+def _no_pair(q_w, q_b, k_w, k_b):
+    """q and k bounded past 2^30 together, scores unchanged: two dims of the first head
+    with 1e6 on one side and zeros on the other."""
+    q_b[0], k_w[0], k_b[0] = 1e6, 0.0, 0.0
+    k_b[1], q_w[1], q_b[1] = 1e6, 0.0, 0.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [144, 180])
+@pytest.mark.parametrize("vs", [1e-6, 1.0, 1e7])
+def test_ocab_behind_the_fp32_attention(c, vs):
+    import hat_amd as hl
+    import oracle
+    rng = np.random.default_rng(41)
+
+    def n(std, *s):
+        return (rng.standard_normal(s) * std).astype(np.float32)
+    h, w = 32, 48
+    x = n(1.0, h * w, c)
+    ws = [n(0.05, *s) for s in [(c,), (c,), (3 * c, c), (3 * c,), (c, c), (c,), (1521, HEADS), (c,), (c,),
+                                (2 * c, c), (2 * c,), (c, 2 * c), (c,)]]
+    ws[0] += 1.0
+    ws[7] += 1.0
+    _no_pair(ws[2][:c], ws[3][:c], ws[2][c:2 * c], ws[3][c:2 * c])
+    # v times vs, the projection over vs: the block's output stays
+    ws[2][2 * c:] *= np.float32(vs)
+    ws[3][2 * c:] *= np.float32(vs)
+    ws[4] /= np.float32(vs)
+    print(f"ocab {c} channels, v times {vs}", flush=True)
+    got = hl.op_ocab(x, h, w, c, HEADS, 2, ws)[0]
+    assert np.isfinite(got).all()
+    assert np.abs(got - oracle.ocab_op(x, h, w, c, HEADS, 2, ws)).max() < OP_TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("net", ["hat-s", "hat"])
+@pytest.mark.parametrize("vs", [1e-6, 1.0, 1e7])
+def test_hab_behind_the_fp32_attention(weights_dir, net, vs):
+    """The same in a HAB, whose FP32 attention also computes the channel gate."""
+    import hat_amd as hl
+    import oracle
+    c = 144 if net == "hat-s" else 180
+
+    def edit(meta, t):
+        for b in (0, 1):
+            p = f"layers.0.residual_group.blocks.{b}.attn."
+            qw, qb = t[p + "qkv.weight"], t[p + "qkv.bias"]
+            _no_pair(qw[:c], qb[:c], qw[c:2 * c], qb[c:2 * c])
+            qw[2 * c:] *= np.float32(vs)
+            qb[2 * c:] *= np.float32(vs)
+            t[p + "proj.weight"] *= np.float32(4.0 / vs)
+    path = edited(make_weights(weights_dir, net, 4, 7, [2]), weights_dir / f"{net}_nopair_{vs}.safetensors", edit)
+    be, om = hl.Backend(hl.Weights(path)), oracle.OracleModel(path)
+    x = np.random.default_rng(42).standard_normal((32 * 48, c), dtype=np.float32)
+    for block in (0, 1):
+        print(f"hab {net} block {block}, v times {vs}", flush=True)
+        got = be.hab(0, block, 32, 48, x)[0]
+        assert np.isfinite(got).all()
+        assert np.abs(got - om.hab(x, 32, 48, 0, block)).max() < OP_TOL
+    be.close()
