@@ -430,7 +430,10 @@ TailPack pack_tail(const float* wp, const float* w1, const float* b1, const floa
         pack_tail_mlp(w1, b1, w2, C, 1.0f, 1.0f, 1.0f, &p.wm, &p.b1x, false);
         return p;
     }
-    float sp = f16_scale(abs_max(wp, (size_t)C * C));
+    // Both sums start from x, times their scale: at most 2^60, so that weights that
+    // have all but vanished do not take an x of 256 past fp32 (two scales of 2^60)
+    const float most = std::ldexp(1.0f, 60);
+    float sp = std::min(f16_scale(abs_max(wp, (size_t)C * C)), most / sv);
     if (cab) {
         // the projection and the gated conv2 add into the same accumulators, so
         // ts gs = sv sp: each of the two as far from its limit as the other, and
@@ -449,7 +452,8 @@ TailPack pack_tail(const float* wp, const float* w1, const float* b1, const floa
     p.w = pack_tail_proj(wp, C, sp);
     // |gelu(v)| <= |v|, and fc1 reads a norm's output
     t.hs = f16_scale(ln_linear_bound(w1, b1, n2w, n2b, 0, 2 * C, C));
-    const float s1 = f16_scale(abs_max(w1, (size_t)2 * C * C)), s2 = f16_scale(abs_max(w2, (size_t)2 * C * C));
+    const float s1 = f16_scale(abs_max(w1, (size_t)2 * C * C)),
+                s2 = std::min(f16_scale(abs_max(w2, (size_t)2 * C * C)), most / t.hs);
     t.h1 = t.hs / (sn * s1);
     t.ms = t.hs * s2;
     pack_tail_mlp(w1, b1, w2, C, s1, s2, t.hs, &p.wm, &p.b1x);

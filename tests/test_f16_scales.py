@@ -120,3 +120,29 @@ def test_swmsa_small_tokens_beside_an_outlier(c, outlier):
     rest[:16, :16] = False
     d = np.abs(got - want)[rest.ravel()].max() / np.abs(want[rest.ravel()]).max()
     assert d < 2e-6, f"worst |diff| over the largest: {d:.3e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [144, 180])
+@pytest.mark.parametrize("dead", ["attention", "mlp"])
+def test_ocab_with_a_dead_branch(c, dead):
+    """A branch whose weights have all but vanished adds nothing to a block input of any
+    size: its scales, which the input shares in the sums, stay clear of overflow."""
+    import hat_amd as hl
+    import oracle
+    rng = np.random.default_rng(44)
+
+    def n(std, *s):
+        return (rng.standard_normal(s) * std).astype(np.float32)
+    h, w = 16, 32
+    x = n(1000.0, h * w, c)
+    ws = [n(0.05, *s) for s in [(c,), (c,), (3 * c, c), (3 * c,), (c, c), (c,), (1521, HEADS), (c,), (c,),
+                                (2 * c, c), (2 * c,), (c, 2 * c), (c,)]]
+    ws[0] += 1.0
+    ws[7] += 1.0
+    for i in (2, 3, 4) if dead == "attention" else (9, 10, 11):
+        ws[i] *= np.float32(1e-18)
+    print(f"ocab {c} channels, dead {dead}", flush=True)
+    got = hl.op_ocab(x, h, w, c, HEADS, 2, ws)[0]
+    assert np.isfinite(got).all()
+    assert np.abs(got - oracle.ocab_op(x, h, w, c, HEADS, 2, ws)).max() < 1000 * OP_TOL
