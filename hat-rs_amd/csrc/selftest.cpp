@@ -148,6 +148,16 @@ std::vector<double> attn_twin(const std::vector<float>& qkv, const std::vector<f
     return out;
 }
 
+// The magnitude that a kernel left in a slot (kargs.h AMAX_SLOTS) against the largest
+// of `plane`, which the kernel's own result is close to by tol.
+void check_slot(const std::string& name, const Dev& slot, const std::vector<double>& plane, double tol)
+{
+    double big = 0.0;
+    for (double v : plane) big = std::max(big, std::fabs(v));
+    const std::vector<float> lanes = slot.get();
+    check_close(name + " output maximum", {*std::max_element(lanes.begin(), lanes.end())}, {big}, tol);
+}
+
 double gelu_d(double v) { return 0.5 * v * (1.0 + std::erf(v / std::sqrt(2.0))); }
 
 }  // namespace
@@ -450,10 +460,13 @@ int gpu_selftest(std::string* err)
                 f.res = dx.p;
                 f.out = dx.p;
                 f.xn = hab ? dxn.p : nullptr;
+                Dev slot(std::vector<float>(AMAX_WORDS, 0.0f));
+                f.amax_out = hab ? nullptr : (unsigned*)slot.p;
                 const std::string k = std::string(hab ? "hat_habx180_hab_ln" : "hat_habx180") + (small ? "_s" : "");
                 launch(s, k.c_str(), (unsigned)wx_tiles(M, small ? WX_ROWS_S : WX_ROWS), 1, 1, WX_THREADS, f);
                 check_close(k, dx.get(), want, 5e-5);
                 if (hab) check_close(k + " next norm", dxn.get(), wxn, 5e-5);
+                else check_slot(k, slot, want, 5e-5);
                 note(k + " (split-f16 C 180 tail, M 600, in place) vs double");
             }
         }
@@ -764,8 +777,11 @@ int gpu_selftest(std::string* err)
                     xof.nw = nullptr;
                     xof.nb = nullptr;
                     xof.M = Mo;
+                    Dev slot(std::vector<float>(AMAX_WORDS, 0.0f));
+                    xof.amax_out = (unsigned*)slot.p;
                     launch(s, ("hat_habx" + sfx).c_str(), (unsigned)wx_tiles(Mo, rows), 1, 1, WX_THREADS, xof);
                     check_close("hat_habx" + sfx, dout_of.get(), wo, 2e-5);
+                    check_slot("hat_habx" + sfx, slot, std::vector<double>(wo.begin(), wo.begin() + (size_t)Mo * C), 2e-5);
                     note("hat_habx" + sfx + " (split-f16 OCAB tail, partial tile) vs the two-kernel path");
                 }
             }
@@ -823,6 +839,8 @@ int gpu_selftest(std::string* err)
                 p.wu = (const unsigned short*)dwu.p;
                 p.uinv = uinv;
                 p.vs = 4096.0f;  // |V| <= 4 max|x| <= 4
+                Dev slot(std::vector<float>(AMAX_WORDS, 0.0f));
+                if (c.wino) p.amax_out = (unsigned*)slot.p;
                 if (c.wino) launch_wino(s, c.k, (W / 16) * (H / 8), c.small ? convwino_small("hat_convwino_resid").ncb : 1, p);
                 else launch(s, c.k, (W / 16) * (H / 16), 1, 1, c.waves * 64, p);  // convw and conv_first: 16 x 16
                 std::vector<double> want((size_t)HW * CO), wxn((size_t)HW * CO);
@@ -848,6 +866,7 @@ int gpu_selftest(std::string* err)
                             wxn[o + co] = (want[o + co] - mean) / std::sqrt(var + 1e-5) * nw[co] + nb[co];
                     }
                 check_close(c.k, dres.get(), want, 5e-5);
+                if (c.wino) check_slot(c.k, slot, want, 5e-5);
                 if (c.epi != EPI_RESID) check_close(std::string(c.k) + " layernorm", dxn.get(), wxn, 5e-5);
                 note(std::string(c.k) + " " + std::to_string(c.CI) + "->" + std::to_string(CO) + ", 32x48");
             }
@@ -1034,11 +1053,11 @@ int gpu_selftest(std::string* err)
                     p.wu = (const unsigned short*)dwu.p;
                     // V's scale from the input's largest magnitude, and the output's
                     // left for the next conv
-                    Dev dmax(std::vector<float>(2 * AMAX_WORDS, 0.0f));
+                    Dev dmax(std::vector<float>(AMAX_WORDS, 0.0f)), slot(std::vector<float>(AMAX_WORDS, 0.0f));
                     AbsMaxArgs am{p.in, (unsigned*)dmax.p, (long)H * W * p.cin_stride};
                     launch(s, "hat_absmax", 3, 1, 1, 256, am);
                     p.amax = (const unsigned*)dmax.p;
-                    p.amax_out = (unsigned*)dmax.p + AMAX_WORDS;
+                    p.amax_out = (unsigned*)slot.p;
                     // the persistent kernels over 5 ncb blocks (2 or 3 of the 12 tiles
                     // each, the next tile's patch fetched under an epilogue)
                     launch_wino(s, k.name.c_str(), (W / 16) * (H / 8), k.ncb, p, 5 * k.ncb);
@@ -1046,12 +1065,12 @@ int gpu_selftest(std::string* err)
                     p.amax = nullptr;
                     p.amax_out = nullptr;
                     check_close(k.name + " " + cc.what, dout4.get(), want, 5e-5);
-                    if (cc.epi != CEPI_COLSUM && cc.act == 0) {
-                        double big = 0.0;
-                        for (double v : want) big = std::max(big, std::fabs(v));
-                        const std::vector<float> lanes = dmax.get();
-                        const float got = *std::max_element(lanes.begin() + AMAX_WORDS, lanes.end());
-                        check_close(k.name + " output maximum", {got}, {big}, 5e-5);
+                    if (cc.epi != CEPI_COLSUM && cc.act != 1) {
+                        // LeakyReLU: what it was given, which bounds what it left
+                        std::vector<double> pre(want);
+                        if (cc.act == 2)
+                            for (double& v : pre) v = v < 0 ? v * 100.0 : v;
+                        check_slot(k.name, slot, pre, 5e-5);
                     }
                     if (cc.epi == CEPI_COLSUM) {
                         // one partial row per 8x16 tile

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from checkpoint_edit import edited
-from conftest import OP_TOL, make_weights
+from conftest import FWD_MEAN_TOL, FWD_TOL, OP_TOL, make_weights
 
 HEADS = 6
 
@@ -146,3 +146,78 @@ def test_ocab_with_a_dead_branch(c, dead):
     got = hl.op_ocab(x, h, w, c, HEADS, 2, ws)[0]
     assert np.isfinite(got).all()
     assert np.abs(got - oracle.ocab_op(x, h, w, c, HEADS, 2, ws)).max() < 1000 * OP_TOL
+
+
+def _planes_times(s):
+    """An edit that takes the trunk's and the head's planes to s times their size and
+    the image back: every branch that adds to them, conv_first and the head's biases
+    times s, conv_last over s."""
+    def edit(meta, t):
+        f = np.float32(s)
+        for k in t:
+            branch = k.endswith((".proj.weight", ".proj.bias", ".fc2.weight", ".fc2.bias", ".cab.2.weight", ".cab.2.bias"))
+            norm = k.startswith("patch_embed.norm.")
+            trunk = k.startswith(("conv_first.", "conv_after_body."))
+            bias = k.endswith(".bias") and (k.startswith(("conv_before_upsample.", "upsample."))
+                                            or k.startswith("layers.") and k.endswith(".conv.bias"))
+            if branch or norm or trunk or bias:
+                t[k] *= f
+        t["conv_last.weight"] /= f
+    return edit
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("net", ["hat-s", "hat"])
+@pytest.mark.parametrize("s", [1e-5, 1e5])
+def test_planes_far_from_one(weights_dir, net, s):
+    """The Winograd convs find their inputs' range on the device."""
+    import hat_amd as hl
+    import oracle
+    path = edited(make_weights(weights_dir, net, 4, 7, [2, 2]), weights_dir / f"{net}_times_{s}.safetensors", _planes_times(s))
+    be, om = hl.Backend(hl.Weights(path)), oracle.OracleModel(path)
+    for h, w in [(32, 48), (70, 100)]:
+        img = np.random.default_rng(45).random((3, h, w), dtype=np.float32)
+        print(f"forward {net} {h}x{w}, planes times {s}", flush=True)
+        d = np.abs(be.forward(h, w, img) - om.forward(h, w, img))
+        assert d.max() < FWD_TOL and d.mean() < FWD_MEAN_TOL
+    be.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("net,scale", [("hat-s", 4), ("hat", 2)])
+def test_no_range_is_kept_from_the_pass_before(weights_dir, net, scale):
+    """After an image of 1e6, one of the usual size comes out as on a new backend,
+    bit for bit."""
+    import hat_amd as hl
+    W = hl.Weights(make_weights(weights_dir, net, scale, 7, [2, 2]))
+    img = np.random.default_rng(46).random((3, 40, 56), dtype=np.float32)
+    be = hl.Backend(W)
+    want = be.forward(40, 56, img)
+    be.close()
+    be = hl.Backend(W)
+    assert np.isfinite(be.forward(40, 56, img * np.float32(1e6))).all()
+    assert np.array_equal(be.forward(40, 56, img), want)
+    be.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cab", [1e-6, 1e3, 1e8])
+def test_folded_conv2_beside_the_projection(weights_dir, cab):
+    """The folded conv2 and the projection share the tail's accumulators: conv2's
+    weights far below the projection's, and far above, where the projection's are
+    scaled down to make room."""
+    import hat_amd as hl
+    import oracle
+
+    def edit(meta, t):
+        for k in t:
+            if k.endswith(".cab.2.weight"):
+                t[k] *= np.float32(cab)
+    path = edited(make_weights(weights_dir, "hat-s", 4, 7, [2]), weights_dir / f"cab_{cab}.safetensors", edit)
+    be, om = hl.Backend(hl.Weights(path)), oracle.OracleModel(path)
+    x = np.random.default_rng(47).standard_normal((32 * 48, 144), dtype=np.float32)
+    for block in (0, 1):
+        print(f"hab block {block}, conv2 times {cab}", flush=True)
+        want = om.hab(x, 32, 48, 0, block)
+        assert np.abs(be.hab(0, block, 32, 48, x)[0] - want).max() < OP_TOL * max(1.0, np.abs(want).max())
+    be.close()
