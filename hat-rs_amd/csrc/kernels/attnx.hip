@@ -16,6 +16,11 @@
 // took 21 MFMAs and ~120. HAT-S 512 x 512 (1024 windows, 6 heads): SW 252.6 ->
 // 178.2 us a launch, OCA 574 -> 383; HAT 512 x 512 OCA 664 -> 458; head_dim 30
 // SW as whole items (two planes fit two blocks a CU; the bf16 planes did not).
+// Those are scores near 0, where the softmax needs no maximum; by the online softmax,
+// where attnx_flat says so, 512 x 512, q . k of 3 units or a table around -3 (base 0
+// tried first, then all again: 333, 374; 634 to 769, 498 to 899): SW 225, 272; OCA
+// 460, 530. Launches where both forms stand, 512 x 512: 197 and 211 us, OCA 396 and
+// 422 (head_dim 24), 250 and 259, 470 and 490 (30).
 // Parts of 288 keys for OCA at head_dim 24 spilled 34 registers (446 us), parts
 // of 192 at 30 27 of them (154 us at 256 x 256 against 122).
 //
@@ -182,13 +187,45 @@ struct AttnxKRows {
     }
 };
 
+// e = exp2(s) for a lane's 16 scores of its item's first 32 keys (in log2 units, the
+// shift mask left out), and whether the base-0 pass is likely to stand
+// (attnx_item_done): no score so large that a later one is likely to reach 2^16, and
+// a share of the denominator that makes 96 of 256 keys. The pass is checked at its end whatever
+// this says; what it decides is that scores of a wider spread, as trained networks
+// have them, go to the SAFE form at once instead of after a whole base-0 pass. A
+// limit of 12 let through waves that met 2^16 later (q . k of 3 units at head_dim
+// 24: 244 us against 228). Wave-uniform.
+__device__ __forceinline__ bool attnx_flat(const f32x16& s, float (&e)[16])
+{
+    float mx = s[0], sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        e[i] = fast_exp2(s[i]);
+        mx = fmaxf(mx, s[i]);
+        sum += e[i];
+    }
+    return __all(sum >= 6.0f && mx <= 10.0f);
+}
+
+// The same from the largest score alone (of 16 keys, one of 576 / 18 for the same
+// denominator; low: whether to ask for that): the OCA kernels have no registers for
+// the probabilities.
+__device__ __forceinline__ bool attnx_flat(const f32x16& s, bool low)
+{
+    float mx = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    return __all(mx <= 10.0f && (!low || mx >= -1.0f));
+}
+
 // O^T (with the softmax denominator in row D) of the lane's query over the
 // item's 256 keys. SAFE: the online softmax (the running base raised when a
 // score exceeds it by more than 8, in log2 units), as the reference subtracts
 // the row maximum (cpu.rs:801-812). Otherwise the base is 0: P = exp2(s)
 // straight from the scores, no maximum, no subtraction, no rescaling (16 VALU
 // a tile fewer); the caller checks the result and runs the SAFE form instead
-// when a sum could have overflowed or lost its range (see attnx_item_done).
+// when a sum could have overflowed or lost its range (see attnx_item_done), or
+// when the first tile says so (attnx_flat: zeros are returned, which fail the check).
 // Either way o / o[row D] is the softmax-weighted sum, the same quantity.
 template <int D, bool MASKED, bool SAFE>
 __device__ __forceinline__ f32x16 attnx_tiles(const AttnArgs& p, const unsigned char* lds, int wi,
@@ -237,10 +274,19 @@ __device__ __forceinline__ f32x16 attnx_tiles(const AttnArgs& p, const unsigned 
             const int key0 = kt * 32 + (i >> 2) * 8 + (i & 3);
             const int ky = key0 >> 4, kx = key0 & 15;
             float b = Tb[sw_rbase + (ky * 31 + kx)];
-            if (MASKED) b += madd[(ky >> 3) & 1][(kx >> 3) & 1];
+            if (MASKED && (SAFE || kt > 0)) b += madd[(ky >> 3) & 1][(kx >> 3) & 1];
             s[i] = b;
         }
         s = kr.qk(kt * 32 * X::KS, qb, s);
+        float e[16];
+        if (!SAFE && kt == 0) {
+            if (!attnx_flat(s, e)) return o;
+            if (MASKED) {
+                // key rows 0 and 1; a masked probability is 2^-132 at most, 0 in f16
+#pragma unroll
+                for (int i = 0; i < 16; ++i) e[i] = madd[0][(i >> 2) & 1] == 0.0f ? e[i] : 0.0f;
+            }
+        }
         if constexpr (SAFE) {
             float mx = -INFINITY;
 #pragma unroll
@@ -260,7 +306,9 @@ __device__ __forceinline__ f32x16 attnx_tiles(const AttnArgs& p, const unsigned 
         for (int st = 0; st < 2; ++st) {
             float pv[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pv[j] = fast_exp2(SAFE ? s[8 * st + j] - (mrun - ATTNX_SAFE_UP) : s[8 * st + j]);
+            for (int j = 0; j < 8; ++j)
+                pv[j] = !SAFE && kt == 0 ? e[8 * st + j]
+                                         : fast_exp2(SAFE ? s[8 * st + j] - (mrun - ATTNX_SAFE_UP) : s[8 * st + j]);
             u32x4 pb[2], va[2];
             split2_x8(pv, pb);
 #pragma unroll
@@ -272,12 +320,12 @@ __device__ __forceinline__ f32x16 attnx_tiles(const AttnArgs& p, const unsigned 
 }
 
 // Whether an item's base-0 pass (attnx_tiles with SAFE false) may stand, for
-// every query of the wave: the denominator within [32, 65504] and every
-// accumulator finite. The upper end means that no probability left f16's range
-// (they are positive, and one that did is infinite, as is then the sum). The
-// lower end bounds what the subnormal parts of the probabilities lose: up to
-// 2^-25 of each of at most 576, under 1e-8 of the denominator. A window of 256
-// scores around 0 has denominator 256; with the row maximum subtracted
+// every query of the wave: the denominator at least 32 and every accumulator
+// finite. A probability that left f16's range is infinite, and with it the sum: a
+// finite one means that none did. The lower end bounds what the subnormal parts of
+// the probabilities lose, up to 2^-25 of each of at most 576: 5.4e-7 of the
+// denominator were all of them to fall the same way, 1e-8 as roundings do. A window
+// of 256 scores around 0 has denominator 256; with the row maximum subtracted
 // (ATTNX_SAFE_UP above it) it lies in [2^6, 576 * 2^14]. Wave-uniform.
 template <int D>
 __device__ __forceinline__ bool attnx_item_done(const f32x16& o)
@@ -285,7 +333,7 @@ __device__ __forceinline__ bool attnx_item_done(const f32x16& o)
     constexpr int RH = (D % 8) / 4, RR = (D / 8) * 4 + D % 4;
     const int ql = threadIdx.x & 31;
     const float ltot = __shfl(o[RR], ql + 32 * RH, 64);
-    bool ok = ltot >= 32.0f && ltot <= 65504.0f;
+    bool ok = ltot >= 32.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) ok = ok && __builtin_isfinite(o[i]);
     return __all(ok);
@@ -375,10 +423,10 @@ __device__ __forceinline__ void attnx_item_kernel(const AttnArgs& p, unsigned ch
 // ---------------------------------------------------------------------------
 // OCA (overlapping cross-attention: 576 keys of the 24x24 unfold with padding
 // 4, zero outside the plane, biased and unmasked; hat_arch.py:373-427,
-// cpu.rs:852-900), one (window, head) item per block. The three-plane K and
-// V^T of 576 keys would need 177 KB of LDS, so an item runs as parts of NK
-// keys (D = 24: three of 192, key rows 0-7, 8-15, 16-23; D = 30: six of 96)
-// that share the online softmax; each part is split into LDS between two
+// cpu.rs:852-900), one (window, head) item per block. The two planes of K and
+// V^T of 576 keys and the table would need 120 KB of LDS (D = 30: 171), so an item
+// runs as parts of NK keys (D = 24: three of 192, key rows 0-7, 8-15, 16-23; D = 30:
+// six of 96) that share the softmax; each part is split into LDS between two
 // barriers and computed, and the next part's fetch into registers is issued
 // before the computing, so that its latency runs under this part's tiles. At
 // most 80 KB of LDS and 128 VGPRs, so that two blocks share a CU and one's
@@ -464,10 +512,36 @@ __device__ __forceinline__ void attnx_oca_stash(unsigned short* Kp, unsigned sho
     }
 }
 
-// One part's key tiles onto the running (o, mrun) of the item; SAFE as in
-// attnx_tiles (without it the base stays 0 and mrun is not used).
+// Whether the scores of one 32-key tile of part 0 are attnx_flat.
+template <int D, int NK>
+__device__ __forceinline__ bool attnx_oca_ask(const unsigned char* lds, int kt, const u32x4 (&qb)[2][2])
+{
+    using X = AttnXOcaShape<D, NK>;
+    const unsigned short* Kp = (const unsigned short*)lds;
+    const float* Tb = (const float*)(Kp + 2 * X::KPL + 2 * X::VPL);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // the addresses are not to be kept for the tiles
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in a scalar register
+    const int ql = lane & 31, h = lane >> 5, q = wave * 32 + ql;
+    AttnxKRows<D, X::KS, X::KPL> kr;
+    kr.init(Kp, ql, h);
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int key = kt * 32 + (i >> 2) * 8 + (i & 3) + 4 * h;
+        s[i] = Tb[600 - ((q >> 4) * 39 + (q & 15)) + key + 15 * (int)((unsigned)key / 24u)];
+    }
+    return attnx_flat(kr.qk(kt * 32 * X::KS, qb, s), true);
+}
+
+// One part's key tiles onto the running (o, mrun) of the item; SAFE as in attnx_tiles
+// (without it the base stays 0 and mrun is not used). False: not SAFE, and the part's
+// first tile was not attnx_flat (the item's first is asked on the low side too);
+// nothing was done. A later part's first tile can turn a wave to SAFE in the middle
+// of the item: base 0 is a maximum of ATTNX_SAFE_UP.
 template <int D, int NK, bool SAFE>
-__device__ __forceinline__ void attnx_oca_compute(const unsigned char* lds, int part, const u32x4 (&qb)[2][2],
+__device__ __forceinline__ bool attnx_oca_compute(const unsigned char* lds, int part, const u32x4 (&qb)[2][2],
                                                   f32x16& o, float& mrun)
 {
     using X = AttnXOcaShape<D, NK>;
@@ -495,11 +569,14 @@ __device__ __forceinline__ void attnx_oca_compute(const unsigned char* lds, int 
             s[i] = Tb[oca_base + key + 15 * ky];
         }
         s = kr.qk(kt * 32 * X::KS, qb, s);
+        if (!SAFE && kt == 0 && !attnx_flat(s, part == 0)) return false;
         if constexpr (SAFE) {
             float mx = -INFINITY;
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-            if ((part == 0 && kt == 0) || __any(mx > mrun + 8.0f)) {  // wave-uniform
+            if (part == 0 && kt == 0) {
+                mrun = fmaxf(mx, __shfl_xor(mx, 32, 64));  // o is zero
+            } else if (__any(mx > mrun + 8.0f)) {  // wave-uniform
                 mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
                 const float mnew = fmaxf(mrun, mx);
                 const float corr = fast_exp2(mrun - mnew);
@@ -520,6 +597,7 @@ __device__ __forceinline__ void attnx_oca_compute(const unsigned char* lds, int 
             o = mfma3(va, pb, o);
         }
     }
+    return true;
 }
 
 template <int D, int NK>
@@ -559,17 +637,26 @@ __device__ __forceinline__ void attnx_oca_kernel(const AttnArgs& p, unsigned cha
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[i] = 0.0f;
     float mrun = 0.0f;
-    // the base-0 pass (see attnx_tiles)
+    bool safe = false;  // this wave's form (attnx_flat)
 #pragma unroll 1
     for (int part = 0; part < X::NPART; ++part) {
         if (part > 0) __syncthreads();  // every read of the previous part's K and V is done
         attnx_oca_stash<D, NK>(Kp, Vp, ks, vs);
         __syncthreads();
+        // In the plane's top windows part 0's first four rows of keys are padding,
+        // which says nothing about the others: at head_dim 24, where a part has eight,
+        // its first tile with others is asked as well (here, where the registers of
+        // the next part's fetch are still free).
+        if (NK > 4 * 24 && part == 0 && wi < p.nx) safe = !attnx_oca_ask<D, NK>(lds, 3, qb);
         // the next part's K and V in flight while this part's tiles run (the
         // registers are free once stashed; same-box with the bf16 split: OCA head_dim
         // 30 677 -> 661 us, head_dim 24 589 -> 585)
         if (part + 1 < X::NPART) attnx_oca_fetch<D, NK>(p, wi, head, part + 1, ks, vs);
-        attnx_oca_compute<D, NK, false>(lds, part, qb, o, mrun);
+        if (!safe) {
+            safe = !attnx_oca_compute<D, NK, false>(lds, part, qb, o, mrun);
+            mrun = ATTNX_SAFE_UP;  // what base 0 is as a maximum
+        }
+        if (safe) attnx_oca_compute<D, NK, true>(lds, part, qb, o, mrun);
     }
     // The parts are staged by the whole block, so the block redoes the item
     // with the max-subtracted softmax if any of its waves needs it.
@@ -583,7 +670,6 @@ __device__ __forceinline__ void attnx_oca_kernel(const AttnArgs& p, unsigned cha
     if (!all_ok) {  // block-uniform
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[i] = 0.0f;
-        mrun = -INFINITY;
 #pragma unroll 1
         for (int part = 0; part < X::NPART; ++part) {
             attnx_oca_fetch<D, NK>(p, wi, head, part, ks, vs);

@@ -23,9 +23,9 @@ __device__ __forceinline__ f32x16 mfma32(float a, float b, f32x16 c)
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-// ---- split-bf16 arithmetic (the BF16 MFMA path at fp32 accuracy): an fp32
-// operand as three bf16 parts, a product as the six terms of order <= 2
-// (attnx.hip states the accuracy).
+// ---- split-bf16 arithmetic (the BF16 MFMA path at fp32 accuracy, conv_last's): an
+// fp32 operand as three bf16 parts, a product as the six terms of order <= 2; what
+// is dropped is below 2^-24 of the product.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
