@@ -609,27 +609,20 @@ void run_gemm(hipStream_t s, const DevLinear& L, const float* a, int lda, long M
            256, p);
 }
 
-// The MLP of one block: x_out = res + fc2(gelu(fc1(a))), for EPI_RESID_LN also
-// xn = LayerNorm(x_out). One fused kernel for C = 144 (hidden 288) and
-// C = 180 (hidden 360), else fc1 and fc2 as two GEMMs through the hidden buffer.
-// The fused MLP kernels: C = 144 (hidden 288) and C = 180 (hidden 360). Other
-// shapes run fc1 and fc2 as two GEMMs through a T x hidden buffer.
-bool mlp_c144(const DevLinear& fc1, const DevLinear& fc2)
+// The MLP of one block that runs no split tail: x_out = res + fc2(gelu(fc1(a))),
+// for EPI_RESID_LN also xn = LayerNorm(x_out). One fused kernel for C = 144
+// (hidden 288) with the norm, else fc1 and fc2 as two GEMMs through a T x hidden
+// buffer.
+bool mlp_fused(const DevLinear& fc1, const DevLinear& fc2, int epi)
 {
-    return fc1.K == 144 && fc1.Kp == 144 && fc1.N == 288 && fc2.K == 288 && fc2.N == 144;
+    return epi == EPI_RESID_LN && fc1.K == 144 && fc1.Kp == 144 && fc1.N == 288 && fc2.K == 288 && fc2.N == 144;
 }
-bool mlp_c180(const DevLinear& fc1, const DevLinear& fc2)
-{
-    return fc1.K == 180 && fc1.Kp == 192 && fc1.N == 360 && fc2.K == 360 && fc2.N == 180;
-}
-bool mlp_fused(const DevLinear& fc1, const DevLinear& fc2) { return mlp_c144(fc1, fc2) || mlp_c180(fc1, fc2); }
 
 void run_mlp(hipStream_t s, const DevLinear& fc1, const DevLinear& fc2, const float* a, long M,
              const float* res, float* out, int epi, const GemmEpilogue& ln, float* hidden)
 {
     if (epi != EPI_RESID && epi != EPI_RESID_LN) throw Error("MLP: bad epilogue");
-    const bool c144 = mlp_c144(fc1, fc2);
-    if (mlp_fused(fc1, fc2)) {
+    if (mlp_fused(fc1, fc2, epi)) {
         if (M > 0x7fffffffL) throw Error("MLP: too many rows");
         if (!fc1.w || !fc2.w) throw Error("MLP: the FP32 weights were not uploaded");
         MlpArgs p{};
@@ -645,19 +638,14 @@ void run_mlp(hipStream_t s, const DevLinear& fc1, const DevLinear& fc2, const fl
         p.nb = ln.nb;
         p.M = (int)M;
         p.eps = 1e-5f;
-        p.K = fc1.K;
-        p.H = fc1.N;
-        p.N = fc2.N;
         p.ldw1 = fc1.Kp;
         p.ldw2 = fc2.Kp;
-        // One block per CU (113 or 151 KB of LDS), persistent over the 128-row tiles.
+        // One block per CU (113 KB of LDS), persistent over the 128-row tiles.
         static const int cus = std::max(1, Runtime::get().cu_count());
         const long ntiles = (M + MLP_ROWS - 1) / MLP_ROWS;
         const long rounds = (ntiles + cus - 1) / cus;
         const long g = std::max(1L, (ntiles + rounds - 1) / rounds);
-        const char* name = epi == EPI_RESID_LN ? (c144 ? "hat_mlp_resid_ln" : "hat_mlp12_resid_ln")
-                                               : (c144 ? "hat_mlp_resid" : "hat_mlp12_resid");
-        launch(s, name, (unsigned)g, 1, 1, MLP_WAVES * 64, p);
+        launch(s, "hat_mlp_resid_ln", (unsigned)g, 1, 1, MLP_WAVES * 64, p);
         return;
     }
     if (!hidden) throw Error("MLP: the unfused form needs a hidden buffer");
@@ -667,14 +655,13 @@ void run_mlp(hipStream_t s, const DevLinear& fc1, const DevLinear& fc2, const fl
     run_gemm(s, fc2, hidden, fc1.N, M, out, fc2.N, epi, e, 0, 0, 0.f);
 }
 
-// Folded CAB, first half: t1 = gelu(conv1(xn)) with its per-tile sums, then
-// the gate and the gate-scaled conv2 weights (w2g) and combined bias (bias2 =
-// bproj + cscale * gate * b2) for the projection GEMM. With `defer`, the gate
-// is not launched: its arguments go to *defer, for the attention launch to run.
-// With `conv_defer`, nor is conv1 (for the qkv linear's launch).
+// Folded CAB, first half: t1 = gelu(conv1(xn)) with its per-tile sums; the gate's
+// arguments go to *gate, for the attention launch to run: the gate-scaled conv2
+// weights (w2gx) and combined bias (bias2 = bproj + cscale * gate * b2) of the
+// tail. With `conv_defer`, conv1 is not launched either (for the qkv linear's launch).
 void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, const float* bproj,
-             float cscale, int sq, float* t1, float* partial, float* w2g, float* bias2, float* gate,
-             unsigned short* w2gx, float ts, float gs, CabGateArgs* defer, CabConvArgs* conv_defer)
+             float cscale, int sq, float* t1, float* partial, float* bias2, float* gate_out,
+             unsigned short* w2gx, float ts, float gs, CabGateArgs* gate, CabConvArgs* conv_defer)
 {
     if (H % 16 != 0 || W % 16 != 0 || H < 16 || W < 16) throw Error("CAB: plane must be 16-aligned");
     if (sq < 1 || sq > 64) throw Error("CAB: squeeze width must be 1..64");
@@ -690,10 +677,10 @@ void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, con
     cab_scales(ts, cb.oscale, &a);
     // Persistent over the 16 x 16 output tiles, two blocks of 4 waves per CU.
     const int tiles = (H / 16) * (W / 16);
-    if (conv_defer && !defer) throw Error("CAB: the gate needs conv1's sums");
     if (conv_defer) *conv_defer = a;
     else launch(s, "hat_cab_conv1", (unsigned)std::min(tiles, 2 * cus), 1, 1, 256, a);
-    CabGateArgs g{};
+    CabGateArgs& g = *gate;
+    g = CabGateArgs{};
     g.partial = partial;
     g.t1 = t1;
     g.tiles = tiles;
@@ -706,71 +693,13 @@ void run_cab(hipStream_t s, const DevCab& cb, const float* xn, int H, int W, con
     g.wb = cb.wb;
     g.bb = cb.bb;
     g.bproj = bproj;
-    g.w2g = w2g;
     g.bias2 = bias2;
-    g.gate = gate;
+    g.gate = gate_out;
     g.cscale = cscale;
     g.sq = sq;
     g.w2gx = w2gx;
     g.ts = ts;
     g.gs = gs;
-    if (defer) {
-        *defer = g;
-        return;
-    }
-    launch(s, "hat_cab_gate", 1, 1, 1, 1024, g);
-}
-
-// x' = res + a . proj^T + conv2-segment + bias2; out = x' + MLP(norm2(x'));
-// xn = norm_next(out). out may alias res; a, t1 and xn must not overlap out.
-// Without t1 (the OCAB): x' = res + a . proj^T + bias2 (the projection bias),
-// out = x' + MLP(norm2(x')), no xn.
-bool hab_tail_fits(const DevLinear& proj, const DevLinear& fc1, const DevLinear& fc2)
-{
-    return proj.K == HT_C && proj.Kp == HT_C && proj.N == HT_C && fc1.K == HT_C && fc1.Kp == HT_C &&
-           fc1.N == 2 * HT_C && fc2.K == 2 * HT_C && fc2.N == HT_C;
-}
-
-void run_hab_tail(hipStream_t s, const DevLinear& proj, const DevLinear& fc1, const DevLinear& fc2,
-                  const float* a, const float* res, float* out, float* xn, const float* t1, const float* w2g,
-                  const float* bias2, const float* n2w, const float* n2b, const float* nw, const float* nb,
-                  int H, int W)
-{
-    const bool cab = t1 != nullptr;
-    if (cab && (!w2g || !xn || !nw || !nb)) throw Error("HAB tail: the CAB form needs w2g and the next norm");
-    if (!hab_tail_fits(proj, fc1, fc2)) throw Error("HAB tail: needs the 144 x 144 projection and 144 -> 288 -> 144 MLP");
-    if (!proj.w || !fc1.w || !fc2.w) throw Error("HAB tail: the FP32 weights were not uploaded");
-    const long M = (long)H * W;
-    if (M > 0x7fffffffL) throw Error("HAB tail: too many rows");
-    HabTailArgs p{};
-    p.a = a;
-    p.res = res;
-    p.out = out;
-    p.xn = xn;
-    p.wp = proj.w;
-    p.w2g = w2g;
-    p.bias2 = bias2;
-    p.t1 = t1;
-    p.n2w = n2w;
-    p.n2b = n2b;
-    p.w1 = fc1.w;
-    p.b1 = fc1.b;
-    p.w2 = fc2.w;
-    p.b2 = fc2.b;
-    p.nw = nw;
-    p.nb = nb;
-    p.M = (int)M;
-    p.H = H;
-    p.W = W;
-    p.eps = 1e-5f;
-    p.ldw1 = fc1.Kp;
-    p.ldw2 = fc2.Kp;
-    // One block per CU (113 KB of LDS), persistent over the 128-row tiles.
-    static const int cus = std::max(1, Runtime::get().cu_count());
-    const long ntiles = (M + MLP_ROWS - 1) / MLP_ROWS;
-    const long rounds = (ntiles + cus - 1) / cus;
-    const long g = std::max(1L, (ntiles + rounds - 1) / rounds);
-    launch(s, cab ? "hat_hab_tail" : "hat_ocab_tail", (unsigned)g, 1, 1, MLP_WAVES * 64, p);
 }
 
 // The tail on split-f16 (tailx.hip): x' = res + a . Wp^T + bias (+ t1: the gated
@@ -1563,7 +1492,7 @@ void GpuBackend::free_plan()
     have_plan_ = false;
 }
 
-// The compress-to-6 CAB at C = 144 (HAT-S) runs folded (cab.hip + habtail.hip).
+// The compress-to-6 CAB at C = 144 (HAT-S) runs folded (cab.hip, tailx.hip).
 bool GpuBackend::cab_folded(const Weights& wt) { return wt.embed == CAB_C && wt.compressed == CAB_CC; }
 
 size_t GpuBackend::plan_bytes(const Weights& wt, int h, int w, bool host_io)
@@ -1603,7 +1532,6 @@ std::vector<std::pair<float**, size_t>> GpuBackend::layout(const Weights& wt_, c
         {&a.xn, T * C},
         {&a.t1, T * t1_stride},
         {&a.cab_part, cab_fold_ ? (size_t)(p.hp / 16) * (p.wp / 16) * CAB_NSUM * CAB_CS : 0},
-        {&a.w2g, cab_fold_ ? C * CAB_K2 : 0},
         {&a.w2gx, cab_fold_ ? (size_t)CAB_W2GX : 0},
         {&a.bias2, cab_fold_ ? C : 0},
         // (the folded CAB's are in w2gx's buffer: magnitude_slots)
@@ -1706,36 +1634,28 @@ void GpuBackend::hab(int stage, int block, float* x_in, float* x_out, const std:
     const int C = wt_.embed, H = plan_.hp, W = plan_.wp;
     if (cab_fold_) {
         // CAB, folded: conv1 + GELU here, the gate inside the attention
-        // launch (its first block), conv2 inside the tail's projection.
-        const DevLinear& proj = lin_.at(p + ".attn.proj");
-        auto tl = tail_.find(p + ".mlp");
-        const bool split = tail_runs(wt_, false);
+        // launch (a block of its own), conv2 inside the tail's projection.
+        if (!tail_runs(wt_, false)) throw Error("HAB: the folded CAB needs an MLP of twice the block's width");
+        const DevTail& tail = tail_.at(p + ".mlp");
         CabGateArgs gate{};
         CabConvArgs conv1{};
         const DevLinear& qkv = lin_.at(p + ".attn.qkv");
         const bool with = qkv_takes_cab1(qkv, wt_.heads, wt_.head_dim, H / 16 * (W / 16));  // conv1 in qkv's launch
-        run_cab(stream_, cab_.at(p), a_.xn, H, W, proj.b, wt_.conv_scale, wt_.squeezed, a_.t1, a_.cab_part,
-                split ? nullptr : a_.w2g, a_.bias2, a_.gate, (unsigned short*)a_.w2gx,
-                split ? tl->second.ts : 1.0f, split ? tl->second.gs : 1.0f, &gate, with ? &conv1 : nullptr);
+        run_cab(stream_, cab_.at(p), a_.xn, H, W, lin_.at(p + ".attn.proj").b, wt_.conv_scale, wt_.squeezed, a_.t1,
+                a_.cab_part, a_.bias2, a_.gate, (unsigned short*)a_.w2gx, tail.ts, tail.gs, &gate, with ? &conv1 : nullptr);
         GemmEpilogue e;
         e.cab = with ? &conv1 : nullptr;
         run_gemm(stream_, qkv, a_.xn, C, T, a_.qkv, 0, EPI_QKV, e, wt_.heads, wt_.head_dim, wt_.conv_scale);
         attention(p + ".attn.relative_position_bias_table", false, block % 2 == 1 ? plan_.shift : 0, &gate);
-        if (split) {
-            // proj + gated conv2 + shortcut, norm2, the MLP + next norm1
-            TailCabIn cab;
-            cab.t1 = a_.t1;
-            cab.w2gx = (const unsigned short*)a_.w2gx;
-            cab.H = H;
-            cab.W = W;
-            run_tailx(stream_, tl->second, a_.ao, x_in, x_out, a_.xn, a_.bias2, lin_.at(p + ".mlp.fc2").b,
-                      raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), raw_.at(next_norm + ".weight"),
-                      raw_.at(next_norm + ".bias"), T, cab);
-            return;
-        }
-        run_hab_tail(stream_, proj, lin_.at(p + ".mlp.fc1"), lin_.at(p + ".mlp.fc2"), a_.ao, x_in, x_out, a_.xn, a_.t1,
-                     a_.w2g, a_.bias2, raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"),
-                     raw_.at(next_norm + ".weight"), raw_.at(next_norm + ".bias"), H, W);
+        // proj + gated conv2 + shortcut, norm2, the MLP + next norm1
+        TailCabIn cab;
+        cab.t1 = a_.t1;
+        cab.w2gx = (const unsigned short*)a_.w2gx;
+        cab.H = H;
+        cab.W = W;
+        run_tailx(stream_, tail, a_.ao, x_in, x_out, a_.xn, a_.bias2, lin_.at(p + ".mlp.fc2").b,
+                  raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), raw_.at(next_norm + ".weight"),
+                  raw_.at(next_norm + ".bias"), T, cab);
         return;
     }
     // CAB: conv3x3 -> GELU -> conv3x3 (+ per-tile channel sums) -> gate; on small
@@ -1791,17 +1711,9 @@ void GpuBackend::ocab(int stage, float* x, Amax* out_max)
     gemm(lin_.at(p + ".qkv"), a_.xn, C, T, a_.qkv, 0, EPI_QKV);
     attention(p + ".relative_position_bias_table", true, 0);
     const DevLinear& proj = lin_.at(p + ".proj");
-    const DevLinear &fc1 = lin_.at(p + ".mlp.fc1"), &fc2 = lin_.at(p + ".mlp.fc2");
     if (tail_runs(wt_, true)) {
-        run_tailx(stream_, tail_.at(p + ".mlp"), a_.ao, x, x, nullptr, proj.b, fc2.b, raw_.at(p + ".norm2.weight"),
+        run_tailx(stream_, tail_.at(p + ".mlp"), a_.ao, x, x, nullptr, proj.b, lin_.at(p + ".mlp.fc2").b, raw_.at(p + ".norm2.weight"),
                   raw_.at(p + ".norm2.bias"), nullptr, nullptr, T, TailCabIn{}, out_max);
-        return;
-    }
-    if (hab_tail_fits(proj, fc1, fc2)) {
-        // projection + shortcut + norm2 + MLP + residual in one kernel
-        run_hab_tail(stream_, proj, fc1, fc2, a_.ao, x, x, nullptr, nullptr,
-                     nullptr, proj.b, raw_.at(p + ".norm2.weight"), raw_.at(p + ".norm2.bias"), nullptr, nullptr,
-                     plan_.hp, plan_.wp);
         return;
     }
     gemm(proj, a_.ao, C, T, x, C, EPI_RESID_LN, x, nullptr, nullptr, a_.xn, p + ".norm2");
@@ -2588,7 +2500,7 @@ void op_ocab(const float* x, float* out, int hp, int wp, int c, int heads, int m
         OpLinear qkv(ar, qkv_w, qkv_b, 3 * c, c, OpLinear::kQkv, osc, 1.0f / s1),
             proj(ar, proj_w, proj_b, c, c, form, nullptr, 1.0f / sc.v), fc1(ar, fc1_w, fc1_b, (int)hid, c, form),
             fc2(ar, fc2_w, fc2_b, c, (int)hid, form);
-        const size_t ih = ar.add(fits || mlp_fused(fc1.L, fc2.L) ? 1 : T * hid);
+        const size_t ih = ar.add(fits ? 1 : T * hid);
         ar.commit();
         if (tail) tail->bind(ar);
         for (OpLinear* l : {&qkv, &proj, &fc1, &fc2}) l->bind(ar);

@@ -227,7 +227,7 @@ private:
         float *x0 = nullptr, *body = nullptr, *xa = nullptr, *xb = nullptr, *xn = nullptr, *t1 = nullptr,
               *t2 = nullptr, *partial = nullptr, *red = nullptr, *gate = nullptr, *qkv = nullptr, *ao = nullptr,
               *hidden = nullptr, *head0 = nullptr, *head1 = nullptr, *din = nullptr, *dout = nullptr,
-              *cab_part = nullptr, *w2g = nullptr, *w2gx = nullptr, *bias2 = nullptr, *amax = nullptr;
+              *cab_part = nullptr, *w2gx = nullptr, *bias2 = nullptr, *amax = nullptr;
     };
     // Each buffer of plan p and its size in floats (0: not used by this
     // network); host_io adds the staging buffers of the host-memory forward.

@@ -65,11 +65,6 @@ struct GemmArgs {
     int heads, hdim;     // EPI_QKV geometry (N = 3 * heads * hdim)
     float cscale;        // EPI_HAB* conv scale
     float eps;           // LayerNorm eps
-    // hat_gemmws_cab_ln only: the CAB's second conv as an extra K segment,
-    // A = 3x3 neighbourhood of t1 on the H x W plane, W = w2g [144][CAB_K2].
-    const float* t1;     // [H*W][CAB_CS]
-    const float* w2g;    // [N][CAB_K2]
-    int H, W;
     // hat_gemmx_qkv*: what takes the operands' scales out of q, k and v (the
     // bias is in the result's scale already)
     float oscale[3];
@@ -81,14 +76,14 @@ struct GemmArgs {
 #define CAB_C 144
 #define CAB_CC 6             // compressed channels
 #define CAB_CS 8             // t1 channel stride (channels 6, 7 are zero)
-#define CAB_K2 56            // 9 taps x 6 channels (k = tap*6 + ci), 2 zero: 3 x 16 + 8
 // conv1's weights split for hat_cab_conv1: per 16-channel step ks (9), row
 // tile nt (2 x 32 rows, row tap*6 + co, rows 54.. zero) and part (2), the
 // 32x32x16 A operand of each lane (row l % 32, channels 16 ks + 8 (l / 32) .. +7)
 #define CX_WPACK (9 * 2 * 2 * 64 * 8)
 // floats of the gated conv2 weights' buffer: CabGateArgs::w2gx, then the forward's
-// magnitude slots (AMAX_SLOTS)
-#define CAB_W2GX 20480
+// magnitude slots (AMAX_SLOTS); the rest is spare, which keeps a plan's size, and with
+// it the tile that a memory budget picks, what they have been
+#define CAB_W2GX 28544
 #define CAB_W2GX_USED (2 * CAB_C * 32)
 #define CAB_NSUM 5           // per-tile sums: whole tile, row 0, row H-1, col 0, col W-1
 
@@ -115,12 +110,12 @@ struct CabGateArgs {
     const float* wb;     // excite [144][sq]
     const float* bb;     // [144]
     const float* bproj;  // attention projection bias [144]
-    float* w2g;          // out (if set): cscale * gate[c] * conv2 weight / ts, [144][CAB_K2] (k = tap*6 + ci)
     float* bias2;        // out: bproj + cscale * gate * b2, [144]
     float* gate;         // out: the gate itself [144]
     float cscale;
     int sq;
-    unsigned short* w2gx;  // out (if set): w2g * gs as the split tail's two steps, [2][144][32] each (ws_slot)
+    unsigned short* w2gx;  // out: cscale * gate[c] * conv2 weight * gs as the split tail's two steps
+                           // (k = tap*6 + ci), [2][144][32] each (ws_slot)
     float ts, gs;        // t1's scale; w2gx's scale (powers of two)
 };
 
@@ -199,8 +194,7 @@ struct AttnArgs {
     int owin, opad;      // OCA: unfold window and padding
     int T;
     float qscale;        // head_dim^-0.5 * log2(e)
-    // with_gate: the launch also computes the folded CAB's gate (hat_cab_gate's
-    // work), which the HAB tail after it needs: the split-f16 SW kernels in a
+    // with_gate: the launch also computes the folded CAB's gate (cab.hip), which the HAB tail after it needs: the split-f16 SW kernels in a
     // block of its own (the grid has one more column, the first), the FP32 ones
     // in block (0, 0) before its item
     int with_gate;
@@ -210,54 +204,25 @@ struct AttnArgs {
     SeArgs se;
 };
 
-// Fused MLP (C = 144, hidden 288; C = 180, hidden 360):
-//   out[m][:] = res[m][:] + fc2(gelu(fc1(a[m][:])))   (+ xn = LayerNorm(out) for EPI_RESID_LN)
+// Fused MLP (C = 144, hidden 288):
+//   out[m][:] = res[m][:] + fc2(gelu(fc1(a[m][:]))),  xn = LayerNorm(out)
 #define MLP_WAVES 8
 #define MLP_ROWS (MLP_WAVES * 16)
 
 struct MlpArgs {
-    const float* a;      // [M][K]
-    const float* w1;     // [H][ldw1] (K used)
-    const float* b1;     // [H]
-    const float* w2;     // [N][ldw2] (H used)
-    const float* b2;     // [N]
-    const float* res;    // [M][N] (may alias out)
-    float* out;          // [M][N]
-    float* xn;           // EPI_RESID_LN: [M][N] (may alias a)
+    const float* a;      // [M][144]
+    const float* w1;     // [288][ldw1]
+    const float* b1;     // [288]
+    const float* w2;     // [144][ldw2]
+    const float* b2;     // [144]
+    const float* res;    // [M][144] (may alias out)
+    float* out;          // [M][144]
+    float* xn;           // [M][144] (may alias a)
     const float* nw;
     const float* nb;
     int M;
     float eps;
-    int K, H, N;         // input width (= N), hidden width, output width
     int ldw1, ldw2;      // packed weight row strides
-};
-
-// The fused block tails' width.
-#define HT_C 144
-
-// The second half of a HAB, C = 144 with the folded CAB (hat_hab_tail):
-//   x' = res + a . wp^T + nb(t1) . w2g^T + bias2,  out = x' + fc2(gelu(fc1(LN2(x')))),
-//   xn = LN_next(out).
-struct HabTailArgs {
-    const float* a;      // [M][144] attention output
-    const float* res;    // [M][144] block input
-    float* out;          // [M][144] (may alias res)
-    float* xn;           // [M][144] LN_next(out)
-    const float* wp;     // [144][144] attention projection (packed, Kp = 144)
-    const float* w2g;    // [144][CAB_K2] gate-scaled conv2 weights
-    const float* bias2;  // [144] projection bias + gated conv2 bias
-    const float* t1;     // [H*W][CAB_CS] CAB conv1 output
-    const float* n2w;    // norm2
-    const float* n2b;
-    const float* w1;     // [288][ldw1]
-    const float* b1;
-    const float* w2;     // [144][ldw2]
-    const float* b2;
-    const float* nw;     // the next block's norm1
-    const float* nb;
-    int M, H, W;         // rows = the H x W plane
-    float eps;
-    int ldw1, ldw2;
 };
 
 // The HAB / OCAB tails on split-f16 MFMA (tailx.hip). Their weights are arrays

@@ -12,8 +12,8 @@
 //     over the tile and over its pixels on the four border lines;
 //   * gate[c] * conv2(t1)[p][c] * cscale is a GEMM of the 3x3 neighbourhood of
 //     t1 at p (9 taps x 6 channels, k = tap*6 + ci) with weights cscale *
-//     gate[c] * w2 - hat_cab_gate folds them, and the attention projection GEMM
-//     (hat_gemmws_cab_ln) runs them as 56 more K.
+//     gate[c] * w2 - the gate folds them, and the block's tail (tailx.hip) runs
+//     them as two more k-steps of the attention's projection.
 // So conv2's T x 144 output is never written or read back.
 #include "common.h"
 
@@ -232,13 +232,9 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
 }
 
 // ---------------------------------------------------------------------------
-// The gate, and conv2 folded with it: one block of 16 waves. Every reduction
-// is a fixed-order per-lane sum followed by a fixed shuffle tree, so the
-// result does not depend on timing.
-#define CG_WAVES 16
-
-// The gate computation for a block of WAVES waves; lds: CAB_GATE_LDS floats. It
-// rides on the attention launch as a block of its own (attnx.hip), so what
+// The gate, and conv2 folded with it, for a block of WAVES waves; lds: CAB_GATE_LDS
+// floats. Every reduction is a fixed-order per-lane sum followed by a fixed shuffle
+// tree, so the result does not depend on timing. It rides on the attention launch as a block of its own (attnx.hip), so what
 // counts is its latency, which small planes would wait for: conv2's weights
 // are read once, coalesced, under the tile sums' loads, and the split chunks
 // go out eight values at a time.
@@ -309,17 +305,10 @@ __device__ __forceinline__ void cab_gate_body(const CabGateArgs& p, float* lds)
         p.bias2[c] = p.bproj[c] + (p.cscale * g) * p.b2[c];
     }
     __syncthreads();
-    // the gated weights for the FP32 tail, where it runs
-    if (p.w2g)
-        for (int i = tid; i < CAB_C * CAB_K2; i += WAVES * 64) {
-            const int c = i / CAB_K2, k = i - c * CAB_K2;
-            const int tap = k / CAB_CC, ci = k - tap * CAB_CC;
-            p.w2g[i] = tap < 9 ? (p.cscale * s_gate[c]) * s_w2[(c * CAB_CC + ci) * 9 + tap] / p.ts : 0.0f;
-        }
-    // the same weights as the split tail's two weight steps: [s][plane][c][32],
-    // row c's k-group g at slot ws_slot(c, g), k = 32 s + j, zeros from k = 54;
-    // one k-group (8 values, 16 bytes a plane) at a time
-    if (p.w2gx) {
+    // cscale * gate[c] * conv2 weight as the split tail's two weight steps:
+    // [s][plane][c][32], row c's k-group g at slot ws_slot(c, g), k = tap*6 + ci =
+    // 32 s + j, zeros from k = 54; one k-group (8 values, 16 bytes a plane) at a time
+    {
         constexpr int PLANE = CAB_C * 32;
         for (int u = tid; u < 2 * CAB_C * 4; u += WAVES * 64) {
             const int s = u / (CAB_C * 4), c = (u >> 2) - s * CAB_C, g = u & 3;
@@ -383,10 +372,4 @@ __device__ __forceinline__ void se_gate_body(const SeArgs& p, float* lds)
         for (int j = 0; j < p.sq; ++j) acc += s_sq[j] * p.w2[(size_t)c * p.sq + j];
         p.gate[c] = 1.0f / (1.0f + __expf(-acc));
     }
-}
-
-extern "C" __global__ __launch_bounds__(CG_WAVES * 64) void hat_cab_gate(CabGateArgs p)
-{
-    __shared__ __attribute__((aligned(16))) float lds[CAB_GATE_LDS];
-    cab_gate_body<CG_WAVES>(p, lds);
 }

@@ -342,7 +342,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& p)
     extern "C" __global__ __launch_bounds__(256) void NAME(GemmArgs p) { gemm_body<NT, EPI>(p); }
 
 // ---------------------------------------------------------------------------
-// Weight-stationary variant for K = 144 (the C = 144 family's qkv, proj and fc1).
+// Weight-stationary variant for K = 144 and 180 (projections and fc1).
 //
 // A block holds a 144 x 144 weight slice (one column block) in LDS and loops
 // over row tiles. The work is the sequence of (column slice, row tile) units,
@@ -359,26 +359,17 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& p)
 // columns).
 // KP: the weight rows' padded K (144, or 192 for K = 180), a multiple of 48;
 // NT: 16-column tiles per block (9, or 12 for the C = 180 family).
-template <int EPI, int MT, int WAVES, bool CAB, int KP, int NT>
+template <int EPI, int MT, int WAVES, int KP, int NT>
 __device__ __forceinline__ void gemm_ws_body(const GemmArgs& p)
 {
     constexpr int ROWS = WAVES * 16 * MT;  // rows per tile
     constexpr int BN = 16 * NT, NCH = KP / 16;
     constexpr int WS_K = KP, WS_KS = KP + 4;  // LDS row stride of the weight slice
     static_assert(NCH % 3 == 0, "the K loop walks groups of three chunks");
-    static_assert(!CAB || (KP == 144 && NT == 9), "the folded CAB is the C = 144 family's");
-    constexpr int S2 = CAB_K2 + 4;         // LDS row stride of the conv2 slice
     __shared__ __attribute__((aligned(16))) float Wsm[BN * WS_KS];
-    __shared__ __attribute__((aligned(16))) float W2s[CAB ? BN * S2 : 1];
-    __shared__ int s_colmap[EPI == EPI_QKV ? BN : 1];
     constexpr bool LNOUT = EPI == EPI_RESID_LN || EPI == EPI_HAB_LN;
     // bias (+ LayerNorm weight and bias) of the block's columns
     __shared__ __attribute__((aligned(16))) float Cs[(LNOUT ? 3 : 1) * BN];
-    // q/k/v staging of the 144-column, head_dim 24 shape: per wave 16 rows x 48
-    // columns (two heads), row stride QS_S.
-    constexpr bool QSTAGE = EPI == EPI_QKV && BN == 144 && MT == 1;
-    constexpr int QS_S = 52;
-    __shared__ __attribute__((aligned(16))) float Qs[QSTAGE ? WAVES * 16 * QS_S : 1];
     // row staging of the whole-row epilogues (N = 144 in one column block)
     constexpr bool RSTAGE = (EPI == EPI_RESID || EPI == EPI_RESID_LN || EPI == EPI_HAB_LN) && BN == 144 && MT == 1;
     __shared__ __attribute__((aligned(16))) float Rs[RSTAGE ? WAVES * 8 * (BN + 4) : 1];
@@ -391,7 +382,7 @@ __device__ __forceinline__ void gemm_ws_body(const GemmArgs& p)
     const int M = p.M, N = p.N;
 
     // The weight slice of the columns from n0: BN rows x KP/4 float4, with the
-    // conv2 slice, the QKV column map and the epilogue constants.
+    // epilogue constants.
     auto load_slice = [&](int n0) {
         for (int idx = tid; idx < BN * (WS_K / 4); idx += WAVES * 64) {
             const int r = idx / (WS_K / 4), c4 = (idx - r * (WS_K / 4)) * 4;
@@ -399,15 +390,6 @@ __device__ __forceinline__ void gemm_ws_body(const GemmArgs& p)
             if (n0 + r < N) v = *(const float4*)(p.w + (size_t)(n0 + r) * p.Kp + c4);
             *(float4*)(Wsm + r * WS_KS + c4) = v;
         }
-        if (CAB) {
-            for (int idx = tid; idx < BN * (CAB_K2 / 4); idx += WAVES * 64) {
-                const int r = idx / (CAB_K2 / 4), c4 = (idx - r * (CAB_K2 / 4)) * 4;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (n0 + r < N) v = *(const float4*)(p.w2g + (size_t)(n0 + r) * CAB_K2 + c4);
-                *(float4*)(W2s + r * S2 + c4) = v;
-            }
-        }
-        build_colmap<BN, EPI>(p, n0, s_colmap);
         for (int i = tid; i < (LNOUT ? 3 : 1) * BN; i += WAVES * 64) {
             const int j = i % BN, n = n0 + j;
             const float* src = i < BN ? p.bias : (i < 2 * BN ? p.nw : p.nb);
@@ -465,36 +447,6 @@ __device__ __forceinline__ void gemm_ws_body(const GemmArgs& p)
         const float* arow_n[MT];
         bool alive_n[MT];
         rows_of(u + gridDim.x < units ? u + gridDim.x : u, arow_n, alive_n);
-        // CAB: the 3x3 neighbourhood of t1 at each row's pixel, k = tap*6 + ci
-        // (54 values, 2 zero): three 16-k chunks, lane group g holding k =
-        // 16 kc2 + 4g .. +3 (two float2 of one or two taps), and an 8-k tail,
-        // g holding k = 48 + 2g, 49 + 2g (tap 8's channels 2g, 2g+1; zero for g = 3).
-        constexpr int K2F = CAB_K2 / 16;
-        f32x4 xg[CAB ? MT : 1][K2F];
-        float2 xh[CAB ? MT : 1];
-        if (CAB) {
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const int m = mbase + mt * 16 + lr;
-                const int y = m / p.W, x = m - y * p.W;
-                // t1[neighbour at tap][ci, ci+1], zero outside the plane
-                // out-of-plane taps read zeros
-                auto pair = [&](int tap, int ci) -> float2 {
-                    const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-                    const bool ok = alive[mt] && tap < 9 && yy >= 0 && yy < p.H && xx >= 0 && xx < p.W;
-                    return *(const float2*)(ok ? p.t1 + ((size_t)yy * p.W + xx) * CAB_CS + ci : hat_zero_row);
-                };
-#pragma unroll
-                for (int kc2 = 0; kc2 < K2F; ++kc2) {
-                    const int k0 = kc2 * 16 + lg * 4, ta = k0 / CAB_CC, ca = k0 - ta * CAB_CC;  // ca: 0, 2 or 4
-                    const float2 lo = pair(ta, ca);
-                    const bool same = ca + 2 < CAB_CC;
-                    const float2 hi = pair(same ? ta : ta + 1, same ? ca + 2 : 0);
-                    xg[mt][kc2] = (f32x4){lo.x, lo.y, hi.x, hi.y};
-                }
-                xh[mt] = pair(lg < 3 ? 8 : 9, 2 * lg);
-            }
-        }
         // The residual for the epilogue, loaded now so its latency hides under
         // the K loop.
         constexpr bool PRE = EPI == EPI_RESID_LN || EPI == EPI_RESID;
@@ -551,80 +503,21 @@ __device__ __forceinline__ void gemm_ws_body(const GemmArgs& p)
             arow[mt] = arow_n[mt];
             alive[mt] = alive_n[mt];
         }
-        if (CAB) {
-#pragma unroll
-            for (int kc2 = 0; kc2 <= K2F; ++kc2) {
-                // keep each chunk's weight reads next to its MFMAs (hoisting
-                // all of them costs more registers than there are)
-                __builtin_amdgcn_sched_barrier(0);
-                if (kc2 < K2F) {
-                    const float* wrow = W2s + lr * S2 + kc2 * 16 + lg * 4;
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) {
-                        const f32x4 wv = *(const f32x4*)(wrow + nt * 16 * S2);
-#pragma unroll
-                        for (int s = 0; s < 4; ++s)
-#pragma unroll
-                            for (int mt = 0; mt < MT; ++mt)
-                                acc[mt][nt] = mfma16(wv[s], xg[mt][kc2][s], acc[mt][nt]);
-                    }
-                } else {
-                    // the 8-k tail: two MFMAs, lane group g's k = 48 + 2g + s
-                    const float* wrow = W2s + lr * S2 + K2F * 16 + lg * 2;
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) {
-                        const float2 wv = *(const float2*)(wrow + nt * 16 * S2);
-#pragma unroll
-                        for (int mt = 0; mt < MT; ++mt) {
-                            acc[mt][nt] = mfma16(wv.x, xh[mt].x, acc[mt][nt]);
-                            acc[mt][nt] = mfma16(wv.y, xh[mt].y, acc[mt][nt]);
-                        }
-                    }
-                }
-            }
-        }
-        if (QSTAGE && p.hdim == 24 && p.heads * 24 == BN) {
-            // A slice is one of q, k, v (6 heads x 24). Two heads at a time go
-            // through the wave's LDS region and leave as 16 consecutive rows of
-            // each head: 1536 contiguous bytes per head, every lane storing
-            // 16 bytes of one run, instead of 16-byte pieces 96 bytes apart.
-            // The stores are non-temporal (measured faster, for this kernel
-            // and for the attention that reads q, k, v next).
-            float* Q = Qs + wave * 16 * QS_S;
-            const int mrows = M - mbase;  // rows of this wave that exist (may exceed 16)
-#pragma unroll
-            for (int ph = 0; ph < 3; ++ph) {
-#pragma unroll
-                for (int t = 0; t < 3; ++t) *(f32x4*)(Q + lr * QS_S + t * 16 + lg * 4) = acc[0][3 * ph + t];
-                __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes are done
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    const int f = lane + 64 * i, hh = f / 96, r = (f - hh * 96) / 6, d4 = f - hh * 96 - r * 6;
-                    const f32x4 v = *(const f32x4*)(Q + r * QS_S + hh * 24 + d4 * 4);
-                    if (r < mrows) {
-                        const int head = 2 * ph + hh;
-                        __builtin_nontemporal_store(v, (f32x4*)(p.out + ((size_t)(slice * p.heads + head) * M + mbase + r) * 24 + d4 * 4));
-                    }
-                }
-                __builtin_amdgcn_s_waitcnt(0xc07f);  // reads done before the next phase's writes
-            }
-            continue;
-        }
         if constexpr (RSTAGE) {
             if (N == BN && p.ldo == BN) {
-                gemm_epilogue<MT, NT, EPI, true, true>(p, kc, acc, mbase, n0, lr, lg, s_colmap, PRE ? rres : nullptr,
+                gemm_epilogue<MT, NT, EPI, true, true>(p, kc, acc, mbase, n0, lr, lg, nullptr, PRE ? rres : nullptr,
                                                        Rs + wave * 8 * (BN + 4));
                 continue;
             }
         }
-        gemm_epilogue<MT, NT, EPI, true>(p, kc, acc, mbase, n0, lr, lg, s_colmap, PRE ? rres : nullptr);
+        gemm_epilogue<MT, NT, EPI, true>(p, kc, acc, mbase, n0, lr, lg, nullptr, PRE ? rres : nullptr);
     }
 }
 
 #define GEMM_WS_INST(NAME, EPI, KP, NT)                                                      \
     extern "C" __global__ __launch_bounds__(ws_waves(EPI) * 64) void NAME(GemmArgs p)          \
     {                                                                                          \
-        gemm_ws_body<EPI, ws_mt(EPI), ws_waves(EPI), false, KP, NT>(p);                        \
+        gemm_ws_body<EPI, ws_mt(EPI), ws_waves(EPI), KP, NT>(p);                               \
     }
 
 // NT = 9: 144-wide column blocks (HAT-S: N = 144, 288, 432 divide exactly).
@@ -642,22 +535,12 @@ GEMM_INST(hat_gemm_n12_resid, 12, EPI_RESID)
 GEMM_INST(hat_gemm_n12_resid_ln, 12, EPI_RESID_LN)
 GEMM_INST(hat_gemm_n12_hab_ln, 12, EPI_HAB_LN)
 
-// K = 144 weight-stationary instances (HAT-S: qkv N = 432, fc1 N = 288, attention
-// proj and OCAB proj N = 144).
-GEMM_WS_INST(hat_gemmws_qkv, EPI_QKV, 144, 9)
+// K = 144 weight-stationary instances: the projections (N = 144) and fc1 of the
+// blocks that run no split tail (a CAB that is not folded, another MLP ratio).
 GEMM_WS_INST(hat_gemmws_gelu, EPI_GELU, 144, 9)
 GEMM_WS_INST(hat_gemmws_resid_ln, EPI_RESID_LN, 144, 9)
 GEMM_WS_INST(hat_gemmws_hab_ln, EPI_HAB_LN, 144, 9)
-// K = 180 (padded to 192), 192-wide column blocks: the C = 180 family's qkv
-// (N = 540 in 3 blocks), fc1 (N = 360 in 2) and projections (N = 180).
-GEMM_WS_INST(hat_gemmws12_qkv, EPI_QKV, 192, 12)
+// K = 180 (padded to 192), 192-wide column blocks: the same at other MLP ratios.
 GEMM_WS_INST(hat_gemmws12_gelu, EPI_GELU, 192, 12)
 GEMM_WS_INST(hat_gemmws12_resid_ln, EPI_RESID_LN, 192, 12)
 GEMM_WS_INST(hat_gemmws12_hab_ln, EPI_HAB_LN, 192, 12)
-
-// HAB attention projection with the CAB's conv2 folded in as 56 more K (the
-// block input as residual, bias = proj bias + folded conv2 bias), then norm2.
-extern "C" __global__ __launch_bounds__(ws_waves(EPI_RESID_LN) * 64) void hat_gemmws_cab_ln(GemmArgs p)
-{
-    gemm_ws_body<EPI_RESID_LN, ws_mt(EPI_RESID_LN), ws_waves(EPI_RESID_LN), true, 144, 9>(p);
-}

@@ -9,7 +9,6 @@
 #include "gemmx.hip"
 #include "tailx.hip"
 #include "mlp.hip"
-#include "habtail.hip"
 #include "convw.hip"
 #include "convwino.hip"
 #include "misc.hip"

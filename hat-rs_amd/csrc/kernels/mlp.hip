@@ -1,5 +1,7 @@
 // Fused MLP on FP32 MFMA:
-//   out = res + fc2(gelu(fc1(a)))   and, for EPI_RESID_LN, xn = LayerNorm(out).
+//   out = res + fc2(gelu(fc1(a))),  xn = LayerNorm(out)
+// at C = 144 (hidden 288): the blocks that run no split tail (a CAB that is not
+// folded).
 //
 // Replaces the reference's two lg_linear launches of the MLP (src/cuda.rs:
 // 162-169; cpu.rs mlp, 1148-1160) with the GELU between them (cuda.rs:195-199)
@@ -22,34 +24,25 @@
 // accumulators then have the layout of the GEMM kernels' epilogue, which is
 // reused (bias, residual, LayerNorm of whole rows).
 //
-// Shapes: C = 144 (KP = 144, hidden 288, NO = 144) and C = 180 (K 180 in
-// KP = 192, hidden 360 in NH = 384, NO = 192). Padding is zero: weights past
-// the real rows / columns are not read, and GELU(0 + 0) = 0 feeds fc2 nothing.
-//
 // Included after gemm.hip (gemm_epilogue) in the one translation unit.
 
 #define MLP_HC 48  // hidden units per chunk
 #define MLP_THREADS (MLP_WAVES * 64)
 
-// The LDS slots that lie past the real weights (the padded C = 180 shape) load
-// from hat_zero_row, since a direct-to-LDS load always writes its slot.
-
 // Swizzle of float4 column c4 in LDS row `row` of a slice whose rows are R
 // float4 long: rows r..r+15 read at one c4 land in 16 distinct groups of four
 // banks (R = 36 or 12: rows 4 apart share a bank offset, the XOR separates
-// them; R = 48: all rows share one, the XOR spreads them over 16).
+// them).
 template <int R>
 __device__ __forceinline__ int mlp_swz(int row)
 {
-    static_assert(R % 16 == 0 || R % 16 == 4 || R % 16 == 12, "slice row length");
-    return R % 16 == 0 ? (row & 15) : ((row >> 2) & 3);
+    static_assert(R % 16 == 4 || R % 16 == 12, "slice row length");
+    return (row >> 2) & 3;
 }
 
-// PAD: the real K, hidden and output widths are below KP, NH, NO (C = 180);
-// without it they are exactly KP, NH, NO and nothing is masked.
-template <int EPI, int KP, int NH, int NO, bool PAD>
-__device__ __forceinline__ void mlp_body(const MlpArgs& p)
+extern "C" __global__ __launch_bounds__(MLP_THREADS) void hat_mlp_resid_ln(MlpArgs p)
 {
+    constexpr int KP = 144, NH = 288, NO = 144;  // input, hidden and output widths
     constexpr int NCH = NH / MLP_HC;             // hidden chunks
     constexpr int R1 = KP / 4;                   // float4 per fc1 slice row [48][R1]
     constexpr int R2 = MLP_HC / 4;               // float4 per fc2 slice row [NO][R2]
@@ -76,7 +69,6 @@ __device__ __forceinline__ void mlp_body(const MlpArgs& p)
     const int lr = lane & 15;
     const int lg = lane >> 4;
     const int M = p.M;
-    const int K = PAD ? p.K : KP, H = PAD ? p.H : NH, N = PAD ? p.N : NO;
     const int ntiles = (M + MLP_ROWS - 1) / MLP_ROWS;
     int tile = blockIdx.x;
     if (tile >= ntiles) return;  // whole block: no barrier has been passed yet
@@ -84,22 +76,19 @@ __device__ __forceinline__ void mlp_body(const MlpArgs& p)
     // This thread's LDS slots of a chunk, float4 idx = tid + 512 i: fc1 slice
     // slots (row = the hidden unit within the chunk) then fc2 slice slots (row =
     // output column); the lane fetches the global float4 whose swizzled column
-    // is the slot's. Without padding the global offsets (relative to the
-    // chunk's bases) are kept in registers; with it they are recomputed and
-    // slots past the real weights read hat_zero_row.
-    unsigned goff[PAD ? 1 : PER];
-    if constexpr (!PAD) {
+    // is the slot's. The global offsets (relative to the chunk's bases) are kept
+    // in registers.
+    unsigned goff[PER];
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = tid + i * MLP_THREADS;
-            if (idx < W1F4) {
-                const int r = idx / R1, c4 = (idx - r * R1) ^ mlp_swz<R1>(r);
-                goff[i] = r * p.ldw1 + c4 * 4;  // + chunk * 48 fc1 rows
-            } else {
-                const int j = idx - W1F4;
-                const int r = j / R2, c4 = (j - r * R2) ^ mlp_swz<R2>(r);
-                goff[i] = r * p.ldw2 + c4 * 4;  // + chunk * 48 fc2 columns
-            }
+    for (int i = 0; i < PER; ++i) {
+        const int idx = tid + i * MLP_THREADS;
+        if (idx < W1F4) {
+            const int r = idx / R1, c4 = (idx - r * R1) ^ mlp_swz<R1>(r);
+            goff[i] = r * p.ldw1 + c4 * 4;  // + chunk * 48 fc1 rows
+        } else {
+            const int j = idx - W1F4;
+            const int r = j / R2, c4 = (j - r * R2) ^ mlp_swz<R2>(r);
+            goff[i] = r * p.ldw2 + c4 * 4;  // + chunk * 48 fc2 columns
         }
     }
     // Chunk c's slices into LDS buffer buf. The LDS side of each load is the
@@ -114,54 +103,24 @@ __device__ __forceinline__ void mlp_body(const MlpArgs& p)
         for (int i = 0; i < PER; ++i) {
             const int base = i * MLP_THREADS + wave * 64;  // wave-uniform
             if (base >= F4) break;
-            int idx = base + lane;
-            // (with padding) an index the compiler cannot see through, so the
-            // per-slot addresses are recomputed here instead of hoisted out of
-            // the loops and kept, 64 bits each
-            if constexpr (PAD) asm volatile("" : "+v"(idx));
-            const float* src;
-            if constexpr (!PAD) {
-                src = (base < W1F4 ? w1c : w2c) + goff[i];
-            } else if (base < W1F4) {
-                const int r = idx / R1, c4 = (idx - r * R1) ^ mlp_swz<R1>(r);
-                src = h0 + r < H ? p.w1 + (size_t)(h0 + r) * p.ldw1 + c4 * 4 : hat_zero_row;
-            } else {
-                const int j = idx - W1F4;
-                const int r = j / R2, c4 = (j - r * R2) ^ mlp_swz<R2>(r);
-                src = r < N && h0 + c4 * 4 < H ? p.w2 + (size_t)r * p.ldw2 + h0 + c4 * 4 : hat_zero_row;
-            }
+            const float* src = (base < W1F4 ? w1c : w2c) + goff[i];
             __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)(B + base * 4),
                                              16, 0, 0);
         }
     };
-    // The residual is loaded a chunk ahead of the epilogue where the registers
-    // allow it (the 144-wide shape).
-    constexpr bool PRE = NO <= 144;
-    constexpr int RN = PRE ? NO / 16 : 1;
+    constexpr int RN = NO / 16;
 
     f32x4 xa[KP / 16];
     auto load_a = [&](int t) {
         const int m = t * MLP_ROWS + wave * 16 + lr;
-        const float* arow = m < M ? p.a + (size_t)m * K + lg * 4 : hat_zero_row;  // + kc*16 stays in it
+        const float* arow = m < M ? p.a + (size_t)m * KP + lg * 4 : hat_zero_row;  // + kc*16 stays in it
 #pragma unroll
-        for (int kc = 0; kc < KP / 16; ++kc) {
-            // k beyond K (180 in 192) reads as zero: past it lies the next row
-            xa[kc] = load_or_zero(arow + kc * 16, !PAD || kc * 16 + lg * 4 < K);
-        }
+        for (int kc = 0; kc < KP / 16; ++kc) xa[kc] = *(const f32x4*)(arow + kc * 16);
     };
 
     for (int i = tid; i < NH + 3 * NO; i += MLP_THREADS) {
-        float v = 0.0f;
-        if (i < NH) {
-            if (i < H) v = p.b1[i];
-        } else {
-            const int j = (i - NH) % NO, which = (i - NH) / NO;
-            if (j < N) {
-                if (which == 0) v = p.b2[j];
-                else if (EPI == EPI_RESID_LN) v = which == 1 ? p.nw[j] : p.nb[j];
-            }
-        }
-        Cs[i] = v;
+        const int j = (i - NH) % NO, which = (i - NH) / NO;
+        Cs[i] = i < NH ? p.b1[i] : (which == 0 ? p.b2 : which == 1 ? p.nw : p.nb)[j];
     }
     GemmArgs g{};
     g.out = p.out;
@@ -169,13 +128,12 @@ __device__ __forceinline__ void mlp_body(const MlpArgs& p)
     g.xn = p.xn;
     const EpiConsts kc{Cs + NH, Cs + NH + NO, Cs + NH + 2 * NO};
     g.M = M;
-    g.N = N;
-    g.ldo = N;
+    g.N = NO;
+    g.ldo = NO;
     g.eps = p.eps;
 
     // The lane's swizzled float4 column in the operand reads: rows nt*16 + lr
     // and n2*16 + lr give (row >> 2) & 3 == (lr >> 2) & 3 and row & 15 == lr.
-    static_assert(R2 % 16 != 0, "the fc2 slice's swizzle is the 2-bit one");
     const int sg = lg ^ mlp_swz<R1>(lr), sg2 = lg ^ mlp_swz<R2>(lr);
     fetch(0, CInt<0>{});
     load_a(tile);
@@ -195,15 +153,11 @@ __device__ __forceinline__ void mlp_body(const MlpArgs& p)
             // the other buffer was last read in the previous chunk, before its barrier
             if (more) fetch(c + 1 < NCH ? c + 1 : 0, CInt<Q ^ 1>{});
             // The residual rows for the epilogue, one chunk ahead of it.
-            if constexpr (PRE) {
-                if (c == NCH - 1) {
-                    const int m = tile * MLP_ROWS + wave * 16 + lr;
-                    const float* rrow = m < M ? p.res + (size_t)m * N + lg * 4 : hat_zero_row;
+            if (c == NCH - 1) {
+                const int m = tile * MLP_ROWS + wave * 16 + lr;
+                const float* rrow = m < M ? p.res + (size_t)m * NO + lg * 4 : hat_zero_row;
 #pragma unroll
-                    for (int n2 = 0; n2 < RN; ++n2) {
-                        rres[0][n2] = load_or_zero(rrow + n2 * 16, n2 * 16 + lg * 4 < N);
-                    }
-                }
+                for (int n2 = 0; n2 < RN; ++n2) rres[0][n2] = *(const f32x4*)(rrow + n2 * 16);
             }
 
             // fc1 for this chunk: h[16 rows][48] = b1 + a . w1[chunk]^T, the
@@ -215,9 +169,9 @@ __device__ __forceinline__ void mlp_body(const MlpArgs& p)
 #pragma unroll
             for (int kc = 0; kc < KP / 16; ++kc) {
                 __builtin_amdgcn_sched_barrier(0);
-                // physical column: (kc*4 + lg) ^ swizzle, which for R1 % 16 != 0
-                // (a 2-bit swizzle) is kc*4 + (lg ^ swizzle)
-                const int pc = R1 % 16 == 0 ? ((kc * 4 + lg) ^ lr) : kc * 4 + sg;
+                // physical column: (kc*4 + lg) ^ swizzle = kc*4 + (lg ^ swizzle), the
+                // swizzle being of two bits
+                const int pc = kc * 4 + sg;
                 f32x4 wv[MLP_HC / 16];
 #pragma unroll
                 for (int nt = 0; nt < MLP_HC / 16; ++nt) wv[nt] = *(const f32x4*)(B + (nt * 16 + lr) * KP + pc * 4);
@@ -258,20 +212,6 @@ __device__ __forceinline__ void mlp_body(const MlpArgs& p)
             chunk(c, CInt<0>{});
             chunk(c + 1, CInt<1>{});
         }
-        if constexpr (PRE)
-            gemm_epilogue<1, NO / 16, EPI>(g, kc, acc2, tile * MLP_ROWS + wave * 16, 0, lr, lg, nullptr, rres);
-        else
-            gemm_epilogue<1, NO / 16, EPI>(g, kc, acc2, tile * MLP_ROWS + wave * 16, 0, lr, lg, nullptr);
+        gemm_epilogue<1, NO / 16, EPI_RESID_LN>(g, kc, acc2, tile * MLP_ROWS + wave * 16, 0, lr, lg, nullptr, rres);
     }
 }
-
-#define MLP_INST(NAME, EPI, KP, NH, NO, PAD)                                                 \
-    extern "C" __global__ __launch_bounds__(MLP_THREADS) void NAME(MlpArgs p)                \
-    {                                                                                        \
-        mlp_body<EPI, KP, NH, NO, PAD>(p);                                                   \
-    }
-
-MLP_INST(hat_mlp_resid, EPI_RESID, 144, 288, 144, false)
-MLP_INST(hat_mlp_resid_ln, EPI_RESID_LN, 144, 288, 144, false)
-MLP_INST(hat_mlp12_resid, EPI_RESID, 192, 384, 192, true)
-MLP_INST(hat_mlp12_resid_ln, EPI_RESID_LN, 192, 384, 192, true)

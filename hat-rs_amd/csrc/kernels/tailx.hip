@@ -13,7 +13,7 @@
 //
 // ao is the attention output, nb(t1) the 3x3 neighbourhood of the folded CAB's
 // conv1 output (k = tap*6 + ci, 54 values) and W2g / bias the gate-scaled conv2
-// weights and combined bias written by the gate (hat_cab_gate's work); aux is
+// weights and combined bias written by the gate (cab.hip); aux is
 // the unfolded CAB's conv2 output. Products are the three-term split-f16 ones of
 // common.h on v_mfma_f32_16x16x32_f16, weights as the A operand, tokens as B; a
 // lane's four accumulators are four consecutive output channels of one token.

@@ -231,7 +231,7 @@ int gpu_selftest(std::string* err)
         // a block walks several tiles.
         auto gemm_case = [&](int C, int epi, bool ws) {
                 const int heads = 6, hd = C / heads;
-                const int M = ws ? 600 : 200;  // not a multiple of the row tile
+                const int M = ws || epi == EPI_QKV ? 600 : 200;  // not a multiple of the row tile
                 const int N = epi == EPI_QKV ? 3 * C : (epi == EPI_GELU ? 2 * C : C);
                 const int K = epi == EPI_RESID ? 2 * C : C;  // RESID at the fc2 shape
                 const bool lnout = epi == EPI_RESID_LN || epi == EPI_HAB_LN;
@@ -268,11 +268,9 @@ int gpu_selftest(std::string* err)
                 const int BN = n9 ? 144 : 192;
                 std::string k;
                 if (ws) {
-                    const int wbn = C == 144 ? 144 : 192;
                     k = std::string(C == 144 ? "hat_gemmws_" : "hat_gemmws12_") + enames[epi];
-                    // 2 blocks: with 3 column slices each block's units
+                    // 2 blocks: with several column slices each block's units
                     // cross from slice to slice
-                    (void)wbn;
                     launch(s, k.c_str(), 2, 1, 1, ws_waves(epi) * 64, p);
                 } else {
                     k = std::string(n9 ? "hat_gemm_n9_" : "hat_gemm_n12_") + enames[epi];
@@ -307,7 +305,7 @@ int gpu_selftest(std::string* err)
                 check_close(k + " C " + std::to_string(C), dout.get(), want, 3e-5);
                 if (lnout) check_close(k + " C " + std::to_string(C) + " layernorm", dxn.get(), wxn, 5e-5);
                 note(k + " C " + std::to_string(C) + " M " + std::to_string(M) + " K " + std::to_string(K));
-                if (ws && epi == EPI_QKV) {
+                if (!ws && epi == EPI_QKV) {
                     // the split-f16 form on the same inputs (the last
                     // subtile partial: 600 rows are 18.75 subtiles of 32),
                     // one group: its 8 waves walk them all; the weights scaled into f16's range
@@ -328,15 +326,13 @@ int gpu_selftest(std::string* err)
         for (int C : {144, 180})
             for (int epi : epis) gemm_case(C, epi, false);
         for (int C : {144, 180})
-            for (int epi : {EPI_QKV, EPI_GELU, EPI_RESID_LN, EPI_HAB_LN}) gemm_case(C, epi, true);
+            for (int epi : {EPI_GELU, EPI_RESID_LN, EPI_HAB_LN}) gemm_case(C, epi, true);
 
-        // ---- fused MLP (C = 144, hidden 288; C = 180, hidden 360 padded to
-        // 384), in place as the backend runs it: out aliases the residual, the
-        // LayerNorm output aliases the input. 600 rows = 5 tiles of 128 (the
-        // last partial) over 2 blocks.
-        for (int C : {144, 180})
-        for (int epi : {EPI_RESID, EPI_RESID_LN}) {
-            const int M = 600, H = 2 * C;
+        // ---- fused MLP (C = 144, hidden 288), in place as the backend runs it: out
+        // aliases the residual, the LayerNorm output aliases the input. 600 rows = 5
+        // tiles of 128 (the last partial) over 2 blocks.
+        {
+            const int C = 144, M = 600, H = 2 * C;
             std::vector<float> a = rng.vec((size_t)M * C, 1.0f), w1 = rng.vec((size_t)H * C, 0.08f),
                                b1 = rng.vec(H, 0.1f), w2 = rng.vec((size_t)C * H, 0.06f), b2 = rng.vec(C, 0.1f),
                                res = rng.vec((size_t)M * C, 1.0f), nw = rng.vec(C, 1.0f), nb = rng.vec(C, 0.1f);
@@ -351,18 +347,14 @@ int gpu_selftest(std::string* err)
             p.b2 = db2.p;
             p.res = dx.p;
             p.out = dx.p;
-            p.xn = epi == EPI_RESID_LN ? da.p : nullptr;
+            p.xn = da.p;
             p.nw = dnw.p;
             p.nb = dnb.p;
             p.M = M;
             p.eps = 1e-5f;
-            p.K = C;
-            p.H = H;
-            p.N = C;
             p.ldw1 = K1;
             p.ldw2 = K2;
-            const char* k = epi == EPI_RESID_LN ? (C == 144 ? "hat_mlp_resid_ln" : "hat_mlp12_resid_ln")
-                                                : (C == 144 ? "hat_mlp_resid" : "hat_mlp12_resid");
+            const char* k = "hat_mlp_resid_ln";
             launch(s, k, 2, 1, 1, MLP_WAVES * 64, p);
             std::vector<double> want((size_t)M * C), wxn((size_t)M * C), hid(H);
             for (int m = 0; m < M; ++m) {
@@ -385,7 +377,7 @@ int gpu_selftest(std::string* err)
                     wxn[(size_t)m * C + n] = (want[(size_t)m * C + n] - mean) / std::sqrt(var + 1e-5) * nw[n] + nb[n];
             }
             check_close(std::string(k), dx.get(), want, 5e-5);
-            if (epi == EPI_RESID_LN) check_close(std::string(k) + " layernorm", da.get(), wxn, 5e-5);
+            check_close(std::string(k) + " layernorm", da.get(), wxn, 5e-5);
             note(std::string(k) + " C " + std::to_string(C) + " M 600 (in place)");
         }
 
@@ -486,13 +478,10 @@ int gpu_selftest(std::string* err)
                                bp = rng.vec(C, 0.1f), res = rng.vec((size_t)T * C, 1.0f),
                                nw = rng.vec(C, 1.0f), nb = rng.vec(C, 0.1f);
             std::vector<unsigned short> w1p = pack_cab_conv1(w1.data(), 1 << 16);
-            int Kp = 0;
-            std::vector<float> wpp = pack_linear(wp.data(), C, C, &Kp);
             const int tiles = (H / 16) * (W / 16);
             Dev dxn(xn), dw1(w1p.size() / 2), db1(b1), dw2(w2), db2(b2), dwa(wa), dba(ba), dwb(wb), dbb(bb), dao(ao),
-                dwp(wpp), dbp(bp), dres(res), dnw(nw), dnb(nb), dt1((size_t)T * CAB_CS),
-                dpart((size_t)tiles * CAB_NSUM * CAB_CS), dw2g((size_t)C * CAB_K2), dw2gx(2 * C * 32), dbias2(C), dgate(C),
-                dout((size_t)T * C), dxo((size_t)T * C);
+                dbp(bp), dnw(nw), dnb(nb), dt1((size_t)T * CAB_CS), dpart((size_t)tiles * CAB_NSUM * CAB_CS),
+                dw2gx(2 * C * 32), dbias2(C), dgate(C);
             Runtime::get().h2d(dw1.p, w1p.data(), w1p.size() * sizeof(unsigned short));
             CabConvArgs ca{dxn.p, (const unsigned short*)dw1.p, db1.p, dt1.p, dpart.p, H, W, 0, 0, 0, 0};
             cab_scales(1.0f, 1.0f / (1 << 16), &ca);
@@ -510,7 +499,6 @@ int gpu_selftest(std::string* err)
             ga.wb = dwb.p;
             ga.bb = dbb.p;
             ga.bproj = dbp.p;
-            ga.w2g = dw2g.p;
             ga.bias2 = dbias2.p;
             ga.gate = dgate.p;
             ga.cscale = cscale;
@@ -518,28 +506,30 @@ int gpu_selftest(std::string* err)
             ga.w2gx = (unsigned short*)dw2gx.p;
             ga.ts = 1.0f;
             ga.gs = 1.0f;
-            launch(s, "hat_cab_gate", 1, 1, 1, 1024, ga);
-            GemmArgs gp{};
-            gp.a = dao.p;
-            gp.w = dwp.p;
-            gp.bias = dbias2.p;
-            gp.out = dout.p;
-            gp.res = dres.p;
-            gp.xn = dxo.p;
-            gp.nw = dnw.p;
-            gp.nb = dnb.p;
-            gp.M = T;
-            gp.N = C;
-            gp.K = C;
-            gp.Kp = Kp;
-            gp.lda = C;
-            gp.ldo = C;
-            gp.eps = 1e-5f;
-            gp.t1 = dt1.p;
-            gp.w2g = dw2g.p;
-            gp.H = H;
-            gp.W = W;
-            launch(s, "hat_gemmws_cab_ln", 3, 1, 1, ws_waves(EPI_RESID_LN) * 64, gp);
+            // The gate rides on an attention launch: as a column of blocks of its own
+            // beside the split-f16 kernel's items, before the first of the FP32 one's.
+            auto launch_gate = [&](const std::string& k) {
+                const int D = 24, heads = 6, TA = 256;
+                Dev dq(rng.vec((size_t)3 * TA * heads * D, 1.0f)), dtab(rng.vec((size_t)961 * heads, 0.5f)),
+                    dat((size_t)TA * heads * D);
+                AttnArgs p{};
+                p.qkv = dq.p;
+                p.table = dtab.p;
+                p.out = dat.p;
+                p.hp = p.wp = 16;
+                p.nx = p.ny = 1;
+                p.heads = heads;
+                p.D = D;
+                p.C = heads * D;
+                p.owin = 24;
+                p.opad = 4;
+                p.T = TA;
+                p.qscale = (float)(1.0 / std::sqrt((double)D) * 1.4426950408889634);
+                p.with_gate = 1;
+                p.gate = ga;
+                launch(s, k.c_str(), k == "hat_attnx_sw_d24" ? 2 : 1, heads, 1, 512, p);
+                rt.sync();
+            };
 
             auto inb = [&](int y, int x) { return y >= 0 && y < H && x >= 0 && x < W; };
             std::vector<double> t1((size_t)T * CAB_CS, 0.0), y2((size_t)T * C);
@@ -569,7 +559,7 @@ int gpu_selftest(std::string* err)
                         y2[((size_t)y * W + x) * C + c] = v;
                         mean2[c] += v / T;
                     }
-            std::vector<double> z(sq), gate(C), bias2(C), w2g((size_t)C * CAB_K2, 0.0);
+            std::vector<double> z(sq), gate(C), bias2(C);
             for (int j = 0; j < sq; ++j) {
                 double v = ba[j];
                 for (int c = 0; c < C; ++c) v += (double)wa[(size_t)j * C + c] * mean2[c];
@@ -580,133 +570,61 @@ int gpu_selftest(std::string* err)
                 for (int j = 0; j < sq; ++j) v += (double)wb[(size_t)c * sq + j] * z[j];
                 gate[c] = 1.0 / (1.0 + std::exp(-v));
                 bias2[c] = bp[c] + cscale * gate[c] * b2[c];
-                for (int tap = 0; tap < 9; ++tap)
-                    for (int ci = 0; ci < CC; ++ci)
-                        w2g[(size_t)c * CAB_K2 + tap * CAB_CC + ci] = cscale * gate[c] * w2[((size_t)c * CC + ci) * 9 + tap];
             }
-            std::vector<double> want((size_t)T * C), wxn((size_t)T * C);
-            for (int m = 0; m < T; ++m) {
-                double mean = 0, var = 0;
+            // x' of the OCAB's tail (no CAB) and of the HAB's
+            std::vector<double> xo((size_t)T * C), xh((size_t)T * C);
+            for (int m = 0; m < T; ++m)
                 for (int c = 0; c < C; ++c) {
+                    const size_t i = (size_t)m * C + c;
                     double v = bp[c];
                     for (int k = 0; k < C; ++k) v += (double)ao[(size_t)m * C + k] * wp[(size_t)c * C + k];
-                    v = res[(size_t)m * C + c] + v + y2[(size_t)m * C + c] * gate[c] * cscale;
-                    want[(size_t)m * C + c] = v;
-                    mean += v / C;
+                    xo[i] = res[i] + v;
+                    xh[i] = xo[i] + y2[i] * gate[c] * cscale;
                 }
-                for (int c = 0; c < C; ++c) var += (want[(size_t)m * C + c] - mean) * (want[(size_t)m * C + c] - mean) / C;
-                for (int c = 0; c < C; ++c)
-                    wxn[(size_t)m * C + c] = (want[(size_t)m * C + c] - mean) / std::sqrt(var + 1e-5) * nw[c] + nb[c];
-            }
             check_close("hat_cab_conv1 t1", dt1.get(), t1, 2e-5);
             note("hat_cab_conv1 144->6 + gelu, 32x48");
-            check_close("hat_cab_gate gate", dgate.get(), gate, 2e-6);
-            check_close("hat_cab_gate bias2", dbias2.get(), bias2, 2e-6);
-            check_close("hat_cab_gate w2g", dw2g.get(), w2g, 1e-7);
-            note("hat_cab_gate (mean by linearity) vs conv2 in full");
-            check_close("hat_gemmws_cab_ln", dout.get(), want, 5e-5);
-            check_close("hat_gemmws_cab_ln layernorm", dxo.get(), wxn, 5e-5);
-            note("hat_gemmws_cab_ln proj + folded conv2 + norm2");
+            for (const char* k : {"hat_attn_sw_d24", "hat_attnx_sw_d24"}) {
+                launch_gate(k);
+                check_close(std::string(k) + " gate", dgate.get(), gate, 2e-6);
+                check_close(std::string(k) + " gate's bias2", dbias2.get(), bias2, 2e-6);
+                note(std::string(k) + "'s gate (mean by linearity) vs conv2 in full");
+            }
 
-            // The fused HAB tail against hat_gemmws_cab_ln followed by the fused
-            // MLP (both checked above against double precision) on the same
-            // inputs: out = x' + MLP(norm2(x')), xn = norm_next(out).
             {
                 const int Hd = 2 * C;
                 std::vector<float> f1 = rng.vec((size_t)Hd * C, 0.05f), fb1 = rng.vec(Hd, 0.1f),
                                    f2 = rng.vec((size_t)C * Hd, 0.05f), fb2 = rng.vec(C, 0.1f),
                                    mw = rng.vec(C, 1.0f), mb = rng.vec(C, 0.1f);
-                int K1 = 0, K2 = 0;
-                std::vector<float> f1p = pack_linear(f1.data(), Hd, C, &K1), f2p = pack_linear(f2.data(), C, Hd, &K2);
-                Dev df1(f1p), dfb1(fb1), df2(f2p), dfb2(fb2), dmw(mw), dmb(mb), dxn_ref((size_t)T * C),
-                    dout_t(res), dxn_t((size_t)T * C);
-                MlpArgs mp{};
-                mp.a = dxo.p;  // norm2(x') from hat_gemmws_cab_ln
-                mp.w1 = df1.p;
-                mp.b1 = dfb1.p;
-                mp.w2 = df2.p;
-                mp.b2 = dfb2.p;
-                mp.res = dout.p;  // x', updated in place
-                mp.out = dout.p;
-                mp.xn = dxn_ref.p;
-                mp.nw = dmw.p;
-                mp.nb = dmb.p;
-                mp.M = T;
-                mp.eps = 1e-5f;
-                mp.K = C;
-                mp.H = Hd;
-                mp.N = C;
-                mp.ldw1 = K1;
-                mp.ldw2 = K2;
-                launch(s, "hat_mlp_resid_ln", 2, 1, 1, MLP_WAVES * 64, mp);
-                HabTailArgs tp{};
-                tp.a = dao.p;
-                tp.res = dout_t.p;  // in place over the block input, as in the forward
-                tp.out = dout_t.p;
-                tp.xn = dxn_t.p;
-                tp.wp = dwp.p;
-                tp.w2g = dw2g.p;
-                tp.bias2 = dbias2.p;
-                tp.t1 = dt1.p;
-                tp.n2w = dnw.p;
-                tp.n2b = dnb.p;
-                tp.w1 = df1.p;
-                tp.b1 = dfb1.p;
-                tp.w2 = df2.p;
-                tp.b2 = dfb2.p;
-                tp.nw = dmw.p;
-                tp.nb = dmb.p;
-                tp.M = T;
-                tp.H = H;
-                tp.W = W;
-                tp.eps = 1e-5f;
-                tp.ldw1 = K1;
-                tp.ldw2 = K2;
-                launch(s, "hat_hab_tail", 5, 1, 1, MLP_WAVES * 64, tp);  // 12 tiles: blocks walk 2 or 3
-                const std::vector<float> ro = dout.get(), rx = dxn_ref.get();
-                check_close("hat_hab_tail", dout_t.get(), std::vector<double>(ro.begin(), ro.end()), 2e-5);
-                check_close("hat_hab_tail next norm", dxn_t.get(), std::vector<double>(rx.begin(), rx.end()), 2e-5);
-                note("hat_hab_tail (proj + folded conv2 + norm2 + MLP + norm) vs the two-kernel path");
-
-                // The OCAB's tail: hat_gemmws_resid_ln (proj + bias + shortcut +
-                // norm2) then hat_mlp_resid, against hat_ocab_tail.
-                Dev dref2(res), dxn2((size_t)T * C), dout_o(res);
-                GemmArgs op{};
-                op.a = dao.p;
-                op.w = dwp.p;
-                op.bias = dbp.p;
-                op.out = dref2.p;
-                op.res = dref2.p;
-                op.xn = dxn2.p;
-                op.nw = dnw.p;
-                op.nb = dnb.p;
-                op.M = T;
-                op.N = C;
-                op.K = C;
-                op.Kp = Kp;
-                op.lda = C;
-                op.ldo = C;
-                op.eps = 1e-5f;
-                launch(s, "hat_gemmws_resid_ln", 3, 1, 1, ws_waves(EPI_RESID_LN) * 64, op);
-                MlpArgs mo = mp;
-                mo.a = dxn2.p;
-                mo.res = dref2.p;
-                mo.out = dref2.p;
-                mo.xn = nullptr;
-                launch(s, "hat_mlp_resid", 2, 1, 1, MLP_WAVES * 64, mo);
-                HabTailArgs to = tp;
-                to.res = dout_o.p;
-                to.out = dout_o.p;
-                to.xn = nullptr;
-                to.t1 = nullptr;
-                to.w2g = nullptr;
-                to.bias2 = dbp.p;
-                to.nw = nullptr;
-                to.nb = nullptr;
-                launch(s, "hat_ocab_tail", 5, 1, 1, MLP_WAVES * 64, to);
-                const std::vector<float> r2 = dref2.get();
-                check_close("hat_ocab_tail", dout_o.get(), std::vector<double>(r2.begin(), r2.end()), 2e-5);
-                note("hat_ocab_tail (proj + norm2 + MLP) vs the two-kernel path");
+                Dev dfb2(fb2), dmw(mw), dmb(mb);
+                // The tails in double from x': out = x' + MLP(norm2(x')), and the next
+                // norm of it.
+                auto norm = [&](const double* v, const std::vector<float>& w, const std::vector<float>& b, double* o) {
+                    double mean = 0, var = 0;
+                    for (int c = 0; c < C; ++c) mean += v[c] / C;
+                    for (int c = 0; c < C; ++c) var += (v[c] - mean) * (v[c] - mean) / C;
+                    for (int c = 0; c < C; ++c) o[c] = (v[c] - mean) / std::sqrt(var + 1e-5) * w[c] + b[c];
+                };
+                auto tail = [&](std::vector<double> x, std::vector<double>* next) {
+                    std::vector<double> y(C), hid(Hd);
+                    next->resize(x.size());
+                    for (int m = 0; m < T; ++m) {
+                        double* v = &x[(size_t)m * C];
+                        norm(v, nw, nb, y.data());
+                        for (int j = 0; j < Hd; ++j) {
+                            double u = fb1[j];
+                            for (int c = 0; c < C; ++c) u += y[c] * f1[(size_t)j * C + c];
+                            hid[j] = gelu_d(u);
+                        }
+                        for (int n = 0; n < C; ++n) {
+                            v[n] += fb2[n];
+                            for (int j = 0; j < Hd; ++j) v[n] += hid[j] * f2[(size_t)n * Hd + j];
+                        }
+                        norm(v, mw, mb, &(*next)[(size_t)m * C]);
+                    }
+                    return x;
+                };
+                std::vector<double> rx, unused;
+                const std::vector<double> ro = tail(xh, &rx), r2 = tail(xo, &unused);
 
                 // The split-f16 tails (tailx.hip) on the same inputs, in place as
                 // the forward runs them (out over the block input); 12 row tiles
@@ -723,16 +641,14 @@ int gpu_selftest(std::string* err)
                 cx.partial = dpartx.p;
                 cab_scales(xt.t.ts, 1.0f / (1 << 16), &cx);
                 launch(s, "hat_cab_conv1", 2, 1, 1, 256, cx);
-                CabGateArgs gx = ga;
-                gx.partial = dpartx.p;
-                gx.t1 = dt1x.p;
-                gx.w2g = nullptr;
-                gx.bias2 = dbias2x.p;
-                gx.gate = dgatex.p;
-                gx.ts = xt.t.ts;
-                gx.gs = xt.t.gs;
-                launch(s, "hat_cab_gate", 1, 1, 1, 1024, gx);
-                check_close("hat_cab_gate gate (scaled t1)", dgatex.get(), gate, 2e-6);
+                ga.partial = dpartx.p;
+                ga.t1 = dt1x.p;
+                ga.bias2 = dbias2x.p;
+                ga.gate = dgatex.p;
+                ga.ts = xt.t.ts;
+                ga.gs = xt.t.gs;
+                launch_gate("hat_attnx_sw_d24");
+                check_close("hat_attnx_sw_d24 gate (scaled t1)", dgatex.get(), gate, 2e-6);
                 TailXArgs xf{};
                 xf.a = dao.p;
                 xf.w = (const unsigned short*)dpw.p;
@@ -754,7 +670,7 @@ int gpu_selftest(std::string* err)
                 // The OCAB form over a partial last tile: rows from Mo on stay
                 // the block input.
                 const int Mo = T - 100;
-                std::vector<double> wo(r2.begin(), r2.end());
+                std::vector<double> wo(r2);
                 for (size_t i = (size_t)Mo * C; i < wo.size(); ++i) wo[i] = res[i];
                 for (bool small : {false, true}) {
                     const std::string sfx = small ? "_s" : "";
@@ -764,9 +680,9 @@ int gpu_selftest(std::string* err)
                     xf.out = dout_f.p;
                     xf.xn = dxn_f.p;
                     launch(s, ("hat_habx_cab_ln" + sfx).c_str(), (unsigned)wx_tiles(T, rows), 1, 1, WX_THREADS, xf);
-                    check_close("hat_habx_cab_ln" + sfx, dout_f.get(), std::vector<double>(ro.begin(), ro.end()), 2e-5);
-                    check_close("hat_habx_cab_ln" + sfx + " next norm", dxn_f.get(), std::vector<double>(rx.begin(), rx.end()), 2e-5);
-                    note("hat_habx_cab_ln" + sfx + " (split-f16 proj + conv2 + MLP + norm) vs the two-kernel path");
+                    check_close("hat_habx_cab_ln" + sfx, dout_f.get(), ro, 2e-5);
+                    check_close("hat_habx_cab_ln" + sfx + " next norm", dxn_f.get(), rx, 2e-5);
+                    note("hat_habx_cab_ln" + sfx + " (split-f16 proj + conv2 + MLP + norm) vs double");
                     TailXArgs xof = xf;
                     xof.res = dout_of.p;
                     xof.out = dout_of.p;
@@ -782,7 +698,7 @@ int gpu_selftest(std::string* err)
                     launch(s, ("hat_habx" + sfx).c_str(), (unsigned)wx_tiles(Mo, rows), 1, 1, WX_THREADS, xof);
                     check_close("hat_habx" + sfx, dout_of.get(), wo, 2e-5);
                     check_slot("hat_habx" + sfx, slot, std::vector<double>(wo.begin(), wo.begin() + (size_t)Mo * C), 2e-5);
-                    note("hat_habx" + sfx + " (split-f16 OCAB tail, partial tile) vs the two-kernel path");
+                    note("hat_habx" + sfx + " (split-f16 OCAB tail, partial tile) vs double");
                 }
             }
         }
