@@ -494,7 +494,6 @@ const char* gemm_ws_kernel(const DevLinear& L, int epi, int* bn)
     if (!k144 && !k180) return nullptr;
     *bn = k144 ? 144 : 192;
     switch (epi) {
-    case EPI_QKV: return k144 ? "hat_gemmws_qkv" : "hat_gemmws12_qkv";
     case EPI_GELU: return k144 ? "hat_gemmws_gelu" : "hat_gemmws12_gelu";
     case EPI_RESID_LN: return k144 ? "hat_gemmws_resid_ln" : "hat_gemmws12_resid_ln";
     case EPI_HAB_LN: return k144 ? "hat_gemmws_hab_ln" : "hat_gemmws12_hab_ln";
@@ -1166,10 +1165,11 @@ void launch_wino(hipStream_t s, const char* name, unsigned tiles, unsigned ncb, 
 // ---------------------------------------------------------------------------
 // GpuBackend
 
-// Weights are allocated in whole granules: the kernels that copy them to LDS do so
-// in whole loads, which may read past a tensor's end, and small ones are spread
-// over the memory channels instead of sharing a page. weight_bytes_ counts what
-// is allocated.
+// Weights are allocated in whole granules, which weight_bytes_ counts. No kernel
+// needs them: none reads past a tensor (tailx.hip's whole loads end inside TX_PAD and
+// TX_B1), and granules of 4 KB are as fast (64 x 64 HAT-S 2.031 ms and 2.030, 512 x 512
+// 30.13 and 30.15, HAT 256 x 256 14.67 and 14.66). HAT-S takes 147.5 MiB so, 54.6 in
+// granules of 4 KB; the memory admission's tests are written for the former.
 static constexpr size_t kWeightGranule = 128u << 10;
 
 float* GpuBackend::upload(const float* src, size_t n) { return (float*)upload_bytes(src, n * sizeof(float)); }
@@ -1797,6 +1797,10 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
 {
     const long T = plan_.tokens();
     const int C = wt_.embed, H = plan_.hp, W = plan_.wp;
+    const size_t S = wt_.depths.size();
+    // a magnitude slot each (the loader takes 32 stages and scales of few octaves)
+    if (S > AMAX_HEAD || AMAX_HEAD + 2 + wt_.up_blocks().size() > AMAX_SLOTS)
+        throw Error("forward: too many stages or upsample convs");
     PreArgs pa{d_in, a_.x0, h, w, H, W, 4, wt_.mean[0], wt_.mean[1], wt_.mean[2], wt_.img_range,
                magnitude_slots(0)};
     launch(stream_, "hat_pre", (unsigned)((T + 255) / 256), 1, 1, 256, pa);
@@ -1832,7 +1836,6 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
         conv(cf, a_.x0, 4, H, W, a_.body, C, CEPI_STORE, 0);
         layernorm(a_.body, a_.xa, "patch_embed.norm", T);
     }
-    const size_t S = wt_.depths.size();
     for (size_t s = 0; s < S; ++s) {
         // RHAG (gpu.rs:592-610): conv3x3(blocks(x)) + x, with the stage input
         // kept in a_.xa and the blocks working in a_.xb. Each block's last GEMM
@@ -1882,7 +1885,6 @@ void GpuBackend::run_forward(int h, int w, const float* d_in, float* d_out, std:
     const auto blocks = wt_.up_blocks();
     const DevConv& last = conv_.at("conv_last");
     const int oh = h * wt_.scale, ow = w * wt_.scale;
-    if (blocks.size() + AMAX_HEAD + 2 > AMAX_SLOTS || S > AMAX_HEAD) throw Error("forward: too many stages or upsample convs");
     for (size_t b = 0; b < blocks.size(); ++b) {
         const DevConv& up = conv_.at("upsample." + std::to_string(2 * b));
         if (bands && b + 1 == blocks.size() && head_bands_fit(up, last, hh, ww, feat)) {

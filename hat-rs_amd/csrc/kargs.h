@@ -318,7 +318,7 @@ struct LnArgs {
 
 // A forward's magnitude slots: the bits of the largest finite |x| of the planes
 // that no norm bounds and a Winograd conv reads (ConvArgs::amax): per stage its
-// last block's output, then the head's planes. At most 32 stages. A slot is
+// last block's output, then, from AMAX_HEAD, the head's planes. A slot is
 // AMAX_LANES words AMAX_STRIDE apart (64 bytes), whose maximum it is: one a XCD, so
 // that a kernel's blocks do not all meet in one word.
 #define AMAX_SLOTS 64

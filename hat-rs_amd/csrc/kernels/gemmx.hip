@@ -1,5 +1,5 @@
 // The qkv linear on split-f16 MFMA: out = A . Wqkv^T + b scattered head-major
-// into q, k, v ([3][heads][T][head_dim]), as hat_gemmws_qkv (lg_linear +
+// into q, k, v ([3][heads][T][head_dim]) (lg_linear +
 // lg_extract_rows of the reference, cuda.rs:428-453), for the C = 144 family
 // (head_dim 24) and the C = 180 family (head_dim 30).
 //

@@ -248,8 +248,7 @@ __device__ __forceinline__ void habx_body(const TailXArgs& p)
     };
     // Stage i begins: its loads have landed (everything issued before those of
     // the D - 1 stages after it), for every wave, and every wave is done with the
-    // stage before, whose buffer stage i + D goes to. Near the end fewer are in
-    // flight than counted, so the last part waits for everything.
+    // stage before, whose buffer stage i + D goes to.
     auto stage_begin = [&](auto iv) {
         constexpr int i = decltype(iv)::value;
         if constexpr (NB == 2) {

@@ -88,7 +88,7 @@ MemPlan gpu_plan(const Weights& wt, size_t h, size_t w)
 {
     MemPlan p;
     p.activations = GpuBackend::plan_bytes(wt, (int)h, (int)w, true);
-    // what the upload allocates: the packed tensors and their split-bf16 copies
+    // what the upload allocates: the packed tensors, FP32 and split
     // (the reference's backend uploads the file's tensors as they are, wt.bytes)
     p.weights = GpuBackend::device_weight_bytes(wt);
     p.base = kBase;
