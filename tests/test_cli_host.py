@@ -168,8 +168,8 @@ def test_auto_tile_returns_a_window_multiple_that_fits_the_budget():
 def test_memory_plan_is_the_reference_formula(weights_dir):
     """memguard.rs:60-75: need = buffers * 1.05 + weights + 128 MiB; the
     buffers are this backend's own per-plan layout (host staging included), the
-    weights what its upload allocates: the packed FP32 tensors and their
-    split-bf16 copies, several times the 38.4 MiB HAT-S file (the reference
+    weights what its upload allocates: the packed FP32 tensors and the
+    split-f16 copies, several times the 38.4 MiB HAT-S file (the reference
     uploads the file's tensors as they are, so it counts wt.bytes; the GPU test
     test_admission_counts_the_weights_the_upload_allocates holds this figure
     to what the upload allocated)."""

@@ -32,7 +32,7 @@ def small(hl, tmp_path_factory):
 
 def test_admission_counts_the_weights_the_upload_allocates(small):
     """The memory plan's weights term is what the backend's upload allocated
-    (packed tensors and split-bf16 copies), computed without a device."""
+    (packed tensors and split-f16 copies), computed without a device."""
     wp, W, be = small
     assert be.weight_bytes() == W.gpu_plan(64, 64)["weights"] > 2 * W.file_bytes()
 
