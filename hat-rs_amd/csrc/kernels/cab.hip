@@ -234,10 +234,10 @@ extern "C" __global__ __launch_bounds__(CX_WAVES * 64, 2) void hat_cab_conv1(Cab
 // ---------------------------------------------------------------------------
 // The gate, and conv2 folded with it, for a block of WAVES waves; lds: CAB_GATE_LDS
 // floats. Every reduction is a fixed-order per-lane sum followed by a fixed shuffle
-// tree, so the result does not depend on timing. It rides on the attention launch as a block of its own (attnx.hip), so what
-// counts is its latency, which small planes would wait for: conv2's weights
-// are read once, coalesced, under the tile sums' loads, and the split chunks
-// go out eight values at a time.
+// tree, so the result does not depend on timing. It rides on the attention launch as
+// a block of its own (attnx.hip), so what counts is its latency, which small planes
+// would wait for: conv2's weights are read once, coalesced, under the tile sums'
+// loads, and the split chunks go out eight values at a time.
 #define CAB_GATE_W2 (CAB_C * CAB_CC * 9)
 #define CAB_GATE_LDS (CAB_GATE_W2 + CAB_NSUM * CAB_CS + 9 * CAB_CC + CAB_C + 64 + CAB_C)
 template <int WAVES>
